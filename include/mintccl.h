@@ -99,10 +99,22 @@ typedef enum {
 } mint_op;
 typedef enum {
     MINT_PLACE_SPREAD = 0,  /* ring neighbours on consecutive blocks (adjacent XCDs) */
-    MINT_PLACE_LOCAL = 1    /* every hop of a channel on the same XCD: each block takes its
+    MINT_PLACE_LOCAL = 1,   /* every hop of a channel on the same XCD: each block takes its
                                work from the XCD it runs on; needs a device that deals
                                every 8 consecutive blocks to 8 different XCDs
                                (mint_device_info reports 8, mint_xcd_map shows the order) */
+    MINT_PLACE_CU = 2       /* every hop of a channel inside one compute unit: a thread
+                               block runs all positions of a channel, the blocks travel
+                               between them through LDS.  Both protocols are the same
+                               there (LDS keeps a wavefront's operations in order, so
+                               whole 1 KiB blocks go first and the step counter behind
+                               them).  staging[], staging_bytes, credit_offset,
+                               slot_bytes, nslots, waves_per_channel_group,
+                               threads_per_block, cache_policy, flag_epoch, epoch_ptr,
+                               row_fetch and origin_cus are not looked at; launches on
+                               different streams share nothing but the status block.
+                               SENDRECV, BROADCAST, REDUCE, ALLGATHER, REDUCESCATTER,
+                               ALLREDUCE and ALLTOALL. */
 } mint_placement;
 
 typedef enum {
@@ -132,7 +144,9 @@ typedef enum {
  * parts).  The same launch with MINT_PLACE_SPREAD (cache_policy 0) will do.
  * The words stay set until the caller zeroes them: every launch that finds
  * word 3 set gives up at its first wait (after at most 64 polls) and leaves
- * unspecified output, and only the first failure is recorded.  After a
+ * unspecified output, and only the first failure is recorded (under
+ * MINT_PLACE_CU a launch runs whatever word 3 says and is counted there; a
+ * position whose wait ran out goes on without waiting, in bounds).  After a
  * non-zero word 0 the caller synchronises the stream, zeroes the block and
  * treats the outputs of every launch since the last clean check as lost;
  * under MINT_PLACE_LOCAL it also zeroes the staging before it is used again
@@ -346,8 +360,8 @@ int mint_ring_grid_blocks(const mint_ring_op* op);
  * 1024 for Simple), recv_offset[i] / send_offset[i] (byte offset of the
  * block's 1 KiB message inside the staging of the rank it is received in /
  * sent to).  Any output array may be NULL; at most max_entries are written,
- * *n_entries is the full count.  Needs no GPU.  The tree ops and the temporal
- * allgather are not listed (MINT_ERR_ARG). */
+ * *n_entries is the full count.  Needs no GPU.  The tree ops, the temporal
+ * allgather and MINT_PLACE_CU are not listed (MINT_ERR_ARG). */
 int mint_ring_schedule(const mint_ring_op* op, int pipeline, int position, int wave,
                        uint32_t max_entries, uint32_t* step, uint32_t* block,
                        uint32_t* recv_offset, uint32_t* send_offset, uint32_t* n_entries);

@@ -18,6 +18,7 @@ _ROOT = os.path.dirname(_PKG)
 SO_PATH = os.getenv("MINTCCL_LIBRARY") or os.path.join(_PKG, "libmintccl.so")
 _CSRC = os.path.join(_PKG, "csrc")
 SRC = os.path.join(_CSRC, "mintccl.hip")
+CU_SRC = os.path.join(_CSRC, "cu_ring.hip")
 FAMILY_SRC = os.path.join(_CSRC, "ring_family.hip")     # compiled once per element type
 BUILD_DIR = os.path.join(_PKG, "_build")
 
@@ -37,7 +38,7 @@ PROTO_LL128, PROTO_SIMPLE = 0, 1
 (OP_SENDRECV, OP_BROADCAST, OP_REDUCE, OP_ALLGATHER, OP_REDUCESCATTER, OP_ALLREDUCE,
  OP_ALLTOALL, OP_TREE_BROADCAST, OP_TREE_REDUCE, OP_ALLGATHER_TEMPORAL,
  OP_HYPERCUBE_REDUCESCATTER, OP_HYPERCUBE_ALLGATHER) = range(12)
-PLACE_SPREAD, PLACE_LOCAL = 0, 1
+PLACE_SPREAD, PLACE_LOCAL, PLACE_CU = 0, 1, 2
 FETCH_INLINE, FETCH_LDS = 0, 1
 
 HIPCC_FLAGS = [
@@ -148,7 +149,7 @@ def stores_with_scalar_offset(asm: str) -> list[str]:
 def build(verbose: bool = False, defines: tuple[str, ...] = (), so_path: str | None = None) -> str:
     """Compile the HIP sources for gfx950 into ``libmintccl.so`` (in-tree).
 
-    The ring kernels are one translation unit per element type; the five
+    The ring kernels are one translation unit per element type; the six
     compilations run side by side and are linked at the end.  ``defines``
     (``-DMINT_RING_STATS``: wait accounting per ring position,
     ``-DMINT_ROW_NOLOAD``: whole blocks of own rows are not loaded - wrong
@@ -158,7 +159,8 @@ def build(verbose: bool = False, defines: tuple[str, ...] = (), so_path: str | N
     out = so_path or os.path.join(_PKG, "libmintccl.so")
     build_dir = BUILD_DIR if so_path is None else out + ".objs"
     os.makedirs(build_dir, exist_ok=True)
-    units = [(SRC, list(defines), os.path.join(build_dir, "mintccl.o"))]
+    units = [(SRC, list(defines), os.path.join(build_dir, "mintccl.o")),
+             (CU_SRC, list(defines), os.path.join(build_dir, "cu_ring.o"))]
     for dt in range(4):
         units.append((FAMILY_SRC, [f"-DMINT_FAMILY_DT={dt}", *defines],
                       os.path.join(build_dir, f"ring_family_{dt}.o")))

@@ -42,12 +42,10 @@ def allgather(buff: torch.Tensor, comm: VirtualComm | None = None,
     row = count // comm.world_size
     ptrs = {r: info["ptr"] for r, info in posted.items()}
     if same_everywhere(posted, "schedule", "the schedule") == "temporal":
-        d = comm.make_op(_lib.OP_ALLGATHER_TEMPORAL, _lib.BYTES, row, ptrs, ptrs, ring_of(comm),
-                         row_stride=row, protocol=_lib.PROTO_LL128)
+        comm.launch(comm.make_op(_lib.OP_ALLGATHER_TEMPORAL, _lib.BYTES, row, ptrs, ptrs,
+                                 ring_of(comm), row_stride=row, protocol=_lib.PROTO_LL128))
     else:
-        d = comm.make_op(_lib.OP_ALLGATHER, _lib.BYTES, row, ptrs, ptrs, ring_of(comm),
-                         row_stride=row)
-    comm.launch(d)
+        comm.enqueue(_lib.OP_ALLGATHER, _lib.BYTES, row, ptrs, ptrs, ring_of(comm), row_stride=row)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

@@ -9,12 +9,12 @@ ranks hold the same bits.
 
 Two ways to run it, same result bit for bit:
 
-* fused (``fused=True`` or ``MINTCCL_ALLREDUCE=fused``; the default below
-  32 MiB per rank): one launch, one pass round the ring of 2 * world - 1
+* fused (``fused=True`` or ``MINTCCL_ALLREDUCE=fused``; the default where the
+  rings run inside compute units, else below 32 MiB per rank): one launch, one pass round the ring of 2 * world - 1
   positions - what the reference plans.  Its two phases share the staging
   slots and the wavefronts.
-* split (``fused=False`` or ``MINTCCL_ALLREDUCE=split``; the default from
-  32 MiB per rank): a reduce-scatter launch followed by an allgather launch on
+* split (``fused=False`` or ``MINTCCL_ALLREDUCE=split``; the default of the
+  rings through staging from 32 MiB per rank): a reduce-scatter launch followed by an allgather launch on
   the same chunks; each launch can use the whole wavefront budget, and the
   allgather's origins get compute units of their own.
 """
@@ -30,10 +30,11 @@ from ._ops import (check_buffer, comm_or_default, nbytes, reduce_dtype, ring_of,
 from .common import VirtualComm
 
 
-# From this size per rank on, two launches are faster than one pass (measured
-# on MI355X, 8 ranks, f16: 104 / 110 us at 16 MiB, 199 / 192 at 32 MiB, 1510 /
+# Through staging, two launches are faster than one pass from this size per rank
+# on (measured on MI355X, 8 ranks, f16: 104 / 110 us at 16 MiB, 199 / 192 at 32 MiB, 1510 /
 # 1384 at 256 MiB; below, the second launch costs more than it gains: 12 / 18 us
-# at 64 KiB).
+# at 64 KiB).  Inside compute units the two phases share nothing: one pass is
+# 205 us at 64 MiB of bf16 where two launches through staging take 368.
 SPLIT_FROM_BYTES = 32 << 20
 
 
@@ -56,16 +57,16 @@ def allreduce(buff: torch.Tensor, comm: VirtualComm | None = None,
     ptrs = {r: info["ptr"] for r, info in posted.items()}
     if fused is None:
         choice = os.getenv("MINTCCL_ALLREDUCE", "").lower()
-        fused = choice != "split" if choice else count < SPLIT_FROM_BYTES
+        fused = choice != "split" if choice else comm.inside_cu or count < SPLIT_FROM_BYTES
     ring = ring_of(comm)
     if fused:
-        comm.launch(comm.make_op(_lib.OP_ALLREDUCE, dtype, count, ptrs, ptrs, ring))
+        comm.enqueue(_lib.OP_ALLREDUCE, dtype, count, ptrs, ptrs, ring)
         return
     row = chunk_bytes(count, comm.world_size)
-    comm.launch(comm.make_op(_lib.OP_REDUCESCATTER, dtype, row, ptrs, ptrs, ring, row_stride=row,
-                             total_bytes=count))
-    comm.launch(comm.make_op(_lib.OP_ALLGATHER, _lib.BYTES, row, ptrs, ptrs, ring, row_stride=row,
-                             total_bytes=count))
+    comm.enqueue(_lib.OP_REDUCESCATTER, dtype, row, ptrs, ptrs, ring, row_stride=row,
+                 total_bytes=count)
+    comm.enqueue(_lib.OP_ALLGATHER, _lib.BYTES, row, ptrs, ptrs, ring, row_stride=row,
+                 total_bytes=count)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

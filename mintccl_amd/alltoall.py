@@ -35,10 +35,9 @@ def alltoall(buff: torch.Tensor, out: torch.Tensor, comm: VirtualComm | None = N
         for b in posted.values():
             if a["in"] < b["out"] + count and b["out"] < a["in"] + count:
                 raise ValueError("alltoall: out overlaps a rank's buff")
-    d = comm.make_op(_lib.OP_ALLTOALL, _lib.BYTES, row, lo,
-                     {r: info["out"] for r, info in posted.items()}, ring_of(comm),
-                     row_stride=row)
-    comm.launch(d)
+    comm.enqueue(_lib.OP_ALLTOALL, _lib.BYTES, row, lo,
+                 {r: info["out"] for r, info in posted.items()}, ring_of(comm),
+                 row_stride=row)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

@@ -24,9 +24,8 @@ def broadcast(buff: torch.Tensor, root: int, comm: VirtualComm | None = None) ->
     root = same_everywhere(posted, "root", "the root")
     ptrs = {r: info["ptr"] for r, info in posted.items()}
     # root has the input, everyone else an output (4_broadcast.py:97-98)
-    d = comm.make_op(_lib.OP_BROADCAST, _lib.BYTES, count, {root: ptrs[root]},
-                     {r: p for r, p in ptrs.items() if r != root}, ring_of(comm), root=root)
-    comm.launch(d)
+    comm.enqueue(_lib.OP_BROADCAST, _lib.BYTES, count, {root: ptrs[root]},
+                 {r: p for r, p in ptrs.items() if r != root}, ring_of(comm), root=root)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

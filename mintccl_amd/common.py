@@ -309,6 +309,14 @@ class VirtualComm:
         # budget of staging per rank
         self.auto_geometry = (tuned and buff_size_ is None and nslots is None
                               and waves_per_rank is None)
+        # With everything about the wire left to the library the operators' rings
+        # run inside compute units; naming a placement, a cache policy, a
+        # block size, who fetches the rows or where the origins sit (arguments
+        # or MINTCCL_*) asks for the rings through staging memory.
+        self.inside_cu = self.auto_geometry and all(
+            v is None for v in (placement, threads_per_block, cache_policy, row_fetch, origin_cus)
+        ) and not any(os.getenv(k) for k in ("MINTCCL_PLACEMENT", "MINTCCL_THREADS", "MINTCCL_CACHE",
+                                             "MINTCCL_ROW_FETCH", "MINTCCL_ORIGIN_CUS"))
         if nslots is None:
             nslots = num_slots() if (reference_geometry or buff_size_ is not None) else TUNED_NSLOTS
         if buff_size_ is None:
@@ -520,6 +528,31 @@ class VirtualComm:
                                      self.stats.data_ptr() if self.stats is not None else NULL)
         return d
 
+    def make_cu_op(self, op: int, dtype: int, count_bytes: int, inputs: dict, outputs: dict,
+                   ring: list[int], root: int = 0, row_stride: int = 0, route_len: int = 0,
+                   total_bytes: int = 0) -> _lib.RingOp:
+        """The descriptor of the same collective with its rings inside compute
+        units: no slots, no staging, no epoch."""
+        d = _lib.RingOp()
+        d.op, d.dtype, d.world, d.protocol = op, dtype, self.world_size, self.protocol
+        for i, r in enumerate(ring):
+            d.ring[i] = r
+        d.route_len, d.root = route_len, root
+        for r, p in inputs.items():
+            d.input[r] = p
+        for r, p in outputs.items():
+            d.output[r] = p
+        d.count_bytes, d.row_stride, d.total_bytes = count_bytes, row_stride, total_bytes
+        d.placement, d.spin_budget, d.status = _lib.PLACE_CU, self.spin_budget, self.status.data_ptr()
+        return d
+
+    def enqueue(self, op: int, *args, **kw) -> None:
+        """Build the descriptor of a ring collective and launch it."""
+        if self.inside_cu and self.stats is None:
+            self.launch(self.make_cu_op(op, *args, **kw))
+        else:
+            self.launch(self.make_op(op, *args, **kw))
+
     def launch(self, d: _lib.RingOp) -> None:
         """Enqueue on the current stream; never synchronises."""
         # The Simple protocol writes raw payload where LL128 keeps its sector
@@ -531,7 +564,8 @@ class VirtualComm:
         # into a graph takes it anew at every replay.  A launch on staging the
         # caller brought (sendrecv_buffer) is the caller's to keep to one
         # protocol or to clear.
-        own_staging = d.staging[0] == self.staging_ptr(0)
+        inside_cu = d.placement == _lib.PLACE_CU       # touches no staging
+        own_staging = not inside_cu and d.staging[0] == self.staging_ptr(0)
         if own_staging and self.epoch_word is None:
             if d.protocol == _lib.PROTO_LL128 and self._last_protocol == _lib.PROTO_SIMPLE:
                 self.staging.zero_()
@@ -539,7 +573,9 @@ class VirtualComm:
             self._last_protocol = d.protocol
         # sector tags hold 12 bits of epoch: when the counter wraps, staging is
         # cleared (a stream-ordered fill) so that no tag of an old launch survives
-        if self.epoch_word is None:
+        if inside_cu:
+            pass
+        elif self.epoch_word is None:
             if self.epoch >= _lib.MAX_EPOCH:
                 self.staging.zero_()
                 self.epoch = 0

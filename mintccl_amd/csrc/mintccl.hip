@@ -60,6 +60,47 @@ static_assert(MINT_OP_TREE_BROADCAST == OP_TREE_BROADCAST && MINT_OP_TREE_REDUCE
                   MINT_OP_HYPERCUBE_ALLGATHER == OP_HYPER_ALLGATHER,
               "op codes");
 
+// The grid of a launch inside compute units (cu_ring.hpp): one thread block per
+// channel, one wavefront per position.
+int plan_cu(Plan* plan) {
+    const RingArgs& a = plan->args;
+    const uint64_t nfull = a.row_bytes / kBlockRawSimple;
+    if (nfull >= (1ull << 31)) return MINT_ERR_TOO_LARGE;
+    constexpr uint64_t kCus = (uint64_t)kXcds * kCusPerXcd;
+    // (4 KiB per step where nothing is added)
+    const bool copying = !reducing(a.op);
+    plan->unroll = copying && nfull / 4 * (uint64_t)a.pipes >= 4 * kCus ? 4 : 1;
+    const uint64_t units = (nfull + plan->unroll - 1) / plan->unroll + (a.row_bytes % kBlockRawSimple ? 1 : 0);
+    const uint64_t per_cu = a.hops == 1 ? 4 : 2;
+    uint64_t channels = per_cu * kCus / (uint64_t)a.pipes;
+    if (channels > units) channels = units ? units : 1;
+    plan->blocks = (int)channels * a.pipes;
+    plan->threads = (a.hops + 1) * 64;
+    CuRingArgs& c = plan->cu_args;
+    for (int i = 0; i < a.cyc_len; ++i) {
+        // (alltoall names ranks, not places on a ring)
+        const int rank = a.op == OP_ALLTOALL ? i : a.cyc[i];
+        c.input[i] = a.input[rank];
+        c.output[i] = a.output[rank];
+    }
+    c.starts = 0;
+    if (a.op != OP_ALLTOALL)
+        for (int p = 0; p < a.pipes; ++p) c.starts |= (uint64_t)a.start[p] << (8 * p);
+    c.row_bytes = a.row_bytes;
+    c.row_stride = a.row_stride;
+    c.total_bytes = a.total_bytes;
+    c.status = a.status;
+    c.op = (uint32_t)a.op;
+    c.pipes = (uint32_t)a.pipes;
+    c.len = (uint32_t)a.cyc_len;
+    c.hops = (uint32_t)a.hops;
+    c.channels = (uint32_t)channels;
+    c.spin_budget = a.spin_budget;
+    plan->lds = false;
+    plan->staging_need = 0;
+    return MINT_OK;
+}
+
 // Everything the launch derives from the descriptor.  `for_launch`: also
 // check what only matters once the kernels run (the size of the staging the
 // caller allocated); the host-side queries do without.
@@ -81,18 +122,25 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
     if (op->cache_policy < 0 || op->cache_policy > 2) return MINT_ERR_ARG;
     // XCD-local staging only makes sense when every hop of a channel shares an XCD
     if (op->cache_policy == 2 && op->placement != MINT_PLACE_LOCAL) return MINT_ERR_ARG;
-    if (op->placement != MINT_PLACE_SPREAD && op->placement != MINT_PLACE_LOCAL) return MINT_ERR_ARG;
+    const bool cu = op->placement == MINT_PLACE_CU;
+    if (!cu && op->placement != MINT_PLACE_SPREAD && op->placement != MINT_PLACE_LOCAL) return MINT_ERR_ARG;
+    // the walks of their own have no form inside a compute unit
+    if (cu && (over_tree(op->op) || temporal || hyper)) return MINT_ERR_ARG;
     if (op->row_fetch != MINT_FETCH_INLINE && op->row_fetch != MINT_FETCH_LDS) return MINT_ERR_ARG;
     if (!op->status) return MINT_ERR_ARG;
-    if (op->epoch_ptr) {
+    if (cu) {
+        // no epoch, no slots, no staging: see there
+    } else if (op->epoch_ptr) {
         if (op->epoch_ptr % 4) return MINT_ERR_ALIGN;        // the epoch lives in device memory
     } else if (op->flag_epoch == 0 || op->flag_epoch > kMaxEpoch) {
         return MINT_ERR_ARG;
     }
-    if (op->threads_per_block == 0 || op->threads_per_block % 64 || op->threads_per_block > 512)
-        return MINT_ERR_ARG;
-    if (op->nslots == 0 || op->slot_bytes == 0) return MINT_ERR_GEOMETRY;
-    if ((uint64_t)op->nslots * op->slot_bytes >= (1ull << 31)) return MINT_ERR_TOO_LARGE;
+    if (!cu) {
+        if (op->threads_per_block == 0 || op->threads_per_block % 64 || op->threads_per_block > 512)
+            return MINT_ERR_ARG;
+        if (op->nslots == 0 || op->slot_bytes == 0) return MINT_ERR_GEOMETRY;
+        if ((uint64_t)op->nslots * op->slot_bytes >= (1ull << 31)) return MINT_ERR_TOO_LARGE;
+    }
 
     RingArgs& a = plan->args;
     a = RingArgs{};
@@ -208,7 +256,7 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
             // caller buffers and rows may start at any byte; staging is ours
             if (load && !op->input[rank]) return MINT_ERR_ARG;
             if (save && !op->output[rank]) return MINT_ERR_ARG;
-            if (!origin && (!op->staging[rank] || !aligned16(op->staging[rank])))
+            if (!cu && !origin && (!op->staging[rank] || !aligned16(op->staging[rank])))
                 return op->staging[rank] ? MINT_ERR_ALIGN : MINT_ERR_ARG;
         }
     }
@@ -224,6 +272,15 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
         a.input[r] = op->input[r];
         a.output[r] = op->output[r];
         a.staging[r] = op->staging[r];
+    }
+
+    a.placement = op->placement;
+    a.spin_budget = op->spin_budget ? op->spin_budget : kDefaultSpinBudget;
+    a.status = reinterpret_cast<uint64_t*>(op->status);
+    plan->cu = cu;
+    if (cu) {
+        if (dbg && (dbg->skip_origin || dbg->stats)) return MINT_ERR_ARG;
+        return plan_cu(plan);
     }
 
     // geometry
@@ -254,8 +311,6 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
     }
     a.epoch = op->flag_epoch;
     a.epoch_word = reinterpret_cast<const uint32_t*>(op->epoch_ptr);
-    a.spin_budget = op->spin_budget ? op->spin_budget : kDefaultSpinBudget;
-    a.status = reinterpret_cast<uint64_t*>(op->status);
     a.skip_origin = dbg ? dbg->skip_origin : 0u;
 #ifdef MINT_RING_STATS
     a.stats = dbg ? reinterpret_cast<uint64_t*>(dbg->stats) : nullptr;
@@ -263,7 +318,6 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
     if (dbg && dbg->stats) return MINT_ERR_ARG;   // this build does not collect wait accounting
     a.stats = nullptr;
 #endif
-    a.placement = op->placement;
     {
         const int npos = a.hops + 1;
         a.seat_turn = (over_tree(op->op) || temporal) && kCusPerXcd % npos == 0
@@ -345,6 +399,7 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
 int launch_ring(const Plan& plan, int protocol, int dtype, int cache_policy, hipStream_t stream) {
     // the copying collectives move bytes whatever element type the caller names
     if (!reducing(plan.args.op)) dtype = MINT_BYTES;
+    if (plan.cu) return launch_cu_ring(plan, dtype, stream);
     switch (dtype) {
         case MINT_F16: return launch_ring_family_f16(plan, protocol, cache_policy, stream);
         case MINT_BF16: return launch_ring_family_bf16(plan, protocol, cache_policy, stream);
@@ -708,8 +763,8 @@ int mint_ring_schedule(const mint_ring_op* op, int pipeline, int position, int w
     const int err = make_plan(op, &plan);
     if (err != MINT_OK) return err;
     if (plan.empty) return MINT_OK;
-    if (over_tree(op->op) || over_hypercube(op->op) || op->op == MINT_OP_ALLGATHER_TEMPORAL)
-        return MINT_ERR_ARG;                        // listed for the ring walks only
+    if (over_tree(op->op) || over_hypercube(op->op) || op->op == MINT_OP_ALLGATHER_TEMPORAL || plan.cu)
+        return MINT_ERR_ARG;                        // listed for the ring walks through staging only
     const RingArgs& a = plan.args;
     if (pipeline < 0 || pipeline >= a.pipes || position < 0 || position > a.hops || wave < 0 ||
         wave >= a.waves)
@@ -774,6 +829,7 @@ int mint_ring_launch_debug(const mint_ring_op* op, const mint_ring_debug* dbg, v
 
 int mint_ring_launch_static(const mint_ring_op* op, void* stream) {
     if (!op) return MINT_ERR_ARG;
+    if (op->placement == MINT_PLACE_CU) return mint_ring_launch(op, stream);    // no staging to bring
     // size limits first: they need no device
     if ((uint64_t)op->nslots * op->slot_bytes > kStaticSlots) return MINT_ERR_TOO_LARGE;
     mint_ring_op d = *op;

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/mintccl.h"
+#include "cu_ring.hpp"
 #include "ring.hpp"
 
 namespace mint {
@@ -16,6 +17,8 @@ struct Plan {
     int blocks_plain;         // the grid without CUs set apart for origins (args.origin_cus)
     size_t staging_need;      // bytes of staging per rank: slots + credit words
     bool empty;
+    bool cu;                  // rings inside compute units: `cu_args` instead of `args`
+    CuRingArgs cu_args;
     bool lds;                 // own rows through LDS: `threads` counts the wave-channels'
                               // threads only, the launch adds the fetcher wavefront
 };
@@ -35,5 +38,6 @@ int launch_ring_family_f16(const Plan& plan, int protocol, int cache_policy, hip
 int launch_ring_family_bf16(const Plan& plan, int protocol, int cache_policy, hipStream_t stream);
 int launch_ring_family_f32(const Plan& plan, int protocol, int cache_policy, hipStream_t stream);
 int launch_ring_family_bytes(const Plan& plan, int protocol, int cache_policy, hipStream_t stream);
+int launch_cu_ring(const Plan& plan, int dtype, hipStream_t stream);
 
 }  // namespace mint

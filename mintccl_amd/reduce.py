@@ -27,9 +27,8 @@ def reduce(buff: torch.Tensor, root: int, comm: VirtualComm | None = None) -> No
     dtype = same_everywhere(posted, "dtype", "the dtype")
     ptrs = {r: info["ptr"] for r, info in posted.items()}
     # inputbuff on every rank, outputbuff only at the root (5_reduce.py:117-118)
-    d = comm.make_op(_lib.OP_REDUCE, dtype, count, ptrs, {root: ptrs[root]}, ring_of(comm),
-                     root=root)
-    comm.launch(d)
+    comm.enqueue(_lib.OP_REDUCE, dtype, count, ptrs, {root: ptrs[root]}, ring_of(comm),
+                 root=root)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

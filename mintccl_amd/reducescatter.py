@@ -30,9 +30,8 @@ def reducescatter(buff: torch.Tensor, comm: VirtualComm | None = None) -> None:
     dtype = same_everywhere(posted, "dtype", "the dtype")
     row = count // comm.world_size
     ptrs = {r: info["ptr"] for r, info in posted.items()}
-    d = comm.make_op(_lib.OP_REDUCESCATTER, dtype, row, ptrs, ptrs, ring_of(comm),
-                     row_stride=row)
-    comm.launch(d)
+    comm.enqueue(_lib.OP_REDUCESCATTER, dtype, row, ptrs, ptrs, ring_of(comm),
+                 row_stride=row)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

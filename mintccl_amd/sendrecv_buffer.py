@@ -49,9 +49,12 @@ def _launch(comm: VirtualComm, s: dict, r: dict, route: list[int] | None,
     if not route or route[0] != s["rank"] or route[-1] != r["rank"]:
         raise ValueError(f"no route {s['rank']} -> {r['rank']}")
     comm.last_route = list(route)
-    d = comm.make_op(_lib.OP_SENDRECV, _lib.BYTES, s["count"], {s["rank"]: s["data_ptr"]},
-                     {r["rank"]: r["data_ptr"]}, route, route_len=len(route))
-    if full_size_staging:
+    args = (_lib.OP_SENDRECV, _lib.BYTES, s["count"], {s["rank"]: s["data_ptr"]},
+            {r["rank"]: r["data_ptr"]}, route)
+    if not full_size_staging:
+        comm.enqueue(*args, route_len=len(route))
+    else:
+        d = comm.make_op(*args, route_len=len(route))
         # every line of the message gets a slot of its own, so no hop ever
         # waits for a credit (2_sendrecv_indirect.py:147-149); zeroed like the
         # reference's, and kept alive until the next transfer replaces it,
@@ -65,7 +68,7 @@ def _launch(comm: VirtualComm, s: dict, r: dict, route: list[int] | None,
             d.staging[k] = hops.data_ptr() + k * per_rank
         d.staging_bytes = per_rank
         d.credit_offset = 0                      # right after this staging's own slots
-    comm.launch(d)
+        comm.launch(d)
 
 
 def sync(comm: VirtualComm | None = None, route: list[int] | None = None) -> None:
