@@ -20,6 +20,8 @@ _CSRC = os.path.join(_PKG, "csrc")
 SRC = os.path.join(_CSRC, "mintccl.hip")
 CU_SRC = os.path.join(_CSRC, "cu_ring.hip")
 FAMILY_SRC = os.path.join(_CSRC, "ring_family.hip")     # compiled once per element type
+HOST_SRC = os.path.join(_CSRC, "host.cpp")              # the extension module _host
+HOST_PATH = os.path.join(_PKG, "_host.so")
 BUILD_DIR = os.path.join(_PKG, "_build")
 
 MAX_RANKS = 8
@@ -38,6 +40,10 @@ PROTO_LL128, PROTO_SIMPLE = 0, 1
 (OP_SENDRECV, OP_BROADCAST, OP_REDUCE, OP_ALLGATHER, OP_REDUCESCATTER, OP_ALLREDUCE,
  OP_ALLTOALL, OP_TREE_BROADCAST, OP_TREE_REDUCE, OP_ALLGATHER_TEMPORAL,
  OP_HYPERCUBE_REDUCESCATTER, OP_HYPERCUBE_ALLGATHER) = range(12)
+# kinds of collectives the host module gathers arguments for (csrc/host.cpp)
+KINDS = ("broadcast", "reduce", "allgather", "reducescatter", "allreduce", "alltoall")
+(KIND_BROADCAST, KIND_REDUCE, KIND_ALLGATHER, KIND_REDUCESCATTER, KIND_ALLREDUCE,
+ KIND_ALLTOALL) = range(6)
 PLACE_SPREAD, PLACE_LOCAL, PLACE_CU = 0, 1, 2
 FETCH_INLINE, FETCH_LDS = 0, 1
 
@@ -146,6 +152,23 @@ def stores_with_scalar_offset(asm: str) -> list[str]:
     return [line.strip() for line in asm.splitlines() if pat.match(line)]
 
 
+def host_command(out: str) -> list[str]:
+    """The compiler call for the extension module (host code only: g++, the
+    headers of Python and of the installed torch)."""
+    import sysconfig
+
+    import torch
+    base = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *[f"-isystem{d}" for d in (os.path.join(base, "include"),
+                                       os.path.join(base, "include", "torch", "csrc", "api", "include"),
+                                       os.path.join(rocm, "include"), sysconfig.get_paths()["include"])],
+            "-o", out, HOST_SRC, "-L" + os.path.join(base, "lib"),
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+
+
 def build(verbose: bool = False, defines: tuple[str, ...] = (), so_path: str | None = None) -> str:
     """Compile the HIP sources for gfx950 into ``libmintccl.so`` (in-tree).
 
@@ -164,6 +187,12 @@ def build(verbose: bool = False, defines: tuple[str, ...] = (), so_path: str | N
     for dt in range(4):
         units.append((FAMILY_SRC, [f"-DMINT_FAMILY_DT={dt}", *defines],
                       os.path.join(build_dir, f"ring_family_{dt}.o")))
+    host = None
+    if so_path is None:           # (a diagnostic build shares the product's host module)
+        cmd = host_command(os.path.join(build_dir, "_host.so"))
+        if verbose:
+            print(" ".join(cmd))
+        host = subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     procs = []
     for src, defs, obj in units:
         # every unit compiles in a directory of its own: the compiler leaves the
@@ -178,6 +207,10 @@ def build(verbose: bool = False, defines: tuple[str, ...] = (), so_path: str | N
         procs.append((cmd, tmp, obj, subprocess.Popen(cmd, stdout=subprocess.PIPE,
                                                       stderr=subprocess.PIPE, text=True)))
     errors, spilling, hazards = [], [], []
+    if host is not None:
+        text, _ = host.communicate()
+        if host.returncode != 0:
+            errors.append(f"{HOST_SRC}\n{text}")
     for cmd, tmp, obj, proc in procs:
         _, err = proc.communicate()
         if proc.returncode != 0:
@@ -210,6 +243,8 @@ def build(verbose: bool = False, defines: tuple[str, ...] = (), so_path: str | N
     proc = subprocess.run(link, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"hipcc link failed:\n{proc.stderr}")
+    if host is not None:
+        os.replace(os.path.join(build_dir, "_host.so"), HOST_PATH)
     return out
 
 
@@ -250,6 +285,29 @@ def lib():
                 "set MINTCCL_ALLOW_DIAGNOSTIC=1 to load it for timing")
         _lib = L
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The native host module, bound to the loaded library.  Raises if it has not
+    been built."""
+    global _host
+    if _host is None:
+        L = lib()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: run `python -c 'import __graft_entry__ as g; "
+                               "g.build()'` in the repository root. There is no Python fallback.")
+        from . import _host as module
+        if (module.DESCRIPTOR_BYTES != ctypes.sizeof(RingOp) or
+                any(getattr(module, k.upper()) != i for i, k in enumerate(KINDS))):
+            raise RuntimeError(f"{HOST_PATH} was built for another descriptor: rebuild it")
+        module.bind(*[ctypes.cast(getattr(L, name), ctypes.c_void_p).value
+                      for name in ("mint_ring_launch", "mint_ring_grid_blocks", "mint_ll128_pack",
+                                   "mint_ll128_unpack", "mint_ll128_packed_bytes")], check)
+        _host = module
+    return _host
 
 
 def build_flags() -> list[str]:

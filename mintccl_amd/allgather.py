@@ -11,37 +11,27 @@ through staging for one row - ``schedule="temporal"`` or
 doubles recursively over a hypercube instead (``mintccl_amd.hypercube``)."""
 from __future__ import annotations
 
-import os
-
 import torch
 
-from . import _lib
-from ._ops import check_buffer, comm_or_default, nbytes, ring_of, same_everywhere
-from .common import VirtualComm
+from . import _lib, hypercube
+from ._ops import ring_of
+from .common import VirtualComm, get_comm
+
+# (what is no schedule is refused by the board; -1: nothing said)
+_SCHEDULE = {None: -1, "spatial": 0, "temporal": 1}
 
 
 def allgather(buff: torch.Tensor, comm: VirtualComm | None = None,
               schedule: str | None = None) -> None:
-    from . import hypercube, tree
-    if schedule is None and tree.topology_env() == "hypercube":
-        return hypercube.allgather(buff, comm)
-    if schedule is None:
-        schedule = os.getenv("MINTCCL_ALLGATHER", "spatial").lower()
-    if schedule not in ("spatial", "temporal"):
-        raise ValueError("allgather schedule is 'spatial' or 'temporal'")
-    comm = comm_or_default(comm)
-    check_buffer(buff, comm)
-    if nbytes(buff) % comm.world_size:
-        raise ValueError("buffer does not split into world_size rows")
-    posted = comm.post("allgather", set(range(comm.world_size)),
-                       {"ptr": buff.data_ptr(), "count": nbytes(buff), "schedule": schedule,
-                        "keep": buff})
-    if posted is None:
+    comm = comm if comm is not None else get_comm()
+    posted = comm._board.post(_lib.KIND_ALLGATHER, buff, 0, _SCHEDULE.get(schedule, 2))
+    if posted is None:               # not all ranks are here yet, or launched
         return
-    count = same_everywhere(posted, "count", "the byte count")
+    if posted is False:
+        return hypercube.allgather(buff, comm)
+    count, _, _, temporal, ptrs, _, _ = posted
     row = count // comm.world_size
-    ptrs = {r: info["ptr"] for r, info in posted.items()}
-    if same_everywhere(posted, "schedule", "the schedule") == "temporal":
+    if temporal:
         comm.launch(comm.make_op(_lib.OP_ALLGATHER_TEMPORAL, _lib.BYTES, row, ptrs, ptrs,
                                  ring_of(comm), row_stride=row, protocol=_lib.PROTO_LL128))
     else:

@@ -20,14 +20,11 @@ Two ways to run it, same result bit for bit:
 """
 from __future__ import annotations
 
-import os
-
 import torch
 
 from . import _lib
-from ._ops import (check_buffer, comm_or_default, nbytes, reduce_dtype, ring_of,
-                   same_everywhere)
-from .common import VirtualComm
+from ._ops import ring_of
+from .common import VirtualComm, get_comm
 
 
 # Through staging, two launches are faster than one pass from this size per rank
@@ -45,19 +42,12 @@ def chunk_bytes(count: int, world: int) -> int:
 
 def allreduce(buff: torch.Tensor, comm: VirtualComm | None = None,
               fused: bool | None = None) -> None:
-    comm = comm_or_default(comm)
-    check_buffer(buff, comm)
-    posted = comm.post("allreduce", set(range(comm.world_size)),
-                       {"ptr": buff.data_ptr(), "count": nbytes(buff),
-                        "dtype": reduce_dtype(buff), "keep": buff})
-    if posted is None:
+    comm = comm if comm is not None else get_comm()
+    posted = comm._board.post(_lib.KIND_ALLREDUCE, buff, 0, -1 if fused is None else int(bool(fused)))
+    if posted is None:               # not all ranks are here yet, or launched
         return
-    count = same_everywhere(posted, "count", "the byte count")
-    dtype = same_everywhere(posted, "dtype", "the dtype")
-    ptrs = {r: info["ptr"] for r, info in posted.items()}
-    if fused is None:
-        choice = os.getenv("MINTCCL_ALLREDUCE", "").lower()
-        fused = choice != "split" if choice else comm.inside_cu or count < SPLIT_FROM_BYTES
+    count, dtype, _, variant, ptrs, _, _ = posted
+    fused = count < SPLIT_FROM_BYTES or comm.inside_cu if variant < 0 else bool(variant)
     ring = ring_of(comm)
     if fused:
         comm.enqueue(_lib.OP_ALLREDUCE, dtype, count, ptrs, ptrs, ring)

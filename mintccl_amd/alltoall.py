@@ -11,33 +11,18 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._ops import check_buffer, comm_or_default, nbytes, ring_of, same_everywhere
-from .common import VirtualComm
+from ._ops import ring_of
+from .common import VirtualComm, get_comm
 
 
 def alltoall(buff: torch.Tensor, out: torch.Tensor, comm: VirtualComm | None = None) -> None:
-    comm = comm_or_default(comm)
-    check_buffer(buff, comm)
-    check_buffer(out, comm)
-    if buff.numel() % comm.world_size:
-        raise ValueError("buffer does not split into world_size rows")
-    if nbytes(buff) != nbytes(out):
-        raise ValueError("buff and out differ in size")
-    posted = comm.post("alltoall", set(range(comm.world_size)),
-                       {"in": buff.data_ptr(), "out": out.data_ptr(), "count": nbytes(buff),
-                        "keep": (buff, out)})
-    if posted is None:
+    comm = comm if comm is not None else get_comm()
+    posted = comm._board.post(_lib.KIND_ALLTOALL, buff, 0, -1, out)
+    if posted is None:               # not all ranks are here yet, or launched
         return
-    count = same_everywhere(posted, "count", "the byte count")
+    count, _, _, _, ins, outs, _ = posted
     row = count // comm.world_size
-    lo = {r: info["in"] for r, info in posted.items()}
-    for a in posted.values():
-        for b in posted.values():
-            if a["in"] < b["out"] + count and b["out"] < a["in"] + count:
-                raise ValueError("alltoall: out overlaps a rank's buff")
-    comm.enqueue(_lib.OP_ALLTOALL, _lib.BYTES, row, lo,
-                 {r: info["out"] for r, info in posted.items()}, ring_of(comm),
-                 row_stride=row)
+    comm.enqueue(_lib.OP_ALLTOALL, _lib.BYTES, row, ins, outs, ring_of(comm), row_stride=row)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

@@ -5,24 +5,19 @@ from __future__ import annotations
 
 import torch
 
-from . import _lib
-from ._ops import check_buffer, comm_or_default, nbytes, ring_of, same_everywhere
-from .common import VirtualComm
+from . import _lib, tree
+from ._ops import ring_of
+from .common import VirtualComm, get_comm
 
 
 def broadcast(buff: torch.Tensor, root: int, comm: VirtualComm | None = None) -> None:
-    from . import tree
-    if tree.topology_env() == "tree":
-        return tree.broadcast(buff, root, comm)
-    comm = comm_or_default(comm)
-    check_buffer(buff, comm)
-    posted = comm.post("broadcast", set(range(comm.world_size)),
-                       {"ptr": buff.data_ptr(), "count": nbytes(buff), "root": root, "keep": buff})
-    if posted is None:
+    comm = comm if comm is not None else get_comm()
+    posted = comm._board.post(_lib.KIND_BROADCAST, buff, root)
+    if posted is None:               # not all ranks are here yet, or launched
         return
-    count = same_everywhere(posted, "count", "the byte count")
-    root = same_everywhere(posted, "root", "the root")
-    ptrs = {r: info["ptr"] for r, info in posted.items()}
+    if posted is False:
+        return tree.broadcast(buff, root, comm)
+    count, _, root, _, ptrs, _, _ = posted
     # root has the input, everyone else an output (4_broadcast.py:97-98)
     comm.enqueue(_lib.OP_BROADCAST, _lib.BYTES, count, {root: ptrs[root]},
                  {r: p for r, p in ptrs.items() if r != root}, ring_of(comm), root=root)

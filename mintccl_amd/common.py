@@ -8,10 +8,8 @@ on one GPU they reduce to a device choice and a pointer mailbox.
 """
 from __future__ import annotations
 
-import contextlib
 import math
 import os
-import threading
 import time
 
 import torch
@@ -276,6 +274,29 @@ def _largest_divisor_at_most(n: int, cap: int) -> int:
     return 1
 
 
+class _RankContext:
+    """``with comm.rank(r):`` - the thread speaks for rank ``r`` inside."""
+
+    __slots__ = ("comm", "r", "before")
+
+    def __init__(self, comm: "VirtualComm", r: int) -> None:
+        if not 0 <= r < comm.world_size:
+            raise ValueError(f"rank {r} outside world of {comm.world_size}")
+        self.comm, self.r = comm, r
+
+    def __enter__(self) -> "VirtualComm":
+        self.before = self.comm._board.enter(self.r)
+        return self.comm
+
+    def __exit__(self, *exc) -> None:
+        self.comm._board.enter(self.before)
+
+
+# attributes a native launch takes from the communicator (VirtualComm._refresh)
+_LAUNCH_ATTRIBUTES = frozenset(("inside_cu", "stats", "epoch_word", "protocol", "spin_budget", "status",
+                                "topology"))
+
+
 class VirtualComm:
     """N virtual ranks on one GPU: stands in for ``MPI.COMM_WORLD``.
 
@@ -352,6 +373,9 @@ class VirtualComm:
             origin_cus = _env_int("MINTCCL_ORIGIN_CUS", 0)
         self.origin_cus = origin_cus
         self._lib = _lib.lib()          # fails loudly if the extension is missing
+        # gathers the ranks' arguments and launches (csrc/host.cpp)
+        self._board = _lib.host().Board(self, self.world_size,
+                                        -1 if self.device.index is None else self.device.index)
         # slots + credit words (never more than slot_bytes / 4), zeroed: flag 0
         # and credit 0 mean "nothing yet" (2_sendrecv_indirect.py:59-60).
         if self.buff_size % 256:
@@ -380,37 +404,52 @@ class VirtualComm:
         # an LL128 launch that follows a Simple one needs the slots cleared)
         self.epoch_word = (torch.zeros(2, dtype=torch.int32, device=self.device)
                            if device_epoch else None)
-        self._tls = threading.local()
         self._pending: dict = {}
         self._mailbox: dict = {}
-        self.last_grid = 0
+
+    def __setattr__(self, name: str, value) -> None:
+        object.__setattr__(self, name, value)
+        if name in _LAUNCH_ATTRIBUTES and "_board" in self.__dict__:
+            self._board.stale()
+
+    def _refresh(self) -> None:
+        """Tell the board what launches take from this communicator (it asks
+        when it has been told that one of them was set)."""
+        from ._ops import ring_of
+        try:
+            ring = ring_of(self)
+        except RuntimeError:
+            ring = []                  # routes only: a collective will say so
+        self._board.configure(self.inside_cu and self.stats is None and self.epoch_word is None,
+                              ring, self.protocol, self.spin_budget, self.status.data_ptr())
+
+    def _find_route(self, src: int, dst: int) -> list[int]:
+        from .topology import find_route, uniform_topology
+        return find_route(src, dst, getattr(self, "topology", None) or uniform_topology(self.world_size))
+
+    @property
+    def last_grid(self) -> int:
+        """Thread blocks of the launch before (0: none yet)."""
+        return self._board.last_grid
+
+    @property
+    def last_route(self) -> list[int]:
+        """Ranks the last send / recv travelled over."""
+        return self._board.last_route
 
     # ---- MPI-like surface -------------------------------------------------
     def Get_size(self) -> int:
         return self.world_size
 
     def Get_rank(self) -> int:
-        r = getattr(self._tls, "rank", None)
-        if r is None:
-            raise RuntimeError("no current rank: use `with comm.rank(r):`")
-        return r
+        return self._board.rank()
 
-    @contextlib.contextmanager
-    def rank(self, r: int):
-        if not 0 <= r < self.world_size:
-            raise ValueError(f"rank {r} outside world of {self.world_size}")
-        prev = getattr(self._tls, "rank", None)
-        self._tls.rank = r
-        try:
-            yield self
-        finally:
-            self._tls.rank = prev
+    def rank(self, r: int) -> _RankContext:
+        return _RankContext(self, r)
 
     def run(self, fn) -> None:
         """SPMD helper: ``fn(rank)`` for every rank in turn (like mpirun)."""
-        for r in range(self.world_size):
-            with self.rank(r):
-                fn(r)
+        self._board.run(fn)
 
     def staging_ptr(self, r: int) -> int:
         return self.staging.data_ptr() + r * self.rank_stride
@@ -583,12 +622,7 @@ class VirtualComm:
             d.flag_epoch = self.epoch
         else:
             d.flag_epoch, d.epoch_ptr = 0, self.epoch_word.data_ptr()
-        # (the grid of a descriptor is asked for once: a small collective is
-        # host-bound, and the answer only depends on fields fixed by make_op)
-        grid = getattr(d, "_grid", None)
-        if grid is None:
-            grid = d._grid = self._lib.mint_ring_grid_blocks(d)
-        self.last_grid = grid
+        self._board.launching(d)
         with torch.cuda.device(self.device):
             stream = torch.cuda.current_stream().cuda_stream
             if self.epoch_word is not None:

@@ -1,0 +1,733 @@
+// mintccl_amd._host: the host side of an operator call, native.
+//
+// A small collective takes the GPU 4 us and used to take the host 30: eight
+// rank contexts, eight sets of tensor checks, dictionaries, a descriptor filled
+// field by field through ctypes and two foreign calls (allgather of 512 B: 50 us
+// per call, 7 of them the kernel).  Here a rank's call is one native call that
+// checks the tensor and notes its address, and the call that completes the set
+// fills the descriptor and launches.
+//
+// Board is the part of a communicator (common.VirtualComm) that gathers the
+// ranks' arguments.  Where the communicator's rings run inside compute units it
+// launches them itself; anything else it hands back to the operator, which goes
+// on in Python.  What a launch takes from the communicator's attributes (ring,
+// protocol, spin limit, status block) is asked for once and again after any of
+// them has been set (VirtualComm._refresh).
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ops/empty.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstdlib>
+#include <cstring>
+#include <strings.h>
+#include <vector>
+
+#include "../../include/mintccl.h"
+
+namespace {
+
+// The library's entry points, by address: ctypes has loaded it (_lib.lib), from
+// wherever MINTCCL_LIBRARY says.
+struct Native {
+    int (*launch)(const mint_ring_op*, void*);
+    int (*grid)(const mint_ring_op*);
+    int (*pack)(const void*, void*, size_t, uint64_t, uint64_t, int, void*);
+    int (*unpack)(const void*, void*, size_t, uint64_t, uint64_t, int, void*, void*);
+    size_t (*packed_bytes)(size_t, int);
+    PyObject* check;             // _lib.check(code, where): raises MintError
+} native = {};
+
+PyObject* raise(PyObject* type, const char* text) {
+    PyErr_SetString(type, text);
+    return nullptr;
+}
+
+PyObject* checked(int code, const char* where) {
+    if (code == MINT_OK) Py_RETURN_NONE;
+    return PyObject_CallFunction(native.check, "is", code, where);
+}
+
+// The current device is `device` for as long as this lives (a launch goes to
+// the current device's context).
+struct OnDevice {
+    int before, device;
+    explicit OnDevice(int d) : before(c10::hip::current_device()), device(d) {
+        if (before != device) c10::hip::set_device((c10::DeviceIndex)device);
+    }
+    ~OnDevice() {
+        if (before != device) c10::hip::set_device((c10::DeviceIndex)before);
+    }
+    void* stream() const { return c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
+};
+
+// C++ exceptions (torch's, out of memory) become Python's.
+template <typename F>
+PyObject* guarded(F&& f) {
+    try {
+        return f();
+    } catch (const std::bad_alloc&) {
+        return PyErr_NoMemory();
+    } catch (const std::exception& e) {
+        if (PyErr_Occurred()) return nullptr;
+        return raise(PyExc_RuntimeError, e.what());
+    }
+}
+
+// ---- kinds of collectives ----------------------------------------------------
+enum Kind { BROADCAST, REDUCE, ALLGATHER, REDUCESCATTER, ALLREDUCE, ALLTOALL, KINDS };
+struct KindInfo {
+    const char* name;
+    int op;
+    bool rows, reducing;         // a buffer of `world` rows; adds elements
+    const char* elsewhere;       // the MINTCCL_TOPOLOGY under which another module does it
+};
+constexpr KindInfo kKinds[KINDS] = {
+    {"broadcast", MINT_OP_BROADCAST, false, false, "tree"},
+    {"reduce", MINT_OP_REDUCE, false, true, "tree"},
+    {"allgather", MINT_OP_ALLGATHER, true, false, "hypercube"},
+    {"reducescatter", MINT_OP_REDUCESCATTER, true, true, "hypercube"},
+    {"allreduce", MINT_OP_ALLREDUCE, false, true, nullptr},
+    {"alltoall", MINT_OP_ALLTOALL, true, false, nullptr},
+};
+// `variant` of an allgather: 0 spatial, 1 temporal; of an allreduce: 0 split, 1 fused; -1: not said
+enum { SPATIAL = 0, TEMPORAL = 1, SPLIT = 0, FUSED = 1, UNSAID = -1 };
+
+struct Post {
+    uint64_t in, out, count;
+    int dtype;
+    long root, variant;
+    PyObject *keep_in, *keep_out;        // alive until the launch is enqueued
+};
+struct Gathering {
+    uint32_t present;
+    Post post[MINT_MAX_RANKS];
+};
+struct Transfer {
+    bool given;
+    int rank;
+    long peer;
+    uint64_t ptr, count;
+    PyObject* keep;
+};
+
+struct Board {
+    PyObject_HEAD
+    PyObject* comm;              // weak reference
+    uint64_t id;                 // of this board, in the threads' lists of ranks
+    int world, device;
+    bool fresh, native_launch;   // `base` is up to date; it is ours to launch
+    bool has_ring;               // (a topology may have routes and no ring)
+    bool launched;
+    mint_ring_op base, last;
+    int8_t last_route[MINT_MAX_RANKS + 1];
+    Gathering gathering[KINDS];
+    Transfer send, recv;
+    int8_t route[MINT_MAX_RANKS][MINT_MAX_RANKS][MINT_MAX_RANKS + 1];   // ranks of the route, its length last
+};
+
+// The rank a thread speaks for, per board: `with comm.rank(r)`.
+struct Here {
+    uint64_t board;
+    int rank;
+};
+thread_local std::vector<Here> here;
+uint64_t next_board = 1;
+
+int current_rank(const Board* b) {
+    for (const Here& h : here)
+        if (h.board == b->id) return h.rank;
+    return -1;
+}
+int enter_rank(const Board* b, int rank) {
+    for (size_t i = 0; i < here.size(); ++i) {
+        if (here[i].board != b->id) continue;
+        const int before = here[i].rank;
+        if (rank >= 0) here[i].rank = rank;
+        else here.erase(here.begin() + (long)i);
+        return before;
+    }
+    if (rank >= 0) here.push_back({b->id, rank});
+    return -1;
+}
+bool rank_or_raise(const Board* b, int* rank) {
+    *rank = current_rank(b);
+    if (*rank >= 0) return true;
+    raise(PyExc_RuntimeError, "no current rank: use `with comm.rank(r):`");
+    return false;
+}
+
+void drop(Gathering* g) {
+    for (int r = 0; r < MINT_MAX_RANKS; ++r)
+        if (g->present >> r & 1u) {
+            Py_CLEAR(g->post[r].keep_in);
+            Py_CLEAR(g->post[r].keep_out);
+        }
+    g->present = 0;
+}
+
+// A device tensor of this communicator, contiguous; or an exception.
+const at::Tensor* tensor_of(const Board* b, PyObject* o) {
+    if (!THPVariable_Check(o) || !THPVariable_Unpack(o).is_cuda()) {
+        raise(PyExc_TypeError, "buffer must be a device tensor");
+        return nullptr;
+    }
+    const at::Tensor& t = THPVariable_Unpack(o);
+    if (t.get_device() != b->device) {
+        raise(PyExc_ValueError, "buffer lives on another device than the communicator");
+        return nullptr;
+    }
+    if (!t.is_contiguous()) {
+        raise(PyExc_ValueError, "buffer must be contiguous");
+        return nullptr;
+    }
+    return &t;
+}
+int dtype_code(const at::Tensor& t) {
+    switch (t.scalar_type()) {
+        case at::kHalf: return MINT_F16;
+        case at::kBFloat16: return MINT_BF16;
+        case at::kFloat: return MINT_F32;
+        default: return -1;
+    }
+}
+
+// Brings `base` up to date with the communicator's attributes.
+bool refresh(Board* b) {
+    if (b->fresh) return true;
+    PyObject* comm = PyWeakref_GetObject(b->comm);
+    if (comm == Py_None) {
+        raise(PyExc_RuntimeError, "the communicator is gone");
+        return false;
+    }
+    PyObject* done = PyObject_CallMethod(comm, "_refresh", nullptr);     // calls configure()
+    Py_XDECREF(done);
+    return done != nullptr;
+}
+
+PyObject* launch(Board* b, const mint_ring_op& op) {
+    b->last = op;
+    b->launched = true;
+    int code;
+    {
+        OnDevice on(b->device);
+        void* const stream = on.stream();
+        Py_BEGIN_ALLOW_THREADS
+        code = native.launch(&op, stream);
+        Py_END_ALLOW_THREADS
+    }
+    return checked(code, "mint_ring_launch");
+}
+
+// What all ranks have to say alike; `what` names it in the message.
+template <typename Field>
+bool alike(const Board* b, const Gathering& g, const char* what, Field field,
+           const char* const* names = nullptr) {
+    bool same = true;
+    for (int r = 1; r < b->world; ++r) same &= field(g.post[r]) == field(g.post[0]);
+    if (same) return true;
+    PyObject* vals = PySet_New(nullptr);
+    for (int r = 0; vals && r < b->world; ++r) {
+        const long long v = (long long)field(g.post[r]);
+        PyObject* s = names ? PyUnicode_FromString(names[v]) : PyUnicode_FromFormat("%lld", v);
+        if (!s || PySet_Add(vals, s) < 0) Py_CLEAR(vals);
+        Py_XDECREF(s);
+    }
+    PyObject* list = vals ? PySequence_List(vals) : nullptr;
+    if (list && PyList_Sort(list) == 0)
+        PyErr_Format(PyExc_ValueError, "ranks disagree on %s: %R", what, list);
+    Py_XDECREF(list);
+    Py_XDECREF(vals);
+    return false;
+}
+
+// All ranks are there: launch, or hand the arguments back as
+// (count, dtype, root, variant, {rank: in}, {rank: out}, kept buffers).
+PyObject* complete(Board* b, Kind kind, const Gathering& g) {
+    const KindInfo& info = kKinds[kind];
+    static const char* const kSchedules[] = {"spatial", "temporal"};
+    if (!alike(b, g, "the byte count", [](const Post& p) { return p.count; })) return nullptr;
+    if (!alike(b, g, "the root", [](const Post& p) { return p.root; })) return nullptr;
+    if (info.reducing && !alike(b, g, "the dtype", [](const Post& p) { return p.dtype; })) return nullptr;
+    if (kind == ALLGATHER &&
+        !alike(b, g, "the schedule", [](const Post& p) { return p.variant; }, kSchedules))
+        return nullptr;
+    const uint64_t count = g.post[0].count;
+    const long root = g.post[0].root;
+    if (kind == ALLTOALL)
+        for (int i = 0; i < b->world; ++i)
+            for (int o = 0; o < b->world; ++o)
+                if (g.post[i].in < g.post[o].out + count && g.post[o].out < g.post[i].in + count)
+                    return raise(PyExc_ValueError, "alltoall: out overlaps a rank's buff");
+    if (!refresh(b)) return nullptr;
+    long variant = g.post[current_rank(b)].variant;
+    if (kind == ALLREDUCE && variant == UNSAID) {
+        const char* e = getenv("MINTCCL_ALLREDUCE");
+        if (e && *e) variant = strcasecmp(e, "split") == 0 ? SPLIT : FUSED;
+        else if (b->native_launch) variant = FUSED;
+    }
+    if (b->native_launch && b->has_ring && !(kind == ALLGATHER && variant == TEMPORAL) &&
+        !(kind == ALLREDUCE && variant == SPLIT)) {
+        mint_ring_op op = b->base;
+        op.op = info.op;
+        op.dtype = info.reducing ? g.post[0].dtype : MINT_BYTES;
+        op.root = (int32_t)root;
+        op.count_bytes = info.rows ? count / (uint64_t)b->world : count;
+        op.row_stride = info.rows ? op.count_bytes : 0;
+        for (int r = 0; r < b->world; ++r) {
+            op.input[r] = kind == BROADCAST && r != root ? 0 : g.post[r].in;
+            // reduce writes at its root, broadcast everywhere else
+            const bool writes = kind == REDUCE ? r == root : !(kind == BROADCAST && r == root);
+            op.output[r] = !writes ? 0 : kind == ALLTOALL ? g.post[r].out : g.post[r].in;
+        }
+        return launch(b, op);
+    }
+    PyObject *ins = PyDict_New(), *outs = PyDict_New(), *kept = PyList_New(0);
+    bool ok = ins && outs && kept;
+    for (int r = 0; ok && r < b->world; ++r) {
+        const Post& p = g.post[r];
+        PyObject *key = PyLong_FromLong(r), *in = PyLong_FromUnsignedLongLong(p.in),
+                 *out = PyLong_FromUnsignedLongLong(p.out);
+        ok = key && in && out && PyDict_SetItem(ins, key, in) == 0 && PyDict_SetItem(outs, key, out) == 0 &&
+             PyList_Append(kept, p.keep_in) == 0 && (!p.keep_out || PyList_Append(kept, p.keep_out) == 0);
+        Py_XDECREF(key);
+        Py_XDECREF(in);
+        Py_XDECREF(out);
+    }
+    PyObject* result = ok ? Py_BuildValue("KillOOO", (unsigned long long)count, g.post[0].dtype, root,
+                                          variant, ins, outs, kept)
+                          : nullptr;
+    Py_XDECREF(ins);
+    Py_XDECREF(outs);
+    Py_XDECREF(kept);
+    return result;
+}
+
+// post(kind, buff[, root[, variant[, out]]]): None (not all ranks are there yet,
+// or launched), the ranks' arguments (complete()), or False: MINTCCL_TOPOLOGY
+// has another module do this collective
+PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+    Board* b = reinterpret_cast<Board*>(self);
+    if (n < 2 || n > 5) return raise(PyExc_TypeError, "post(kind, buff[, root[, variant[, out]]])");
+    const long k = PyLong_AsLong(args[0]);
+    if (k < 0 || k >= KINDS) return PyErr_Occurred() ? nullptr : raise(PyExc_ValueError, "no such collective");
+    const Kind kind = (Kind)k;
+    const KindInfo& info = kKinds[kind];
+    return guarded([&]() -> PyObject* {
+        Post p{};
+        p.variant = UNSAID;
+        if (n > 2) p.root = PyLong_AsLong(args[2]);
+        if (n > 3) p.variant = PyLong_AsLong(args[3]);
+        if (PyErr_Occurred()) return nullptr;
+        if (info.elsewhere && p.variant == UNSAID) {
+            const char* e = getenv("MINTCCL_TOPOLOGY");
+            if (e && strcasecmp(e, info.elsewhere) == 0) Py_RETURN_FALSE;
+        }
+        if (kind == ALLGATHER && p.variant == UNSAID) {
+            const char* e = getenv("MINTCCL_ALLGATHER");
+            p.variant = !e || strcasecmp(e, "spatial") == 0 ? SPATIAL : strcasecmp(e, "temporal") == 0 ? TEMPORAL : 2;
+        }
+        if (kind == ALLGATHER && (p.variant < SPATIAL || p.variant > TEMPORAL))
+            return raise(PyExc_ValueError, "allgather schedule is 'spatial' or 'temporal'");
+        const at::Tensor* t = tensor_of(b, args[1]);
+        if (!t) return nullptr;
+        p.in = (uint64_t)t->data_ptr();
+        p.count = (uint64_t)t->numel() * (uint64_t)t->element_size();
+        p.dtype = MINT_BYTES;
+        if (info.rows &&
+            (kind == ALLGATHER ? p.count % (uint64_t)b->world : (uint64_t)t->numel() % (uint64_t)b->world))
+            return raise(PyExc_ValueError, "buffer does not split into world_size rows");
+        if (info.reducing && (p.dtype = dtype_code(*t)) < 0)
+            return raise(PyExc_TypeError, "reductions take float16, bfloat16 or float32 tensors");
+        if (n > 4) {
+            const at::Tensor* o = tensor_of(b, args[4]);
+            if (!o) return nullptr;
+            if ((uint64_t)o->numel() * (uint64_t)o->element_size() != p.count)
+                return raise(PyExc_ValueError, "buff and out differ in size");
+            p.out = (uint64_t)o->data_ptr();
+        }
+        int rank;
+        if (!rank_or_raise(b, &rank)) return nullptr;
+        Gathering& g = b->gathering[kind];
+        if (g.present >> rank & 1u) {
+            PyErr_Format(PyExc_RuntimeError, "rank %d called %s twice before the others joined", rank, info.name);
+            return nullptr;
+        }
+        p.keep_in = Py_NewRef(args[1]);
+        p.keep_out = n > 4 ? Py_NewRef(args[4]) : nullptr;
+        g.post[rank] = p;
+        g.present |= 1u << rank;
+        if (g.present != (1u << b->world) - 1u) Py_RETURN_NONE;
+        // (taken out before anything can call back or raise)
+        Gathering all = g;
+        g.present = 0;
+        PyObject* result = complete(b, kind, all);
+        drop(&all);
+        return result;
+    });
+}
+
+PyObject* transfer(Board* b, Transfer* t, PyObject* const* args, Py_ssize_t n) {
+    if (n != 2) return raise(PyExc_TypeError, "takes a buffer and a peer");
+    return guarded([&]() -> PyObject* {
+        const at::Tensor* x = tensor_of(b, args[0]);
+        if (!x) return nullptr;
+        const long peer = PyLong_AsLong(args[1]);
+        if (peer == -1 && PyErr_Occurred()) return nullptr;
+        int rank;
+        if (!rank_or_raise(b, &rank)) return nullptr;
+        PyObject* before = t->given ? t->keep : nullptr;
+        *t = Transfer{true, rank, peer, (uint64_t)x->data_ptr(),
+                      (uint64_t)x->numel() * (uint64_t)x->element_size(), Py_NewRef(args[0])};
+        Py_XDECREF(before);
+        Py_RETURN_NONE;
+    });
+}
+PyObject* board_send(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+    return transfer(reinterpret_cast<Board*>(self), &reinterpret_cast<Board*>(self)->send, args, n);
+}
+PyObject* board_recv(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+    return transfer(reinterpret_cast<Board*>(self), &reinterpret_cast<Board*>(self)->recv, args, n);
+}
+
+// Route into op.ring / op.route_len; `given`: the caller's list, or None for the
+// topology's (searched once per pair, by VirtualComm._find_route).
+bool take_route(Board* b, PyObject* given, int src, int dst, int8_t (&route)[MINT_MAX_RANKS + 1]) {
+    const bool cache = given == Py_None && src < b->world && dst < b->world;
+    if (cache && b->route[src][dst][MINT_MAX_RANKS]) {
+        memcpy(route, b->route[src][dst], sizeof(route));
+        return true;
+    }
+    PyObject* list;
+    if (given == Py_None) {
+        PyObject* comm = PyWeakref_GetObject(b->comm);
+        if (comm == Py_None) return raise(PyExc_RuntimeError, "the communicator is gone") != nullptr;
+        PyObject* found = PyObject_CallMethod(comm, "_find_route", "ii", src, dst);
+        list = found ? PySequence_Fast(found, "a route is a sequence of ranks") : nullptr;
+        Py_XDECREF(found);
+    } else {
+        list = PySequence_Fast(given, "a route is a sequence of ranks");
+    }
+    if (!list) return false;
+    const Py_ssize_t len = PySequence_Fast_GET_SIZE(list);
+    memset(route, 0, sizeof(route));
+    bool ok = len > 0;
+    for (Py_ssize_t i = 0; ok && i < len; ++i) {
+        const long r = PyLong_AsLong(PySequence_Fast_GET_ITEM(list, i));
+        if (r == -1 && PyErr_Occurred()) {
+            Py_DECREF(list);
+            return false;
+        }
+        ok = !(i == 0 && r != src) && !(i == len - 1 && r != dst);
+        // (a route longer than the world, or over ranks that are not there, is
+        // refused by the library: what does not fit is written as no rank)
+        if (i < MINT_MAX_RANKS) route[i] = r < 0 || r >= MINT_MAX_RANKS ? (int8_t)-1 : (int8_t)r;
+    }
+    Py_DECREF(list);
+    if (!ok) {
+        PyErr_Format(PyExc_ValueError, "no route %d -> %d", src, dst);
+        return false;
+    }
+    route[MINT_MAX_RANKS] = (int8_t)(len > MINT_MAX_RANKS ? MINT_MAX_RANKS + 1 : len);
+    if (cache) memcpy(b->route[src][dst], route, sizeof(route));
+    return true;
+}
+
+// sync(route, staged): the first call that finds a matched pair launches it, or
+// hands it back as (source, destination, from, to, bytes, route, kept buffers)
+PyObject* board_sync(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+    Board* b = reinterpret_cast<Board*>(self);
+    if (n != 2) return raise(PyExc_TypeError, "sync(route, staged)");
+    if (!b->send.given || !b->recv.given) Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        const Transfer s = b->send, r = b->recv;
+        b->send.given = b->recv.given = false;
+        auto go = [&]() -> PyObject* {
+            if (s.peer != r.rank || r.peer != s.rank)
+                return raise(PyExc_ValueError, "send and recv do not name each other");
+            if (s.count != r.count) return raise(PyExc_ValueError, "send and recv sizes differ");
+            if (!refresh(b)) return nullptr;
+            int8_t route[MINT_MAX_RANKS + 1];
+            if (!take_route(b, args[0], s.rank, r.rank, route)) return nullptr;
+            const int len = route[MINT_MAX_RANKS];
+            memcpy(b->last_route, route, sizeof(route));
+            mint_ring_op op = b->base;
+            op.op = MINT_OP_SENDRECV;
+            op.dtype = MINT_BYTES;
+            op.route_len = len;
+            for (int i = 0; i < MINT_MAX_RANKS; ++i) op.ring[i] = i < len ? route[i] : 0;
+            op.input[s.rank] = s.ptr;
+            op.output[r.rank] = r.ptr;
+            op.count_bytes = s.count;
+            if (b->native_launch && args[1] == Py_False) return launch(b, op);
+            PyObject* list = PyList_New(0);
+            bool ok = list != nullptr;
+            for (int i = 0; ok && i < len && i < MINT_MAX_RANKS; ++i) {
+                PyObject* v = PyLong_FromLong(route[i]);
+                ok = v && PyList_Append(list, v) == 0;
+                Py_XDECREF(v);
+            }
+            PyObject* result = ok ? Py_BuildValue("iiKKKO(OO)", s.rank, r.rank, (unsigned long long)s.ptr,
+                                                  (unsigned long long)r.ptr, (unsigned long long)s.count,
+                                                  list, s.keep, r.keep)
+                                  : nullptr;
+            Py_XDECREF(list);
+            return result;
+        };
+        PyObject* result = go();
+        Py_DECREF(s.keep);
+        Py_DECREF(r.keep);
+        return result;
+    });
+}
+
+PyObject* board_enter(PyObject* self, PyObject* arg) {
+    const long r = PyLong_AsLong(arg);
+    if (r == -1 && PyErr_Occurred()) return nullptr;
+    return PyLong_FromLong(enter_rank(reinterpret_cast<Board*>(self), (int)r));
+}
+PyObject* board_rank(PyObject* self, PyObject*) {
+    int rank;
+    return rank_or_raise(reinterpret_cast<Board*>(self), &rank) ? PyLong_FromLong(rank) : nullptr;
+}
+// run(fn): fn(rank) for every rank in turn
+PyObject* board_run(PyObject* self, PyObject* fn) {
+    Board* b = reinterpret_cast<Board*>(self);
+    const int before = current_rank(b);
+    PyObject* result = Py_NewRef(Py_None);
+    for (int r = 0; result && r < b->world; ++r) {
+        enter_rank(b, r);
+        PyObject* arg = PyLong_FromLong(r);
+        PyObject* got = arg ? PyObject_CallOneArg(fn, arg) : nullptr;
+        Py_XDECREF(arg);
+        if (!got) Py_CLEAR(result);
+        Py_XDECREF(got);
+    }
+    enter_rank(b, before);
+    return result;
+}
+
+PyObject* board_stale(PyObject* self, PyObject*) {
+    reinterpret_cast<Board*>(self)->fresh = false;
+    Py_RETURN_NONE;
+}
+// launching(descriptor): what a launch from Python is about to enqueue (last_grid)
+PyObject* board_launching(PyObject* self, PyObject* arg) {
+    Board* b = reinterpret_cast<Board*>(self);
+    Py_buffer view;
+    if (PyObject_GetBuffer(arg, &view, PyBUF_SIMPLE) < 0) return nullptr;
+    if (view.len == (Py_ssize_t)sizeof(mint_ring_op)) {
+        memcpy(&b->last, view.buf, sizeof(mint_ring_op));
+        b->launched = true;
+    }
+    PyBuffer_Release(&view);
+    Py_RETURN_NONE;
+}
+// configure(native_launch, ring, protocol, spin_budget, status): what launches
+// take from the communicator; an empty ring where the topology has none
+PyObject* board_configure(PyObject* self, PyObject* args) {
+    Board* b = reinterpret_cast<Board*>(self);
+    int native_launch, protocol;
+    unsigned long spin;
+    unsigned long long status;
+    PyObject* ring;
+    if (!PyArg_ParseTuple(args, "pOikK", &native_launch, &ring, &protocol, &spin, &status)) return nullptr;
+    mint_ring_op& d = b->base;
+    d = mint_ring_op{};
+    PyObject* list = PySequence_Fast(ring, "a ring is a sequence of ranks");
+    if (!list) return nullptr;
+    for (Py_ssize_t i = 0; i < PySequence_Fast_GET_SIZE(list) && i <= MINT_MAX_RANKS; ++i)
+        d.ring[i] = (int32_t)PyLong_AsLong(PySequence_Fast_GET_ITEM(list, i));
+    Py_DECREF(list);
+    if (PyErr_Occurred()) return nullptr;
+    b->has_ring = PySequence_Size(ring) == b->world + 1;
+    d.protocol = protocol;
+    d.world = b->world;
+    d.placement = MINT_PLACE_CU;
+    d.spin_budget = (uint32_t)spin;
+    d.status = status;
+    memset(b->route, 0, sizeof(b->route));
+    b->native_launch = native_launch;
+    b->fresh = true;
+    Py_RETURN_NONE;
+}
+
+PyObject* board_last_grid(PyObject* self, void*) {
+    Board* b = reinterpret_cast<Board*>(self);
+    return PyLong_FromLong(b->launched ? native.grid(&b->last) : 0);
+}
+PyObject* board_last_route(PyObject* self, void*) {
+    const int8_t* route = reinterpret_cast<Board*>(self)->last_route;
+    PyObject* list = PyList_New(0);
+    for (int i = 0; list && i < route[MINT_MAX_RANKS] && i < MINT_MAX_RANKS; ++i) {
+        PyObject* v = PyLong_FromLong(route[i]);
+        if (!v || PyList_Append(list, v) < 0) Py_CLEAR(list);
+        Py_XDECREF(v);
+    }
+    return list;
+}
+
+// Board(comm, world, device index)
+PyObject* board_new(PyTypeObject* type, PyObject* args, PyObject*) {
+    PyObject* comm;
+    int world, device;
+    if (!PyArg_ParseTuple(args, "Oii", &comm, &world, &device)) return nullptr;
+    if (world < 1 || world > MINT_MAX_RANKS) return raise(PyExc_ValueError, "world is 1..8");
+    Board* b = reinterpret_cast<Board*>(type->tp_alloc(type, 0));       // (zeroed)
+    if (!b) return nullptr;
+    b->id = next_board++;
+    b->world = world;
+    b->device = device;
+    b->comm = PyWeakref_NewRef(comm, nullptr);
+    if (!b->comm) Py_CLEAR(b);
+    return reinterpret_cast<PyObject*>(b);
+}
+void board_dealloc(PyObject* self) {
+    Board* b = reinterpret_cast<Board*>(self);
+    for (Gathering& g : b->gathering) drop(&g);
+    if (b->send.given) Py_DECREF(b->send.keep);
+    if (b->recv.given) Py_DECREF(b->recv.keep);
+    Py_XDECREF(b->comm);
+    Py_TYPE(self)->tp_free(self);
+}
+
+PyMethodDef board_methods[] = {
+    {"post", (PyCFunction)(void (*)(void))board_post, METH_FASTCALL, nullptr},
+    {"send", (PyCFunction)(void (*)(void))board_send, METH_FASTCALL, nullptr},
+    {"recv", (PyCFunction)(void (*)(void))board_recv, METH_FASTCALL, nullptr},
+    {"sync", (PyCFunction)(void (*)(void))board_sync, METH_FASTCALL, nullptr},
+    {"enter", board_enter, METH_O, nullptr},
+    {"rank", board_rank, METH_NOARGS, nullptr},
+    {"run", board_run, METH_O, nullptr},
+    {"stale", board_stale, METH_NOARGS, nullptr},
+    {"launching", board_launching, METH_O, nullptr},
+    {"configure", board_configure, METH_VARARGS, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyGetSetDef board_getset[] = {{"last_grid", board_last_grid, nullptr, nullptr, nullptr},
+                              {"last_route", board_last_route, nullptr, nullptr, nullptr},
+                              {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyTypeObject board_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ---- codec ---------------------------------------------------------------------
+const at::Tensor* device_tensor(PyObject* o) {
+    if (!THPVariable_Check(o)) return nullptr;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    return t.is_cuda() ? &t : nullptr;
+}
+size_t bytes_of(const at::Tensor& t) { return (size_t)t.numel() * (size_t)t.element_size(); }
+
+// pack(raw, flag_base, layout, flag_stride, out or None)
+PyObject* host_pack(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 5) return raise(PyExc_TypeError, "pack(raw, flag_base, layout, flag_stride, out)");
+    const uint64_t base = PyLong_AsUnsignedLongLongMask(args[1]), stride = PyLong_AsUnsignedLongLongMask(args[3]);
+    const int layout = (int)PyLong_AsLong(args[2]);
+    if (PyErr_Occurred()) return nullptr;
+    return guarded([&]() -> PyObject* {
+        const at::Tensor* raw = device_tensor(args[0]);
+        if (!raw || !raw->is_contiguous())
+            return raise(PyExc_ValueError, "pack needs a contiguous device tensor");
+        const size_t nbytes = bytes_of(*raw), need = native.packed_bytes(nbytes, layout);
+        PyObject* result;
+        if (args[4] == Py_None) {
+            result = THPVariable_Wrap(at::empty({(int64_t)need}, raw->options().dtype(at::kByte).requires_grad(false)));
+            if (!result) return nullptr;
+        } else {
+            const at::Tensor* out = device_tensor(args[4]);
+            if (!out) return raise(PyExc_ValueError, "pack needs a contiguous device tensor");
+            if (bytes_of(*out) < need) return raise(PyExc_ValueError, "output too small");
+            result = Py_NewRef(args[4]);
+        }
+        OnDevice on(raw->get_device());
+        void *const from = raw->data_ptr(), *const to = THPVariable_Unpack(result).data_ptr(), *const stream = on.stream();
+        int code;
+        Py_BEGIN_ALLOW_THREADS
+        code = native.pack(from, to, nbytes, base, stride, layout, stream);
+        Py_END_ALLOW_THREADS
+        if (code != MINT_OK) {
+            Py_DECREF(result);
+            return checked(code, "mint_ll128_pack");
+        }
+        return result;
+    });
+}
+
+// unpack(msg, out, flag_base, layout, flag_stride, bad_flags or None)
+PyObject* host_unpack(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != 6) return raise(PyExc_TypeError, "unpack(msg, out, flag_base, layout, flag_stride, bad_flags)");
+    const uint64_t base = PyLong_AsUnsignedLongLongMask(args[2]), stride = PyLong_AsUnsignedLongLongMask(args[4]);
+    const int layout = (int)PyLong_AsLong(args[3]);
+    if (PyErr_Occurred()) return nullptr;
+    return guarded([&]() -> PyObject* {
+        const at::Tensor *msg = device_tensor(args[0]), *out = device_tensor(args[1]);
+        if (!msg || !out || !out->is_contiguous())
+            return raise(PyExc_ValueError, "unpack needs contiguous device tensors");
+        const size_t nbytes = bytes_of(*out);
+        if (bytes_of(*msg) < native.packed_bytes(nbytes, layout))
+            return raise(PyExc_ValueError, "message too small");
+        void* bad = nullptr;
+        if (args[5] != Py_None) {
+            if (!THPVariable_Check(args[5])) return raise(PyExc_TypeError, "bad_flags is a tensor");
+            bad = THPVariable_Unpack(args[5]).data_ptr();
+        }
+        OnDevice on(out->get_device());
+        void *const from = msg->data_ptr(), *const to = out->data_ptr(), *const stream = on.stream();
+        int code;
+        Py_BEGIN_ALLOW_THREADS
+        code = native.unpack(from, to, nbytes, base, stride, layout, bad, stream);
+        Py_END_ALLOW_THREADS
+        if (code != MINT_OK) return checked(code, "mint_ll128_unpack");
+        return Py_NewRef(args[1]);
+    });
+}
+
+// bind(launch, grid, pack, unpack, packed_bytes, check): addresses, and what raises
+PyObject* host_bind(PyObject*, PyObject* args) {
+    unsigned long long launch, grid, pack, unpack, packed;
+    PyObject* check;
+    if (!PyArg_ParseTuple(args, "KKKKKO", &launch, &grid, &pack, &unpack, &packed, &check)) return nullptr;
+    native.launch = reinterpret_cast<decltype(native.launch)>(launch);
+    native.grid = reinterpret_cast<decltype(native.grid)>(grid);
+    native.pack = reinterpret_cast<decltype(native.pack)>(pack);
+    native.unpack = reinterpret_cast<decltype(native.unpack)>(unpack);
+    native.packed_bytes = reinterpret_cast<decltype(native.packed_bytes)>(packed);
+    Py_INCREF(check);
+    Py_XSETREF(native.check, check);
+    Py_RETURN_NONE;
+}
+
+PyMethodDef host_methods[] = {
+    {"bind", host_bind, METH_VARARGS, nullptr},
+    {"pack", (PyCFunction)(void (*)(void))host_pack, METH_FASTCALL, nullptr},
+    {"unpack", (PyCFunction)(void (*)(void))host_unpack, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef host_module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, host_methods,
+                           nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) {
+    board_type.tp_name = "mintccl_amd._host.Board";
+    board_type.tp_basicsize = sizeof(Board);
+    board_type.tp_flags = Py_TPFLAGS_DEFAULT;
+    board_type.tp_new = board_new;
+    board_type.tp_dealloc = board_dealloc;
+    board_type.tp_methods = board_methods;
+    board_type.tp_getset = board_getset;
+    if (PyType_Ready(&board_type) < 0) return nullptr;
+    PyObject* m = PyModule_Create(&host_module);
+    if (!m) return nullptr;
+    Py_INCREF(&board_type);
+    PyModule_AddObject(m, "Board", reinterpret_cast<PyObject*>(&board_type));
+    for (int k = 0; k < KINDS; ++k) {
+        char name[32];
+        size_t i = 0;
+        for (; kKinds[k].name[i]; ++i) name[i] = (char)toupper(kKinds[k].name[i]);
+        name[i] = 0;
+        PyModule_AddIntConstant(m, name, k);
+    }
+    PyModule_AddIntConstant(m, "DESCRIPTOR_BYTES", sizeof(mint_ring_op));
+    return m;
+}

@@ -29,25 +29,10 @@ def packed_bytes(nbytes: int, layout: int = LAYOUT_WAVE64) -> int:
     return _lib.lib().mint_ll128_packed_bytes(nbytes, layout)
 
 
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
-
-
 def pack(raw: torch.Tensor, flag_base: int = 1, layout: int = LAYOUT_WAVE64,
          flag_stride: int = 1, out: torch.Tensor | None = None) -> torch.Tensor:
     """Device tensor (any dtype, contiguous) -> uint8 tensor of LL128 lines."""
-    if not raw.is_cuda or not raw.is_contiguous():
-        raise ValueError("pack needs a contiguous device tensor")
-    nbytes = raw.numel() * raw.element_size()
-    need = packed_bytes(nbytes, layout)
-    if out is None:
-        out = torch.empty(need, dtype=torch.uint8, device=raw.device)
-    elif out.numel() * out.element_size() < need:
-        raise ValueError("output too small")
-    with torch.cuda.device(raw.device):
-        _lib.check(_lib.lib().mint_ll128_pack(raw.data_ptr(), out.data_ptr(), nbytes, flag_base,
-                                              flag_stride, layout, _stream(raw)), "mint_ll128_pack")
-    return out
+    return _lib.host().pack(raw, flag_base, layout, flag_stride, out)
 
 
 def unpack(msg: torch.Tensor, out: torch.Tensor, flag_base: int = 1,
@@ -55,14 +40,4 @@ def unpack(msg: torch.Tensor, out: torch.Tensor, flag_base: int = 1,
            bad_flags: torch.Tensor | None = None) -> torch.Tensor:
     """LL128 lines -> ``out`` (its byte size says how much to unpack).
     ``bad_flags`` (int64[1], device) counts lines with an unexpected flag."""
-    if not msg.is_cuda or not out.is_cuda or not out.is_contiguous():
-        raise ValueError("unpack needs contiguous device tensors")
-    nbytes = out.numel() * out.element_size()
-    if msg.numel() * msg.element_size() < packed_bytes(nbytes, layout):
-        raise ValueError("message too small")
-    with torch.cuda.device(out.device):
-        _lib.check(_lib.lib().mint_ll128_unpack(
-            msg.data_ptr(), out.data_ptr(), nbytes, flag_base, flag_stride, layout,
-            bad_flags.data_ptr() if bad_flags is not None else 0, _stream(out)),
-            "mint_ll128_unpack")
-    return out
+    return _lib.host().unpack(msg, out, flag_base, layout, flag_stride, bad_flags)

@@ -7,31 +7,21 @@ from __future__ import annotations
 
 import torch
 
-from . import _lib
-from ._ops import (check_buffer, comm_or_default, nbytes, reduce_dtype, ring_of,
-                   same_everywhere)
-from .common import VirtualComm
+from . import _lib, hypercube
+from ._ops import ring_of
+from .common import VirtualComm, get_comm
 
 
 def reducescatter(buff: torch.Tensor, comm: VirtualComm | None = None) -> None:
-    from . import hypercube, tree
-    if tree.topology_env() == "hypercube":
-        return hypercube.reducescatter(buff, comm)
-    comm = comm_or_default(comm)
-    check_buffer(buff, comm)
-    if buff.numel() % comm.world_size:
-        raise ValueError("buffer does not split into world_size rows")
-    posted = comm.post("reducescatter", set(range(comm.world_size)),
-                       {"ptr": buff.data_ptr(), "count": nbytes(buff),
-                        "dtype": reduce_dtype(buff), "keep": buff})
-    if posted is None:
+    comm = comm if comm is not None else get_comm()
+    posted = comm._board.post(_lib.KIND_REDUCESCATTER, buff)
+    if posted is None:               # not all ranks are here yet, or launched
         return
-    count = same_everywhere(posted, "count", "the byte count")
-    dtype = same_everywhere(posted, "dtype", "the dtype")
+    if posted is False:
+        return hypercube.reducescatter(buff, comm)
+    count, dtype, _, _, ptrs, _, _ = posted
     row = count // comm.world_size
-    ptrs = {r: info["ptr"] for r, info in posted.items()}
-    comm.enqueue(_lib.OP_REDUCESCATTER, dtype, row, ptrs, ptrs, ring_of(comm),
-                 row_stride=row)
+    comm.enqueue(_lib.OP_REDUCESCATTER, dtype, row, ptrs, ptrs, ring_of(comm), row_stride=row)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

@@ -4,21 +4,17 @@ its own (``:147-149``), so no hop ever waits for a credit."""
 from __future__ import annotations
 
 from . import sendrecv_buffer as _buffered
-from ._ops import comm_or_default
-from .common import VirtualComm
+from .common import VirtualComm, get_comm
 
 send = _buffered.send
 recv = _buffered.recv
 
 
 def sync(comm: VirtualComm | None = None, route: list[int] | None = None) -> None:
-    comm = comm_or_default(comm)
-    st = _buffered._state(comm)
-    if st["send"] is None or st["recv"] is None:
-        return
-    s, r = st["send"], st["recv"]
-    st["send"] = st["recv"] = None
-    _buffered._launch(comm, s, r, route, full_size_staging=True)
+    comm = comm if comm is not None else get_comm()
+    matched = comm._board.sync(route, True)
+    if matched is not None:
+        _buffered._launch(comm, matched, full_size_staging=True)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

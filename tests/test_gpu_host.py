@@ -1,0 +1,139 @@
+"""The native host side of the operators: what it refuses, that it follows the
+communicator's attributes and the environment, and whose rank a thread speaks for."""
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ring
+from tests.helpers import as_bytes, rank_rows
+
+pytestmark = pytest.mark.gpu
+
+
+def make_comm(world, **kw):
+    from mintccl_amd.common import VirtualComm
+    return VirtualComm(world_size=world, spin_budget=400000, **kw)
+
+
+def test_refusals_leave_the_communicator_usable(dev):
+    from mintccl_amd.allgather import allgather
+    from mintccl_amd.alltoall import alltoall
+    from mintccl_amd.broadcast import broadcast
+    from mintccl_amd.reduce import reduce
+    comm = make_comm(2)
+    a, b = torch.zeros(8, device=dev), torch.zeros(8, device=dev, dtype=torch.float16)
+
+    def pair(first, second, match):
+        with comm.rank(0):
+            first()
+        with comm.rank(1), pytest.raises(ValueError, match=match):
+            second()
+
+    pair(lambda: broadcast(a, 0, comm), lambda: broadcast(a, 1, comm), "ranks disagree on the root")
+    pair(lambda: broadcast(a, 0, comm), lambda: broadcast(b, 0, comm), "byte count: .'16', '32'.")
+    pair(lambda: reduce(b, 0, comm), lambda: reduce(b.bfloat16(), 0, comm), "the dtype")
+    pair(lambda: allgather(a, comm), lambda: allgather(a, comm, schedule="temporal"),
+         "the schedule: .'spatial', 'temporal'.")
+    pair(lambda: alltoall(a, torch.zeros_like(a), comm), lambda: alltoall(b.float(), a, comm), "overlaps")
+    with comm.rank(0):
+        with pytest.raises(ValueError, match="schedule is"):
+            allgather(a, comm, schedule="both")
+        with pytest.raises(ValueError, match="differ in size"):
+            alltoall(a, b, comm)
+        reduce(a, 0, comm)
+        with pytest.raises(RuntimeError, match="called reduce twice"):
+            reduce(a, 0, comm)
+    with comm.rank(1):
+        reduce(a, 0, comm)
+    with pytest.raises(ValueError):
+        comm.rank(2)
+    comm.check()
+
+
+def test_launches_follow_attributes_and_environment(dev, monkeypatch):
+    """A ring set after the first launch is the ring of the next one (f16 sums
+    depend on the order), and MINTCCL_TOPOLOGY / _ALLREDUCE / _ALLGATHER are read
+    when an operator runs."""
+    from mintccl_amd._ops import ring_of
+    from mintccl_amd.allgather import allgather
+    from mintccl_amd.allreduce import allreduce
+    from mintccl_amd.reducescatter import reducescatter
+    world, n = 4, 5000
+    comm = make_comm(world)
+    host = rank_rows(world, n, "f16", seed0=70)
+    raw = [as_bytes(h) for h in host]
+
+    def summed():
+        bufs = [h.to(dev) for h in host]
+        comm.run(lambda r: reducescatter(bufs[r], comm))
+        comm.check()
+        return [as_bytes(x) for x in bufs]
+
+    plain = summed()
+    assert all(np.array_equal(x, y) for x, y in zip(plain, ring.reducescatter(raw, "f16")))
+    # only the links of the ring 0 -> 2 -> 1 -> 3 -> 0
+    links = [(0, 2), (2, 1), (1, 3), (3, 0)]
+    comm.topology = {u: [(v, 1.0) for a, b in links for v in ((b,) if a == u else (a,) if b == u else ())]
+                     for u in range(world)}
+    turned = summed()
+    order = ring_of(comm)
+    assert order in ([0, 2, 1, 3, 0], [0, 3, 1, 2, 0])
+    assert all(np.array_equal(x, y) for x, y in zip(turned, ring.reducescatter(raw, "f16", order)))
+    assert any(not np.array_equal(x, y) for x, y in zip(plain, turned))
+    comm.topology = None
+    monkeypatch.setenv("MINTCCL_TOPOLOGY", "hypercube")
+    cube = summed()
+    assert all(np.array_equal(x, y) for x, y in zip(cube, ring.hypercube_reducescatter(raw, "f16")))
+    monkeypatch.delenv("MINTCCL_TOPOLOGY")
+    for var, value, op, want in (("MINTCCL_ALLREDUCE", "split", allreduce, ring.allreduce(raw, "f16")),
+                                 ("MINTCCL_ALLGATHER", "temporal", allgather, ring.allgather(raw))):
+        monkeypatch.setenv(var, value)
+        bufs = [h.to(dev) for h in host]
+        comm.run(lambda r: op(bufs[r], comm))
+        comm.check()
+        assert all(np.array_equal(as_bytes(b), w) for b, w in zip(bufs, want)), var
+        monkeypatch.delenv(var)
+
+
+def test_a_rank_belongs_to_its_thread_and_communicator(dev):
+    from mintccl_amd.broadcast import broadcast
+    comm, other = make_comm(3), make_comm(2)
+    bufs = [torch.full((1000,), float(r), device=dev) for r in range(3)]
+    seen = []
+
+    def rank(r):
+        with comm.rank(r), other.rank(0):
+            with comm.rank((r + 1) % 3):
+                assert comm.Get_rank() == (r + 1) % 3
+            assert comm.Get_rank() == r and other.Get_rank() == 0
+            broadcast(bufs[r], 1, comm)
+        try:
+            comm.Get_rank()
+        except RuntimeError:
+            seen.append(r)
+
+    threads = [threading.Thread(target=rank, args=(r,)) for r in range(3)]
+    for t in threads:
+        t.start()
+        t.join()
+    comm.check()
+    assert seen == [0, 1, 2]
+    assert all(torch.all(b == 1.0) for b in bufs)
+
+
+def test_codec_refuses_what_it_cannot_take(dev):
+    from mintccl_amd import _lib, protocol
+    raw = torch.zeros(960, dtype=torch.uint8, device=dev)
+    msg = protocol.pack(raw)
+    for bad in (lambda: protocol.pack(raw.cpu()), lambda: protocol.pack(raw.view(2, 480).t()),
+                lambda: protocol.pack(raw, out=raw), lambda: protocol.unpack(msg[:512], raw),
+                lambda: protocol.unpack(msg.cpu(), raw)):
+        with pytest.raises(ValueError):
+            bad()
+    with pytest.raises(_lib.MintError):
+        protocol.pack(raw, layout=7)
+    with pytest.raises(_lib.MintError) as e:
+        protocol.pack(torch.zeros(976, dtype=torch.uint8, device=dev)[1:961])
+    assert e.value.code == _lib.ERR_ALIGN
