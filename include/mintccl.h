@@ -103,16 +103,16 @@ typedef enum {
                                work from the XCD it runs on; needs a device that deals
                                every 8 consecutive blocks to 8 different XCDs
                                (mint_device_info reports 8, mint_xcd_map shows the order) */
-    MINT_PLACE_CU = 2       /* every hop of a channel inside one compute unit: a thread
-                               block runs all positions of a channel, the blocks travel
-                               between them through LDS.  Both protocols are the same
-                               there (LDS keeps a wavefront's operations in order, so
-                               whole 1 KiB blocks go first and the step counter behind
-                               them).  staging[], staging_bytes, credit_offset,
+    MINT_PLACE_CU = 2       /* every hop inside a compute unit: a lane stands at all
+                               positions of a ring in turn, the partial sum stays in its
+                               registers from one to the next (same additions, same
+                               order).  Nobody waits, so both protocols are the same
+                               there.  staging[], staging_bytes, credit_offset,
                                slot_bytes, nslots, waves_per_channel_group,
                                threads_per_block, cache_policy, flag_epoch, epoch_ptr,
-                               row_fetch and origin_cus are not looked at; launches on
-                               different streams share nothing but the status block.
+                               row_fetch, origin_cus and spin_budget are not looked at;
+                               launches on different streams share nothing but the
+                               status block.
                                SENDRECV, BROADCAST, REDUCE, ALLGATHER, REDUCESCATTER,
                                ALLREDUCE and ALLTOALL. */
 } mint_placement;
@@ -145,8 +145,8 @@ typedef enum {
  * The words stay set until the caller zeroes them: every launch that finds
  * word 3 set gives up at its first wait (after at most 64 polls) and leaves
  * unspecified output, and only the first failure is recorded (under
- * MINT_PLACE_CU a launch runs whatever word 3 says and is counted there; a
- * position whose wait ran out goes on without waiting, in bounds).  After a
+ * MINT_PLACE_CU a launch waits for nothing: it runs whatever word 3 says and is
+ * only counted there).  After a
  * non-zero word 0 the caller synchronises the stream, zeroes the block and
  * treats the outputs of every launch since the last clean check as lost;
  * under MINT_PLACE_LOCAL it also zeroes the staging before it is used again

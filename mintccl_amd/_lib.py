@@ -56,6 +56,8 @@ HIPCC_FLAGS = [
     # refuses a kernel that uses scratch (see there)
     "-Rpass-analysis=kernel-resource-usage",
 ]
+# the first ten words of a launch's arguments (CuShape) arrive in registers
+CU_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=10"]
 
 
 class RingOp(ctypes.Structure):
@@ -183,7 +185,7 @@ def build(verbose: bool = False, defines: tuple[str, ...] = (), so_path: str | N
     build_dir = BUILD_DIR if so_path is None else out + ".objs"
     os.makedirs(build_dir, exist_ok=True)
     units = [(SRC, list(defines), os.path.join(build_dir, "mintccl.o")),
-             (CU_SRC, list(defines), os.path.join(build_dir, "cu_ring.o"))]
+             (CU_SRC, [*CU_FLAGS, *defines], os.path.join(build_dir, "cu_ring.o"))]
     for dt in range(4):
         units.append((FAMILY_SRC, [f"-DMINT_FAMILY_DT={dt}", *defines],
                       os.path.join(build_dir, f"ring_family_{dt}.o")))

@@ -1,276 +1,242 @@
-// Rings inside a compute unit: the ring collectives of ring.hpp with every
-// position of a channel in ONE thread block and the hops between them in LDS.
+// Rings inside a compute unit: the ring collectives of ring.hpp with all
+// positions of a ring in one lane and the hops between them in its registers.
 //
 // The walks of ring.hpp put neighbouring positions on different compute units
 // and their staging into the L2 of an XCD.  A hop then costs a 1 KiB store and
 // a 1 KiB load through the L2 beside the rows from HBM, and a compute unit
 // keeps only some 130 requests in flight: an 8-rank reduce-scatter spends half
-// of its time on staging.  Virtual ranks share one GPU, so a channel's whole
-// ring fits one compute unit: wavefront h of the block is position h (the rank
-// `h` places after the pipeline's root), it loads its own rank's row from HBM
-// ahead of time, takes the block its predecessor left in LDS, adds or copies,
-// and leaves the result for its successor.  What crosses the memory system is
-// each row once; LDS carries 2 KiB per hop and KiB of row, an eighth of its rate.
+// of its time on staging.  Virtual ranks share one GPU, so one lane can stand
+// at every position in turn: it loads its 16 bytes of every rank's row, all of
+// them at once, walks the ring from the pipeline's root with the partial sum in
+// registers - the additions and their order are those of the hops - and stores
+// the result at the positions that keep it.  Each row crosses the memory system
+// once; there is no staging, no epoch, no seat to claim and nobody to wait for,
+// and both protocols (which say how a hop is made safe) are the same.
 //
-// The wire between two positions: NS slots of U KiB in LDS, and two words,
-//   head   steps the sender has put into the slots   (sender writes)
-//   tail   steps the receiver has taken out          (receiver writes)
-// the pair of the Simple protocol (post / wait, protocol.py:161-189).  LDS
-// executes a wavefront's operations in issue order, so a `head` stored behind
-// the data is seen behind the data: what LL128's flag inside every line is for
-// holds by itself, and both protocols move whole 1 KiB blocks here.  There is
-// no epoch, no staging memory and no seat to claim: the words start at zero in
-// every block, all positions of a channel are resident together because they
-// are one block, and a grid of any size drains.  Waits stay bounded and report
-// like those of ring.hpp.
+// Bound by HBM (6.4 - 6.8 TB/s of rows read and written).  A thread block moves
+// one tile and ends, and the tiles of a pipeline follow each other in the order
+// the blocks are dealt: what is in flight over the device is one window of
+// consecutive bytes per row that moves through memory.  Wavefronts that stay
+// resident and stride through the rows drift apart and lose a tenth of the rate.
+// 8 ranks: one ring per resident thread block, hops through LDS / one lane and
+// resident / a block per tile / and the wavefronts held down (cu_threads):
+// reduce-scatter of 256 MiB f16 447 / 470 / 391 / 375 us, allgather of 8 x 128 MiB
+// 1675 / 1660 / 1540 / 1380, allreduce of 64 MiB bf16 205 / 198 / 190 / 165.
 #pragma once
 #include "ring.hpp"
 
 namespace mint {
 
-// One launch.  The ranks' buffers come in the order of the ring (or route), so
-// that position h of a pipeline that starts at index i works for index
-// (i + h) % len of these tables.
-struct CuRingArgs {
-    uint64_t input[kMaxRanks], output[kMaxRanks];
+// One launch.  Grid: tiles of a row, then one block for its ragged ends if it has
+// any, in x (large form) or y; pipelines (alltoall: destinations) in the other;
+// the sources of an alltoall in z.
+//
+// A block lives for one trip to memory, so what it does before its loads are out
+// counts: the numbers come as kernel arguments of their own, which the compiler
+// has the hardware put into scalar registers before the first instruction
+// (kernarg preload), and one round of scalar loads brings the addresses.
+struct CuShape {
     uint64_t starts;               // byte p: index in the ring of pipeline p's root
     uint64_t row_bytes, row_stride;
-    uint64_t total_bytes;          // 0, or clip row p to total_bytes - p * row_stride
+    uint64_t short_bytes;          // bytes of row `full`; rows behind it are empty
+    uint32_t full;                 // rows before this one have row_bytes
+    uint32_t tiles;                // thread blocks that share the whole vectors of a row
+};
+// The ranks' buffers in the order of the ring (or route), twice over, so that
+// those of a pipeline that starts at index i are the `len` entries from i on.
+struct CuTables {
+    uint64_t input[2 * kMaxRanks], output[2 * kMaxRanks];
     uint64_t* status;
-    uint32_t op, pipes, len, hops;
-    uint32_t channels;             // per pipeline
-    uint32_t spin_budget;
+};
+struct CuRingArgs {
+    CuShape shape;
+    CuTables tables;
+    uint32_t op, pipes, len, ends;
 };
 
-// Row p in whole 1 KiB blocks, dealt in units of `unit`: unit i belongs to
-// channel i % channels, which walks its units in steps.  The bytes behind the
-// last whole block are a step of their own of the channel that comes next.
-struct CuWalk {
-    uint32_t steps;          // units of this channel
-    uint32_t nfull;          // whole blocks of the row
-    bool tail;               // this channel moves the bytes behind them
-    uint64_t row_bytes;
+// Two forms of a launch (which: plan_cu in mintccl.hip).
+//
+// LARGE, rows beyond the last-level cache: one wavefront per block and 1 KiB
+// tiles (with several copies two), the pipelines one after the other, as few
+// wavefronts on a compute unit as keep HBM busy (cu_waves).  More of them widen
+// the window over which the loads and stores of 8 or 16 rows are scattered: 8
+// ranks, 256 MiB of f16, reduce-scatter 390 us with 32 to a compute unit, 368 with
+// 9, 460 with 4; allreduce of 8 x 64 MiB 204 with 32, 163 with 4; allgather of
+// 8 x 32 MiB 429 / 338 with 32 / 8.
+//
+// Otherwise: blocks of 128 threads and 2 KiB, dealt to the pipelines in turn,
+// loads through the cache (8 ranks, reduce-scatter of 8 MiB 10.9 us; 15.5 in the
+// large form, 13.0 with one pipeline after the other; blocks of 64 threads lose up
+// to a third where rows are copied once, 512 up to a tenth where they are added).
+#ifndef PROBE
+constexpr uint32_t cu_threads(bool large, bool copies) { return large && !copies ? 64u : 128u; }
+#endif
+
+// Rows that are read once, by nobody soon, are streamed past the last-level
+// cache, and so are stores nobody waits for.
+template <bool STREAM>
+__device__ __forceinline__ u32x4 cu_load(const uint8_t* uniform, uint32_t lane) {
+    MINT_GLOBAL const u32x4_unaligned* const p = (MINT_GLOBAL const u32x4_unaligned*)(as_global(uniform) + lane);
+    if constexpr (STREAM) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <bool STREAM>
+__device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 v) {
+    MINT_GLOBAL u32x4_unaligned* const p = (MINT_GLOBAL u32x4_unaligned*)(as_global(uniform) + lane);
+    if constexpr (STREAM) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
+// A row cut into vectors of 16 bytes whose stores are aligned: vector i covers
+// the bytes from 16 i - `shift` on.  Vectors that are not wholly inside the row
+// are left out; the bytes they would have brought, fewer than 16 at either end,
+// are moved one element per lane.
+struct CuRow {
+    uint64_t bytes;
+    uint32_t shift;
+    __device__ __forceinline__ CuRow(const CuShape& a, uint32_t p, const uint8_t* stored, uint32_t size) {
+        bytes = p < a.full ? a.row_bytes : p == a.full ? a.short_bytes : 0u;
+        // (whole elements: a row may start at any byte)
+        shift = (uint32_t)(uintptr_t)stored & 127u & ~(size - 1u);
+    }
+    __device__ __forceinline__ bool whole(int64_t off) const {
+        return off >= 0 && (uint64_t)off + 16u <= bytes;
+    }
+    // Element of `size` bytes that this lane (of the first 32) moves, or none.
+    __device__ __forceinline__ bool end_element(uint32_t size, uint64_t& off) const {
+        uint32_t head = (0u - shift) & 15u;
+        head = bytes < head ? (uint32_t)bytes : head;
+        const uint32_t tail = (uint32_t)(bytes - head) & 15u;
+        const uint32_t at = (threadIdx.x & 15u) * size;
+        const bool first = threadIdx.x < 16u;
+        off = first ? at : bytes - tail + at;
+        return threadIdx.x < 32u && at < (first ? head : tail);
+    }
 };
-__host__ __device__ __forceinline__ CuWalk cu_walk_of(const CuRingArgs& a, uint32_t p, uint32_t c,
-                                                      uint32_t unit) {
-    CuWalk k;
-    k.row_bytes = a.row_bytes;
-    if (a.total_bytes) {
-        const uint64_t off = (uint64_t)p * a.row_stride;
-        const uint64_t left = a.total_bytes > off ? a.total_bytes - off : 0;
-        k.row_bytes = left < a.row_bytes ? left : a.row_bytes;
-    }
-    k.nfull = (uint32_t)(k.row_bytes / kBlockRawSimple);
-    const uint32_t units = (k.nfull + unit - 1) / unit;
-    k.steps = units > c ? (units - 1 - c) / a.channels + 1 : 0;
-    k.tail = k.row_bytes % kBlockRawSimple != 0 && units % a.channels == c;
-    return k;
+
+// A launch that finds the abort flag of its status block set (an earlier launch
+// through staging gave up) is counted there, as in take_seat; by the last
+// wavefront of the first block, which has nothing else to do in a launch so
+// small that this load would show.
+template <uint32_t THREADS>
+__device__ __forceinline__ void cu_count_if_aborted(uint64_t* status) {
+    if (blockIdx.x == 0u && blockIdx.y == 0u && blockIdx.z == 0u && threadIdx.x >= THREADS - 64u)
+        count_launch_if_aborted(status, 0);
 }
 
-// The words of a channel, in LDS in front of the slots: head and tail of every hop.
-constexpr int kCuMaxHops = 2 * kMaxRanks - 2;
-constexpr uint32_t kCuWordBytes = 128;
-static_assert(2 * kCuMaxHops * 4 <= (int)kCuWordBytes, "head and tail of every hop");
-
-// What a position does, in flags that are compile-time constants of its walk.
-template <bool LOAD, bool RECV, bool REDUCE, bool SAVE, bool SEND>
-struct CuRole {
-    static constexpr bool load = LOAD, recv = RECV, reduce = REDUCE, save = SAVE, send = SEND;
-};
-
-// Polls `word` until it has reached `need` or `patience` further polls have
-// gone by; `seen` comes back as what the last poll saw.
-__device__ __forceinline__ void cu_spin(MINT_LDS const uint32_t* word, uint32_t need, uint32_t patience,
-                                        uint32_t& seen) {
-    uint32_t v, gap;
-    asm volatile(
-        "1:\n\t"
-        "ds_read_b32 %[v], %[word]\n\t"
-        "s_waitcnt lgkmcnt(0)\n\t"
-        "v_readfirstlane_b32 %[seen], %[v]\n\t"
-        "s_sub_i32 %[gap], %[seen], %[need]\n\t"
-        "s_cmp_ge_i32 %[gap], 0\n\t"
-        "s_cbranch_scc1 2f\n\t"
-        "s_sub_u32 %[left], %[left], 1\n\t"
-        "s_cbranch_scc1 2f\n\t"
-        "s_sleep 1\n\t"
-        "s_branch 1b\n"
-        "2:"
-        : [v] "=&v"(v), [seen] "=&s"(seen), [gap] "=&s"(gap), [left] "+s"(patience)
-        : [word] "v"(word), [need] "s"(need)
-        : "memory", "scc");
+typedef uint32_t u32_unaligned __attribute__((aligned(1)));
+typedef uint16_t u16_unaligned __attribute__((aligned(1)));
+template <int DT>
+__device__ __forceinline__ uint32_t cu_load_element(const uint8_t* p) {
+    if constexpr (DT == DT_F32) return *(MINT_GLOBAL const u32_unaligned*)p;
+    else return *(MINT_GLOBAL const u16_unaligned*)p;
+}
+template <int DT>
+__device__ __forceinline__ void cu_store_element(uint8_t* p, uint32_t v) {
+    if constexpr (DT == DT_F32) *(MINT_GLOBAL u32_unaligned*)p = v;
+    else *(MINT_GLOBAL u16_unaligned*)p = (uint16_t)v;
 }
 
-template <int DT, int U, int NS, int D, typename Role>
-__device__ __forceinline__ void cu_walk(const CuRingArgs& a, const uint32_t p, const uint32_t h,
-                                        const uint32_t c, const uint8_t* in_row, uint8_t* out_row,
-                                        MINT_LDS uint8_t* lds, Role) {
-    static_assert((NS & (NS - 1)) == 0 && D == 4, "masks; the loop below is unrolled by the depth");
-    constexpr uint32_t kSlot = (uint32_t)U * kBlockRawSimple, kHop = (uint32_t)NS * kSlot;
-    const uint32_t lane_off = (uint32_t)lane_id() * 16u;
-    const CuWalk k = cu_walk_of(a, p, c, (uint32_t)U);
-    MINT_LDS uint32_t* const head = reinterpret_cast<MINT_LDS uint32_t*>(lds);
-    MINT_LDS uint32_t* const tail = head + kCuMaxHops;
-    MINT_LDS uint8_t* const slots = lds + kCuWordBytes;
-    MINT_LDS uint8_t* const rx = slots + (h - 1u) * kHop + lane_off;
-    MINT_LDS uint8_t* const tx = slots + h * kHop + lane_off;
-    const uint32_t C = a.channels, last = k.nfull - 1u;
-
-    // Own rows, D steps ahead.  Block numbers are clamped to the last whole
-    // block, so that every step issues the same loads and the wait for the
-    // oldest leaves the others in flight.  The walk is whole rounds of D steps
-    // with one way out (the compiler sets each wait from the path with the
-    // fewest younger loads, and an exit in the middle of a round would be
-    // such a path): what the steps leave over D comes first, so buffer j
-    // starts with step (j + rest) % D.
-    u32x4 v[D][U];
-    auto fetch = [&](uint32_t s, u32x4 (&x)[U]) MINT_INLINE_LAMBDA {
+// The next addresses of a table, and a point where they have to be there: the
+// compiler would fetch each where it is first used, a scalar load and a wait at
+// a time.
+template <int N, typename P>
+__device__ __forceinline__ void cu_addresses(const uint64_t* table, P* (&x)[N]) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            uint32_t g = (s * C + c) * (uint32_t)U + (uint32_t)u;
-            g = g < last ? g : last;
-            x[u] = ld128_row(in_row + (uint64_t)g * kBlockRawSimple + lane_off);
-        }
-    };
-    const uint32_t rest = k.steps % (uint32_t)D;
-    if (Role::load && k.steps) {
+    for (int i = 0; i < N; ++i) x[i] = reinterpret_cast<P*>(table[i]);
+}
+template <int N, typename P>
+__device__ __forceinline__ void cu_here(P* (&x)[N]) {
 #pragma unroll
-        for (int d = 0; d < D; ++d) fetch(((uint32_t)d + rest) % (uint32_t)D, v[d]);
-    }
-    // The words are cleared while the first rows are on their way; the barrier
-    // must not wait for those.
-    if (threadIdx.x < kCuWordBytes / 4) head[threadIdx.x] = 0u;
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-
-    // wait_ll128 (protocol.py:161-180) on either word.  A wait that runs out
-    // marks the walk as failed and lets it go on without waiting any further:
-    // the outputs are unspecified from there on, every access stays where it
-    // was, the neighbours see their words move and the grid drains.  (Written
-    // as one statement, with no way out of the walk behind it, so that the
-    // compiler keeps exact count of the loads in flight around it.)
-    uint32_t head_seen = 0, tail_seen = 0, patience = a.spin_budget, failed_at = ~0u;
-    auto wait_for = [&](MINT_LDS uint32_t* word, uint32_t need, uint32_t& seen, uint32_t s) MINT_INLINE_LAMBDA {
-        if ((int32_t)(seen - need) >= 0) return;
-        cu_spin(word, need, patience, seen);
-        if ((int32_t)(seen - need) < 0) {
-            failed_at = failed_at < s ? failed_at : s;
-            patience = 0;
-        }
-    };
-    // One step between this position's neighbours: take the blocks out of the
-    // predecessor's slot, combine them with `own`, leave them for the successor.
-    auto pass_on = [&](uint32_t s, const u32x4 (&own)[U], u32x4 (&x)[U]) MINT_INLINE_LAMBDA {
-        const uint32_t slot = (s & (uint32_t)(NS - 1)) * kSlot;
-#pragma unroll
-        for (int u = 0; u < U; ++u) x[u] = own[u];
-        if (Role::recv) {
-            wait_for(head + (h - 1u), s + 1u, head_seen, s);
-            compiler_fence();
-            u32x4 r[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                r[u] = *reinterpret_cast<MINT_LDS const u32x4*>(rx + slot + (uint32_t)u * kBlockRawSimple);
-            // post_ll128 (protocol.py:183-189): executed behind the reads
-            compiler_fence();
-            lds_set(tail + (h - 1u), s + 1u);
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if constexpr (DT != DT_BYTES) x[u] = Role::reduce ? ll_comp<DT>(x[u], r[u]) : r[u];
-                else x[u] = r[u];
-            }
-        }
-        if (Role::send) {
-            wait_for(tail + h, s + 1u - (uint32_t)NS, tail_seen, s);
-            compiler_fence();
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                *reinterpret_cast<MINT_LDS u32x4*>(tx + slot + (uint32_t)u * kBlockRawSimple) = x[u];
-            compiler_fence();
-            lds_set(head + h, s + 1u);
-        }
-    };
-    uint32_t s = 0;
-    auto step = [&](auto phase) MINT_INLINE_LAMBDA {
-        constexpr int B = decltype(phase)::value;
-        u32x4 x[U];
-        pass_on(s, v[B], x);
-        if (Role::save) {
-            const uint32_t g = (s * C + c) * (uint32_t)U;
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (U == 1 || g + (uint32_t)u < k.nfull)
-                    st128_row(out_row + (uint64_t)(g + (uint32_t)u) * kBlockRawSimple + lane_off, x[u]);
-        }
-        if (Role::load) {
-            compiler_fence();
-            fetch(s + (uint32_t)D, v[B]);
-        }
-        ++s;
-    };
-    if (rest >= 3u) step(std::integral_constant<int, 1>{});
-    if (rest >= 2u) step(std::integral_constant<int, 2>{});
-    if (rest >= 1u) step(std::integral_constant<int, 3>{});
-    while (s != k.steps) {
-        step(std::integral_constant<int, 0>{});
-        step(std::integral_constant<int, 1>{});
-        step(std::integral_constant<int, 2>{});
-        step(std::integral_constant<int, 3>{});
-    }
-    if (k.tail) {
-        // fewer than 1 KiB, byte by byte where a lane's 16 are not all there
-        u32x4 own[U], x[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) own[u] = u32x4{0u, 0u, 0u, 0u};
-        const uint64_t off = (uint64_t)k.nfull * kBlockRawSimple + lane_off;
-        if (Role::load) own[0] = load_guarded(in_row, off, 16u, k.row_bytes);
-        pass_on(k.steps, own, x);
-        if (Role::save) store_guarded(out_row, off, 16u, k.row_bytes, x[0]);
-    }
-    if (failed_at != ~0u) report_timeout(a.status, (int)p, (int)h, (int)c, failed_at);
-    // a launch that finds the abort flag set is counted, as in take_seat
-    if (!Role::recv) count_launch_if_aborted(a.status, (int)h);
+    for (int i = 0; i < N; ++i) asm volatile("" : "+s"(x[i]));
 }
 
-// One thread block per channel: wavefront h is position h (the roles: role_of).
-template <int DT, int U, int NS, int D>
-__global__ void __launch_bounds__((2 * kMaxRanks - 1) * 64) cu_ring_kernel(const CuRingArgs a) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    MINT_LDS uint8_t* lds = (MINT_LDS uint8_t*)lds_raw;
-    const uint32_t h = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)wave_in_block());
-    const uint32_t c = blockIdx.x / a.pipes, p = blockIdx.x - c * a.pipes;
-    uint32_t row_in = p, row_out = p, idx;
-    if (a.op == OP_ALLTOALL) {
-        // pipeline source * len + destination
-        row_out = p / a.len;
-        row_in = p - row_out * a.len;
-        idx = h == 0u ? row_out : row_in;
-    } else {
-        idx = (uint32_t)(a.starts >> (8u * p)) & 0xFFu;
-        idx += h;
-        while (idx >= a.len) idx -= a.len;
-    }
-    const uint8_t* in_row = reinterpret_cast<const uint8_t*>(a.input[idx]) + (uint64_t)row_in * a.row_stride;
-    uint8_t* out_row = reinterpret_cast<uint8_t*>(a.output[idx]) + (uint64_t)row_out * a.row_stride;
-    const bool sink = h == a.hops, allreduce = a.op == OP_ALLREDUCE;
-    if (h == 0u) {
-        cu_walk<DT, U, NS, D>(a, p, h, c, in_row, out_row, lds, CuRole<true, false, false, false, true>{});
+#define CU_SHAPE uint64_t starts, uint64_t row_bytes, uint64_t row_stride, uint64_t short_bytes, uint32_t full, uint32_t tiles
+
+// Rings that add: N ranks, the sum goes to the root of the pipeline (reduce,
+// reduce-scatter) or, EVERYWHERE, to all of them (allreduce).
+template <int DT, int N, bool EVERYWHERE, bool LARGE>
+__global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(CU_SHAPE, const CuTables a) {
+    const CuShape shape = {starts, row_bytes, row_stride, short_bytes, full, tiles};
+    constexpr uint32_t kSize = DT == DT_F32 ? 4u : 2u, kThreads = cu_threads(LARGE, false), kTile = kThreads * 16u;
+    const uint32_t tile = LARGE ? blockIdx.x : blockIdx.y, p = LARGE ? blockIdx.y : blockIdx.x;
+    const uint32_t root = (uint32_t)(starts >> (8u * p)) & 0xFFu;
+    const uint64_t row_off = (uint64_t)p * row_stride;
+    constexpr int kStored = EVERYWHERE ? N : 1;
+    const uint8_t* from[N];
+    uint8_t* to[kStored];
+    cu_addresses(a.input + root, from);
+    cu_addresses(a.output + root, to);
+    cu_here(from);
+    cu_here(to);
+    const CuRow row(shape, p, to[0] + row_off, kSize);
+    cu_count_if_aborted<kThreads>(a.status);
+    if (__builtin_expect(tile == tiles, 0)) {
+        uint64_t off;
+        if (!row.end_element(kSize, off)) return;
+        uint32_t v[N];
+#pragma unroll
+        for (int h = 0; h < N; ++h) v[h] = cu_load_element<DT>(from[h] + row_off + off);
+        uint32_t x = v[0];
+#pragma unroll
+        for (int h = 1; h < N; ++h) x = add_rn<DT>(v[h], x);
+#pragma unroll
+        for (int h = 0; h < kStored; ++h) cu_store_element<DT>(to[h] + row_off + off, x);
         return;
     }
-    if constexpr (DT != DT_BYTES) {
-        if (allreduce ? h < a.len : !sink) {
-            if (allreduce && h == a.len - 1u)
-                cu_walk<DT, U, NS, D>(a, p, h, c, in_row, out_row, lds, CuRole<true, true, true, true, true>{});
-            else
-                cu_walk<DT, U, NS, D>(a, p, h, c, in_row, out_row, lds, CuRole<true, true, true, false, true>{});
-            return;
-        }
+    const uint32_t lane = threadIdx.x * 16u;
+    for (uint64_t t = tile; t * kTile < row.bytes + row.shift; t += tiles) {
+        // (a uniform part and a lane's: scalar base and 32-bit offset of one instruction)
+        const int64_t base = (int64_t)(t * kTile) - row.shift;
+        if (!row.whole(base + lane)) continue;
+        u32x4 v[N];
+#pragma unroll
+        for (int h = 0; h < N; ++h) v[h] = cu_load<LARGE>(from[h] + ((int64_t)row_off + base), lane);
+        u32x4 x = v[0];
+#pragma unroll
+        for (int h = 1; h < N; ++h) x = ll_comp<DT>(v[h], x);
+#pragma unroll
+        for (int h = 0; h < kStored; ++h) cu_store<LARGE || !EVERYWHERE>(to[h] + ((int64_t)row_off + base), lane, x);
     }
-    if (sink)
-        cu_walk<DT, U, NS, D>(a, p, h, c, in_row, out_row, lds, CuRole<false, true, false, true, false>{});
-    else if (a.op == OP_SENDRECV)
-        cu_walk<DT, U, NS, D>(a, p, h, c, in_row, out_row, lds, CuRole<false, true, false, false, true>{});
-    else
-        cu_walk<DT, U, NS, D>(a, p, h, c, in_row, out_row, lds, CuRole<false, true, false, true, true>{});
 }
+
+// Rings and routes that copy: a row of the root to the COPIES positions behind
+// it: the last one (sendrecv) or every other one (broadcast, allgather).
+// ALLTOALL: row `destination` of the source goes to row `source` of the
+// destination, and the tables are by rank.
+template <int COPIES, bool ALLTOALL, bool LARGE>
+__global__ void __launch_bounds__(cu_threads(LARGE, (COPIES > 1))) cu_ring_copy_kernel(CU_SHAPE, const CuTables a) {
+    const CuShape shape = {starts, row_bytes, row_stride, short_bytes, full, tiles};
+    constexpr uint32_t kThreads = cu_threads(LARGE, COPIES > 1), kTile = kThreads * 16u;
+    const uint32_t tile = LARGE ? blockIdx.x : blockIdx.y, p = LARGE ? blockIdx.y : blockIdx.x;
+    const uint32_t root = ALLTOALL ? blockIdx.z : (uint32_t)(starts >> (8u * p)) & 0xFFu;
+    const uint64_t in_off = (uint64_t)p * row_stride, out_off = (uint64_t)(ALLTOALL ? root : p) * row_stride;
+    const uint8_t* from[1];
+    uint8_t* to[COPIES];
+    cu_addresses(a.input + root, from);
+    cu_addresses(a.output + (ALLTOALL ? p : root + 1u), to);
+    cu_here(from);
+    cu_here(to);
+    const CuRow row(shape, p, to[0] + out_off, 1u);
+    cu_count_if_aborted<kThreads>(a.status);
+    if (__builtin_expect(tile == tiles, 0)) {
+        uint64_t off;
+        if (!row.end_element(1u, off)) return;
+        const uint8_t x = as_global(from[0])[in_off + off];
+#pragma unroll
+        for (int k = 0; k < COPIES; ++k) as_global(to[k])[out_off + off] = x;
+        return;
+    }
+    const uint32_t lane = threadIdx.x * 16u;
+    for (uint64_t t = tile; t * kTile < row.bytes + row.shift; t += tiles) {
+        const int64_t base = (int64_t)(t * kTile) - row.shift;
+        if (!row.whole(base + lane)) continue;
+        const u32x4 x = cu_load<LARGE && COPIES == 1>(from[0] + ((int64_t)in_off + base), lane);
+#pragma unroll
+        for (int k = 0; k < COPIES; ++k) cu_store<LARGE || COPIES == 1>(to[k] + ((int64_t)out_off + base), lane, x);
+    }
+}
+
+#undef CU_SHAPE
 
 }  // namespace mint

@@ -60,42 +60,90 @@ static_assert(MINT_OP_TREE_BROADCAST == OP_TREE_BROADCAST && MINT_OP_TREE_REDUCE
                   MINT_OP_HYPERCUBE_ALLGATHER == OP_HYPER_ALLGATHER,
               "op codes");
 
-// The grid of a launch inside compute units (cu_ring.hpp): one thread block per
-// channel, one wavefront per position.
+// The wavefronts that a compute unit is to hold of the large form of a launch
+// inside compute units (cu_ring.hpp; one copy of a row: all 32).  Some 64 KiB
+// of rows on their way to or from a compute unit keep HBM busy: fewer
+// wavefronts leave it idle, more only scatter its accesses.  Each holds a KiB of
+// N rows to be added, of a row that goes to N - 1 others, or (allreduce) of N rows
+// and then N results.  Fastest counts on MI355X at 0.25 - 2 GiB, f16, bf16 and
+// f32, for N = 2 / 3 / 4 / 5 / 6 / 7 / 8: reduce-scatter 20 / 14 / 12 / 11 / 10 / 9 /
+// 9, allreduce 16 / 10 / 8 / 5 - 7 / 5 - 6 / 5 / 4 - 5, allgather 32 / 18 / 16 / 10 /
+// 10 / - / 8; one or two off is 1 - 3 % slower, but twice as many 5 - 20 %.
+int cu_waves(int op, int ranks) {
+    if (op == OP_ALLREDUCE) return 32 / ranks + 1;
+    if (reducing(op)) return 24 / ranks + 6;
+    return 64 / ranks;
+}
+
+// The grid of a launch inside compute units: a thread block per tile of a row,
+// one 16-byte vector per thread.
 int plan_cu(Plan* plan) {
     const RingArgs& a = plan->args;
-    const uint64_t nfull = a.row_bytes / kBlockRawSimple;
-    if (nfull >= (1ull << 31)) return MINT_ERR_TOO_LARGE;
-    constexpr uint64_t kCus = (uint64_t)kXcds * kCusPerXcd;
-    // (4 KiB per step where nothing is added)
-    const bool copying = !reducing(a.op);
-    plan->unroll = copying && nfull / 4 * (uint64_t)a.pipes >= 4 * kCus ? 4 : 1;
-    const uint64_t units = (nfull + plan->unroll - 1) / plan->unroll + (a.row_bytes % kBlockRawSimple ? 1 : 0);
-    const uint64_t per_cu = a.hops == 1 ? 4 : 2;
-    uint64_t channels = per_cu * kCus / (uint64_t)a.pipes;
-    if (channels > units) channels = units ? units : 1;
-    plan->blocks = (int)channels * a.pipes;
-    plan->threads = (a.hops + 1) * 64;
-    CuRingArgs& c = plan->cu_args;
-    for (int i = 0; i < a.cyc_len; ++i) {
-        // (alltoall names ranks, not places on a ring)
-        const int rank = a.op == OP_ALLTOALL ? i : a.cyc[i];
-        c.input[i] = a.input[rank];
-        c.output[i] = a.output[rank];
+    const bool sums = reducing(a.op), alltoall = a.op == OP_ALLTOALL;
+    const bool copies = (a.op == OP_BROADCAST || a.op == OP_ALLGATHER) && a.cyc_len > 2;
+    // Large: the last-level cache (256 MiB) would not hold the rows from one use
+    // to the next.  Measured with three such sets of buffers in turn, the two
+    // forms meet at 64 - 128 MiB, where rows are only copied once at 128 - 256
+    // (8 ranks: reduce-scatter of 64 MiB 11.0 us small / 15.5 large, 128 MiB
+    // 28.6 / 26.9; alltoall of 128 MiB 17.0 / 24.5, 256 MiB 45.2 / 43.3).
+    const uint64_t touched = (uint64_t)a.pipes * a.row_bytes *
+                             (alltoall || a.op == OP_SENDRECV ? 2u : (uint64_t)a.cyc_len);
+    plan->cu_large = touched > ((uint64_t)(sums || copies ? 96 : 192) << 20);
+    plan->threads = (int)cu_threads(plan->cu_large, copies);
+    // (held to that number by the share of LDS its blocks ask for; LDS is handed
+    // out in units of 1280 bytes)
+    plan->cu_lds = 0;
+    if (plan->cu_large && (sums || copies)) {
+        const int blocks = cu_waves(a.op, a.cyc_len) / (plan->threads / 64);
+        if (blocks * (plan->threads / 64) < 32) plan->cu_lds = (160 << 10) / blocks / 1280 * 1280;
     }
-    c.starts = 0;
-    if (a.op != OP_ALLTOALL)
-        for (int p = 0; p < a.pipes; ++p) c.starts |= (uint64_t)a.start[p] << (8 * p);
-    c.row_bytes = a.row_bytes;
-    c.row_stride = a.row_stride;
-    c.total_bytes = a.total_bytes;
-    c.status = a.status;
+    CuRingArgs& c = plan->cu_args;
     c.op = (uint32_t)a.op;
     c.pipes = (uint32_t)a.pipes;
     c.len = (uint32_t)a.cyc_len;
-    c.hops = (uint32_t)a.hops;
-    c.channels = (uint32_t)channels;
-    c.spin_budget = a.spin_budget;
+    uint64_t stored = 0;           // what the stored rows' addresses have in their low bits
+    if (a.op == OP_SENDRECV) {
+        // a route: only its ends touch the caller's buffers
+        c.len = 2;
+        c.tables.input[0] = a.input[a.cyc[0]];
+        stored = c.tables.output[1] = a.output[a.cyc[a.cyc_len - 1]];
+    } else {
+        for (int i = 0; i < a.cyc_len; ++i) {
+            // (alltoall names ranks, not places on a ring)
+            const int rank = alltoall ? i : a.cyc[i];
+            c.tables.input[i] = c.tables.input[a.cyc_len + i] = a.input[rank];
+            c.tables.output[i] = c.tables.output[a.cyc_len + i] = a.output[rank];
+            stored |= a.output[rank];
+        }
+    }
+    c.tables.status = a.status;
+    CuShape& s = c.shape;
+    s.starts = 0;
+    if (!alltoall)
+        for (int p = 0; p < a.pipes; ++p) s.starts |= (uint64_t)a.start[p] << (8 * p);
+    s.row_bytes = a.row_bytes;
+    s.row_stride = a.pipes > 1 ? a.row_stride : 0;
+    s.full = (uint32_t)a.pipes;
+    s.short_bytes = 0;
+    if (a.total_bytes && a.row_stride) {
+        // rows cut from one buffer: those that end inside it, then a shorter one
+        const uint64_t whole = a.total_bytes < a.row_bytes ? 0 : (a.total_bytes - a.row_bytes) / a.row_stride + 1;
+        if (whole < (uint64_t)a.pipes) {
+            s.full = (uint32_t)whole;
+            const uint64_t off = whole * a.row_stride;
+            s.short_bytes = a.total_bytes > off ? a.total_bytes - off : 0;
+        }
+    }
+    stored |= s.row_stride;
+    // a row's first tile may start up to 127 bytes before it (CuRow::shift)
+    const uint64_t tile = (uint64_t)plan->threads * 16, slack = stored & 127 ? 127 : 0;
+    uint64_t tiles = (a.row_bytes + slack + tile - 1) / tile;
+    // (a launch is at most 2^32 - 1 threads; beyond that the blocks take several tiles each)
+    const uint64_t most = ((1ull << 31) / plan->threads) / (uint64_t)a.pipes;
+    if (tiles > most) tiles = most;
+    s.tiles = (uint32_t)tiles;
+    c.ends = ((stored | a.row_bytes | s.short_bytes) & 15) != 0;
+    plan->blocks = (int)(s.tiles + c.ends) * a.pipes;
     plan->lds = false;
     plan->staging_need = 0;
     return MINT_OK;

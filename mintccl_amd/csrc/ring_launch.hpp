@@ -17,10 +17,12 @@ struct Plan {
     int blocks_plain;         // the grid without CUs set apart for origins (args.origin_cus)
     size_t staging_need;      // bytes of staging per rank: slots + credit words
     bool empty;
-    bool cu;                  // rings inside compute units: `cu_args` instead of `args`
-    CuRingArgs cu_args;
     bool lds;                 // own rows through LDS: `threads` counts the wave-channels'
                               // threads only, the launch adds the fetcher wavefront
+    bool cu;                  // rings inside compute units: `cu_args` instead of `args`
+    CuRingArgs cu_args;
+    bool cu_large;            // which form of the kernels
+    int cu_lds;               // bytes of LDS per block, to bound how many a compute unit holds
 };
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? MINT_OK : MINT_ERR_HIP; }

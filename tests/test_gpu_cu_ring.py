@@ -1,8 +1,8 @@
 """Rings inside compute units (what the operators run when nothing about the
 wire is named): rows around every edge of the walk - less than a lane's 16
-bytes, around one 1 KiB block, around the rounds of four steps, one channel
-more or less than a grid holds, around the size from which the copying
-collectives move 4 KiB per step - bit for bit against the oracle."""
+bytes, around a wavefront's 1 KiB and a tile's 2, at any byte, in both forms of
+the kernels - bit for bit against the oracle or, for the large rows, against the
+same additions in torch."""
 import numpy as np
 import pytest
 import torch
@@ -13,7 +13,7 @@ from tests.helpers import as_bytes, rank_rows
 pytestmark = pytest.mark.gpu
 
 # bytes of a row (even: whole f16 values)
-ROWS = [2, 14, 16, 18, 1022, 1024, 1026, 3 * 1024, 4 * 1024 + 2, 64 * 1024 - 2, 65 * 1024 + 16,
+ROWS = [2, 14, 16, 18, 1022, 1024, 1026, 2046, 2050, 3 * 1024, 4 * 1024 - 2, 4 * 1024 + 2, 64 * 1024 - 2, 65 * 1024 + 16,
         5 * 64 * 1024 + 1040, 7 * 64 * 1024 - 6]
 
 
@@ -24,7 +24,8 @@ def make_comm(world, **kw):
     return comm
 
 
-@pytest.mark.parametrize("world,dt", [(8, "f16"), (8, "bf16"), (8, "f32"), (3, "f16"), (2, "bf16")])
+@pytest.mark.parametrize("world,dt", [(8, "f16"), (8, "bf16"), (8, "f32"), (7, "bf16"), (6, "f32"), (5, "f16"),
+                                      (4, "bf16"), (3, "f16"), (2, "bf16")])
 def test_reducing_rows(dev, world, dt):
     from mintccl_amd.allreduce import allreduce
     from mintccl_amd.reduce import reduce
@@ -52,7 +53,7 @@ def test_reducing_rows(dev, world, dt):
 
 
 @pytest.mark.parametrize("world", [2, 3, 8])
-@pytest.mark.parametrize("nbytes", ROWS + [4 << 20, (4 << 20) - 1, (4 << 20) + 4097, (9 << 20) + 5 * 1024 + 3])
+@pytest.mark.parametrize("nbytes", ROWS + [(4 << 20) + 4097, (8 << 20) - 1, (9 << 20) + 5 * 1024 + 3])
 def test_copying_rows(dev, world, nbytes):
     from mintccl_amd import sendrecv_buffer
     from mintccl_amd.allgather import allgather
@@ -83,7 +84,7 @@ def test_copying_rows(dev, world, nbytes):
         assert torch.equal(flat[r].cpu(), host[world - 1][world - 1]), r
 
 
-@pytest.mark.parametrize("shift", [1, 3, 8])
+@pytest.mark.parametrize("shift", [1, 3, 8, 16, 30])
 def test_rows_at_any_byte_touch_nothing_else(dev, shift):
     from mintccl_amd import _lib
     from mintccl_amd.broadcast import broadcast
@@ -110,23 +111,72 @@ def test_rows_at_any_byte_touch_nothing_else(dev, shift):
         assert torch.all(backing[r][:shift] == 0x5A) and torch.all(backing[r][shift + world * n * 2:] == 0x5A)
 
 
-def test_a_wait_that_runs_out_is_reported_and_the_grid_drains(dev):
-    """A spin limit of one poll: the positions behind the origin find nothing in
-    their first slot - the row is still on its way from HBM - and say so."""
+@pytest.mark.parametrize("world,dt", [(8, "bf16"), (7, "f16"), (5, "f32"), (3, "f16"), (2, "f32")])
+def test_rows_beyond_the_cache(dev, world, dt):
+    """The large form (more than 96 MiB touched), buffers that start 6 or 12 bytes
+    behind a 16-byte boundary and rows that end in the middle of a vector."""
+    from mintccl_amd.allgather import allgather
+    from mintccl_amd.allreduce import allreduce
+    from mintccl_amd.broadcast import broadcast
+    from mintccl_amd.reduce import reduce
+    from mintccl_amd.reducescatter import reducescatter
+    dtype = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[dt]
+    comm = make_comm(world)
+    n = (100 << 20) // (world * world * dtype.itemsize) + 13
+    g = torch.Generator(device=dev).manual_seed(world)
+    made = [torch.randn(world * n + 3, generator=g, device=dev, dtype=dtype)[3:] for _ in range(world)]
+    total = made[0].numel()
+    per = (-(-total * dtype.itemsize // world) + 15) // 16 * 16 // dtype.itemsize     # a chunk of the allreduce
+
+    def summed(start, lo, hi):
+        x = made[start][lo:hi]
+        for h in range(1, world):
+            x = made[(start + h) % world][lo:hi] + x
+        return x
+
+    def run(op):
+        bufs = [torch.empty(total + 3, device=dev, dtype=dtype)[3:].copy_(m) for m in made]
+        comm.run(lambda r: op(bufs[r]))
+        comm.check()
+        return bufs
+
+    def same(a, b):
+        return torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+    scattered = run(lambda b: reducescatter(b.view(world, n), comm))
+    reduced = run(lambda b: reduce(b, world - 1, comm))
+    everywhere = run(lambda b: allreduce(b, comm))
+    gathered = run(lambda b: allgather(b.view(world, n), comm))
+    cast = run(lambda b: broadcast(b, world - 1, comm))
+    want = torch.cat([summed(c, c * per, min(total, (c + 1) * per)) for c in range(world)])
+    rows = torch.cat([made[r][r * n: (r + 1) * n] for r in range(world)])
+    for r in range(world):
+        own = made[r].clone()
+        own[r * n: (r + 1) * n] = summed(r, r * n, (r + 1) * n)
+        assert same(scattered[r], own), r
+        assert same(reduced[r], summed(r, 0, total) if r == world - 1 else made[r]), r
+        assert same(everywhere[r], want) and same(gathered[r], rows) and same(cast[r], made[world - 1]), r
+
+
+def test_nothing_waits(dev):
+    """A spin limit of one poll, and the abort flag of an earlier launch: the
+    launch has nobody to wait for, runs all the same and is counted."""
     from mintccl_amd.broadcast import broadcast
     from mintccl_amd.common import RingTimeout
     world, n = 8, 1 << 22
     comm = make_comm(world)
     comm.spin_budget = 1
     host = torch.randint(0, 256, (n,), dtype=torch.uint8, generator=torch.Generator().manual_seed(1))
-    bufs = [host.to(dev) if r == 0 else torch.zeros(n, dtype=torch.uint8, device=dev) for r in range(world)]
-    comm.run(lambda r: broadcast(bufs[r], 0, comm))
-    with pytest.raises(RingTimeout):
-        comm.check()
-    comm.spin_budget = 400000
-    comm.run(lambda r: broadcast(bufs[r], 0, comm))
-    comm.check()
-    assert all(torch.equal(b.cpu(), host) for b in bufs)
+    for flag in (0, 1):
+        bufs = [host.to(dev) if r == 0 else torch.zeros(n, dtype=torch.uint8, device=dev) for r in range(world)]
+        comm.status[0] = comm.status[3] = flag
+        comm.run(lambda r: broadcast(bufs[r], 0, comm))
+        if flag:
+            with pytest.raises(RingTimeout, match="1 later launch"):
+                comm.check()
+        else:
+            comm.check()
+        assert all(torch.equal(b.cpu(), host) for b in bufs)
 
 
 def test_naming_anything_about_the_wire_goes_through_staging(dev, monkeypatch):
