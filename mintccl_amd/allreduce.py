@@ -26,6 +26,8 @@ from . import _lib
 from ._ops import ring_of
 from .common import VirtualComm, get_comm
 
+_KIND = _lib.KIND_ALLREDUCE
+
 
 # Through staging, two launches are faster than one pass from this size per rank
 # on (measured on MI355X, 8 ranks, f16: 104 / 110 us at 16 MiB, 199 / 192 at 32 MiB, 1510 /
@@ -43,7 +45,7 @@ def chunk_bytes(count: int, world: int) -> int:
 def allreduce(buff: torch.Tensor, comm: VirtualComm | None = None,
               fused: bool | None = None) -> None:
     comm = comm if comm is not None else get_comm()
-    posted = comm._board.post(_lib.KIND_ALLREDUCE, buff, 0, -1 if fused is None else int(bool(fused)))
+    posted = comm._post(_KIND, buff, 0, -1 if fused is None else int(bool(fused)))
     if posted is None:               # not all ranks are here yet, or launched
         return
     count, dtype, _, variant, ptrs, _, _ = posted

@@ -14,10 +14,12 @@ from . import _lib
 from ._ops import ring_of
 from .common import VirtualComm, get_comm
 
+_KIND = _lib.KIND_ALLTOALL
+
 
 def alltoall(buff: torch.Tensor, out: torch.Tensor, comm: VirtualComm | None = None) -> None:
     comm = comm if comm is not None else get_comm()
-    posted = comm._board.post(_lib.KIND_ALLTOALL, buff, 0, -1, out)
+    posted = comm._post(_KIND, buff, 0, -1, out)
     if posted is None:               # not all ranks are here yet, or launched
         return
     count, _, _, _, ins, outs, _ = posted

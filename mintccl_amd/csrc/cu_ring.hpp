@@ -36,22 +36,31 @@ namespace mint {
 // has the hardware put into scalar registers before the first instruction
 // (kernarg preload), and one round of scalar loads brings the addresses.
 struct CuShape {
-    uint64_t starts;               // byte p: index in the ring of pipeline p's root
     uint64_t row_bytes, row_stride;
     uint64_t short_bytes;          // bytes of row `full`; rows behind it are empty
+    uint32_t starts;               // bits 3 p: index in the ring of pipeline p's root
     uint32_t full;                 // rows before this one have row_bytes
     uint32_t tiles;                // thread blocks that share the whole vectors of a row
 };
-// The ranks' buffers in the order of the ring (or route), twice over, so that
-// those of a pipeline that starts at index i are the `len` entries from i on.
+#define CU_SHAPE uint64_t row_bytes, uint64_t row_stride, uint64_t short_bytes, uint32_t starts, uint32_t full, uint32_t tiles
+
+// The ranks' buffers in the order of the ring.  One address per rank where they
+// work in place, as the operators do: a launch with up to 112 bytes of arguments
+// takes the host 2.6 us, one with more 3.3.  SPLIT: N addresses to load from, then
+// N to store to.
+template <int N, bool SPLIT>
 struct CuTables {
-    uint64_t input[2 * kMaxRanks], output[2 * kMaxRanks];
+    uint64_t rank[SPLIT ? 2 * N : N];
     uint64_t* status;
 };
+static_assert(sizeof(CuShape) + sizeof(CuTables<kMaxRanks, false>) <= 112, "arguments of a launch in place");
+// (host side: the whole of a launch)
 struct CuRingArgs {
     CuShape shape;
-    CuTables tables;
+    uint64_t input[kMaxRanks], output[kMaxRanks];
+    uint64_t* status;
     uint32_t op, pipes, len, ends;
+    bool split;
 };
 
 // Two forms of a launch (which: plan_cu in mintccl.hip).
@@ -94,8 +103,9 @@ __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 
 struct CuRow {
     uint64_t bytes;
     uint32_t shift;
-    __device__ __forceinline__ CuRow(const CuShape& a, uint32_t p, const uint8_t* stored, uint32_t size) {
-        bytes = p < a.full ? a.row_bytes : p == a.full ? a.short_bytes : 0u;
+    __device__ __forceinline__ CuRow(uint64_t row_bytes, uint64_t short_bytes, uint32_t full, uint32_t p,
+                                     const uint8_t* stored, uint32_t size) {
+        bytes = p < full ? row_bytes : p == full ? short_bytes : 0u;
         // (whole elements: a row may start at any byte)
         shift = (uint32_t)(uintptr_t)stored & 127u & ~(size - 1u);
     }
@@ -137,39 +147,36 @@ __device__ __forceinline__ void cu_store_element(uint8_t* p, uint32_t v) {
     else *(MINT_GLOBAL u16_unaligned*)p = (uint16_t)v;
 }
 
-// The next addresses of a table, and a point where they have to be there: the
-// compiler would fetch each where it is first used, a scalar load and a wait at
-// a time.
-template <int N, typename P>
-__device__ __forceinline__ void cu_addresses(const uint64_t* table, P* (&x)[N]) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) x[i] = reinterpret_cast<P*>(table[i]);
-}
+// Where the addresses have to be there: the compiler would fetch each where it is
+// first used, a scalar load and a wait at a time.
 template <int N, typename P>
 __device__ __forceinline__ void cu_here(P* (&x)[N]) {
 #pragma unroll
     for (int i = 0; i < N; ++i) asm volatile("" : "+s"(x[i]));
 }
 
-#define CU_SHAPE uint64_t starts, uint64_t row_bytes, uint64_t row_stride, uint64_t short_bytes, uint32_t full, uint32_t tiles
-
 // Rings that add: N ranks, the sum goes to the root of the pipeline (reduce,
 // reduce-scatter) or, EVERYWHERE, to all of them (allreduce).
-template <int DT, int N, bool EVERYWHERE, bool LARGE>
-__global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(CU_SHAPE, const CuTables a) {
-    const CuShape shape = {starts, row_bytes, row_stride, short_bytes, full, tiles};
+template <int DT, int N, bool EVERYWHERE, bool LARGE, bool SPLIT>
+__global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(CU_SHAPE, const CuTables<N, SPLIT> a) {
     constexpr uint32_t kSize = DT == DT_F32 ? 4u : 2u, kThreads = cu_threads(LARGE, false), kTile = kThreads * 16u;
     const uint32_t tile = LARGE ? blockIdx.x : blockIdx.y, p = LARGE ? blockIdx.y : blockIdx.x;
-    const uint32_t root = (uint32_t)(starts >> (8u * p)) & 0xFFu;
+    const uint32_t root = starts >> (3u * p) & 7u;
     const uint64_t row_off = (uint64_t)p * row_stride;
-    constexpr int kStored = EVERYWHERE ? N : 1;
+    constexpr int kStored = EVERYWHERE ? N : 1, kOut = SPLIT ? N : 0;
     const uint8_t* from[N];
     uint8_t* to[kStored];
-    cu_addresses(a.input + root, from);
-    cu_addresses(a.output + root, to);
+    uint32_t idx = root;
+#pragma unroll
+    for (int h = 0; h < N; ++h) {
+        from[h] = reinterpret_cast<const uint8_t*>(a.rank[idx]);
+        idx = idx + 1u == (uint32_t)N ? 0u : idx + 1u;
+    }
+#pragma unroll
+    for (int i = 0; i < kStored; ++i) to[i] = reinterpret_cast<uint8_t*>(a.rank[kOut + (EVERYWHERE ? (uint32_t)i : root)]);
     cu_here(from);
     cu_here(to);
-    const CuRow row(shape, p, to[0] + row_off, kSize);
+    const CuRow row(row_bytes, short_bytes, full, p, to[0] + row_off, kSize);
     cu_count_if_aborted<kThreads>(a.status);
     if (__builtin_expect(tile == tiles, 0)) {
         uint64_t off;
@@ -181,7 +188,7 @@ __global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(C
 #pragma unroll
         for (int h = 1; h < N; ++h) x = add_rn<DT>(v[h], x);
 #pragma unroll
-        for (int h = 0; h < kStored; ++h) cu_store_element<DT>(to[h] + row_off + off, x);
+        for (int i = 0; i < kStored; ++i) cu_store_element<DT>(to[i] + row_off + off, x);
         return;
     }
     const uint32_t lane = threadIdx.x * 16u;
@@ -196,45 +203,68 @@ __global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(C
 #pragma unroll
         for (int h = 1; h < N; ++h) x = ll_comp<DT>(v[h], x);
 #pragma unroll
-        for (int h = 0; h < kStored; ++h) cu_store<LARGE || !EVERYWHERE>(to[h] + ((int64_t)row_off + base), lane, x);
+        for (int i = 0; i < kStored; ++i) cu_store<LARGE || !EVERYWHERE>(to[i] + ((int64_t)row_off + base), lane, x);
     }
 }
 
-// Rings and routes that copy: a row of the root to the COPIES positions behind
-// it: the last one (sendrecv) or every other one (broadcast, allgather).
-// ALLTOALL: row `destination` of the source goes to row `source` of the
-// destination, and the tables are by rank.
-template <int COPIES, bool ALLTOALL, bool LARGE>
-__global__ void __launch_bounds__(cu_threads(LARGE, (COPIES > 1))) cu_ring_copy_kernel(CU_SHAPE, const CuTables a) {
-    const CuShape shape = {starts, row_bytes, row_stride, short_bytes, full, tiles};
-    constexpr uint32_t kThreads = cu_threads(LARGE, COPIES > 1), kTile = kThreads * 16u;
-    const uint32_t tile = LARGE ? blockIdx.x : blockIdx.y, p = LARGE ? blockIdx.y : blockIdx.x;
-    const uint32_t root = ALLTOALL ? blockIdx.z : (uint32_t)(starts >> (8u * p)) & 0xFFu;
-    const uint64_t in_off = (uint64_t)p * row_stride, out_off = (uint64_t)(ALLTOALL ? root : p) * row_stride;
-    const uint8_t* from[1];
-    uint8_t* to[COPIES];
-    cu_addresses(a.input + root, from);
-    cu_addresses(a.output + (ALLTOALL ? p : root + 1u), to);
-    cu_here(from);
-    cu_here(to);
-    const CuRow row(shape, p, to[0] + out_off, 1u);
-    cu_count_if_aborted<kThreads>(a.status);
+// A row from one place to COPIES others.
+template <int COPIES, bool LARGE>
+__device__ __forceinline__ void cu_copy_row(const CuRow& row, uint32_t tile, uint32_t tiles, const uint8_t* in,
+                                            uint8_t* const (&out)[COPIES]) {
+    constexpr uint32_t kTile = cu_threads(LARGE, COPIES > 1) * 16u;
     if (__builtin_expect(tile == tiles, 0)) {
         uint64_t off;
         if (!row.end_element(1u, off)) return;
-        const uint8_t x = as_global(from[0])[in_off + off];
+        const uint8_t x = as_global(in)[off];
 #pragma unroll
-        for (int k = 0; k < COPIES; ++k) as_global(to[k])[out_off + off] = x;
+        for (int k = 0; k < COPIES; ++k) as_global(out[k])[off] = x;
         return;
     }
     const uint32_t lane = threadIdx.x * 16u;
     for (uint64_t t = tile; t * kTile < row.bytes + row.shift; t += tiles) {
         const int64_t base = (int64_t)(t * kTile) - row.shift;
         if (!row.whole(base + lane)) continue;
-        const u32x4 x = cu_load<LARGE && COPIES == 1>(from[0] + ((int64_t)in_off + base), lane);
+        const u32x4 x = cu_load<LARGE && COPIES == 1>(in + base, lane);
 #pragma unroll
-        for (int k = 0; k < COPIES; ++k) cu_store<LARGE || COPIES == 1>(to[k] + ((int64_t)out_off + base), lane, x);
+        for (int k = 0; k < COPIES; ++k) cu_store<LARGE || COPIES == 1>(out[k] + base, lane, x);
     }
+}
+
+// Rings that copy: N ranks, the root's row to every other one (broadcast,
+// allgather).  A route is a ring of its two ends (sendrecv).
+template <int N, bool LARGE, bool SPLIT>
+__global__ void __launch_bounds__(cu_threads(LARGE, (N > 2))) cu_ring_copy_kernel(CU_SHAPE, const CuTables<N, SPLIT> a) {
+    const uint32_t tile = LARGE ? blockIdx.x : blockIdx.y, p = LARGE ? blockIdx.y : blockIdx.x;
+    const uint32_t root = starts >> (3u * p) & 7u;
+    const uint64_t row_off = (uint64_t)p * row_stride;
+    constexpr uint32_t kOut = SPLIT ? N : 0;
+    const uint8_t* from[1] = {reinterpret_cast<const uint8_t*>(a.rank[root])};
+    uint8_t* to[N - 1];
+#pragma unroll
+    for (int k = 0; k < N - 1; ++k)
+        to[k] = reinterpret_cast<uint8_t*>((uint32_t)k < root ? a.rank[kOut + k] : a.rank[kOut + k + 1]);
+    cu_here(from);
+    cu_here(to);
+    from[0] += row_off;
+#pragma unroll
+    for (int k = 0; k < N - 1; ++k) to[k] += row_off;
+    cu_count_if_aborted<cu_threads(LARGE, (N > 2))>(a.status);
+    cu_copy_row<N - 1, LARGE>(CuRow(row_bytes, short_bytes, full, p, to[0], 1u), tile, tiles, from[0], to);
+}
+
+// Row `destination` of the source goes to row `source` of the destination.
+template <bool LARGE>
+__global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_alltoall_kernel(CU_SHAPE, const CuTables<kMaxRanks, true> a) {
+    const uint32_t tile = LARGE ? blockIdx.x : blockIdx.y, p = LARGE ? blockIdx.y : blockIdx.x;
+    const uint32_t source = blockIdx.z;
+    const uint8_t* from[1] = {reinterpret_cast<const uint8_t*>(a.rank[source])};
+    uint8_t* to[1] = {reinterpret_cast<uint8_t*>(a.rank[kMaxRanks + p])};
+    cu_here(from);
+    cu_here(to);
+    from[0] += (uint64_t)p * row_stride;
+    to[0] += (uint64_t)source * row_stride;
+    cu_count_if_aborted<cu_threads(LARGE, false)>(a.status);
+    cu_copy_row<1, LARGE>(CuRow(row_bytes, short_bytes, full, p, to[0], 1u), tile, tiles, from[0], to);
 }
 
 #undef CU_SHAPE

@@ -104,6 +104,8 @@ struct Post {
 };
 struct Gathering {
     uint32_t present;
+    bool asked;                  // a rank of this collective has looked at the environment:
+    long env_variant;            // what it says (the others go by the same)
     Post post[MINT_MAX_RANKS];
 };
 struct Transfer {
@@ -322,13 +324,21 @@ PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
         if (n > 2) p.root = PyLong_AsLong(args[2]);
         if (n > 3) p.variant = PyLong_AsLong(args[3]);
         if (PyErr_Occurred()) return nullptr;
+        Gathering& g = b->gathering[kind];
+        bool asked = g.present && g.asked;
+        long env_variant = g.env_variant;
         if (info.elsewhere && p.variant == UNSAID) {
-            const char* e = getenv("MINTCCL_TOPOLOGY");
-            if (e && strcasecmp(e, info.elsewhere) == 0) Py_RETURN_FALSE;
-        }
-        if (kind == ALLGATHER && p.variant == UNSAID) {
-            const char* e = getenv("MINTCCL_ALLGATHER");
-            p.variant = !e || strcasecmp(e, "spatial") == 0 ? SPATIAL : strcasecmp(e, "temporal") == 0 ? TEMPORAL : 2;
+            if (!asked) {
+                const char* e = getenv("MINTCCL_TOPOLOGY");
+                if (e && strcasecmp(e, info.elsewhere) == 0) Py_RETURN_FALSE;
+                env_variant = UNSAID;
+                if (kind == ALLGATHER) {
+                    e = getenv("MINTCCL_ALLGATHER");
+                    env_variant = !e || strcasecmp(e, "spatial") == 0 ? SPATIAL : strcasecmp(e, "temporal") == 0 ? TEMPORAL : 2;
+                }
+                asked = true;
+            }
+            p.variant = env_variant;
         }
         if (kind == ALLGATHER && (p.variant < SPATIAL || p.variant > TEMPORAL))
             return raise(PyExc_ValueError, "allgather schedule is 'spatial' or 'temporal'");
@@ -351,7 +361,6 @@ PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
         }
         int rank;
         if (!rank_or_raise(b, &rank)) return nullptr;
-        Gathering& g = b->gathering[kind];
         if (g.present >> rank & 1u) {
             PyErr_Format(PyExc_RuntimeError, "rank %d called %s twice before the others joined", rank, info.name);
             return nullptr;
@@ -360,6 +369,8 @@ PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
         p.keep_out = n > 4 ? Py_NewRef(args[4]) : nullptr;
         g.post[rank] = p;
         g.present |= 1u << rank;
+        g.asked = asked;
+        g.env_variant = env_variant;
         if (g.present != (1u << b->world) - 1u) Py_RETURN_NONE;
         // (taken out before anything can call back or raise)
         Gathering all = g;

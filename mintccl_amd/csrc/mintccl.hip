@@ -101,26 +101,29 @@ int plan_cu(Plan* plan) {
     c.op = (uint32_t)a.op;
     c.pipes = (uint32_t)a.pipes;
     c.len = (uint32_t)a.cyc_len;
+    c.split = alltoall;
+    c.status = a.status;
     uint64_t stored = 0;           // what the stored rows' addresses have in their low bits
     if (a.op == OP_SENDRECV) {
         // a route: only its ends touch the caller's buffers
         c.len = 2;
-        c.tables.input[0] = a.input[a.cyc[0]];
-        stored = c.tables.output[1] = a.output[a.cyc[a.cyc_len - 1]];
+        c.input[0] = a.input[a.cyc[0]];
+        c.output[0] = c.input[1] = 0;
+        stored = c.output[1] = a.output[a.cyc[a.cyc_len - 1]];
     } else {
         for (int i = 0; i < a.cyc_len; ++i) {
             // (alltoall names ranks, not places on a ring)
             const int rank = alltoall ? i : a.cyc[i];
-            c.tables.input[i] = c.tables.input[a.cyc_len + i] = a.input[rank];
-            c.tables.output[i] = c.tables.output[a.cyc_len + i] = a.output[rank];
+            c.input[i] = a.input[rank];
+            c.output[i] = a.output[rank];
+            c.split |= a.input[rank] && a.output[rank] && a.input[rank] != a.output[rank];
             stored |= a.output[rank];
         }
     }
-    c.tables.status = a.status;
     CuShape& s = c.shape;
     s.starts = 0;
     if (!alltoall)
-        for (int p = 0; p < a.pipes; ++p) s.starts |= (uint64_t)a.start[p] << (8 * p);
+        for (int p = 0; p < a.pipes; ++p) s.starts |= (uint32_t)a.start[p] << (3 * p);
     s.row_bytes = a.row_bytes;
     s.row_stride = a.pipes > 1 ? a.row_stride : 0;
     s.full = (uint32_t)a.pipes;
@@ -292,7 +295,17 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
         if (!op->staging[r] || !aligned16(op->staging[r]))
             return op->staging[r] ? MINT_ERR_ALIGN : MINT_ERR_ARG;
     }
-    for (int p = 0; p < a.pipes && !plan->empty && !over_tree(op->op) && !temporal && !hyper; ++p) {
+    if (cu && !plan->empty) {
+        // (no staging: a rank has what it loads and what it stores)
+        const bool route = op->op == MINT_OP_SENDRECV, cast = op->op == MINT_OP_BROADCAST;
+        for (int i = 0; i < a.cyc_len; ++i) {
+            const bool root = i == a.start[0];
+            const bool load = root || !(route || cast);
+            const bool save = route ? i == a.cyc_len - 1 : cast ? !root : root || op->op != MINT_OP_REDUCE;
+            if ((load && !op->input[a.cyc[i]]) || (save && !op->output[a.cyc[i]])) return MINT_ERR_ARG;
+        }
+    }
+    for (int p = 0; p < a.pipes && !cu && !plan->empty && !over_tree(op->op) && !temporal && !hyper; ++p) {
         for (int h = 0; h <= a.hops; ++h) {
             const int rank = alltoall ? (h == 0 ? p / op->world : p % op->world)
                                       : a.cyc[(a.start[p] + h) % a.cyc_len];
@@ -304,7 +317,7 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
             // caller buffers and rows may start at any byte; staging is ours
             if (load && !op->input[rank]) return MINT_ERR_ARG;
             if (save && !op->output[rank]) return MINT_ERR_ARG;
-            if (!cu && !origin && (!op->staging[rank] || !aligned16(op->staging[rank])))
+            if (!origin && (!op->staging[rank] || !aligned16(op->staging[rank])))
                 return op->staging[rank] ? MINT_ERR_ALIGN : MINT_ERR_ARG;
         }
     }
@@ -718,16 +731,12 @@ int mint_ll128_pack(const void* raw, void* msg, size_t nbytes, uint64_t flag_bas
     const uint64_t cap = (uint64_t)device_cus() * 8;
     if (cap && blocks > cap) blocks = cap;
     if (layout == MINT_LAYOUT_WAVE64)
-        hipLaunchKernelGGL(pack_wave64_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                           as_stream(stream), static_cast<const uint8_t*>(raw),
+        return Launch<&pack_wave64_kernel>::go(dim3((unsigned)blocks), 256, 0, as_stream(stream), static_cast<const uint8_t*>(raw),
                            static_cast<uint8_t*>(msg), (uint64_t)nbytes, (uint32_t)(lines / 8),
                            flag_base, flag_stride);
-    else
-        hipLaunchKernelGGL(pack_pair_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                           as_stream(stream), static_cast<const uint8_t*>(raw),
+    return Launch<&pack_pair_kernel>::go(dim3((unsigned)blocks), 256, 0, as_stream(stream), static_cast<const uint8_t*>(raw),
                            static_cast<uint8_t*>(msg), (uint64_t)nbytes, lines, flag_base,
                            flag_stride);
-    return launch_status();
 }
 
 int mint_ll128_unpack(const void* msg, void* raw, size_t nbytes, uint64_t flag_base,
@@ -743,16 +752,12 @@ int mint_ll128_unpack(const void* msg, void* raw, size_t nbytes, uint64_t flag_b
     const uint64_t cap = (uint64_t)device_cus() * 8;
     if (cap && blocks > cap) blocks = cap;
     if (layout == MINT_LAYOUT_WAVE64)
-        hipLaunchKernelGGL(unpack_wave64_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                           as_stream(stream), static_cast<const uint8_t*>(msg),
+        return Launch<&unpack_wave64_kernel>::go(dim3((unsigned)blocks), 256, 0, as_stream(stream), static_cast<const uint8_t*>(msg),
                            static_cast<uint8_t*>(raw), (uint64_t)nbytes, (uint32_t)(lines / 8),
                            flag_base, flag_stride, static_cast<unsigned long long*>(bad_flags));
-    else
-        hipLaunchKernelGGL(unpack_pair_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                           as_stream(stream), static_cast<const uint8_t*>(msg),
+    return Launch<&unpack_pair_kernel>::go(dim3((unsigned)blocks), 256, 0, as_stream(stream), static_cast<const uint8_t*>(msg),
                            static_cast<uint8_t*>(raw), (uint64_t)nbytes, lines, flag_base,
                            flag_stride, static_cast<unsigned long long*>(bad_flags));
-    return launch_status();
 }
 
 int mint_elementwise_sum(const void* a, const void* b, void* out, size_t nelem, int dtype,

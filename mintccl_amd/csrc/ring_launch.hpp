@@ -5,6 +5,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include "../../include/mintccl.h"
 #include "cu_ring.hpp"
 #include "ring.hpp"
@@ -27,13 +29,40 @@ struct Plan {
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? MINT_OK : MINT_ERR_HIP; }
 
+constexpr int kDevices = 16;      // per-device facts are kept for the first so many
 inline int device_cus() {
+    static std::atomic<int> known[kDevices];
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
+    if (dev < kDevices && (cus = known[dev].load(std::memory_order_relaxed)) != 0) return cus;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return 0;
+    if (dev < kDevices) known[dev].store(cus, std::memory_order_relaxed);
     return cus;
 }
+
+// Launches KERNEL.  A launch costs the host 2.4 us and is most of what a small
+// collective takes, so the symbol is looked up once per device and not on every
+// launch (hipLaunchKernelGGL: 2.6).
+template <auto KERNEL>
+struct Launch;
+template <typename... P, void (*KERNEL)(P...)>
+struct Launch<KERNEL> {
+    static int go(dim3 grid, unsigned threads, unsigned lds_bytes, hipStream_t stream, P... args) {
+        static std::atomic<hipFunction_t> known[kDevices];
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return MINT_ERR_HIP;
+        hipFunction_t f = dev < kDevices ? known[dev].load(std::memory_order_acquire) : nullptr;
+        if (!f) {
+            if (hipGetFuncBySymbol(&f, reinterpret_cast<const void*>(KERNEL)) != hipSuccess) return MINT_ERR_HIP;
+            if (dev < kDevices) known[dev].store(f, std::memory_order_release);
+        }
+        void* list[] = {const_cast<void*>(static_cast<const void*>(&args))...};
+        const hipError_t e = hipModuleLaunchKernel(f, grid.x, grid.y, grid.z, threads, 1, 1, lds_bytes, stream,
+                                                   list, nullptr);
+        return e == hipSuccess ? MINT_OK : MINT_ERR_HIP;
+    }
+};
 
 // protocol: MINT_PROTO_*; cache_policy: 0 agent, 1 system, 2 XCD-local
 int launch_ring_family_f16(const Plan& plan, int protocol, int cache_policy, hipStream_t stream);

@@ -9,10 +9,12 @@ from . import _lib, tree
 from ._ops import ring_of
 from .common import VirtualComm, get_comm
 
+_KIND = _lib.KIND_REDUCE
+
 
 def reduce(buff: torch.Tensor, root: int, comm: VirtualComm | None = None) -> None:
     comm = comm if comm is not None else get_comm()
-    posted = comm._board.post(_lib.KIND_REDUCE, buff, root)
+    posted = comm._post(_KIND, buff, root)
     if posted is None:               # not all ranks are here yet, or launched
         return
     if posted is False:

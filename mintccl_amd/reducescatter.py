@@ -11,10 +11,12 @@ from . import _lib, hypercube
 from ._ops import ring_of
 from .common import VirtualComm, get_comm
 
+_KIND = _lib.KIND_REDUCESCATTER
+
 
 def reducescatter(buff: torch.Tensor, comm: VirtualComm | None = None) -> None:
     comm = comm if comm is not None else get_comm()
-    posted = comm._board.post(_lib.KIND_REDUCESCATTER, buff)
+    posted = comm._post(_KIND, buff)
     if posted is None:               # not all ranks are here yet, or launched
         return
     if posted is False:
