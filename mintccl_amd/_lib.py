@@ -168,7 +168,7 @@ def host_command(out: str) -> list[str]:
                                        os.path.join(base, "include", "torch", "csrc", "api", "include"),
                                        os.path.join(rocm, "include"), sysconfig.get_paths()["include"])],
             "-o", out, HOST_SRC, "-L" + os.path.join(base, "lib"),
-            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
 
 
 def build(verbose: bool = False, defines: tuple[str, ...] = (), so_path: str | None = None) -> str:

@@ -16,7 +16,7 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
-#include <ATen/ops/empty.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -643,7 +643,8 @@ PyObject* host_pack(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const size_t nbytes = bytes_of(*raw), need = native.packed_bytes(nbytes, layout);
         PyObject* result;
         if (args[4] == Py_None) {
-            result = THPVariable_Wrap(at::empty({(int64_t)need}, raw->options().dtype(at::kByte).requires_grad(false)));
+            // (the allocator's own entry: half of what the dispatcher takes)
+            result = THPVariable_Wrap(at::Tensor(at::detail::empty_cuda({(int64_t)need}, at::kByte, raw->device(), {})));
             if (!result) return nullptr;
         } else {
             const at::Tensor* out = device_tensor(args[4]);

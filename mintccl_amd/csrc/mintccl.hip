@@ -718,6 +718,17 @@ size_t mint_ll128_packed_bytes(size_t nbytes, int layout) {
     return (nbytes + 959) / 960 * 1024;
 }
 
+namespace {
+// Thread blocks of the codec: one wavefront per block of the message, but no
+// more threads than a launch may have; pair layout: 8 blocks per compute unit.
+uint32_t codec_blocks(uint64_t lines, int layout) {
+    const uint64_t waves = layout == MINT_LAYOUT_WAVE64 ? lines / 8 : (lines * 8 + 63) / 64;
+    const uint64_t blocks = (waves + kCodecThreads / 64 - 1) / (kCodecThreads / 64);
+    const uint64_t cap = layout == MINT_LAYOUT_WAVE64 ? (1ull << 31) / kCodecThreads : (uint64_t)device_cus() * 8;
+    return (uint32_t)(cap && blocks > cap ? cap : blocks);
+}
+}  // namespace
+
 int mint_ll128_pack(const void* raw, void* msg, size_t nbytes, uint64_t flag_base,
                     uint64_t flag_stride, int layout, void* stream) {
     if (layout != MINT_LAYOUT_PAIR && layout != MINT_LAYOUT_WAVE64) return MINT_ERR_ARG;
@@ -726,17 +737,15 @@ int mint_ll128_pack(const void* raw, void* msg, size_t nbytes, uint64_t flag_bas
     if (!aligned16(raw) || !aligned16(msg)) return MINT_ERR_ALIGN;
     const uint64_t lines = mint_ll128_packed_bytes(nbytes, layout) / 128;
     if (lines >= (1ull << 31)) return MINT_ERR_TOO_LARGE;
-    const uint64_t waves = layout == MINT_LAYOUT_WAVE64 ? lines / 8 : (lines * 8 + 63) / 64;
-    uint64_t blocks = (waves + 3) / 4;
-    const uint64_t cap = (uint64_t)device_cus() * 8;
-    if (cap && blocks > cap) blocks = cap;
+    const uint32_t blocks = codec_blocks(lines, layout);
+    const uint8_t* from = static_cast<const uint8_t*>(raw);
+    uint8_t* to = static_cast<uint8_t*>(msg);
     if (layout == MINT_LAYOUT_WAVE64)
-        return Launch<&pack_wave64_kernel>::go(dim3((unsigned)blocks), 256, 0, as_stream(stream), static_cast<const uint8_t*>(raw),
-                           static_cast<uint8_t*>(msg), (uint64_t)nbytes, (uint32_t)(lines / 8),
-                           flag_base, flag_stride);
-    return Launch<&pack_pair_kernel>::go(dim3((unsigned)blocks), 256, 0, as_stream(stream), static_cast<const uint8_t*>(raw),
-                           static_cast<uint8_t*>(msg), (uint64_t)nbytes, lines, flag_base,
-                           flag_stride);
+        return Launch<&pack_wave64_kernel>::go(blocks, kCodecThreads, 0, as_stream(stream), from, to, nbytes,
+                                               (uint32_t)(lines / 8), blocks * (kCodecThreads / 64), flag_base,
+                                               flag_stride);
+    return Launch<&pack_pair_kernel>::go(blocks, kCodecThreads, 0, as_stream(stream), from, to, nbytes, lines,
+                                         flag_base, flag_stride);
 }
 
 int mint_ll128_unpack(const void* msg, void* raw, size_t nbytes, uint64_t flag_base,
@@ -747,17 +756,16 @@ int mint_ll128_unpack(const void* msg, void* raw, size_t nbytes, uint64_t flag_b
     if (!aligned16(raw) || !aligned16(msg)) return MINT_ERR_ALIGN;
     const uint64_t lines = mint_ll128_packed_bytes(nbytes, layout) / 128;
     if (lines >= (1ull << 31)) return MINT_ERR_TOO_LARGE;
-    const uint64_t waves = layout == MINT_LAYOUT_WAVE64 ? lines / 8 : (lines * 8 + 63) / 64;
-    uint64_t blocks = (waves + 3) / 4;
-    const uint64_t cap = (uint64_t)device_cus() * 8;
-    if (cap && blocks > cap) blocks = cap;
+    const uint32_t blocks = codec_blocks(lines, layout);
+    const uint8_t* from = static_cast<const uint8_t*>(msg);
+    uint8_t* to = static_cast<uint8_t*>(raw);
+    unsigned long long* bad = static_cast<unsigned long long*>(bad_flags);
     if (layout == MINT_LAYOUT_WAVE64)
-        return Launch<&unpack_wave64_kernel>::go(dim3((unsigned)blocks), 256, 0, as_stream(stream), static_cast<const uint8_t*>(msg),
-                           static_cast<uint8_t*>(raw), (uint64_t)nbytes, (uint32_t)(lines / 8),
-                           flag_base, flag_stride, static_cast<unsigned long long*>(bad_flags));
-    return Launch<&unpack_pair_kernel>::go(dim3((unsigned)blocks), 256, 0, as_stream(stream), static_cast<const uint8_t*>(msg),
-                           static_cast<uint8_t*>(raw), (uint64_t)nbytes, lines, flag_base,
-                           flag_stride, static_cast<unsigned long long*>(bad_flags));
+        return Launch<&unpack_wave64_kernel>::go(blocks, kCodecThreads, 0, as_stream(stream), from, to, nbytes,
+                                                 (uint32_t)(lines / 8), blocks * (kCodecThreads / 64), flag_base,
+                                                 flag_stride, bad);
+    return Launch<&unpack_pair_kernel>::go(blocks, kCodecThreads, 0, as_stream(stream), from, to, nbytes, lines,
+                                           flag_base, flag_stride, bad);
 }
 
 int mint_elementwise_sum(const void* a, const void* b, void* out, size_t nelem, int dtype,
