@@ -19,14 +19,11 @@ from .common import VirtualComm, get_comm
 
 _KIND = _lib.KIND_ALLGATHER
 
-# (what is no schedule is refused by the board; -1: nothing said)
-_SCHEDULE = {None: -1, "spatial": 0, "temporal": 1}
-
 
 def allgather(buff: torch.Tensor, comm: VirtualComm | None = None,
               schedule: str | None = None) -> None:
     comm = comm if comm is not None else get_comm()
-    posted = comm._post(_KIND, buff, 0, _SCHEDULE.get(schedule, 2))
+    posted = comm._post(_KIND, buff, 0, schedule)
     if posted is None:               # not all ranks are here yet, or launched
         return
     if posted is False:

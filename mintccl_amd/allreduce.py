@@ -45,7 +45,7 @@ def chunk_bytes(count: int, world: int) -> int:
 def allreduce(buff: torch.Tensor, comm: VirtualComm | None = None,
               fused: bool | None = None) -> None:
     comm = comm if comm is not None else get_comm()
-    posted = comm._post(_KIND, buff, 0, -1 if fused is None else int(bool(fused)))
+    posted = comm._post(_KIND, buff, 0, fused)
     if posted is None:               # not all ranks are here yet, or launched
         return
     count, dtype, _, variant, ptrs, _, _ = posted

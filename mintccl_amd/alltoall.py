@@ -19,7 +19,7 @@ _KIND = _lib.KIND_ALLTOALL
 
 def alltoall(buff: torch.Tensor, out: torch.Tensor, comm: VirtualComm | None = None) -> None:
     comm = comm if comm is not None else get_comm()
-    posted = comm._post(_KIND, buff, 0, -1, out)
+    posted = comm._post(_KIND, buff, 0, None, out)
     if posted is None:               # not all ranks are here yet, or launched
         return
     count, _, _, _, ins, outs, _ = posted

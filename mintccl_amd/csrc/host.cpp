@@ -94,7 +94,7 @@ constexpr KindInfo kKinds[KINDS] = {
     {"alltoall", MINT_OP_ALLTOALL, true, false, nullptr},
 };
 // `variant` of an allgather: 0 spatial, 1 temporal; of an allreduce: 0 split, 1 fused; -1: not said
-enum { SPATIAL = 0, TEMPORAL = 1, SPLIT = 0, FUSED = 1, UNSAID = -1 };
+enum { SPATIAL = 0, TEMPORAL = 1, NO_SCHEDULE = 2, SPLIT = 0, FUSED = 1, UNSAID = -1 };
 
 struct Post {
     uint64_t in, out, count;
@@ -308,12 +308,12 @@ PyObject* complete(Board* b, Kind kind, const Gathering& g) {
     return result;
 }
 
-// post(kind, buff[, root[, variant[, out]]]): None (not all ranks are there yet,
+// post(kind, buff[, root[, schedule or fused, or None[, out]]]): None (not all ranks are there yet,
 // or launched), the ranks' arguments (complete()), or False: MINTCCL_TOPOLOGY
 // has another module do this collective
 PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     Board* b = reinterpret_cast<Board*>(self);
-    if (n < 2 || n > 5) return raise(PyExc_TypeError, "post(kind, buff[, root[, variant[, out]]])");
+    if (n < 2 || n > 5) return raise(PyExc_TypeError, "post(kind, buff[, root[, variant or None[, out]]])");
     const long k = PyLong_AsLong(args[0]);
     if (k < 0 || k >= KINDS) return PyErr_Occurred() ? nullptr : raise(PyExc_ValueError, "no such collective");
     const Kind kind = (Kind)k;
@@ -321,9 +321,19 @@ PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
         Post p{};
         p.variant = UNSAID;
-        if (n > 2) p.root = PyLong_AsLong(args[2]);
-        if (n > 3) p.variant = PyLong_AsLong(args[3]);
-        if (PyErr_Occurred()) return nullptr;
+        if (n > 2 && (p.root = PyLong_AsLong(args[2])) == -1 && PyErr_Occurred()) return nullptr;
+        if (n > 3 && args[3] != Py_None) {
+            if (kind == ALLGATHER) {
+                if (!PyUnicode_Check(args[3])) p.variant = NO_SCHEDULE;
+                else p.variant = PyUnicode_CompareWithASCIIString(args[3], "spatial") == 0    ? SPATIAL
+                                 : PyUnicode_CompareWithASCIIString(args[3], "temporal") == 0 ? TEMPORAL
+                                                                                             : NO_SCHEDULE;
+            } else {
+                const int fused = PyObject_IsTrue(args[3]);
+                if (fused < 0) return nullptr;
+                p.variant = fused ? FUSED : SPLIT;
+            }
+        }
         Gathering& g = b->gathering[kind];
         bool asked = g.present && g.asked;
         long env_variant = g.env_variant;
@@ -334,7 +344,7 @@ PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
                 env_variant = UNSAID;
                 if (kind == ALLGATHER) {
                     e = getenv("MINTCCL_ALLGATHER");
-                    env_variant = !e || strcasecmp(e, "spatial") == 0 ? SPATIAL : strcasecmp(e, "temporal") == 0 ? TEMPORAL : 2;
+                    env_variant = !e || strcasecmp(e, "spatial") == 0 ? SPATIAL : strcasecmp(e, "temporal") == 0 ? TEMPORAL : NO_SCHEDULE;
                 }
                 asked = true;
             }
