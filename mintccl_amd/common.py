@@ -274,24 +274,6 @@ def _largest_divisor_at_most(n: int, cap: int) -> int:
     return 1
 
 
-class _RankContext:
-    """``with comm.rank(r):`` - the thread speaks for rank ``r`` inside."""
-
-    __slots__ = ("comm", "r", "before")
-
-    def __init__(self, comm: "VirtualComm", r: int) -> None:
-        if not 0 <= r < comm.world_size:
-            raise ValueError(f"rank {r} outside world of {comm.world_size}")
-        self.comm, self.r = comm, r
-
-    def __enter__(self) -> "VirtualComm":
-        self.before = self.comm._board.enter(self.r)
-        return self.comm
-
-    def __exit__(self, *exc) -> None:
-        self.comm._board.enter(self.before)
-
-
 # attributes a native launch takes from the communicator (VirtualComm._refresh)
 _LAUNCH_ATTRIBUTES = frozenset(("inside_cu", "stats", "epoch_word", "protocol", "spin_budget", "status",
                                 "topology"))
@@ -376,7 +358,7 @@ class VirtualComm:
         # gathers the ranks' arguments and launches (csrc/host.cpp)
         self._board = _lib.host().Board(self, self.world_size,
                                         -1 if self.device.index is None else self.device.index)
-        self._post = self._board.post
+        self._post, self._sync = self._board.post, self._board.sync
         # slots + credit words (never more than slot_bytes / 4), zeroed: flag 0
         # and credit 0 mean "nothing yet" (2_sendrecv_indirect.py:59-60).
         if self.buff_size % 256:
@@ -445,8 +427,9 @@ class VirtualComm:
     def Get_rank(self) -> int:
         return self._board.rank()
 
-    def rank(self, r: int) -> _RankContext:
-        return _RankContext(self, r)
+    def rank(self, r: int):
+        """``with comm.rank(r):`` - the thread speaks for rank ``r`` inside."""
+        return self._board.speak(r)
 
     def run(self, fn) -> None:
         """SPMD helper: ``fn(rank)`` for every rank in turn (like mpirun)."""

@@ -505,10 +505,48 @@ PyObject* board_sync(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     });
 }
 
-PyObject* board_enter(PyObject* self, PyObject* arg) {
+// speak(rank): a context in which the thread speaks for that rank
+struct RankContext {
+    PyObject_HEAD
+    PyObject* comm;              // owns the board
+    Board* board;
+    int rank, before;
+};
+PyTypeObject context_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+void context_dealloc(PyObject* self) {
+    Py_DECREF(reinterpret_cast<RankContext*>(self)->comm);
+    Py_DECREF(reinterpret_cast<RankContext*>(self)->board);
+    Py_TYPE(self)->tp_free(self);
+}
+PyObject* context_enter(PyObject* self, PyObject*) {
+    RankContext* c = reinterpret_cast<RankContext*>(self);
+    c->before = enter_rank(c->board, c->rank);
+    return Py_NewRef(c->comm);
+}
+PyObject* context_exit(PyObject* self, PyObject* const*, Py_ssize_t) {
+    RankContext* c = reinterpret_cast<RankContext*>(self);
+    enter_rank(c->board, c->before);
+    Py_RETURN_NONE;
+}
+PyMethodDef context_methods[] = {
+    {"__enter__", context_enter, METH_NOARGS, nullptr},
+    {"__exit__", (PyCFunction)(void (*)(void))context_exit, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyObject* board_speak(PyObject* self, PyObject* arg) {
+    Board* b = reinterpret_cast<Board*>(self);
     const long r = PyLong_AsLong(arg);
     if (r == -1 && PyErr_Occurred()) return nullptr;
-    return PyLong_FromLong(enter_rank(reinterpret_cast<Board*>(self), (int)r));
+    if (r < 0 || r >= b->world) {
+        PyErr_Format(PyExc_ValueError, "rank %ld outside world of %d", r, b->world);
+        return nullptr;
+    }
+    RankContext* c = PyObject_New(RankContext, &context_type);
+    if (!c) return nullptr;
+    c->comm = Py_NewRef(PyWeakref_GetObject(b->comm));
+    c->board = reinterpret_cast<Board*>(Py_NewRef(self));
+    c->rank = (int)r;
+    c->before = -1;
+    return reinterpret_cast<PyObject*>(c);
 }
 PyObject* board_rank(PyObject* self, PyObject*) {
     int rank;
@@ -620,7 +658,7 @@ PyMethodDef board_methods[] = {
     {"send", (PyCFunction)(void (*)(void))board_send, METH_FASTCALL, nullptr},
     {"recv", (PyCFunction)(void (*)(void))board_recv, METH_FASTCALL, nullptr},
     {"sync", (PyCFunction)(void (*)(void))board_sync, METH_FASTCALL, nullptr},
-    {"enter", board_enter, METH_O, nullptr},
+    {"speak", board_speak, METH_O, nullptr},
     {"rank", board_rank, METH_NOARGS, nullptr},
     {"run", board_run, METH_O, nullptr},
     {"stale", board_stale, METH_NOARGS, nullptr},
@@ -738,7 +776,13 @@ PyMODINIT_FUNC PyInit__host(void) {
     board_type.tp_dealloc = board_dealloc;
     board_type.tp_methods = board_methods;
     board_type.tp_getset = board_getset;
-    if (PyType_Ready(&board_type) < 0) return nullptr;
+    context_type.tp_name = "mintccl_amd._host.RankContext";
+    context_type.tp_basicsize = sizeof(RankContext);
+    context_type.tp_flags = Py_TPFLAGS_DEFAULT;
+    context_type.tp_doc = "with comm.rank(r): the thread speaks for rank r inside";
+    context_type.tp_dealloc = context_dealloc;
+    context_type.tp_methods = context_methods;
+    if (PyType_Ready(&board_type) < 0 || PyType_Ready(&context_type) < 0) return nullptr;
     PyObject* m = PyModule_Create(&host_module);
     if (!m) return nullptr;
     Py_INCREF(&board_type);

@@ -49,7 +49,7 @@ def sync(comm: VirtualComm | None = None, route: list[int] | None = None) -> Non
     """Every rank calls this; the first call that finds a matched send / recv
     pair launches, the others find nothing left to do."""
     comm = comm if comm is not None else get_comm()
-    matched = comm._board.sync(route, False)
+    matched = comm._sync(route, False)
     if matched is not None:                  # (not launched by the board)
         _launch(comm, matched)
 
