@@ -2,6 +2,8 @@
 launch once every participating rank has posted its buffer."""
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import _lib
@@ -20,6 +22,22 @@ def check_buffer(t: torch.Tensor, comm: VirtualComm) -> None:
         raise ValueError("buffer lives on another device than the communicator")
     if not t.is_contiguous():
         raise ValueError("buffer must be contiguous")
+
+
+def front(action: int, go_on=None):
+    """Decorator: the operator behind a native front (csrc/host.cpp), which takes
+    the calls that need no Python: a rank's arguments are noted, the last one's
+    call launches.  ``go_on(comm, posted)`` does what is left where the board
+    hands the arguments back.  Without the host module (before the first
+    build) the operator stands alone."""
+    def wrap(op):
+        try:
+            from . import _host
+        except ImportError:
+            return op
+        made = getattr(_host, "Front", None)
+        return op if made is None else functools.update_wrapper(made(op, action, go_on), op)
+    return wrap
 
 
 def ring_of(comm: VirtualComm) -> list[int]:

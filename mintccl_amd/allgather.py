@@ -14,20 +14,14 @@ from __future__ import annotations
 import torch
 
 from . import _lib, hypercube
-from ._ops import ring_of
+from ._ops import front, ring_of
 from .common import VirtualComm, get_comm
 
 _KIND = _lib.KIND_ALLGATHER
 
 
-def allgather(buff: torch.Tensor, comm: VirtualComm | None = None,
-              schedule: str | None = None) -> None:
-    comm = comm if comm is not None else get_comm()
-    posted = comm._post(_KIND, buff, 0, schedule)
-    if posted is None:               # not all ranks are here yet, or launched
-        return
-    if posted is False:
-        return hypercube.allgather(buff, comm)
+def _go_on(comm: VirtualComm, posted: tuple) -> None:
+    """All ranks are here, and it is not the board's to launch."""
     count, _, _, temporal, ptrs, _, _ = posted
     row = count // comm.world_size
     if temporal:
@@ -35,6 +29,17 @@ def allgather(buff: torch.Tensor, comm: VirtualComm | None = None,
                                  ring_of(comm), row_stride=row, protocol=_lib.PROTO_LL128))
     else:
         comm.enqueue(_lib.OP_ALLGATHER, _lib.BYTES, row, ptrs, ptrs, ring_of(comm), row_stride=row)
+
+
+@front(_KIND, _go_on)
+def allgather(buff: torch.Tensor, comm: VirtualComm | None = None,
+              schedule: str | None = None) -> None:
+    comm = comm if comm is not None else get_comm()
+    posted = comm._post(_KIND, buff, 0, schedule)
+    if posted is False:
+        return hypercube.allgather(buff, comm)
+    if posted is not None:           # (None: not all ranks are here yet, or launched)
+        _go_on(comm, posted)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

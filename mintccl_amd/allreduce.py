@@ -23,7 +23,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._ops import ring_of
+from ._ops import front, ring_of
 from .common import VirtualComm, get_comm
 
 _KIND = _lib.KIND_ALLREDUCE
@@ -42,12 +42,8 @@ def chunk_bytes(count: int, world: int) -> int:
     return (-(-count // world) + 15) // 16 * 16
 
 
-def allreduce(buff: torch.Tensor, comm: VirtualComm | None = None,
-              fused: bool | None = None) -> None:
-    comm = comm if comm is not None else get_comm()
-    posted = comm._post(_KIND, buff, 0, fused)
-    if posted is None:               # not all ranks are here yet, or launched
-        return
+def _go_on(comm: VirtualComm, posted: tuple) -> None:
+    """All ranks are here, and it is not the board's to launch."""
     count, dtype, _, variant, ptrs, _, _ = posted
     fused = count < SPLIT_FROM_BYTES or comm.inside_cu if variant < 0 else bool(variant)
     ring = ring_of(comm)
@@ -59,6 +55,15 @@ def allreduce(buff: torch.Tensor, comm: VirtualComm | None = None,
                  total_bytes=count)
     comm.enqueue(_lib.OP_ALLGATHER, _lib.BYTES, row, ptrs, ptrs, ring, row_stride=row,
                  total_bytes=count)
+
+
+@front(_KIND, _go_on)
+def allreduce(buff: torch.Tensor, comm: VirtualComm | None = None,
+              fused: bool | None = None) -> None:
+    comm = comm if comm is not None else get_comm()
+    posted = comm._post(_KIND, buff, 0, fused)
+    if posted is not None:           # (None: not all ranks are here yet, or launched)
+        _go_on(comm, posted)
 
 
 if __name__ == "__main__":      # the reference runs its self-test from here

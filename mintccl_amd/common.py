@@ -358,7 +358,7 @@ class VirtualComm:
         # gathers the ranks' arguments and launches (csrc/host.cpp)
         self._board = _lib.host().Board(self, self.world_size,
                                         -1 if self.device.index is None else self.device.index)
-        self._post, self._sync = self._board.post, self._board.sync
+        self._post = self._board.post
         # slots + credit words (never more than slot_bytes / 4), zeroed: flag 0
         # and credit 0 mean "nothing yet" (2_sendrecv_indirect.py:59-60).
         if self.buff_size % 256:

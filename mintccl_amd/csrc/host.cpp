@@ -61,7 +61,11 @@ struct OnDevice {
     ~OnDevice() {
         if (before != device) c10::hip::set_device((c10::DeviceIndex)before);
     }
-    void* stream() const { return c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
+    // (stream() goes through a device guard; the default stream, whose id is 0, is null)
+    void* stream() const {
+        const auto current = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device);
+        return current.id() == 0 ? nullptr : (void*)current.stream();
+    }
 };
 
 // C++ exceptions (torch's, out of memory) become Python's.
@@ -311,25 +315,20 @@ PyObject* complete(Board* b, Kind kind, const Gathering& g) {
 // post(kind, buff[, root[, schedule or fused, or None[, out]]]): None (not all ranks are there yet,
 // or launched), the ranks' arguments (complete()), or False: MINTCCL_TOPOLOGY
 // has another module do this collective
-PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
-    Board* b = reinterpret_cast<Board*>(self);
-    if (n < 2 || n > 5) return raise(PyExc_TypeError, "post(kind, buff[, root[, variant or None[, out]]])");
-    const long k = PyLong_AsLong(args[0]);
-    if (k < 0 || k >= KINDS) return PyErr_Occurred() ? nullptr : raise(PyExc_ValueError, "no such collective");
-    const Kind kind = (Kind)k;
+PyObject* post(Board* b, Kind kind, PyObject* buff, PyObject* root, PyObject* variant, PyObject* out) {
     const KindInfo& info = kKinds[kind];
     return guarded([&]() -> PyObject* {
         Post p{};
         p.variant = UNSAID;
-        if (n > 2 && (p.root = PyLong_AsLong(args[2])) == -1 && PyErr_Occurred()) return nullptr;
-        if (n > 3 && args[3] != Py_None) {
+        if (root && (p.root = PyLong_AsLong(root)) == -1 && PyErr_Occurred()) return nullptr;
+        if (variant && variant != Py_None) {
             if (kind == ALLGATHER) {
-                if (!PyUnicode_Check(args[3])) p.variant = NO_SCHEDULE;
-                else p.variant = PyUnicode_CompareWithASCIIString(args[3], "spatial") == 0    ? SPATIAL
-                                 : PyUnicode_CompareWithASCIIString(args[3], "temporal") == 0 ? TEMPORAL
+                if (!PyUnicode_Check(variant)) p.variant = NO_SCHEDULE;
+                else p.variant = PyUnicode_CompareWithASCIIString(variant, "spatial") == 0    ? SPATIAL
+                                 : PyUnicode_CompareWithASCIIString(variant, "temporal") == 0 ? TEMPORAL
                                                                                              : NO_SCHEDULE;
             } else {
-                const int fused = PyObject_IsTrue(args[3]);
+                const int fused = PyObject_IsTrue(variant);
                 if (fused < 0) return nullptr;
                 p.variant = fused ? FUSED : SPLIT;
             }
@@ -352,7 +351,7 @@ PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
         }
         if (kind == ALLGATHER && (p.variant < SPATIAL || p.variant > TEMPORAL))
             return raise(PyExc_ValueError, "allgather schedule is 'spatial' or 'temporal'");
-        const at::Tensor* t = tensor_of(b, args[1]);
+        const at::Tensor* t = tensor_of(b, buff);
         if (!t) return nullptr;
         p.in = (uint64_t)t->data_ptr();
         p.count = (uint64_t)t->numel() * (uint64_t)t->element_size();
@@ -362,8 +361,8 @@ PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
             return raise(PyExc_ValueError, "buffer does not split into world_size rows");
         if (info.reducing && (p.dtype = dtype_code(*t)) < 0)
             return raise(PyExc_TypeError, "reductions take float16, bfloat16 or float32 tensors");
-        if (n > 4) {
-            const at::Tensor* o = tensor_of(b, args[4]);
+        if (out) {
+            const at::Tensor* o = tensor_of(b, out);
             if (!o) return nullptr;
             if ((uint64_t)o->numel() * (uint64_t)o->element_size() != p.count)
                 return raise(PyExc_ValueError, "buff and out differ in size");
@@ -375,8 +374,8 @@ PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
             PyErr_Format(PyExc_RuntimeError, "rank %d called %s twice before the others joined", rank, info.name);
             return nullptr;
         }
-        p.keep_in = Py_NewRef(args[1]);
-        p.keep_out = n > 4 ? Py_NewRef(args[4]) : nullptr;
+        p.keep_in = Py_NewRef(buff);
+        p.keep_out = Py_XNewRef(out);
         g.post[rank] = p;
         g.present |= 1u << rank;
         g.asked = asked;
@@ -389,6 +388,14 @@ PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
         drop(&all);
         return result;
     });
+}
+
+PyObject* board_post(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+    if (n < 2 || n > 5) return raise(PyExc_TypeError, "post(kind, buff[, root[, variant or None[, out]]])");
+    const long k = PyLong_AsLong(args[0]);
+    if (k < 0 || k >= KINDS) return PyErr_Occurred() ? nullptr : raise(PyExc_ValueError, "no such collective");
+    return post(reinterpret_cast<Board*>(self), (Kind)k, args[1], n > 2 ? args[2] : nullptr,
+                n > 3 ? args[3] : nullptr, n > 4 ? args[4] : nullptr);
 }
 
 PyObject* transfer(Board* b, Transfer* t, PyObject* const* args, Py_ssize_t n) {
@@ -670,6 +677,108 @@ PyGetSetDef board_getset[] = {{"last_grid", board_last_grid, nullptr, nullptr, n
                               {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyTypeObject board_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
+// ---- fronts of the operators ---------------------------------------------------
+// Front(operator, action, go_on) stands before an operator written in Python: a
+// call that names its communicator goes straight to the board; what is left to
+// do where the board has not done it all, go_on(comm, posted) does in
+// Python, and any other call (the default communicator, arguments that do not
+// fit) is the operator's.  A collective of eight ranks is eight such calls: 0.1 us
+// each in place of 0.2.
+enum Action { SEND = KINDS, RECV, SYNC, ACTIONS };
+constexpr int kParams = 3;
+// the parameters in their order; what is not required comes last
+struct FrontInfo {
+    const char* names[kParams];
+    int required;
+} kFronts[ACTIONS] = {
+    {{"buff", "root", "comm"}, 2},  {{"buff", "root", "comm"}, 2},     {{"buff", "comm", "schedule"}, 1},
+    {{"buff", "comm", nullptr}, 1}, {{"buff", "comm", "fused"}, 1},    {{"buff", "out", "comm"}, 2},
+    {{"buff", "peer", "comm"}, 2},  {{"buff", "peer", "comm"}, 2},     {{"comm", "route", nullptr}, 0}};
+PyObject* param_names[ACTIONS][kParams];     // interned
+PyObject* board_name;
+
+struct Front {
+    PyObject_HEAD
+    vectorcallfunc call;
+    PyObject *op, *go_on, *dict;
+    int action;
+};
+
+PyObject* front_call(PyObject* self, PyObject* const* args, size_t nargsf, PyObject* kwnames) {
+    Front* f = reinterpret_cast<Front*>(self);
+    PyObject* const* names = param_names[f->action];
+    PyObject* given[kParams] = {};
+    const Py_ssize_t n = PyVectorcall_NARGS(nargsf), nk = kwnames ? PyTuple_GET_SIZE(kwnames) : 0;
+    bool fits = n <= kParams && (n == 0 || names[n - 1]);
+    for (Py_ssize_t i = 0; fits && i < n; ++i) given[i] = args[i];
+    for (Py_ssize_t i = 0; fits && i < nk; ++i) {
+        int k = 0;
+        while (k < kParams && names[k] != PyTuple_GET_ITEM(kwnames, i)) ++k;
+        fits = k < kParams && !given[k];
+        if (fits) given[k] = args[n + i];
+    }
+    PyObject* comm = nullptr;
+    for (int k = 0; fits && k < kParams && names[k]; ++k) {
+        if (k < kFronts[f->action].required && !given[k]) fits = false;
+        if (kFronts[f->action].names[k][0] == 'c') comm = given[k];
+    }
+    PyObject* board = fits && comm && comm != Py_None ? PyObject_GetAttr(comm, board_name) : nullptr;
+    if (!board || Py_TYPE(board) != &board_type) {
+        Py_XDECREF(board);
+        PyErr_Clear();
+        return PyObject_Vectorcall(f->op, args, nargsf, kwnames);
+    }
+    Board* b = reinterpret_cast<Board*>(board);
+    PyObject* result;
+    switch (f->action) {
+        case BROADCAST:
+        case REDUCE: result = post(b, (Kind)f->action, given[0], given[1], nullptr, nullptr); break;
+        case ALLTOALL: result = post(b, ALLTOALL, given[0], nullptr, nullptr, given[1]); break;
+        case SEND: result = transfer(b, &b->send, given, 2); break;
+        case RECV: result = transfer(b, &b->recv, given, 2); break;
+        case SYNC: {
+            PyObject* const pair[2] = {given[1] ? given[1] : Py_None, Py_False};
+            result = board_sync(board, pair, 2);
+            break;
+        }
+        default: result = post(b, (Kind)f->action, given[0], nullptr, given[2], nullptr);
+    }
+    Py_DECREF(board);
+    if (!result || result == Py_None) return result;
+    PyObject* const rest[2] = {comm, result};
+    // (False: MINTCCL_TOPOLOGY has another module do it)
+    PyObject* done = result == Py_False ? PyObject_Vectorcall(f->op, args, nargsf, kwnames)
+                                        : PyObject_Vectorcall(f->go_on, rest, 2, nullptr);
+    Py_DECREF(result);
+    return done;
+}
+
+// Front(operator, action, go_on)
+PyObject* front_new(PyTypeObject* type, PyObject* args, PyObject*) {
+    PyObject *op, *go_on;
+    int action;
+    if (!PyArg_ParseTuple(args, "OiO", &op, &action, &go_on)) return nullptr;
+    if (action < 0 || action >= ACTIONS) return raise(PyExc_ValueError, "no such action");
+    Front* f = reinterpret_cast<Front*>(type->tp_alloc(type, 0));
+    if (!f) return nullptr;
+    f->call = front_call;
+    f->op = Py_NewRef(op);
+    f->go_on = Py_NewRef(go_on);
+    f->action = action;
+    return reinterpret_cast<PyObject*>(f);
+}
+void front_dealloc(PyObject* self) {
+    Front* f = reinterpret_cast<Front*>(self);
+    Py_XDECREF(f->op);
+    Py_XDECREF(f->go_on);
+    Py_XDECREF(f->dict);
+    Py_TYPE(self)->tp_free(self);
+}
+PyTypeObject front_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+// (functools.update_wrapper gives it the operator's name, documentation and signature)
+PyGetSetDef front_getset[] = {{"__dict__", PyObject_GenericGetDict, PyObject_GenericSetDict, nullptr, nullptr},
+                              {nullptr, nullptr, nullptr, nullptr, nullptr}};
+
 // ---- codec ---------------------------------------------------------------------
 const at::Tensor* device_tensor(PyObject* o) {
     if (!THPVariable_Check(o)) return nullptr;
@@ -783,8 +892,28 @@ PyMODINIT_FUNC PyInit__host(void) {
     context_type.tp_dealloc = context_dealloc;
     context_type.tp_methods = context_methods;
     if (PyType_Ready(&board_type) < 0 || PyType_Ready(&context_type) < 0) return nullptr;
+    front_type.tp_name = "mintccl_amd._host.Front";
+    front_type.tp_basicsize = sizeof(Front);
+    front_type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL;
+    front_type.tp_new = front_new;
+    front_type.tp_dealloc = front_dealloc;
+    front_type.tp_call = PyVectorcall_Call;
+    front_type.tp_vectorcall_offset = offsetof(Front, call);
+    front_type.tp_dictoffset = offsetof(Front, dict);
+    front_type.tp_getset = front_getset;
+    if (PyType_Ready(&front_type) < 0) return nullptr;
+    for (int k = 0; k < ACTIONS; ++k)
+        for (int i = 0; i < kParams; ++i)
+            if (kFronts[k].names[i] && !(param_names[k][i] = PyUnicode_InternFromString(kFronts[k].names[i])))
+                return nullptr;
+    if (!(board_name = PyUnicode_InternFromString("_board"))) return nullptr;
     PyObject* m = PyModule_Create(&host_module);
     if (!m) return nullptr;
+    Py_INCREF(&front_type);
+    PyModule_AddObject(m, "Front", reinterpret_cast<PyObject*>(&front_type));
+    PyModule_AddIntConstant(m, "SEND", SEND);
+    PyModule_AddIntConstant(m, "RECV", RECV);
+    PyModule_AddIntConstant(m, "SYNC", SYNC);
     Py_INCREF(&board_type);
     PyModule_AddObject(m, "Board", reinterpret_cast<PyObject*>(&board_type));
     for (int k = 0; k < KINDS; ++k) {

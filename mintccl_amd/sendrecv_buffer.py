@@ -10,14 +10,17 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+from ._ops import front
 from .common import VirtualComm, get_comm
 from .protocol import packed_bytes
 
 
+@front(_lib.SEND)
 def send(buff: torch.Tensor, peer: int, comm: VirtualComm | None = None) -> None:
     (comm if comm is not None else get_comm())._board.send(buff, peer)
 
 
+@front(_lib.RECV)
 def recv(buff: torch.Tensor, peer: int, comm: VirtualComm | None = None) -> None:
     (comm if comm is not None else get_comm())._board.recv(buff, peer)
 
@@ -45,11 +48,12 @@ def _launch(comm: VirtualComm, matched: tuple, full_size_staging: bool = False) 
     comm.launch(d)
 
 
+@front(_lib.SYNC, _launch)
 def sync(comm: VirtualComm | None = None, route: list[int] | None = None) -> None:
     """Every rank calls this; the first call that finds a matched send / recv
     pair launches, the others find nothing left to do."""
     comm = comm if comm is not None else get_comm()
-    matched = comm._sync(route, False)
+    matched = comm._board.sync(route, False)
     if matched is not None:                  # (not launched by the board)
         _launch(comm, matched)
 

@@ -137,3 +137,51 @@ def test_codec_refuses_what_it_cannot_take(dev):
     with pytest.raises(_lib.MintError) as e:
         protocol.pack(torch.zeros(976, dtype=torch.uint8, device=dev)[1:961])
     assert e.value.code == _lib.ERR_ALIGN
+
+
+def test_operators_take_their_arguments_in_every_form(dev, monkeypatch):
+    """Positional, by name, the default communicator; what does not fit is the
+    operator's own TypeError; MINTCCL_TOPOLOGY still reaches the other modules."""
+    from mintccl_amd import sendrecv_buffer
+    from mintccl_amd.allgather import allgather
+    from mintccl_amd.alltoall import alltoall
+    from mintccl_amd.broadcast import broadcast
+    from mintccl_amd.common import get_comm, set_comm
+    world, n = 4, 999
+    comm, before = make_comm(world), get_comm()
+    src = [torch.full((world, n), r + 1, dtype=torch.int32, device=dev) for r in range(world)]
+    out = [torch.zeros_like(s) for s in src]
+    rows = torch.arange(1, world + 1, dtype=torch.int32, device=dev)[:, None].expand(world, n)
+
+    def fresh():
+        return [s.clone() for s in src]
+    set_comm(comm)
+    try:
+        for call in (lambda b: allgather(b), lambda b: allgather(b, comm), lambda b: allgather(buff=b, comm=comm),
+                     lambda b: allgather(b, comm=comm, schedule="spatial"), lambda b: allgather(b, None, "temporal"),
+                     lambda b: allgather(b, **{"co" + "mm": comm})):
+            bufs = fresh()
+            comm.run(lambda r: call(bufs[r]))
+            comm.check()
+            assert all(torch.equal(b, rows) for b in bufs)
+        for topology in ("", "tree"):
+            monkeypatch.setenv("MINTCCL_TOPOLOGY", topology)
+            bufs = fresh()
+            comm.run(lambda r: broadcast(bufs[r], comm=comm, root=2))
+            comm.check()
+            assert all(torch.equal(b, src[2]) for b in bufs)
+        comm.run(lambda r: alltoall(src[r], comm=comm, out=out[r]))
+        with comm.rank(1):
+            sendrecv_buffer.send(peer=3, buff=src[1])
+        with comm.rank(3):
+            sendrecv_buffer.recv(bufs[3], 1, comm=comm)
+        comm.run(lambda r: sendrecv_buffer.sync(route=[1, 0, 3], comm=comm))
+        assert comm.last_route == [1, 0, 3]
+        comm.check()
+        assert all(torch.equal(o, rows) for o in out) and torch.equal(bufs[3], src[1])
+        for bad in (lambda: allgather(), lambda: allgather(src[0], comm, None, None),
+                    lambda: allgather(src[0], comm, comm=comm), lambda: broadcast(src[0], comm=comm)):
+            with pytest.raises(TypeError, match="allgather|broadcast"):
+                bad()
+    finally:
+        set_comm(before)
