@@ -69,9 +69,9 @@ struct CuRingArgs {
 // tiles (with several copies two), the pipelines one after the other, as few
 // wavefronts on a compute unit as keep HBM busy (cu_waves).  More of them widen
 // the window over which the loads and stores of 8 or 16 rows are scattered: 8
-// ranks, 256 MiB of f16, reduce-scatter 390 us with 32 to a compute unit, 368 with
-// 9, 460 with 4; allreduce of 8 x 64 MiB 204 with 32, 163 with 4; allgather of
-// 8 x 32 MiB 429 / 338 with 32 / 8.
+// ranks, reduce-scatter of 256 MiB 392 us with 32 to a compute unit, 376 with 9;
+// allreduce of 64 MiB 202 with 20, 158 with 4; allgather of 8 x 64 MiB 89 with 32,
+// 67 with 8.
 //
 // Otherwise: blocks of 128 threads and 2 KiB, dealt to the pipelines in turn,
 // loads through the cache (8 ranks, reduce-scatter of 8 MiB 10.9 us; 15.5 in the
@@ -81,19 +81,35 @@ struct CuRingArgs {
 constexpr uint32_t cu_threads(bool large, bool copies) { return large && !copies ? 64u : 128u; }
 #endif
 
-// Rows that are read once, by nobody soon, are streamed past the last-level
-// cache, and so are stores nobody waits for.
+// How rows are loaded: through the caches, or streamed past the last-level one.
 template <bool STREAM>
 __device__ __forceinline__ u32x4 cu_load(const uint8_t* uniform, uint32_t lane) {
     MINT_GLOBAL const u32x4_unaligned* const p = (MINT_GLOBAL const u32x4_unaligned*)(as_global(uniform) + lane);
     if constexpr (STREAM) return __builtin_nontemporal_load(p);
     else return *p;
 }
-template <bool STREAM>
+// How results are stored: past the last-level cache (nt), through the XCD's L2
+// (sc1), or both.  Through the L2 a block's results are on their way while others
+// still load, and nothing is left to write back when the launch ends.  8 ranks,
+// kept in the L2 / nt / sc1 / sc1 nt:
+//   small, a row to several places: allgather of 8 x 8 MiB  9.9 / 10.5 /  8.2 / 10.1 us
+//   small, a row to one place:      sendrecv of 48 MiB     18.8 / 13.7 / 16.4 / 13.4
+//   large, several:                 allgather of 8 x 64 MiB   - / 73.4 / 94.3 / 67.7
+//   large, one:                     reduce-scatter of 64 MiB 86.9 / 88.6 / 82.1 / 88.0
+// No builtin stores 16 bytes with sc1 at any address; the gap behind the store
+// keeps the next instruction off its data registers.
+enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
+constexpr int cu_stores(bool large, bool several) {
+    return several ? (large ? CU_SC1_NT : CU_SC1) : large ? CU_SC1 : CU_NT;
+}
+template <int HOW>
 __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 v) {
-    MINT_GLOBAL u32x4_unaligned* const p = (MINT_GLOBAL u32x4_unaligned*)(as_global(uniform) + lane);
-    if constexpr (STREAM) __builtin_nontemporal_store(v, p);
-    else *p = v;
+    if constexpr (HOW == CU_NT)
+        __builtin_nontemporal_store(v, (MINT_GLOBAL u32x4_unaligned*)(as_global(uniform) + lane));
+    else if constexpr (HOW == CU_SC1)
+        asm volatile("global_store_dwordx4 %0, %1, %2 sc1\n\ts_nop 0" ::"v"(lane), "v"(v), "s"(uniform) : "memory");
+    else
+        asm volatile("global_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 0" ::"v"(lane), "v"(v), "s"(uniform) : "memory");
 }
 
 // A row cut into vectors of 16 bytes whose stores are aligned: vector i covers
@@ -203,7 +219,7 @@ __global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(C
 #pragma unroll
         for (int h = 1; h < N; ++h) x = ll_comp<DT>(v[h], x);
 #pragma unroll
-        for (int i = 0; i < kStored; ++i) cu_store<LARGE || !EVERYWHERE>(to[i] + ((int64_t)row_off + base), lane, x);
+        for (int i = 0; i < kStored; ++i) cu_store<cu_stores(LARGE, EVERYWHERE)>(to[i] + ((int64_t)row_off + base), lane, x);
     }
 }
 
@@ -226,7 +242,7 @@ __device__ __forceinline__ void cu_copy_row(const CuRow& row, uint32_t tile, uin
         if (!row.whole(base + lane)) continue;
         const u32x4 x = cu_load<LARGE && COPIES == 1>(in + base, lane);
 #pragma unroll
-        for (int k = 0; k < COPIES; ++k) cu_store<LARGE || COPIES == 1>(out[k] + base, lane, x);
+        for (int k = 0; k < COPIES; ++k) cu_store<cu_stores(LARGE, (COPIES > 1))>(out[k] + base, lane, x);
     }
 }
 

@@ -65,14 +65,18 @@ static_assert(MINT_OP_TREE_BROADCAST == OP_TREE_BROADCAST && MINT_OP_TREE_REDUCE
 // of rows on their way to or from a compute unit keep HBM busy: fewer
 // wavefronts leave it idle, more only scatter its accesses.  Each holds a KiB of
 // N rows to be added, of a row that goes to N - 1 others, or (allreduce) of N rows
-// and then N results.  Fastest counts on MI355X at 0.25 - 2 GiB, f16, bf16 and
-// f32, for N = 2 / 3 / 4 / 5 / 6 / 7 / 8: reduce-scatter 20 / 14 / 12 / 11 / 10 / 9 /
-// 9, allreduce 16 / 10 / 8 / 5 - 7 / 5 - 6 / 5 / 4 - 5, allgather 32 / 18 / 16 / 10 /
-// 10 / - / 8; one or two off is 1 - 3 % slower, but twice as many 5 - 20 %.
-int cu_waves(int op, int ranks) {
-    if (op == OP_ALLREDUCE) return 32 / ranks + 1;
-    if (reducing(op)) return 24 / ranks + 6;
-    return 64 / ranks;
+// and then N results.  Fastest counts on MI355X at 0.5 - 2 GiB, f16 and bf16, for
+// N = 2 / 3 / 4 / 5 / 6 / 7 / 8: reduce-scatter 16 - 18 / 14 / 12 / 10 - 11 / 11 - 12 /
+// 10 / 9, allreduce 14 / 9 / 7 - 8 / 6 - 7 / 5 - 6 / 5 / 4 - 5, allgather - / 18 / 16 /
+// 14 / 12 / 10 / 10 and up; one or two off is 1 - 3 % slower, but twice as many 5 -
+// 20 %.  Rows that are copied from the last-level cache arrive sooner: there 7 and
+// 8 ranks are fastest with 6 - 8 (allgather of 8 x 64 MiB 67 us with 8, 71 with 10;
+// of 8 x 128 MiB 179 / 174).
+int cu_waves(int op, int ranks, uint64_t copied) {
+    if (op == OP_ALLREDUCE) return (26 + ranks - 1) / ranks + 1;
+    if (reducing(op)) return (24 + ranks - 1) / ranks + 6;
+    if (ranks >= 7) return copied <= (72ull << 20) ? 8 : 10;
+    return 24 - 2 * ranks;
 }
 
 // The grid of a launch inside compute units: a thread block per tile of a row,
@@ -82,19 +86,19 @@ int plan_cu(Plan* plan) {
     const bool sums = reducing(a.op), alltoall = a.op == OP_ALLTOALL;
     const bool copies = (a.op == OP_BROADCAST || a.op == OP_ALLGATHER) && a.cyc_len > 2;
     // Large: the last-level cache (256 MiB) would not hold the rows from one use
-    // to the next.  Measured with three such sets of buffers in turn, the two
-    // forms meet at 64 - 128 MiB, where rows are only copied once at 128 - 256
-    // (8 ranks: reduce-scatter of 64 MiB 11.0 us small / 15.5 large, 128 MiB
-    // 28.6 / 26.9; alltoall of 128 MiB 17.0 / 24.5, 256 MiB 45.2 / 43.3).
+    // to the next.  Measured with three sets of buffers in turn (8 ranks, small /
+    // large, us): allgather 11.5 / 12.0 at 80 MiB, 17.7 / 15.5 at 96; reduce-scatter
+    // 17.8 / 19.6 at 96, 28.2 / 25.0 at 128; allreduce 34.9 / 35.3, 52.3 / 46.6; one
+    // copy of a row 19.8 / 20.7 at 128, 45.2 / 41.5 at 256.
     const uint64_t touched = (uint64_t)a.pipes * a.row_bytes *
                              (alltoall || a.op == OP_SENDRECV ? 2u : (uint64_t)a.cyc_len);
-    plan->cu_large = touched > ((uint64_t)(sums || copies ? 96 : 192) << 20);
+    plan->cu_large = touched > ((uint64_t)(copies ? 88 : sums ? 100 : 192) << 20);
     plan->threads = (int)cu_threads(plan->cu_large, copies);
     // (held to that number by the share of LDS its blocks ask for; LDS is handed
     // out in units of 1280 bytes)
     plan->cu_lds = 0;
     if (plan->cu_large && (sums || copies)) {
-        const int blocks = cu_waves(a.op, a.cyc_len) / (plan->threads / 64);
+        const int blocks = cu_waves(a.op, a.cyc_len, (uint64_t)a.pipes * a.row_bytes) / (plan->threads / 64);
         if (blocks * (plan->threads / 64) < 32) plan->cu_lds = (160 << 10) / blocks / 1280 * 1280;
     }
     CuRingArgs& c = plan->cu_args;
