@@ -89,15 +89,11 @@ __device__ __forceinline__ u32x4 cu_load(const uint8_t* uniform, uint32_t lane) 
     else return *p;
 }
 // How results are stored: past the last-level cache (nt), through the XCD's L2
-// (sc1), or both.  Through the L2 a block's results are on their way while others
-// still load, and nothing is left to write back when the launch ends.  8 ranks,
-// kept in the L2 / nt / sc1 / sc1 nt:
+// (sc1), or both.  8 ranks, kept in the L2 / nt / sc1 / sc1 nt:
 //   small, a row to several places: allgather of 8 x 8 MiB  9.9 / 10.5 /  8.2 / 10.1 us
 //   small, a row to one place:      sendrecv of 48 MiB     18.8 / 13.7 / 16.4 / 13.4
 //   large, several:                 allgather of 8 x 64 MiB   - / 73.4 / 94.3 / 67.7
 //   large, one:                     reduce-scatter of 64 MiB 86.9 / 88.6 / 82.1 / 88.0
-// No builtin stores 16 bytes with sc1 at any address; the gap behind the store
-// keeps the next instruction off its data registers.
 enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
 constexpr int cu_stores(bool large, bool several) {
     return several ? (large ? CU_SC1_NT : CU_SC1) : large ? CU_SC1 : CU_NT;
@@ -106,10 +102,8 @@ template <int HOW>
 __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 v) {
     if constexpr (HOW == CU_NT)
         __builtin_nontemporal_store(v, (MINT_GLOBAL u32x4_unaligned*)(as_global(uniform) + lane));
-    else if constexpr (HOW == CU_SC1)
-        asm volatile("global_store_dwordx4 %0, %1, %2 sc1\n\ts_nop 0" ::"v"(lane), "v"(v), "s"(uniform) : "memory");
     else
-        asm volatile("global_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 0" ::"v"(lane), "v"(v), "s"(uniform) : "memory");
+        st128_through<HOW == CU_SC1_NT>(uniform, lane, v);
 }
 
 // A row cut into vectors of 16 bytes whose stores are aligned: vector i covers

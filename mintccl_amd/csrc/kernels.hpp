@@ -267,11 +267,13 @@ __global__ void __launch_bounds__(256) step_mix_deep_kernel(const uint8_t* rows,
 // ---- LL128 codec, wave64 layout: one wavefront per block -------------------
 // Bound by memory from some MiB on.  A wavefront moves one block and ends (the
 // loop is for messages beyond 2^31 threads), so that what is in flight is one
-// window that moves through memory; the lines stay in the last-level cache for
-// whoever unpacks them, the raw bytes that unpack leaves are streamed past it.
-// pack + unpack, resident wavefronts that stride / this: 4 MiB 5.6 / 5.1 us, 24 MiB
-// 19.6 / 18.3, 32 MiB 25.6 / 22.9, 64 MiB 47.0 / 45.7 (both streamed: 27, 49).
-constexpr uint32_t kCodecThreads = 256;
+// window that moves through memory; the lines go through the L2 into the last-level
+// cache for whoever unpacks them, the raw bytes that unpack leaves past it.
+// pack + unpack, resident wavefronts that stride / a wavefront per block and plain
+// stores / this: 16 MiB 14.1 / 13.7 / 13.0 us, 32 MiB 25.6 / 22.8 / 22.2, 48 MiB 36.7 /
+// 34.7 / 32.4, 64 MiB 47.0 / 45.4 / 42.4 (blocks of 256 threads 2 % slower, of 64 2 %
+// faster from 8 MiB on and a tenth slower at 4).
+constexpr uint32_t kCodecThreads = 128;
 __global__ void __launch_bounds__(kCodecThreads) pack_wave64_kernel(const uint8_t* __restrict__ raw,
                                                                     uint8_t* __restrict__ msg, uint64_t nbytes,
                                                                     uint32_t nblocks, uint32_t waves,
@@ -288,7 +290,7 @@ __global__ void __launch_bounds__(kCodecThreads) pack_wave64_kernel(const uint8_
         // line = two sectors; both carry the low 32 bits of the line's flag
         const uint64_t flag = flag_base + ((uint64_t)g * 8u + (m.sector >> 1)) * flag_stride;
         if (m.flag_lane) v.w = (uint32_t)flag;
-        *(MINT_GLOBAL u32x4*)(as_global(msg + (uint64_t)g * kBlockMsg) + m.lane * 16u) = v;
+        st128_through<false>(msg + (uint64_t)g * kBlockMsg, m.lane * 16u, v);
     }
 }
 __global__ void __launch_bounds__(kCodecThreads) unpack_wave64_kernel(const uint8_t* __restrict__ msg,
@@ -309,7 +311,10 @@ __global__ void __launch_bounds__(kCodecThreads) unpack_wave64_kernel(const uint
             wrong |= wrong << 4;
             bad += (uint32_t)__popcll(wrong & 0x8080808080808080ull);
         }
-        ll_save_raw(raw, nbytes, g, m, v);
+        const uint64_t base = (uint64_t)g * kBlockRawLL;
+        if (base + kBlockRawLL > nbytes) store_guarded(raw, base + m.raw_off, m.raw_len, nbytes, v);
+        else if (m.flag_lane) st96_through<true>(raw + base, m.raw_off, u32x3{v.x, v.y, v.z});
+        else st128_through<true>(raw + base, m.raw_off, v);
     }
     if (bad && lane_id() == 0) atomicAdd(bad_flags, (unsigned long long)bad);
 }

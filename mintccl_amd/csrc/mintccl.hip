@@ -725,10 +725,12 @@ size_t mint_ll128_packed_bytes(size_t nbytes, int layout) {
 namespace {
 // Thread blocks of the codec: one wavefront per block of the message, but no
 // more threads than a launch may have; pair layout: 8 blocks per compute unit.
+constexpr uint32_t kPairThreads = 256;
 uint32_t codec_blocks(uint64_t lines, int layout) {
-    const uint64_t waves = layout == MINT_LAYOUT_WAVE64 ? lines / 8 : (lines * 8 + 63) / 64;
-    const uint64_t blocks = (waves + kCodecThreads / 64 - 1) / (kCodecThreads / 64);
-    const uint64_t cap = layout == MINT_LAYOUT_WAVE64 ? (1ull << 31) / kCodecThreads : (uint64_t)device_cus() * 8;
+    const bool wave64 = layout == MINT_LAYOUT_WAVE64;
+    const uint64_t threads = wave64 ? kCodecThreads : kPairThreads, work = lines * 8;     // (one thread each)
+    const uint64_t cap = wave64 ? (1ull << 31) / threads : (uint64_t)device_cus() * 8;
+    const uint64_t blocks = (work + threads - 1) / threads;
     return (uint32_t)(cap && blocks > cap ? cap : blocks);
 }
 }  // namespace
@@ -748,7 +750,7 @@ int mint_ll128_pack(const void* raw, void* msg, size_t nbytes, uint64_t flag_bas
         return Launch<&pack_wave64_kernel>::go(blocks, kCodecThreads, 0, as_stream(stream), from, to, nbytes,
                                                (uint32_t)(lines / 8), blocks * (kCodecThreads / 64), flag_base,
                                                flag_stride);
-    return Launch<&pack_pair_kernel>::go(blocks, kCodecThreads, 0, as_stream(stream), from, to, nbytes, lines,
+    return Launch<&pack_pair_kernel>::go(blocks, kPairThreads, 0, as_stream(stream), from, to, nbytes, lines,
                                          flag_base, flag_stride);
 }
 
@@ -768,7 +770,7 @@ int mint_ll128_unpack(const void* msg, void* raw, size_t nbytes, uint64_t flag_b
         return Launch<&unpack_wave64_kernel>::go(blocks, kCodecThreads, 0, as_stream(stream), from, to, nbytes,
                                                  (uint32_t)(lines / 8), blocks * (kCodecThreads / 64), flag_base,
                                                  flag_stride, bad);
-    return Launch<&unpack_pair_kernel>::go(blocks, kCodecThreads, 0, as_stream(stream), from, to, nbytes, lines,
+    return Launch<&unpack_pair_kernel>::go(blocks, kPairThreads, 0, as_stream(stream), from, to, nbytes, lines,
                                            flag_base, flag_stride, bad);
 }
 

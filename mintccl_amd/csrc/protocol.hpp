@@ -34,6 +34,26 @@ typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 typedef u32x3 u32x3_a1 __attribute__((aligned(1)));
 typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
 
+// Stores to `uniform + lane` (uniform: the same in every lane) that go through the
+// L2 of the XCD (sc1) and, NT, past the last-level cache, at any address: no builtin
+// has both.  What is stored so is on its way while the rest of the launch runs; what
+// stays in the L2 is written back when the launch ends.  The gap behind the store
+// keeps the next instruction off its data registers.
+template <bool NT>
+__device__ __forceinline__ void st128_through(uint8_t* uniform, uint32_t lane, u32x4 v) {
+    if constexpr (NT)
+        asm volatile("global_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 0" ::"v"(lane), "v"(v), "s"(uniform) : "memory");
+    else
+        asm volatile("global_store_dwordx4 %0, %1, %2 sc1\n\ts_nop 0" ::"v"(lane), "v"(v), "s"(uniform) : "memory");
+}
+template <bool NT>
+__device__ __forceinline__ void st96_through(uint8_t* uniform, uint32_t lane, u32x3 v) {
+    if constexpr (NT)
+        asm volatile("global_store_dwordx3 %0, %1, %2 sc1 nt\n\ts_nop 0" ::"v"(lane), "v"(v), "s"(uniform) : "memory");
+    else
+        asm volatile("global_store_dwordx3 %0, %1, %2 sc1\n\ts_nop 0" ::"v"(lane), "v"(v), "s"(uniform) : "memory");
+}
+
 constexpr uint32_t kLineBytes = 128, kLinePayload = 120;
 constexpr uint32_t kBlockMsg = 1024, kBlockRawLL = 960, kBlockRawSimple = 1024;
 constexpr uint32_t kFlagLaneRaw = 768;    // first raw byte carried by a flag lane
