@@ -1,4 +1,6 @@
 // The kernels of rings inside compute units (cu_ring.hpp) and their launcher.
+#include <algorithm>
+
 #include "ring_launch.hpp"
 
 namespace mint {
@@ -14,8 +16,8 @@ int launch_as(const Plan& plan, hipStream_t stream) {
         if (SPLIT) tables.rank[N + i] = a.output[i];
     }
     tables.status = a.status;
-    const uint32_t x = s.tiles + a.ends, y = a.op == OP_ALLTOALL ? a.len : a.pipes;
-    const dim3 grid(plan.cu_large ? x : y, plan.cu_large ? y : x, a.op == OP_ALLTOALL ? a.len : 1u);
+    const uint32_t x = s.tiles + a.ends;
+    const dim3 grid(plan.cu_large ? x : a.pipes, plan.cu_large ? a.pipes : x);
     return Launch<KERNEL>::go(grid, (unsigned)plan.threads, (unsigned)plan.cu_lds, stream, s.row_bytes,
                               s.row_stride, s.short_bytes, s.starts, s.full, s.tiles, tables);
 }
@@ -49,12 +51,39 @@ int launch_ranks(const Plan& plan, int dtype, hipStream_t stream) {
     }
 }
 
+int launch_alltoall(const Plan& plan, hipStream_t stream) {
+    const CuRingArgs& a = plan.cu_args;
+    const CuShape& s = a.shape;
+    CuPairs<uint64_t> far = {};
+    CuPairs<uint32_t> near = {};
+    uint64_t lowest = ~0ull, rest = 0;            // rest: what the short form cannot say
+    for (uint32_t i = 0; i < a.len; ++i) {
+        far.rank[i] = a.input[i];
+        far.rank[kMaxRanks + i] = a.output[i];
+        lowest = std::min({lowest, a.input[i], a.output[i]});
+    }
+    for (uint32_t i = 0; i < 2 * kMaxRanks; ++i) {
+        const uint64_t off = far.rank[i] ? far.rank[i] - lowest : 0;
+        near.rank[i] = (uint32_t)(off >> kCuNearShift);
+        rest |= off ^ (uint64_t)near.rank[i] << kCuNearShift;
+    }
+    const uint32_t x = s.tiles + a.ends;
+    const dim3 grid(plan.cu_large ? x : a.len, plan.cu_large ? a.len : x, a.len);
+    const unsigned threads = (unsigned)plan.threads;
+    if (plan.cu_large)
+        return Launch<&cu_alltoall_kernel<true, uint64_t>>::go(grid, threads, 0, stream, s.row_bytes, s.row_stride,
+                                                               lowest, a.status, s.tiles, far);
+    if (rest)
+        return Launch<&cu_alltoall_kernel<false, uint64_t>>::go(grid, threads, 0, stream, s.row_bytes, s.row_stride,
+                                                                lowest, a.status, s.tiles, far);
+    return Launch<&cu_alltoall_kernel<false, uint32_t>>::go(grid, threads, 0, stream, s.row_bytes, s.row_stride,
+                                                            lowest, a.status, s.tiles, near);
+}
+
 }  // namespace
 
 int launch_cu_ring(const Plan& plan, int dtype, hipStream_t stream) {
-    if (plan.cu_args.op == OP_ALLTOALL)
-        return plan.cu_large ? launch_as<&cu_alltoall_kernel<true>, kMaxRanks, true>(plan, stream)
-                             : launch_as<&cu_alltoall_kernel<false>, kMaxRanks, true>(plan, stream);
+    if (plan.cu_args.op == OP_ALLTOALL) return launch_alltoall(plan, stream);
     switch (plan.cu_args.len) {
         case 2: return launch_ranks<2>(plan, dtype, stream);
         case 3: return launch_ranks<3>(plan, dtype, stream);

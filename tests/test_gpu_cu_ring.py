@@ -87,6 +87,7 @@ def test_copying_rows(dev, world, nbytes):
 @pytest.mark.parametrize("shift", [1, 3, 8, 16, 30])
 def test_rows_at_any_byte_touch_nothing_else(dev, shift):
     from mintccl_amd import _lib
+    from mintccl_amd.alltoall import alltoall
     from mintccl_amd.broadcast import broadcast
     world, n = 8, 3001
     comm = make_comm(world)
@@ -103,6 +104,15 @@ def test_rows_at_any_byte_touch_nothing_else(dev, shift):
         assert np.array_equal(as_bytes(backing[r])[shift: shift + world * n * 2], want[r]), r
         assert torch.all(backing[r][:shift] == 0x5A) and torch.all(backing[r][shift + world * n * 2:] == 0x5A)
     views = [b[shift: shift + world * n * 2] for b in backing]
+    # (addresses that are no multiples of 256 bytes from each other)
+    taken = [torch.full((world * n * 2 + 32 + 2 * r,), 0x5A, dtype=torch.uint8, device=dev)[2 * r:] for r in range(world)]
+    outs = [t[shift: shift + world * n * 2] for t in taken]
+    comm.run(lambda r: alltoall(views[r], outs[r], comm))
+    comm.check()
+    for r in range(world):
+        row = slice(r * n * 2, (r + 1) * n * 2)
+        assert torch.equal(outs[r], torch.cat([v[row] for v in views])), r
+        assert torch.all(taken[r][:shift] == 0x5A) and torch.all(taken[r][shift + world * n * 2:] == 0x5A)
     root = views[2].clone()
     comm.run(lambda r: broadcast(views[r], 2, comm))
     comm.check()
