@@ -25,6 +25,9 @@ int launch_as(const Plan& plan, hipStream_t stream) {
 // (in place only in the small form: to the large one the host's time is nothing)
 template <int DT, int N, bool EVERYWHERE>
 int launch_sum(const Plan& plan, hipStream_t stream) {
+    if constexpr (N >= kCuStreamRanks && !EVERYWHERE)
+        if (plan.cu_stream)
+            return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, true, true, CU_NT>, N, true>(plan, stream);
     if (plan.cu_large) return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, true, true>, N, true>(plan, stream);
     if (plan.cu_args.split)
         return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, false, true>, N, true>(plan, stream);

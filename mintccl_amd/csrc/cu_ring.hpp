@@ -98,6 +98,12 @@ enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
 constexpr int cu_stores(bool large, bool several) {
     return several ? (large ? CU_SC1_NT : CU_SC1) : large ? CU_SC1 : CU_NT;
 }
+// Sums to one place that are far larger than the last-level cache (plan_cu): with
+// many rows to read nt is the faster one.  sc1 / nt, us, 8 / 7 / 6 / 5 / 4 ranks:
+// bf16, 0.5 GiB touched 83 / 88, 84 / 90, 90 / 92, 93 / 95,  98 /  98;
+//       1 GiB          175 / 173, 190 / 182, 186 / 179, 186 / 184, 195 / 198;
+// f16,  1 GiB          180 / 178, 192 / 186, 196 / 190, 194 / 193, 197 / 202.
+constexpr int kCuStreamRanks = 6;
 template <int HOW>
 __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 v) {
     if constexpr (HOW == CU_NT)
@@ -167,7 +173,7 @@ __device__ __forceinline__ void cu_here(P* (&x)[N]) {
 
 // Rings that add: N ranks, the sum goes to the root of the pipeline (reduce,
 // reduce-scatter) or, EVERYWHERE, to all of them (allreduce).
-template <int DT, int N, bool EVERYWHERE, bool LARGE, bool SPLIT>
+template <int DT, int N, bool EVERYWHERE, bool LARGE, bool SPLIT, int STORES = cu_stores(LARGE, EVERYWHERE)>
 __global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(CU_SHAPE, const CuTables<N, SPLIT> a) {
     constexpr uint32_t kSize = DT == DT_F32 ? 4u : 2u, kThreads = cu_threads(LARGE, false), kTile = kThreads * 16u;
     const uint32_t tile = LARGE ? blockIdx.x : blockIdx.y, p = LARGE ? blockIdx.y : blockIdx.x;
@@ -213,7 +219,7 @@ __global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(C
 #pragma unroll
         for (int h = 1; h < N; ++h) x = ll_comp<DT>(v[h], x);
 #pragma unroll
-        for (int i = 0; i < kStored; ++i) cu_store<cu_stores(LARGE, EVERYWHERE)>(to[i] + ((int64_t)row_off + base), lane, x);
+        for (int i = 0; i < kStored; ++i) cu_store<STORES>(to[i] + ((int64_t)row_off + base), lane, x);
     }
 }
 

@@ -93,6 +93,8 @@ int plan_cu(Plan* plan) {
     const uint64_t touched = (uint64_t)a.pipes * a.row_bytes *
                              (alltoall || a.op == OP_SENDRECV ? 2u : (uint64_t)a.cyc_len);
     plan->cu_large = touched > ((uint64_t)(copies ? 88 : sums ? 100 : 192) << 20);
+    // Far beyond it the sums of many ranks are as well streamed (kCuStreamRanks).
+    plan->cu_stream = sums && a.op != OP_ALLREDUCE && a.cyc_len >= kCuStreamRanks && touched > (640ull << 20);
     plan->threads = (int)cu_threads(plan->cu_large, copies);
     // (held to that number by the share of LDS its blocks ask for; LDS is handed
     // out in units of 1280 bytes)

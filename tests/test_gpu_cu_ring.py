@@ -84,6 +84,30 @@ def test_copying_rows(dev, world, nbytes):
         assert torch.equal(flat[r].cpu(), host[world - 1][world - 1]), r
 
 
+@pytest.mark.parametrize("world,dt", [(8, "f16"), (7, "bf16"), (6, "f32")])
+def test_sums_far_beyond_the_cache(dev, world, dt):
+    """More than 640 MiB touched, rows that end in the middle of a vector."""
+    from mintccl_amd.reduce import reduce
+    from mintccl_amd.reducescatter import reducescatter
+    dtype = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[dt]
+    comm = make_comm(world)
+    n = (648 << 20) // (world * world * dtype.itemsize) + 5
+    g = torch.Generator(device=dev).manual_seed(world)
+    made = [torch.randn((world, n), generator=g, device=dev, dtype=torch.float32).to(dtype) for _ in range(world)]
+    for op, root in ((reducescatter, None), (reduce, 2)):
+        bufs = [m.clone() for m in made]
+        comm.run(lambda r: op(bufs[r], comm) if root is None else op(bufs[r], root, comm))
+        comm.check()
+        for r in range(world):
+            want = made[r].clone()
+            for row in [r] if root is None else range(world) if r == root else []:
+                x = made[r][row]
+                for h in range(1, world):
+                    x = made[(r + h) % world][row] + x
+                want[row] = x
+            assert torch.equal(bufs[r].view(torch.uint8), want.view(torch.uint8)), (op.__name__, r)
+
+
 @pytest.mark.parametrize("shift", [1, 3, 8, 16, 30])
 def test_rows_at_any_byte_touch_nothing_else(dev, shift):
     from mintccl_amd import _lib
