@@ -30,6 +30,8 @@ are already resident in HBM.  Prints ONE JSON line:
   step_mix  the same number of wavefronts doing the loads and stores of the
             same number of ring steps with no flags and no waiting
             (mint_step_mix): what the device needs for this mix of accesses.
+  operator_defaults  the same collective, inputs and checks on a communicator
+            that names nothing about the wire: rings inside compute units.
   copy_* / read_*  measured HBM copy and read bandwidth of the library's own
             16 B / lane kernels on 1 GiB.
   cpu_baseline  the PyTorch-CPU walk of the same collective through the same
@@ -276,6 +278,22 @@ def main() -> int:
         return 1
     kernel_ms = sum(s.elapsed_time(e) for s, e in zip(starts, stops)) / args.steps
 
+    # the same with nothing named about the wire: what a program gets by default
+    default_comm = VirtualComm(world_size=WORLD, device=dev)
+    for i in range(args.warmup + args.steps):
+        restore()
+        if i >= args.warmup:
+            starts[i - args.warmup].record()
+        default_comm.run(lambda r: reducescatter(bufs[r], default_comm))
+        if i >= args.warmup:
+            stops[i - args.warmup].record()
+    torch.cuda.synchronize()
+    default_comm.check()
+    if not verify():
+        print("bench.py: the reduce-scatter at the operators' defaults is wrong", file=sys.stderr)
+        return 1
+    default_ms = sum(s.elapsed_time(e) for s, e in zip(starts, stops)) / args.steps
+
     small_ms = None
     if args.also_64mib:
         # the other reading of the baseline's headline (its config 4: 32 Mi
@@ -362,6 +380,11 @@ def main() -> int:
                      "kernel_over_mix": round(kernel_ms / mix_ms, 4),
                      "what": "own-row load + staging load + staging store per step, no flags, "
                              "no waiting (mint_step_mix)"},
+        "operator_defaults": {"ms_per_step": round(default_ms, 4),
+                              "hbm_gbps": round(hbm_bytes / default_ms / 1e6, 1),
+                              "frac": round(hbm_bytes / default_ms / 1e6 / HBM_PEAK_GBPS, 4),
+                              "what": "the same collective with nothing named about the wire: all hops of "
+                                      "a ring inside a compute unit, no staging"},
         "algbw_gbps": round(algbw, 1), "busbw_gbps": round(algbw * (WORLD - 1) / WORLD, 1),
         "flag_bytes_frac_of_staging": round(8 / 128, 4),
     }
