@@ -33,7 +33,7 @@ _KIND = _lib.KIND_ALLREDUCE
 # on (measured on MI355X, 8 ranks, f16: 104 / 110 us at 16 MiB, 199 / 192 at 32 MiB, 1510 /
 # 1384 at 256 MiB; below, the second launch costs more than it gains: 12 / 18 us
 # at 64 KiB).  Inside compute units the two phases share nothing: one pass is
-# 205 us at 64 MiB of bf16 where two launches through staging take 368.
+# 161 us at 64 MiB of bf16 where two launches through staging take 368.
 SPLIT_FROM_BYTES = 32 << 20
 
 
