@@ -700,7 +700,7 @@ PyObject* board_name;
 struct Front {
     PyObject_HEAD
     vectorcallfunc call;
-    PyObject *op, *go_on, *dict;
+    PyObject *op, *go_on, *dict, *weak;
     int action;
 };
 
@@ -769,11 +769,19 @@ PyObject* front_new(PyTypeObject* type, PyObject* args, PyObject*) {
 }
 void front_dealloc(PyObject* self) {
     Front* f = reinterpret_cast<Front*>(self);
+    if (f->weak) PyObject_ClearWeakRefs(self);
     Py_XDECREF(f->op);
     Py_XDECREF(f->go_on);
     Py_XDECREF(f->dict);
     Py_TYPE(self)->tp_free(self);
 }
+// It is handed on like the function it stands for: pickled and copied by its name
+// in its module, bound where a class holds it, referred to weakly.
+PyObject* front_reduce(PyObject* self, PyObject*) { return PyObject_GetAttrString(self, "__qualname__"); }
+PyObject* front_bind(PyObject* self, PyObject* object, PyObject*) {
+    return object && object != Py_None ? PyMethod_New(self, object) : Py_NewRef(self);
+}
+PyMethodDef front_methods[] = {{"__reduce__", front_reduce, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyTypeObject front_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 // (functools.update_wrapper gives it the operator's name, documentation and signature)
 PyGetSetDef front_getset[] = {{"__dict__", PyObject_GenericGetDict, PyObject_GenericSetDict, nullptr, nullptr},
@@ -900,6 +908,9 @@ PyMODINIT_FUNC PyInit__host(void) {
     front_type.tp_call = PyVectorcall_Call;
     front_type.tp_vectorcall_offset = offsetof(Front, call);
     front_type.tp_dictoffset = offsetof(Front, dict);
+    front_type.tp_weaklistoffset = offsetof(Front, weak);
+    front_type.tp_descr_get = front_bind;
+    front_type.tp_methods = front_methods;
     front_type.tp_getset = front_getset;
     if (PyType_Ready(&front_type) < 0) return nullptr;
     for (int k = 0; k < ACTIONS; ++k)
