@@ -8,6 +8,7 @@ on one GPU they reduce to a device choice and a pointer mailbox.
 """
 from __future__ import annotations
 
+import functools
 import math
 import os
 import time
@@ -428,8 +429,16 @@ class VirtualComm:
         return self._board.rank()
 
     def rank(self, r: int):
-        """``with comm.rank(r):`` - the thread speaks for rank ``r`` inside."""
+        """``with comm.rank(r):`` - the thread speaks for rank ``r`` inside (as a
+        decorator: in the function)."""
         return self._board.speak(r)
+
+    def _speaking(self, r: int, fn):
+        @functools.wraps(fn)
+        def speaks(*args, **kw):
+            with self.rank(r):
+                return fn(*args, **kw)
+        return speaks
 
     def run(self, fn) -> None:
         """SPMD helper: ``fn(rank)`` for every rank in turn (like mpirun)."""

@@ -535,6 +535,14 @@ PyObject* context_exit(PyObject* self, PyObject* const*, Py_ssize_t) {
     enter_rank(c->board, c->before);
     Py_RETURN_NONE;
 }
+// (as a decorator: every call of the function enters a context of its own)
+PyObject* context_call(PyObject* self, PyObject* args, PyObject* kwargs) {
+    RankContext* c = reinterpret_cast<RankContext*>(self);
+    PyObject* fn;
+    if (kwargs && PyDict_GET_SIZE(kwargs)) return raise(PyExc_TypeError, "a rank's decorator takes a function");
+    if (!PyArg_ParseTuple(args, "O", &fn)) return nullptr;
+    return PyObject_CallMethod(c->comm, "_speaking", "iO", c->rank, fn);
+}
 PyMethodDef context_methods[] = {
     {"__enter__", context_enter, METH_NOARGS, nullptr},
     {"__exit__", (PyCFunction)(void (*)(void))context_exit, METH_FASTCALL, nullptr},
@@ -896,8 +904,9 @@ PyMODINIT_FUNC PyInit__host(void) {
     context_type.tp_name = "mintccl_amd._host.RankContext";
     context_type.tp_basicsize = sizeof(RankContext);
     context_type.tp_flags = Py_TPFLAGS_DEFAULT;
-    context_type.tp_doc = "with comm.rank(r): the thread speaks for rank r inside";
+    context_type.tp_doc = "with comm.rank(r): the thread speaks for rank r inside; @comm.rank(r): in the function";
     context_type.tp_dealloc = context_dealloc;
+    context_type.tp_call = context_call;
     context_type.tp_methods = context_methods;
     if (PyType_Ready(&board_type) < 0 || PyType_Ready(&context_type) < 0) return nullptr;
     front_type.tp_name = "mintccl_amd._host.Front";

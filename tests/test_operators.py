@@ -1,4 +1,5 @@
-"""The operators as Python objects (no GPU needed): what a function can do."""
+"""The operators and the communicator as Python objects (no GPU needed): what a
+function and a context manager can do."""
 import copy
 import importlib
 import inspect
@@ -7,9 +8,21 @@ import weakref
 
 import pytest
 
+from mintccl_amd import common
+
 OPERATORS = [("broadcast", "broadcast"), ("reduce", "reduce"), ("allgather", "allgather"),
              ("reducescatter", "reducescatter"), ("allreduce", "allreduce"), ("alltoall", "alltoall"),
              ("sendrecv_buffer", "send"), ("sendrecv_buffer", "recv"), ("sendrecv_buffer", "sync")]
+
+
+@pytest.fixture
+def make_comm(monkeypatch):
+    """A communicator whose memory lies on the host: nothing can be launched."""
+    monkeypatch.setattr(common, "_xcd_count", lambda device: 8)
+    for knob in ("NUM_BLOCKS", "NUM_WARPS", "BUFFSIZE", "NSLOTS", "PLACEMENT", "THREADS", "CACHE",
+                 "ROW_FETCH", "ORIGIN_CUS", "PROTOCOL"):
+        monkeypatch.delenv("MINTCCL_" + knob, raising=False)
+    return lambda world=4, cls=common.VirtualComm, **kw: cls(world, device="cpu", **kw)
 
 
 @pytest.mark.parametrize("module,name", OPERATORS)
@@ -27,3 +40,24 @@ def test_an_operator_can_be_handed_on_like_a_function(module, name):
     holder = Holder()
     assert Holder.held is op
     assert holder.held.__self__ is holder and holder.held.__func__ is op
+
+
+def test_a_rank_as_a_decorator(make_comm):
+    comm = make_comm()
+
+    @comm.rank(2)
+    def who(x, *, y):
+        """docs"""
+        return comm.Get_rank(), x, y
+    assert who.__name__ == "who" and who.__doc__ == "docs"
+    for _ in range(2):
+        assert who(1, y=3) == (2, 1, 3)
+        with comm.rank(1):
+            assert who(4, y=5) == (2, 4, 5) and comm.Get_rank() == 1
+
+    @comm.rank(3)
+    def nested(depth):
+        return nested(depth - 1) if depth else comm.Get_rank()
+    assert nested(2) == 3
+    with pytest.raises(RuntimeError, match="no current rank"):
+        comm.Get_rank()
