@@ -518,6 +518,7 @@ struct RankContext {
     PyObject* comm;              // owns the board
     Board* board;
     int rank, before;
+    bool inside;
 };
 PyTypeObject context_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 void context_dealloc(PyObject* self) {
@@ -527,11 +528,15 @@ void context_dealloc(PyObject* self) {
 }
 PyObject* context_enter(PyObject* self, PyObject*) {
     RankContext* c = reinterpret_cast<RankContext*>(self);
+    // (a second way in would forget whose rank the thread had before the first)
+    if (c->inside) return raise(PyExc_RuntimeError, "this context of a rank is entered already");
+    c->inside = true;
     c->before = enter_rank(c->board, c->rank);
     return Py_NewRef(c->comm);
 }
 PyObject* context_exit(PyObject* self, PyObject* const*, Py_ssize_t) {
     RankContext* c = reinterpret_cast<RankContext*>(self);
+    c->inside = false;
     enter_rank(c->board, c->before);
     Py_RETURN_NONE;
 }
@@ -561,6 +566,7 @@ PyObject* board_speak(PyObject* self, PyObject* arg) {
     c->board = reinterpret_cast<Board*>(Py_NewRef(self));
     c->rank = (int)r;
     c->before = -1;
+    c->inside = false;
     return reinterpret_cast<PyObject*>(c);
 }
 PyObject* board_rank(PyObject* self, PyObject*) {

@@ -61,3 +61,16 @@ def test_a_rank_as_a_decorator(make_comm):
     assert nested(2) == 3
     with pytest.raises(RuntimeError, match="no current rank"):
         comm.Get_rank()
+
+
+def test_a_rank_context_is_not_entered_twice_at_a_time(make_comm):
+    """The second way in would forget whose rank the thread had before the first."""
+    comm = make_comm()
+    context = comm.rank(1)
+    with context:
+        with pytest.raises(RuntimeError, match="entered"):
+            with context:
+                pass
+        assert comm.Get_rank() == 1
+    with pytest.raises(RuntimeError, match="no current rank"):
+        comm.Get_rank()
