@@ -45,7 +45,7 @@ def chunk_bytes(count: int, world: int) -> int:
 def _go_on(comm: VirtualComm, posted: tuple) -> None:
     """All ranks are here, and it is not the board's to launch."""
     count, dtype, _, variant, ptrs, _, _ = posted
-    fused = count < SPLIT_FROM_BYTES or comm.inside_cu if variant < 0 else bool(variant)
+    fused = count < SPLIT_FROM_BYTES or comm._runs_inside() if variant < 0 else bool(variant)
     ring = ring_of(comm)
     if fused:
         comm.enqueue(_lib.OP_ALLREDUCE, dtype, count, ptrs, ptrs, ring)

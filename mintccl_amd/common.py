@@ -275,9 +275,11 @@ def _largest_divisor_at_most(n: int, cap: int) -> int:
     return 1
 
 
-# attributes a native launch takes from the communicator (VirtualComm._refresh)
+# what the board takes from the communicator (VirtualComm._refresh): attributes
+# of a launch, and methods that it passes by unless they have been replaced
 _LAUNCH_ATTRIBUTES = frozenset(("inside_cu", "stats", "epoch_word", "protocol", "spin_budget", "status",
                                 "topology"))
+_PASSED_BY = frozenset(("launch", "enqueue", "make_op", "make_cu_op", "Get_rank", "rank"))
 
 
 class VirtualComm:
@@ -393,8 +395,22 @@ class VirtualComm:
 
     def __setattr__(self, name: str, value) -> None:
         object.__setattr__(self, name, value)
-        if name in _LAUNCH_ATTRIBUTES and "_board" in self.__dict__:
+        if (name in _LAUNCH_ATTRIBUTES or name in _PASSED_BY) and "_board" in self.__dict__:
             self._board.stale()
+
+    def __delattr__(self, name: str) -> None:
+        object.__delattr__(self, name)
+        if (name in _LAUNCH_ATTRIBUTES or name in _PASSED_BY) and "_board" in self.__dict__:
+            self._board.stale()
+
+    def _replaced(self, *methods: str) -> bool:
+        """Whether a subclass or this object brings one of ``methods`` itself."""
+        return any(m in self.__dict__ or getattr(type(self), m) is not _METHODS[m] for m in methods)
+
+    def _runs_inside(self) -> bool:
+        """Whether rings run inside compute units (a make_op of one's own
+        describes launches through staging)."""
+        return self.inside_cu and self.stats is None and not self._replaced("make_op")
 
     def _refresh(self) -> None:
         """Tell the board what launches take from this communicator (it asks
@@ -402,9 +418,11 @@ class VirtualComm:
         from ._ops import ring_of
         try:
             ring = ring_of(self)
-        except RuntimeError:
+        except Exception:
             ring = []                  # routes only: a collective will say so
-        self._board.configure(self.inside_cu and self.stats is None and self.epoch_word is None,
+        self._board.configure(self._runs_inside() and self.epoch_word is None and
+                              not self._replaced("launch", "enqueue", "make_cu_op"),
+                              self._replaced("Get_rank"), self._replaced("rank"),
                               ring, self.protocol, self.spin_budget, self.status.data_ptr())
 
     def _find_route(self, src: int, dst: int) -> list[int]:
@@ -443,6 +461,11 @@ class VirtualComm:
     def run(self, fn) -> None:
         """SPMD helper: ``fn(rank)`` for every rank in turn (like mpirun)."""
         self._board.run(fn)
+
+    def _in_turn(self, fn) -> None:
+        for r in range(self.world_size):
+            with self.rank(r):
+                fn(r)
 
     def staging_ptr(self, r: int) -> int:
         return self.staging.data_ptr() + r * self.rank_stride
@@ -580,7 +603,7 @@ class VirtualComm:
 
     def enqueue(self, op: int, *args, **kw) -> None:
         """Build the descriptor of a ring collective and launch it."""
-        if self.inside_cu and self.stats is None:
+        if self._runs_inside():
             self.launch(self.make_cu_op(op, *args, **kw))
         else:
             self.launch(self.make_op(op, *args, **kw))
@@ -662,6 +685,8 @@ class VirtualComm:
                 "launch(es) found the abort flag set and gave up "
                 "(outputs of every launch since the last check are unspecified)")
 
+
+_METHODS = {name: VirtualComm.__dict__[name] for name in _PASSED_BY}
 
 _default_comm: VirtualComm | None = None
 

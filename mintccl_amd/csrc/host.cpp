@@ -11,8 +11,9 @@
 // ranks' arguments.  Where the communicator's rings run inside compute units it
 // launches them itself; anything else it hands back to the operator, which goes
 // on in Python.  What a launch takes from the communicator's attributes (ring,
-// protocol, spin limit, status block) is asked for once and again after any of
-// them has been set (VirtualComm._refresh).
+// protocol, spin limit, status block, which methods a subclass or the object has
+// replaced) is asked for once and again after any of them has been set, or the
+// class has been changed (VirtualComm._refresh).
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -126,6 +127,9 @@ struct Board {
     uint64_t id;                 // of this board, in the threads' lists of ranks
     int world, device;
     bool fresh, native_launch;   // `base` is up to date; it is ours to launch
+    bool asks_rank, in_turn;     // Get_rank, rank are the communicator's own: called, not passed by
+    PyTypeObject* type;          // the communicator's class and its version when last asked
+    unsigned version;
     bool has_ring;               // (a topology may have routes and no ring)
     bool launched;
     mint_ring_op base, last;
@@ -166,6 +170,12 @@ bool rank_or_raise(const Board* b, int* rank) {
     return false;
 }
 
+// A strong reference to the communicator, or an exception.
+PyObject* comm_of(const Board* b) {
+    PyObject* comm = PyWeakref_GetObject(b->comm);
+    return comm == Py_None ? raise(PyExc_RuntimeError, "the communicator is gone") : Py_NewRef(comm);
+}
+
 void drop(Gathering* g) {
     for (int r = 0; r < MINT_MAX_RANKS; ++r)
         if (g->present >> r & 1u) {
@@ -201,17 +211,39 @@ int dtype_code(const at::Tensor& t) {
     }
 }
 
-// Brings `base` up to date with the communicator's attributes.
+// Brings `base` up to date with the communicator's attributes and methods.  A class
+// has another version, or none, once anything of it or its bases has been changed.
 bool refresh(Board* b) {
-    if (b->fresh) return true;
     PyObject* comm = PyWeakref_GetObject(b->comm);
-    if (comm == Py_None) {
-        raise(PyExc_RuntimeError, "the communicator is gone");
-        return false;
-    }
+    const PyTypeObject* type = Py_TYPE(comm);
+    if (b->fresh && b->type == type && (type->tp_flags & Py_TPFLAGS_VALID_VERSION_TAG) &&
+        b->version == type->tp_version_tag)
+        return true;
+    if (!(comm = comm_of(b))) return false;
     PyObject* done = PyObject_CallMethod(comm, "_refresh", nullptr);     // calls configure()
+    b->type = Py_TYPE(comm);
+    b->version = b->type->tp_version_tag;
+    Py_DECREF(comm);
     Py_XDECREF(done);
     return done != nullptr;
+}
+
+// The rank this call is made for.
+bool calling_rank(Board* b, int* rank) {
+    if (!refresh(b)) return false;
+    if (!b->asks_rank) return rank_or_raise(b, rank);
+    PyObject* comm = comm_of(b);
+    PyObject* got = comm ? PyObject_CallMethod(comm, "Get_rank", nullptr) : nullptr;
+    const long r = got ? PyLong_AsLong(got) : -1;
+    Py_XDECREF(got);
+    Py_XDECREF(comm);
+    if (PyErr_Occurred()) return false;
+    if (r < 0 || r >= b->world) {
+        PyErr_Format(PyExc_ValueError, "rank %ld outside world of %d", r, b->world);
+        return false;
+    }
+    *rank = (int)r;
+    return true;
 }
 
 PyObject* launch(Board* b, const mint_ring_op& op) {
@@ -250,9 +282,9 @@ bool alike(const Board* b, const Gathering& g, const char* what, Field field,
     return false;
 }
 
-// All ranks are there: launch, or hand the arguments back as
+// All ranks are there, `last` came last: launch, or hand the arguments back as
 // (count, dtype, root, variant, {rank: in}, {rank: out}, kept buffers).
-PyObject* complete(Board* b, Kind kind, const Gathering& g) {
+PyObject* complete(Board* b, Kind kind, const Gathering& g, int last) {
     const KindInfo& info = kKinds[kind];
     static const char* const kSchedules[] = {"spatial", "temporal"};
     if (!alike(b, g, "the byte count", [](const Post& p) { return p.count; })) return nullptr;
@@ -269,7 +301,7 @@ PyObject* complete(Board* b, Kind kind, const Gathering& g) {
                 if (g.post[i].in < g.post[o].out + count && g.post[o].out < g.post[i].in + count)
                     return raise(PyExc_ValueError, "alltoall: out overlaps a rank's buff");
     if (!refresh(b)) return nullptr;
-    long variant = g.post[current_rank(b)].variant;
+    long variant = g.post[last].variant;
     if (kind == ALLREDUCE && variant == UNSAID) {
         const char* e = getenv("MINTCCL_ALLREDUCE");
         if (e && *e) variant = strcasecmp(e, "split") == 0 ? SPLIT : FUSED;
@@ -369,7 +401,7 @@ PyObject* post(Board* b, Kind kind, PyObject* buff, PyObject* root, PyObject* va
             p.out = (uint64_t)o->data_ptr();
         }
         int rank;
-        if (!rank_or_raise(b, &rank)) return nullptr;
+        if (!calling_rank(b, &rank)) return nullptr;
         if (g.present >> rank & 1u) {
             PyErr_Format(PyExc_RuntimeError, "rank %d called %s twice before the others joined", rank, info.name);
             return nullptr;
@@ -384,7 +416,7 @@ PyObject* post(Board* b, Kind kind, PyObject* buff, PyObject* root, PyObject* va
         // (taken out before anything can call back or raise)
         Gathering all = g;
         g.present = 0;
-        PyObject* result = complete(b, kind, all);
+        PyObject* result = complete(b, kind, all, rank);
         drop(&all);
         return result;
     });
@@ -406,7 +438,7 @@ PyObject* transfer(Board* b, Transfer* t, PyObject* const* args, Py_ssize_t n) {
         const long peer = PyLong_AsLong(args[1]);
         if (peer == -1 && PyErr_Occurred()) return nullptr;
         int rank;
-        if (!rank_or_raise(b, &rank)) return nullptr;
+        if (!calling_rank(b, &rank)) return nullptr;
         PyObject* before = t->given ? t->keep : nullptr;
         *t = Transfer{true, rank, peer, (uint64_t)x->data_ptr(),
                       (uint64_t)x->numel() * (uint64_t)x->element_size(), Py_NewRef(args[0])};
@@ -431,9 +463,9 @@ bool take_route(Board* b, PyObject* given, int src, int dst, int8_t (&route)[MIN
     }
     PyObject* list;
     if (given == Py_None) {
-        PyObject* comm = PyWeakref_GetObject(b->comm);
-        if (comm == Py_None) return raise(PyExc_RuntimeError, "the communicator is gone") != nullptr;
-        PyObject* found = PyObject_CallMethod(comm, "_find_route", "ii", src, dst);
+        PyObject* comm = comm_of(b);
+        PyObject* found = comm ? PyObject_CallMethod(comm, "_find_route", "ii", src, dst) : nullptr;
+        Py_XDECREF(comm);
         list = found ? PySequence_Fast(found, "a route is a sequence of ranks") : nullptr;
         Py_XDECREF(found);
     } else {
@@ -576,6 +608,13 @@ PyObject* board_rank(PyObject* self, PyObject*) {
 // run(fn): fn(rank) for every rank in turn
 PyObject* board_run(PyObject* self, PyObject* fn) {
     Board* b = reinterpret_cast<Board*>(self);
+    if (!refresh(b)) return nullptr;
+    if (b->in_turn) {
+        PyObject* comm = comm_of(b);
+        PyObject* done = comm ? PyObject_CallMethod(comm, "_in_turn", "O", fn) : nullptr;
+        Py_XDECREF(comm);
+        return done;
+    }
     const int before = current_rank(b);
     PyObject* result = Py_NewRef(Py_None);
     for (int r = 0; result && r < b->world; ++r) {
@@ -606,15 +645,16 @@ PyObject* board_launching(PyObject* self, PyObject* arg) {
     PyBuffer_Release(&view);
     Py_RETURN_NONE;
 }
-// configure(native_launch, ring, protocol, spin_budget, status): what launches
-// take from the communicator; an empty ring where the topology has none
+// configure(native_launch, asks_rank, in_turn, ring, protocol, spin_budget, status):
+// what launches take from the communicator; an empty ring where the topology has none
 PyObject* board_configure(PyObject* self, PyObject* args) {
     Board* b = reinterpret_cast<Board*>(self);
-    int native_launch, protocol;
+    int native_launch, asks_rank, in_turn, protocol;
     unsigned long spin;
     unsigned long long status;
     PyObject* ring;
-    if (!PyArg_ParseTuple(args, "pOikK", &native_launch, &ring, &protocol, &spin, &status)) return nullptr;
+    if (!PyArg_ParseTuple(args, "pppOikK", &native_launch, &asks_rank, &in_turn, &ring, &protocol, &spin, &status))
+        return nullptr;
     mint_ring_op& d = b->base;
     d = mint_ring_op{};
     PyObject* list = PySequence_Fast(ring, "a ring is a sequence of ranks");
@@ -631,6 +671,8 @@ PyObject* board_configure(PyObject* self, PyObject* args) {
     d.status = status;
     memset(b->route, 0, sizeof(b->route));
     b->native_launch = native_launch;
+    b->asks_rank = asks_rank;
+    b->in_turn = in_turn;
     b->fresh = true;
     Py_RETURN_NONE;
 }

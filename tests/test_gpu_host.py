@@ -185,3 +185,77 @@ def test_operators_take_their_arguments_in_every_form(dev, monkeypatch):
                 bad()
     finally:
         set_comm(before)
+
+
+def test_methods_of_ones_own_are_called(dev, monkeypatch):
+    """A subclass's launch, make_op, Get_rank and rank are what an operator goes
+    through, on the object and on the class as well, also when they are set
+    after a launch."""
+    from mintccl_amd import _lib, common
+    from mintccl_amd.allgather import allgather
+    from mintccl_amd.broadcast import broadcast
+    world, n = 3, 1000
+    src = [torch.full((world, n), float(r), device=dev) for r in range(world)]
+    rows = torch.arange(world, device=dev, dtype=torch.float32)[:, None].expand(world, n)
+    calls = []
+
+    class Own(common.VirtualComm):
+        def launch(self, d):
+            calls.append(("launch", d.op, d.placement))
+            super().launch(d)
+
+    class Described(common.VirtualComm):
+        def make_op(self, *args, **kw):
+            calls.append("make_op")
+            return super().make_op(*args, **kw)
+
+    class Elsewhere(common.VirtualComm):
+        speaker = None
+
+        def Get_rank(self):
+            return self.speaker
+
+        def rank(self, r):
+            calls.append(r)
+            return super().rank(r)
+
+    def gather(comm, run=None):
+        calls.clear()
+        bufs = [s.clone() for s in src]
+        (run or comm.run)(lambda r: allgather(bufs[r], comm))
+        comm.check()
+        assert all(torch.equal(b, rows) for b in bufs)
+    gather(Own(world, dev))
+    assert calls == [("launch", _lib.OP_ALLGATHER, _lib.PLACE_CU)]
+    comm = Described(world, dev)
+    gather(comm)
+    assert calls == ["make_op"] and comm.epoch == 1
+    comm = Elsewhere(world, dev)
+
+    def in_turn(fn):
+        for comm.speaker in range(world):
+            fn(comm.speaker)
+    gather(comm, in_turn)
+    comm.speaker = world
+    with pytest.raises(ValueError, match="rank 3"):
+        broadcast(src[0], 0, comm)
+    comm.speaker = 0
+    comm.run(calls.append)
+    assert calls == [0, 0, 1, 1, 2, 2]
+    # after launches of an ordinary communicator: on the object, on its class
+    comm = make_comm(world)
+    gather(comm)
+    assert not calls
+    comm.launch = lambda d: (calls.append("own"), common.VirtualComm.launch(comm, d))
+    gather(comm)
+    assert calls == ["own"]
+    del comm.launch
+    gather(comm)
+    assert not calls
+    plain = common.VirtualComm.launch
+    with monkeypatch.context() as m:
+        m.setattr(common.VirtualComm, "launch", lambda self, d: (calls.append("class"), plain(self, d)))
+        gather(comm)
+        assert calls == ["class"]
+    gather(comm)
+    assert not calls

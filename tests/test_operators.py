@@ -8,7 +8,7 @@ import weakref
 
 import pytest
 
-from mintccl_amd import common
+from mintccl_amd import _lib, common
 
 OPERATORS = [("broadcast", "broadcast"), ("reduce", "reduce"), ("allgather", "allgather"),
              ("reducescatter", "reducescatter"), ("allreduce", "allreduce"), ("alltoall", "alltoall"),
@@ -74,3 +74,20 @@ def test_a_rank_context_is_not_entered_twice_at_a_time(make_comm):
         assert comm.Get_rank() == 1
     with pytest.raises(RuntimeError, match="no current rank"):
         comm.Get_rank()
+
+
+def test_a_make_op_of_ones_own_is_the_one_that_is_used(make_comm):
+    """In a subclass or on the object: it describes launches through staging."""
+    class Own(common.VirtualComm):
+        def make_op(self, *args, **kw):
+            d = super().make_op(*args, **kw)
+            d.nslots = 2
+            return d
+    comm, plain = make_comm(cls=Own), make_comm()
+    plain.make_op = lambda *args, **kw: "mine"
+    seen = []
+    for c in (comm, plain):
+        c.launch = seen.append
+        ptrs = {r: 4096 * (r + 1) for r in range(4)}
+        c.enqueue(_lib.OP_BROADCAST, _lib.BYTES, 64, {0: ptrs[0]}, ptrs, [0, 1, 2, 3, 0])
+    assert seen[0].nslots == 2 and seen[0].placement != _lib.PLACE_CU and seen[1] == "mine"
