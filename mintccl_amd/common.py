@@ -279,6 +279,10 @@ def _largest_divisor_at_most(n: int, cap: int) -> int:
 # of a launch, and methods that it passes by unless they have been replaced
 _LAUNCH_ATTRIBUTES = frozenset(("inside_cu", "stats", "epoch_word", "protocol", "spin_budget", "status",
                                 "topology"))
+# ... and attributes of launches through staging: to set one asks for staging
+_STAGING_ATTRIBUTES = frozenset(("placement", "cache_policy", "row_fetch", "origin_cus", "threads_per_block",
+                                 "threads_explicit", "waves_per_rank", "nslots", "slot_bytes", "buff_size",
+                                 "auto_geometry"))
 _PASSED_BY = frozenset(("launch", "enqueue", "make_op", "make_cu_op", "Get_rank", "rank"))
 
 
@@ -317,8 +321,9 @@ class VirtualComm:
                               and waves_per_rank is None)
         # With everything about the wire left to the library the operators' rings
         # run inside compute units; naming a placement, a cache policy, a
-        # block size, who fetches the rows or where the origins sit (arguments
-        # or MINTCCL_*) asks for the rings through staging memory.
+        # block size, who fetches the rows or where the origins sit (arguments,
+        # MINTCCL_*, or the attribute set later) asks for the rings through
+        # staging memory.
         self.inside_cu = self.auto_geometry and all(
             v is None for v in (placement, threads_per_block, cache_policy, row_fetch, origin_cus)
         ) and not any(os.getenv(k) for k in ("MINTCCL_PLACEMENT", "MINTCCL_THREADS", "MINTCCL_CACHE",
@@ -395,6 +400,8 @@ class VirtualComm:
 
     def __setattr__(self, name: str, value) -> None:
         object.__setattr__(self, name, value)
+        if name in _STAGING_ATTRIBUTES and "_board" in self.__dict__:
+            self.inside_cu = False     # as naming it in the constructor
         if (name in _LAUNCH_ATTRIBUTES or name in _PASSED_BY) and "_board" in self.__dict__:
             self._board.stale()
 

@@ -259,3 +259,17 @@ def test_methods_of_ones_own_are_called(dev, monkeypatch):
         assert calls == ["class"]
     gather(comm)
     assert not calls
+
+
+def test_an_attribute_of_the_wire_set_after_a_launch_is_in_the_next_one(dev):
+    from mintccl_amd.allgather import allgather
+    world, n = 8, 5000
+    comm = make_comm(world)
+    for launch in range(3):
+        bufs = [torch.zeros(world, n, device=dev) for _ in range(world)]
+        for r, b in enumerate(bufs):
+            b[r] = r + 1
+        comm.run(lambda r: allgather(bufs[r], comm))
+        comm.check()
+        assert comm.epoch == launch and all(torch.equal(b, bufs[0]) and b[-1, -1] == world for b in bufs)
+        comm.threads_per_block = 128

@@ -91,3 +91,29 @@ def test_a_make_op_of_ones_own_is_the_one_that_is_used(make_comm):
         ptrs = {r: 4096 * (r + 1) for r in range(4)}
         c.enqueue(_lib.OP_BROADCAST, _lib.BYTES, 64, {0: ptrs[0]}, ptrs, [0, 1, 2, 3, 0])
     assert seen[0].nslots == 2 and seen[0].placement != _lib.PLACE_CU and seen[1] == "mine"
+
+
+@pytest.mark.parametrize("name,value", [("placement", _lib.PLACE_SPREAD), ("cache_policy", 0),
+                                        ("row_fetch", _lib.FETCH_LDS), ("origin_cus", 9),
+                                        ("threads_per_block", 512), ("waves_per_rank", 64), ("nslots", 2),
+                                        ("slot_bytes", 1 << 16), ("auto_geometry", False)])
+def test_naming_the_wire_after_construction_goes_through_staging(make_comm, name, value):
+    """As naming it in the constructor does, and what is named is in the next
+    launch's descriptor."""
+    comm = make_comm(8)
+    launched = []
+    comm.launch = launched.append
+    ptrs = {r: 4096 * (r + 1) for r in range(8)}
+    ring = list(range(8)) + [0]
+
+    def launch():
+        comm.enqueue(_lib.OP_ALLGATHER, _lib.BYTES, 1 << 20, ptrs, ptrs, ring, row_stride=1 << 20)
+        return launched[-1]
+    assert comm.inside_cu and launch().placement == _lib.PLACE_CU
+    if name == "placement":
+        comm.cache_policy = 0           # (agent scope: what the spread placement takes)
+    setattr(comm, name, value)
+    d = launch()
+    assert not comm.inside_cu and d.placement != _lib.PLACE_CU and d.nslots
+    if name in ("placement", "cache_policy", "row_fetch", "origin_cus", "threads_per_block", "nslots"):
+        assert getattr(d, name) == value
