@@ -430,7 +430,7 @@ class VirtualComm:
         self._board.configure(self._runs_inside() and self.epoch_word is None and
                               not self._replaced("launch", "enqueue", "make_cu_op"),
                               self._replaced("Get_rank"), self._replaced("rank"),
-                              ring, self.protocol, self.spin_budget, self.status.data_ptr())
+                              getattr(self, "topology", None) is None, ring, self.protocol, self.spin_budget, self.status.data_ptr())
 
     def _find_route(self, src: int, dst: int) -> list[int]:
         from .topology import find_route, uniform_topology

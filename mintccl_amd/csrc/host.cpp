@@ -131,6 +131,7 @@ struct Board {
     PyTypeObject* type;          // the communicator's class and its version when last asked
     unsigned version;
     bool has_ring;               // (a topology may have routes and no ring)
+    bool keeps_routes;           // no topology of the caller's, who may change it in place
     bool launched;
     mint_ring_op base, last;
     int8_t last_route[MINT_MAX_RANKS + 1];
@@ -454,9 +455,9 @@ PyObject* board_recv(PyObject* self, PyObject* const* args, Py_ssize_t n) {
 }
 
 // Route into op.ring / op.route_len; `given`: the caller's list, or None for the
-// topology's (searched once per pair, by VirtualComm._find_route).
+// topology's (VirtualComm._find_route; where all ranks are alike once per pair).
 bool take_route(Board* b, PyObject* given, int src, int dst, int8_t (&route)[MINT_MAX_RANKS + 1]) {
-    const bool cache = given == Py_None && src < b->world && dst < b->world;
+    const bool cache = given == Py_None && b->keeps_routes && src < b->world && dst < b->world;
     if (cache && b->route[src][dst][MINT_MAX_RANKS]) {
         memcpy(route, b->route[src][dst], sizeof(route));
         return true;
@@ -645,15 +646,16 @@ PyObject* board_launching(PyObject* self, PyObject* arg) {
     PyBuffer_Release(&view);
     Py_RETURN_NONE;
 }
-// configure(native_launch, asks_rank, in_turn, ring, protocol, spin_budget, status):
-// what launches take from the communicator; an empty ring where the topology has none
+// configure(native_launch, asks_rank, in_turn, keeps_routes, ring, protocol, spin_budget,
+// status): what launches take from the communicator; an empty ring where the topology has none
 PyObject* board_configure(PyObject* self, PyObject* args) {
     Board* b = reinterpret_cast<Board*>(self);
-    int native_launch, asks_rank, in_turn, protocol;
+    int native_launch, asks_rank, in_turn, keeps_routes, protocol;
     unsigned long spin;
     unsigned long long status;
     PyObject* ring;
-    if (!PyArg_ParseTuple(args, "pppOikK", &native_launch, &asks_rank, &in_turn, &ring, &protocol, &spin, &status))
+    if (!PyArg_ParseTuple(args, "ppppOikK", &native_launch, &asks_rank, &in_turn, &keeps_routes, &ring, &protocol,
+                          &spin, &status))
         return nullptr;
     mint_ring_op& d = b->base;
     d = mint_ring_op{};
@@ -673,6 +675,7 @@ PyObject* board_configure(PyObject* self, PyObject* args) {
     b->native_launch = native_launch;
     b->asks_rank = asks_rank;
     b->in_turn = in_turn;
+    b->keeps_routes = keeps_routes;
     b->fresh = true;
     Py_RETURN_NONE;
 }

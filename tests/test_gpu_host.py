@@ -273,3 +273,31 @@ def test_an_attribute_of_the_wire_set_after_a_launch_is_in_the_next_one(dev):
         comm.check()
         assert comm.epoch == launch and all(torch.equal(b, bufs[0]) and b[-1, -1] == world for b in bufs)
         comm.threads_per_block = 128
+
+
+def test_a_topology_changed_in_place_changes_the_next_route(dev):
+    from mintccl_amd import sendrecv_buffer
+    comm = make_comm(4)
+    comm.topology = {0: [(1, 2.0)], 1: [(0, 2.0), (3, 2.0)], 2: [], 3: [(1, 2.0)]}
+    src, dst = torch.arange(1000, device=dev), torch.zeros(1000, dtype=torch.int64, device=dev)
+
+    def route():
+        dst.zero_()
+        with comm.rank(0):
+            sendrecv_buffer.send(src, 3, comm)
+        with comm.rank(3):
+            sendrecv_buffer.recv(dst, 0, comm)
+        comm.run(lambda r: sendrecv_buffer.sync(comm))
+        comm.check()
+        assert torch.equal(src, dst)
+        return comm.last_route
+    assert route() == [0, 1, 3]
+    comm.topology[0].append((2, 5.0))
+    comm.topology[2].append((3, 5.0))
+    assert route() == [0, 2, 3]
+    comm.topology[0].append((3, 1.0))
+    assert route() == [0, 3]
+    del comm.topology[0][-1]
+    assert route() == [0, 2, 3]
+    del comm.topology
+    assert route() == [0, 3]
