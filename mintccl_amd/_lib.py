@@ -309,9 +309,15 @@ def host():
             raise RuntimeError(f"{HOST_PATH} was built for another descriptor: rebuild it")
         module.bind(*[ctypes.cast(getattr(L, name), ctypes.c_void_p).value
                       for name in ("mint_ring_launch", "mint_ring_grid_blocks", "mint_ll128_pack",
-                                   "mint_ll128_unpack", "mint_ll128_packed_bytes")], check)
+                                   "mint_ll128_unpack", "mint_ll128_packed_bytes")], check, empty_bytes)
         _host = module
     return _host
+
+
+def empty_bytes(n: int, like):
+    """``n`` bytes on the device of the tensor ``like``."""
+    import torch
+    return torch.empty(n, dtype=torch.uint8, device=like.device)
 
 
 def build_flags() -> list[str]:

@@ -17,7 +17,8 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
-#include <ATen/hip/EmptyTensor.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/ops/empty.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -40,6 +41,7 @@ struct Native {
     int (*unpack)(const void*, void*, size_t, uint64_t, uint64_t, int, void*, void*);
     size_t (*packed_bytes)(size_t, int);
     PyObject* check;             // _lib.check(code, where): raises MintError
+    PyObject* empty_bytes;       // _lib.empty_bytes(n, like): torch.empty
 } native = {};
 
 PyObject* raise(PyObject* type, const char* text) {
@@ -854,6 +856,16 @@ const at::Tensor* device_tensor(PyObject* o) {
 }
 size_t bytes_of(const at::Tensor& t) { return (size_t)t.numel() * (size_t)t.element_size(); }
 
+// A message of n bytes beside `like`, allocated where whoever looks at allocations
+// sees it: dispatch modes and the profiler through the dispatcher (pack and unpack
+// of 1 MiB 7.16 us, 6.96 with the allocator's own entry, which they do not see),
+// function modes through torch.empty itself.
+PyObject* empty_bytes(size_t n, PyObject* like) {
+    if (at::impl::torch_function_mode_enabled())
+        return PyObject_CallFunction(native.empty_bytes, "nO", (Py_ssize_t)n, like);
+    return THPVariable_Wrap(at::empty({(int64_t)n}, THPVariable_Unpack(like).options().dtype(at::kByte)));
+}
+
 // pack(raw, flag_base, layout, flag_stride, out or None)
 PyObject* host_pack(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != 5) return raise(PyExc_TypeError, "pack(raw, flag_base, layout, flag_stride, out)");
@@ -867,8 +879,7 @@ PyObject* host_pack(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const size_t nbytes = bytes_of(*raw), need = native.packed_bytes(nbytes, layout);
         PyObject* result;
         if (args[4] == Py_None) {
-            // (the allocator's own entry: half of what the dispatcher takes)
-            result = THPVariable_Wrap(at::Tensor(at::detail::empty_cuda({(int64_t)need}, at::kByte, raw->device(), {})));
+            result = empty_bytes(need, args[0]);
             if (!result) return nullptr;
         } else {
             const at::Tensor* out = device_tensor(args[4]);
@@ -919,11 +930,11 @@ PyObject* host_unpack(PyObject*, PyObject* const* args, Py_ssize_t n) {
     });
 }
 
-// bind(launch, grid, pack, unpack, packed_bytes, check): addresses, and what raises
+// bind(launch, grid, pack, unpack, packed_bytes, check, empty_bytes): addresses, what raises, what allocates
 PyObject* host_bind(PyObject*, PyObject* args) {
     unsigned long long launch, grid, pack, unpack, packed;
-    PyObject* check;
-    if (!PyArg_ParseTuple(args, "KKKKKO", &launch, &grid, &pack, &unpack, &packed, &check)) return nullptr;
+    PyObject *check, *empty;
+    if (!PyArg_ParseTuple(args, "KKKKKOO", &launch, &grid, &pack, &unpack, &packed, &check, &empty)) return nullptr;
     native.launch = reinterpret_cast<decltype(native.launch)>(launch);
     native.grid = reinterpret_cast<decltype(native.grid)>(grid);
     native.pack = reinterpret_cast<decltype(native.pack)>(pack);
@@ -931,6 +942,8 @@ PyObject* host_bind(PyObject*, PyObject* args) {
     native.packed_bytes = reinterpret_cast<decltype(native.packed_bytes)>(packed);
     Py_INCREF(check);
     Py_XSETREF(native.check, check);
+    Py_INCREF(empty);
+    Py_XSETREF(native.empty_bytes, empty);
     Py_RETURN_NONE;
 }
 

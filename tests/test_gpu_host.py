@@ -301,3 +301,34 @@ def test_a_topology_changed_in_place_changes_the_next_route(dev):
     assert route() == [0, 2, 3]
     del comm.topology
     assert route() == [0, 3]
+
+
+def test_the_allocation_of_a_message_is_seen(dev):
+    """By dispatch modes, function modes and the profiler, as any allocation."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from mintccl_amd import protocol
+    raw = torch.arange(2000, dtype=torch.int32, device=dev)
+    seen = []
+
+    class Dispatched(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+    want = protocol.pack(raw)
+    with Dispatched():
+        msg = protocol.pack(raw)
+    assert any("aten.empty" in str(f) for f in seen) and torch.equal(msg, want)
+    seen.clear()
+    with Functions():
+        msg = protocol.pack(raw)
+    assert torch.empty in seen and torch.equal(msg, want)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        protocol.pack(raw)
+    assert any(e.key == "aten::empty" for e in prof.key_averages())
