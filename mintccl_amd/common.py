@@ -278,7 +278,7 @@ def _largest_divisor_at_most(n: int, cap: int) -> int:
 # what the board takes from the communicator (VirtualComm._refresh): attributes
 # of a launch, and methods that it passes by unless they have been replaced
 _LAUNCH_ATTRIBUTES = frozenset(("inside_cu", "stats", "epoch_word", "protocol", "spin_budget", "status",
-                                "topology"))
+                                "topology", "__class__"))
 # ... and attributes of launches through staging: to set one asks for staging
 _STAGING_ATTRIBUTES = frozenset(("placement", "cache_policy", "row_fetch", "origin_cus", "threads_per_block",
                                  "threads_explicit", "waves_per_rank", "nslots", "slot_bytes", "buff_size",

@@ -131,7 +131,7 @@ struct Board {
     bool fresh, native_launch;   // `base` is up to date; it is ours to launch
     bool asks_rank, in_turn;     // Get_rank, rank are the communicator's own: called, not passed by
     PyTypeObject* type;          // the communicator's class and its version when last asked
-    unsigned version;
+    unsigned version;            // (assigning __class__ is an attribute set: fresh says so)
     bool has_ring;               // (a topology may have routes and no ring)
     bool keeps_routes;           // no topology of the caller's, who may change it in place
     bool launched;
@@ -216,19 +216,21 @@ int dtype_code(const at::Tensor& t) {
 
 // Brings `base` up to date with the communicator's attributes and methods.  A class
 // has another version, or none, once anything of it or its bases has been changed.
-bool refresh(Board* b) {
-    PyObject* comm = PyWeakref_GetObject(b->comm);
-    const PyTypeObject* type = Py_TYPE(comm);
-    if (b->fresh && b->type == type && (type->tp_flags & Py_TPFLAGS_VALID_VERSION_TAG) &&
-        b->version == type->tp_version_tag)
-        return true;
-    if (!(comm = comm_of(b))) return false;
+bool ask(Board* b) {
+    PyObject* comm = comm_of(b);
+    if (!comm) return false;
     PyObject* done = PyObject_CallMethod(comm, "_refresh", nullptr);     // calls configure()
-    b->type = Py_TYPE(comm);
+    Py_INCREF(Py_TYPE(comm));
+    Py_XSETREF(b->type, Py_TYPE(comm));
     b->version = b->type->tp_version_tag;
     Py_DECREF(comm);
     Py_XDECREF(done);
     return done != nullptr;
+}
+// (asked for by every rank's call: a few loads)
+inline bool refresh(Board* b) {
+    return (b->fresh && b->type && (b->type->tp_flags & Py_TPFLAGS_VALID_VERSION_TAG) &&
+            b->version == b->type->tp_version_tag) || ask(b);
 }
 
 // The rank this call is made for.
@@ -718,6 +720,7 @@ void board_dealloc(PyObject* self) {
     if (b->send.given) Py_DECREF(b->send.keep);
     if (b->recv.given) Py_DECREF(b->recv.keep);
     Py_XDECREF(b->comm);
+    Py_XDECREF(b->type);
     Py_TYPE(self)->tp_free(self);
 }
 
