@@ -277,8 +277,8 @@ def _largest_divisor_at_most(n: int, cap: int) -> int:
 
 # what the board takes from the communicator (VirtualComm._refresh): attributes
 # of a launch, and methods that it passes by unless they have been replaced
-_LAUNCH_ATTRIBUTES = frozenset(("inside_cu", "stats", "epoch_word", "protocol", "spin_budget", "status",
-                                "topology", "__class__"))
+_LAUNCH_ATTRIBUTES = frozenset(("inside_cu", "stats", "protocol", "spin_budget", "status", "topology",
+                                "__class__"))
 # ... and attributes of launches through staging: to set one asks for staging
 _STAGING_ATTRIBUTES = frozenset(("placement", "cache_policy", "row_fetch", "origin_cus", "threads_per_block",
                                  "threads_explicit", "waves_per_rank", "nslots", "slot_bytes", "buff_size",
@@ -386,8 +386,9 @@ class VirtualComm:
         self._last_protocol = None
         # Launches that are captured into a HIP graph and replayed cannot carry
         # their epoch as an argument: with device_epoch (or MINTCCL_DEVICE_EPOCH=1)
-        # it lives in device memory and every launch is preceded by a tiny
-        # kernel that advances it (and clears staging when it starts over).
+        # it lives in device memory and every launch through staging is preceded
+        # by a tiny kernel that advances it (and clears staging when it starts
+        # over).
         if device_epoch is None:
             device_epoch = bool(os.getenv("MINTCCL_DEVICE_EPOCH", ""))
         # (two words: the epoch, and the protocol of the launch before - the
@@ -427,10 +428,10 @@ class VirtualComm:
             ring = ring_of(self)
         except Exception:
             ring = []                  # routes only: a collective will say so
-        self._board.configure(self._runs_inside() and self.epoch_word is None and
-                              not self._replaced("launch", "enqueue", "make_cu_op"),
+        self._board.configure(self._runs_inside() and not self._replaced("launch", "enqueue", "make_cu_op"),
                               self._replaced("Get_rank"), self._replaced("rank"),
-                              getattr(self, "topology", None) is None, ring, self.protocol, self.spin_budget, self.status.data_ptr())
+                              getattr(self, "topology", None) is None, ring, self.protocol,
+                              self.spin_budget, self.status.data_ptr())
 
     def _find_route(self, src: int, dst: int) -> list[int]:
         from .topology import find_route, uniform_topology
@@ -648,7 +649,7 @@ class VirtualComm:
         self._board.launching(d)
         with torch.cuda.device(self.device):
             stream = torch.cuda.current_stream().cuda_stream
-            if self.epoch_word is not None:
+            if self.epoch_word is not None and not inside_cu:
                 _lib.check(self._lib.mint_epoch_advance(
                     self.epoch_word.data_ptr(), self.staging.data_ptr(),
                     self.staging.numel() * self.staging.element_size(),

@@ -332,3 +332,27 @@ def test_the_allocation_of_a_message_is_seen(dev):
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
         protocol.pack(raw)
     assert any(e.key == "aten::empty" for e in prof.key_averages())
+
+
+def test_a_launch_without_an_epoch_advances_none(dev):
+    """With the epoch in device memory: a ring inside compute units leaves it (and
+    the staging that is cleared when it starts over) alone, one through staging
+    advances it."""
+    from mintccl_amd.allgather import allgather
+    world = 4
+    comm = make_comm(world, device_epoch=True)
+    comm.epoch_word[0] = 4094
+    comm.staging.fill_(7)
+    bufs = [torch.zeros(world, 1000, device=dev) for _ in range(world)]
+    for r, b in enumerate(bufs):
+        b[r] = r + 1
+    rows = torch.arange(1, world + 1, dtype=torch.float32, device=dev)[:, None].expand(world, 1000)
+    for _ in range(3):
+        comm.run(lambda r: allgather(bufs[r], comm))
+    comm.check()
+    assert all(torch.equal(b, rows) for b in bufs)
+    assert int(comm.epoch_word[0]) == 4094 and torch.all(comm.staging == 7)
+    comm.staging.zero_()
+    comm.run(lambda r: allgather(bufs[r], comm, schedule="temporal"))
+    comm.check()
+    assert int(comm.epoch_word[0]) == 4095 and all(torch.equal(b, rows) for b in bufs)

@@ -196,11 +196,13 @@ def test_reference_style_self_tests_pass(monkeypatch, capsys, world, count):
 
 @pytest.mark.gpu
 def test_device_epoch_wraps_and_clears(dev):
-    """With the epoch in device memory every launch advances it; when it starts
-    over the staging is cleared, so results stay right across the wrap."""
+    """With the epoch in device memory every launch through staging advances it;
+    when it starts over the staging is cleared, so results stay right across
+    the wrap."""
+    from mintccl_amd import _lib
     from mintccl_amd.reducescatter import reducescatter
     world, n = 4, 3000
-    comm = make_comm(world, device_epoch=True)
+    comm = make_comm(world, device_epoch=True, placement=_lib.PLACE_LOCAL)
     host = rank_rows(world, n, "f16")
     want = ring.reducescatter([as_bytes(h) for h in host], "f16")
     bufs = [h.to(dev) for h in host]
