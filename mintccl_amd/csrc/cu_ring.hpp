@@ -77,9 +77,7 @@ struct CuRingArgs {
 // loads through the cache (8 ranks, reduce-scatter of 8 MiB 10.9 us; 15.5 in the
 // large form, 13.0 with one pipeline after the other; blocks of 64 threads lose up
 // to a third where rows are copied once, 512 up to a tenth where they are added).
-#ifndef PROBE
 constexpr uint32_t cu_threads(bool large, bool copies) { return large && !copies ? 64u : 128u; }
-#endif
 
 // How rows are loaded: through the caches, or streamed past the last-level one.
 template <bool STREAM>
