@@ -46,7 +46,7 @@ struct CuShape {
 
 // The ranks' buffers in the order of the ring.  One address per rank where they
 // work in place, as the operators do: a launch with up to 112 bytes of arguments
-// takes the host 2.6 us, one with more 3.3.  SPLIT: N addresses to load from, then
+// takes the host 2.7 us, one with more 3.3 - 3.5.  SPLIT: N addresses to load from, then
 // N to store to.
 template <int N, bool SPLIT>
 struct CuTables {
@@ -97,10 +97,16 @@ constexpr int cu_stores(bool large, bool several) {
     return several ? (large ? CU_SC1_NT : CU_SC1) : large ? CU_SC1 : CU_NT;
 }
 // Sums to one place that are far larger than the last-level cache (plan_cu): with
-// many rows to read nt is the faster one.  sc1 / nt, us, 8 / 7 / 6 / 5 / 4 ranks:
-// bf16, 0.5 GiB touched 83 / 88, 84 / 90, 90 / 92, 93 / 95,  98 /  98;
-//       1 GiB          175 / 173, 190 / 182, 186 / 179, 186 / 184, 195 / 198;
-// f16,  1 GiB          180 / 178, 192 / 186, 196 / 190, 194 / 193, 197 / 202.
+// many rows to read nt is the faster one, on buffers that have not just been used.
+// Four sets of buffers in turn, reduce-scatter and reduce of f16 and bf16, nt over
+// sc1: 0.94 - 1.01 for 6, 7 and 8 ranks at 560 MiB touched and up; three sets, f16
+// reduce-scatter, sc1 / nt, us, 8 / 7 / 6 / 5 / 4 ranks (f32 the same):
+//   448 MiB  75 / 80,  77 / 82,  80 / 86,  84 / 88,  90 / 96;
+//   800     144 / 141, 152 / 145, 154 / 151, 153 / 156, 158 / 168;
+//   1 GiB   181 / 179, 192 / 185, 198 / 194, 200 / 200, 204 / 213;
+//   2 GiB   386 / 378, 381 / 369, 401 / 391, 410 / 399, 415 / 428.
+// The same buffers again and again keep a part of the sums in the cache with sc1:
+// there nt takes 1 - 11 % longer up to 1.5 GiB and is ahead from 2.3 GiB on.
 constexpr int kCuStreamRanks = 6;
 template <int HOW>
 __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 v) {
@@ -269,7 +275,7 @@ __global__ void __launch_bounds__(cu_threads(LARGE, (N > 2))) cu_ring_copy_kerne
 // The addresses of an alltoall, N to load from and N to store to.  T = uint32_t
 // where they lie whole multiples of 256 bytes from the lowest, as allocations do:
 // their distances from it in those units, which keeps a launch below 112 bytes of
-// arguments (3.5 us for the host with 64-bit ones, 2.9 so).
+// arguments (2.7 us for the host; with 64-bit ones, 168 bytes, 3.4 - 3.5).
 template <typename T>
 struct CuPairs {
     T rank[2 * kMaxRanks];

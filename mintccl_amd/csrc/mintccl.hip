@@ -69,9 +69,12 @@ static_assert(MINT_OP_TREE_BROADCAST == OP_TREE_BROADCAST && MINT_OP_TREE_REDUCE
 // N = 2 / 3 / 4 / 5 / 6 / 7 / 8: reduce-scatter 16 - 18 / 14 / 12 / 10 - 11 / 11 - 12 /
 // 10 / 9, allreduce 14 / 9 / 7 - 8 / 6 - 7 / 5 - 6 / 5 / 4 - 5, allgather - / 18 / 16 /
 // 14 / 12 / 10 / 10 and up; one or two off is 1 - 3 % slower, but twice as many 5 -
-// 20 %.  Rows that are copied from the last-level cache arrive sooner: there 7 and
-// 8 ranks are fastest with 6 - 8 (allgather of 8 x 64 MiB 67 us with 8, 71 with 10;
-// of 8 x 128 MiB 179 / 174).
+// 20 %.  Rows that are copied from the last-level cache arrive sooner: with 7 and
+// 8 ranks, 8 wavefronts instead of 10 are up to 5 % faster where the same buffers
+// are used again (8 ranks, allgather of 24 MiB in all 27.6 / 29.1 us) and within 1 -
+// 2 % either way on others up to 64 MiB; three sets of buffers in turn, 8 ranks, 8 /
+// 10: 64 MiB 72.7 / 73.0, 72 88.1 / 87.7, 80 97.8 / 97.4, 96 125 / 123, 128 178 / 174,
+// 256 358 / 348.
 int cu_waves(int op, int ranks, uint64_t copied) {
     if (op == OP_ALLREDUCE) return (26 + ranks - 1) / ranks + 1;
     if (reducing(op)) return (24 + ranks - 1) / ranks + 6;
@@ -93,7 +96,9 @@ int plan_cu(Plan* plan) {
     const uint64_t touched = (uint64_t)a.pipes * a.row_bytes *
                              (alltoall || a.op == OP_SENDRECV ? 2u : (uint64_t)a.cyc_len);
     plan->cu_large = touched > ((uint64_t)(copies ? 88 : sums ? 100 : 192) << 20);
-    // Far beyond it the sums of many ranks are as well streamed (kCuStreamRanks).
+    // Far beyond it the sums of many ranks are streamed past it (kCuStreamRanks): the
+    // line lies where three sets of buffers in turn cross over, 600 MiB (6 ranks) to
+    // 740 (8; 640 MiB 110 / 114 us).
     plan->cu_stream = sums && a.op != OP_ALLREDUCE && a.cyc_len >= kCuStreamRanks && touched > (640ull << 20);
     plan->threads = (int)cu_threads(plan->cu_large, copies);
     // (held to that number by the share of LDS its blocks ask for; LDS is handed
