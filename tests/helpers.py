@@ -24,6 +24,24 @@ def rank_rows(world: int, n: int, dt: str, seed0: int = 3000) -> list[torch.Tens
     return [normal(world * n, seed0 + r, TORCH_DT[dt]).reshape(world, n) for r in range(world)]
 
 
+#: How the rings of a communicator at the library's own geometry run: inside compute
+#: units (the operators' default), through staging as LL128 lines, or by the Simple
+#: protocol (naming a placement asks for staging).
+WIRES = ["inside", "ll128", "simple"]
+
+
+def comm_over(wire: str, world: int, **kw):
+    from mintccl_amd import _lib
+    from mintccl_amd.common import VirtualComm
+    kw.setdefault("spin_budget", 400000)      # ~ a second: a lost line fails, never hangs
+    if wire != "inside":
+        kw.update(placement=_lib.PLACE_LOCAL,
+                  protocol=_lib.PROTO_SIMPLE if wire == "simple" else _lib.PROTO_LL128)
+    comm = VirtualComm(world_size=world, **kw)
+    assert comm.inside_cu == (wire == "inside") and comm.auto_geometry
+    return comm
+
+
 def as_bytes(t: torch.Tensor) -> np.ndarray:
     return t.detach().cpu().contiguous().view(torch.uint8).numpy().reshape(-1)
 

@@ -150,10 +150,10 @@ def test_hypercube_64mib_and_back_to_back_launches(dev):
     then a ring reduce-scatter on the same communicator; checked against torch
     additions in the hypercube's order and, for the allgather that follows,
     through the round trip."""
-    from mintccl_amd import hypercube, primitive
+    from mintccl_amd import _lib, hypercube, primitive
     from mintccl_amd.reducescatter import reducescatter as ring_reducescatter
     world, n = 8, (64 << 20) // 2 // 8
-    comm = make_comm(world)
+    comm = make_comm(world, placement=_lib.PLACE_LOCAL)       # (the ring reduce-scatter through staging too)
     g = torch.Generator(device=dev).manual_seed(78)
     src = [torch.empty(world, n, dtype=torch.float16, device=dev).uniform_(-1, 1, generator=g)
            for _ in range(world)]

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import ring
-from tests.helpers import TORCH_DT, as_bytes, normal, rank_rows, uniform
+from tests.helpers import TORCH_DT, WIRES, as_bytes, comm_over, normal, rank_rows, uniform
 
 pytestmark = pytest.mark.gpu
 
@@ -59,9 +59,9 @@ def test_reducescatter_f16(dev, world, n):
     assert same(bufs, ring.reducescatter([as_bytes(h) for h in host], "f16"))
 
 
-@pytest.mark.parametrize("proto", [0, 1])
+@pytest.mark.parametrize("wire", WIRES)
 @pytest.mark.parametrize("shift", [1, 2, 6, 9])
-def test_buffers_and_rows_at_any_byte(dev, proto, shift):
+def test_buffers_and_rows_at_any_byte(dev, wire, shift):
     """Neither the buffers nor the rows of a (world, n) tensor need any
     alignment: buffers carved `shift` elements into an allocation, rows of an
     odd number of elements (many full blocks and a ragged end)."""
@@ -73,7 +73,7 @@ def test_buffers_and_rows_at_any_byte(dev, proto, shift):
     for b, h in zip(bufs, host):
         b.copy_(h)
     assert all(b.data_ptr() % 16 == (2 * shift) % 16 for b in bufs)
-    comm = make_comm(world, protocol=proto)
+    comm = comm_over(wire, world)
     run_reducescatter(comm, bufs)
     assert same(bufs, ring.reducescatter([as_bytes(h) for h in host], "f16"))
     # nothing written outside the buffers
@@ -142,26 +142,30 @@ def test_reduce_and_allreduce_with_own_rows_through_lds(dev, world):
     assert same(bufs, ring.broadcast(raw, 0))
 
 
-@pytest.mark.parametrize("proto", [0, 1])
+@pytest.mark.parametrize("wire", WIRES)
 @pytest.mark.parametrize("world", WORLDS)
 @pytest.mark.parametrize("n", [1, 479, 480, 481, 100003])
-def test_alltoall(dev, proto, world, n):
+def test_alltoall(dev, wire, world, n):
     """Row d of rank s arrives as row s of rank d, bit for bit, and the inputs
     are left alone (oracle: the transpose of rows)."""
     from mintccl_amd.alltoall import alltoall
     host = [uniform(world * n, -1.0, 1.0, 70 + r).reshape(world, n) for r in range(world)]
     want = ring.alltoall([as_bytes(h) for h in host])
-    for kw in (dict(), dict(buff_size_=world * 8 * 3072, nslots=3, waves_per_rank=2 * 8 * world)):
+    comms = [comm_over(wire, world)]
+    if wire != "inside":
+        comms.append(make_comm(world, protocol=comms[0].protocol, buff_size_=world * 8 * 3072, nslots=3,
+                               waves_per_rank=2 * 8 * world))
+    for comm in comms:
         bufs = [h.to(dev) for h in host]
         outs = [torch.full_like(b, 7.0) for b in bufs]
-        comm = make_comm(world, protocol=proto, **kw)
         comm.run(lambda r: alltoall(bufs[r], outs[r], comm))
         comm.check()
-        assert same(outs, want), kw
+        assert same(outs, want), comm.nslots
         assert same(bufs, [as_bytes(h) for h in host])
 
 
-def test_alltoall_64mib_and_argument_checks(dev):
+@pytest.mark.parametrize("wire", WIRES)
+def test_alltoall_64mib_and_argument_checks(dev, wire):
     from mintccl_amd.alltoall import alltoall
     world, n = 8, 4194304                                   # 8 ranks x 64 MiB fp16
     bufs = []
@@ -169,7 +173,7 @@ def test_alltoall_64mib_and_argument_checks(dev):
         g = torch.Generator(device=dev).manual_seed(90 + r)
         bufs.append(torch.randn(world, n, generator=g, device=dev, dtype=torch.float16))
     outs = [torch.zeros_like(b) for b in bufs]
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     comm.run(lambda r: alltoall(bufs[r], outs[r], comm))
     comm.check()
     for d in range(world):
@@ -182,7 +186,8 @@ def test_alltoall_64mib_and_argument_checks(dev):
         comm.run(lambda r: alltoall(bufs[r], bufs[(r + 1) % world], comm))    # out is somebody's buff
 
 
-def test_reducescatter_special_values(dev):
+@pytest.mark.parametrize("wire", WIRES)
+def test_reducescatter_special_values(dev, wire):
     # overflow to inf, inf - inf, subnormals, signed zeros ride the ring unharmed
     world, n = 4, 960
     vals = torch.tensor([65504.0, -65504.0, 6e-8, -6e-8, 0.0, -0.0, float("inf"), float("-inf"),
@@ -191,14 +196,15 @@ def test_reducescatter_special_values(dev):
     host = [vals[torch.randint(0, len(vals), (world * n,), generator=g)].reshape(world, n)
             for _ in range(world)]
     bufs = [h.to(dev) for h in host]
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     run_reducescatter(comm, bufs)
     want = ring.reducescatter([as_bytes(h) for h in host], "f16")
     for b, w in zip(bufs, want):
         assert ring.same_values(as_bytes(b), w, "f16")
 
 
-def test_reducescatter_order_is_the_reference_ring_order(dev):
+@pytest.mark.parametrize("wire", WIRES)
+def test_reducescatter_order_is_the_reference_ring_order(dev, wire):
     # binary16 has ulp 2 at 2048, so 2048 + 1 ties back to 2048 while
     # (1 + 1) + 2048 = 2050: where the large value enters the fold is visible.
     # rows[r][c] = rank r's value for chunk c; chunk c folds in the order
@@ -209,7 +215,7 @@ def test_reducescatter_order_is_the_reference_ring_order(dev):
     host = [torch.tensor(rows[r], dtype=torch.float16).repeat_interleave(n).reshape(world, n).contiguous()
             for r in range(world)]
     bufs = [h.to(dev) for h in host]
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     run_reducescatter(comm, bufs)
     got = [float(bufs[c][c, 0]) for c in range(world)]
     assert got[0] == 2048.0   # 2048, +1 -> 2048, +1 -> 2048, +1 -> 2048
@@ -222,24 +228,25 @@ def test_reducescatter_order_is_the_reference_ring_order(dev):
 @pytest.mark.parametrize("world", WORLDS)
 @pytest.mark.parametrize("root", [0, 1])
 @pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
-def test_reduce(dev, world, root, dt):
+@pytest.mark.parametrize("wire", WIRES)
+def test_reduce(dev, world, root, dt, wire):
     n = 70001
     host = [normal(n, 3000 + r, TORCH_DT[dt]) for r in range(world)]
     bufs = [h.to(dev) for h in host]
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     run_reduce(comm, bufs, root)
     assert same(bufs, ring.reduce([as_bytes(h) for h in host], root, dt))
 
 
 @pytest.mark.parametrize("world", WORLDS)
 @pytest.mark.parametrize("nbytes", [1, 7, 960, 961, 1 << 20, (1 << 20) + 3])
-@pytest.mark.parametrize("proto", [0, 1])
-def test_broadcast_bytes(dev, world, nbytes, proto):
+@pytest.mark.parametrize("wire", WIRES)
+def test_broadcast_bytes(dev, world, nbytes, wire):
     root = world - 1
     g = torch.Generator().manual_seed(nbytes)
     host = [torch.randint(0, 256, (nbytes,), dtype=torch.uint8, generator=g) for _ in range(world)]
     bufs = [h.to(dev) for h in host]
-    comm = make_comm(world, protocol=proto)
+    comm = comm_over(wire, world)
     run_broadcast(comm, bufs, root)
     for b in bufs:
         assert torch.equal(b.cpu(), host[root])
@@ -278,11 +285,11 @@ def test_an_origin_needs_no_staging(dev, proto, policy):
 
 @pytest.mark.parametrize("world", WORLDS)
 @pytest.mark.parametrize("n", [8, 480, 488, 65536])
-@pytest.mark.parametrize("proto", [0, 1])
-def test_allgather(dev, world, n, proto):
+@pytest.mark.parametrize("wire", WIRES)
+def test_allgather(dev, world, n, wire):
     host = [uniform(world * n, -1.0, 1.0, 4 + r).reshape(world, n) for r in range(world)]
     bufs = [h.to(dev) for h in host]
-    comm = make_comm(world, protocol=proto)
+    comm = comm_over(wire, world)
     run_allgather(comm, bufs)
     assert same(bufs, ring.allgather([as_bytes(h) for h in host]))
 
@@ -402,12 +409,13 @@ def run_allreduce(comm, bufs, fused=False):
 @pytest.mark.parametrize("fused", [False, True])
 @pytest.mark.parametrize("world", WORLDS)
 @pytest.mark.parametrize("n", [1, 7, 8, 63, 64, 4000, 100003, (1 << 20) + 9])
-def test_allreduce_f16(dev, world, n, fused):
+@pytest.mark.parametrize("wire", WIRES)
+def test_allreduce_f16(dev, world, n, fused, wire):
     # ragged sizes: with few elements some chunks are short or empty; as one
     # pass round the ring, and as a reduce-scatter followed by an allgather
     host = [normal(n, 3000 + r) for r in range(world)]
     bufs = [h.to(dev) for h in host]
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     run_allreduce(comm, bufs, fused)
     want = ring.allreduce([as_bytes(h) for h in host], "f16")
     assert same(bufs, want)
@@ -427,13 +435,14 @@ def test_allreduce_dtypes_protocols_policies(dev, dt, proto, place, cp, fused):
 
 
 @pytest.mark.parametrize("fused", [False, True])
-def test_allreduce_64mib_against_device_fold(dev, fused):
+@pytest.mark.parametrize("wire", WIRES)
+def test_allreduce_64mib_against_device_fold(dev, fused, wire):
     from mintccl_amd import primitive
     world, n = 8, 33554432          # 64 MiB per rank
     g = torch.Generator(device=dev).manual_seed(11)
     bufs = [torch.randn(n, generator=g, device=dev, dtype=torch.float16) for _ in range(world)]
     orig = [b.clone() for b in bufs]
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     run_allreduce(comm, bufs, fused)
     row = n // world
     for c in range(world):
@@ -444,7 +453,8 @@ def test_allreduce_64mib_against_device_fold(dev, fused):
             assert torch.equal(bufs[r][c * row:(c + 1) * row].view(torch.int16), acc.view(torch.int16))
 
 
-def test_permuted_ring(dev):
+@pytest.mark.parametrize("wire", WIRES)
+def test_permuted_ring(dev, wire):
     # a non-uniform topology whose best ring is not the identity
     from mintccl_amd.topology import find_ring
     world, n = 4, 5000
@@ -458,7 +468,7 @@ def test_permuted_ring(dev):
     assert ring_ in ([0, 2, 1, 3, 0], [0, 3, 1, 2, 0])
     host = rank_rows(world, n + (-n) % 8, "f16")
     bufs = [h.to(dev) for h in host]
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     comm.topology = topo
     run_reducescatter(comm, bufs)
     assert same(bufs, ring.reducescatter([as_bytes(h) for h in host], "f16", ring_))
@@ -468,7 +478,8 @@ def test_permuted_ring(dev):
     assert same(bufs2, ring.reduce([as_bytes(h) for h in host2], 1, "f16", ring_))
 
 
-def test_topology_file_drives_ring_and_route_end_to_end(dev, tmp_path):
+@pytest.mark.parametrize("wire", WIRES)
+def test_topology_file_drives_ring_and_route_end_to_end(dev, tmp_path, wire):
     """A non-uniform ``topo.json`` (the reference's file format), written with
     ``save_topology`` and loaded with ``get_topology``: the collectives run
     round the ring it implies, and the deferred send / recv takes the widest
@@ -484,7 +495,7 @@ def test_topology_file_drives_ring_and_route_end_to_end(dev, tmp_path):
         topo[b].append((a, bw))
     path = str(tmp_path / "topo.json")
     save_topology(topo, path)
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     comm.topology = get_topology(path)
     ring_ = find_ring(comm.topology)
     assert ring_ in ([0, 1, 3, 2, 0], [0, 2, 3, 1, 0])          # the two cycles there are
@@ -512,7 +523,7 @@ def test_many_launches_reuse_staging_without_clearing(dev):
     # flags carry a per-launch epoch: stale lines of earlier launches, of other
     # sizes and other collectives, are never mistaken for data
     world = 8
-    comm = make_comm(world)
+    comm = comm_over("ll128", world)
     for i, n in enumerate([4096, 480, 100000, 8, 4096, 52000]):
         host = rank_rows(world, n, "f16", seed0=100 * i)
         bufs = [h.to(dev) for h in host]
@@ -522,6 +533,7 @@ def test_many_launches_reuse_staging_without_clearing(dev):
         bufs = [h.to(dev) for h in host]
         run_allgather(comm, bufs)
         assert same(bufs, ring.allgather([as_bytes(h) for h in host]))
+        assert comm.epoch == 2 * i + 2
 
 
 def test_epoch_wraps_after_4095_launches(dev):
@@ -530,11 +542,12 @@ def test_epoch_wraps_after_4095_launches(dev):
     from mintccl_amd import _lib
     from mintccl_amd.broadcast import broadcast
     world, n = 4, 2048
-    comm = make_comm(world)
+    comm = comm_over("ll128", world)
     host = [torch.full((n,), float(r + 1), dtype=torch.float16) for r in range(world)]
     bufs = [h.to(dev) for h in host]
     ptrs = {r: bufs[r].data_ptr() for r in range(world)}
     comm.run(lambda r: broadcast(bufs[r], 0, comm))
+    assert comm.epoch == 1
     d = comm.make_op(_lib.OP_BROADCAST, _lib.BYTES, n * 2, {0: ptrs[0]},
                      {r: ptrs[r] for r in range(1, world)}, [0, 1, 2, 3, 0], root=0)
     for _ in range(_lib.MAX_EPOCH + 5):
@@ -557,7 +570,7 @@ def test_payload_that_looks_like_credit_words_is_harmless(dev):
     from mintccl_amd import sendrecv_buffer
     from mintccl_amd.broadcast import broadcast
     world = 8
-    comm = make_comm(world)
+    comm = comm_over("ll128", world)
     n64 = 1 << 20
     for round_ in range(3):
         words = torch.arange(n64, dtype=torch.int64)
@@ -580,6 +593,7 @@ def test_payload_that_looks_like_credit_words_is_harmless(dev):
         rs = [h.to(dev) for h in host]
         run_reducescatter(comm, rs)
         assert same(rs, ring.reducescatter([as_bytes(h) for h in host], "f16"))
+        assert comm.epoch == 3 * round_ + 3
 
 
 def test_simple_payload_that_looks_like_ll128_tags_is_harmless(dev):
@@ -618,7 +632,7 @@ def test_a_lost_producer_times_out_instead_of_hanging(dev):
     from mintccl_amd import _lib
     from mintccl_amd.common import RingTimeout
     world, n = 4, 4096
-    comm = make_comm(world, spin_budget=2000)
+    comm = comm_over("ll128", world, spin_budget=2000)
     bufs = [torch.zeros(n, dtype=torch.float16, device=dev) for _ in range(world)]
     d = comm.make_op(_lib.OP_BROADCAST, _lib.BYTES, n * 2, {0: bufs[0].data_ptr()},
                      {r: bufs[r].data_ptr() for r in range(1, world)}, [0, 1, 2, 3, 0],
@@ -883,17 +897,19 @@ def test_config4_reducescatter_and_reduce_32m_elements(dev, dt):
         assert torch.equal(flat[r], orig[r].reshape(-1))
 
 
-def test_headline_reducescatter_256mib_fp16(dev):
-    """8 ranks x 256 MiB fp16 with the library's default geometry (the one
-    bench.py times): every owner row, all 32 MiB of it, against the oracle's
-    fold computed on the host, and every other row untouched."""
+@pytest.mark.parametrize("wire", ["inside", "ll128"])
+def test_headline_reducescatter_256mib_fp16(dev, wire):
+    """8 ranks x 256 MiB fp16 inside compute units and through staging at the
+    library's tuned geometry (bench.py times both): every owner row, all 32 MiB
+    of it, against the oracle's fold computed on the host, and every other row
+    untouched."""
     from mintccl_amd import primitive
     world, n_total = 8, 134217728
     n = n_total // world
     g = torch.Generator(device=dev).manual_seed(7)
     bufs = [torch.randn(world, n, generator=g, device=dev, dtype=torch.float16) for _ in range(world)]
     orig = [b.clone() for b in bufs]
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     run_reducescatter(comm, bufs)
     for c in range(world):
         rows = [as_bytes(orig[r][c]) for r in range(world)]
@@ -909,7 +925,8 @@ def test_headline_reducescatter_256mib_fp16(dev):
                 assert torch.equal(bufs[r][c].view(torch.int16), orig[r][c].view(torch.int16)), (r, c)
 
 
-def test_empty_buffers_are_a_no_op(dev):
+@pytest.mark.parametrize("wire", WIRES)
+def test_empty_buffers_are_a_no_op(dev, wire):
     """Zero bytes: every collective returns without launching and touches nothing."""
     from mintccl_amd.allgather import allgather
     from mintccl_amd.allreduce import allreduce
@@ -917,7 +934,7 @@ def test_empty_buffers_are_a_no_op(dev):
     from mintccl_amd.reduce import reduce
     from mintccl_amd.reducescatter import reducescatter
     world = 4
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     rows = [torch.empty(world, 0, dtype=torch.float16, device=dev) for _ in range(world)]
     flat = [torch.empty(0, dtype=torch.float16, device=dev) for _ in range(world)]
     comm.run(lambda r: reducescatter(rows[r], comm))
@@ -928,7 +945,8 @@ def test_empty_buffers_are_a_no_op(dev):
     comm.check()
 
 
-def test_rows_beyond_4_gib(dev):
+@pytest.mark.parametrize("wire", WIRES)
+def test_rows_beyond_4_gib(dev, wire):
     """Offsets inside a row are 64-bit: a 4 GiB + 960 KiB + 40 B message through two
     hops (rank 0 -> 1 -> 2 as a broadcast over 3 ranks) arrives bit for bit."""
     from mintccl_amd.broadcast import broadcast
@@ -943,7 +961,7 @@ def test_rows_beyond_4_gib(dev):
         src[lo:hi] = ((i * 2654435761) >> 7).to(torch.uint8)
         del i
     bufs = [src, torch.zeros(n, dtype=torch.uint8, device=dev), torch.zeros(n, dtype=torch.uint8, device=dev)]
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     run_broadcast(comm, bufs, 0)
     for b in bufs[1:]:
         assert torch.equal(b, src)

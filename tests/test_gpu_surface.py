@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import ring
-from tests.helpers import as_bytes, normal, rank_rows, uniform
+from tests.helpers import WIRES, as_bytes, comm_over, normal, rank_rows, uniform
 
 pytestmark = pytest.mark.gpu
 
@@ -33,10 +33,11 @@ def test_direct_send_recv(dev, nbytes):
 @pytest.mark.parametrize("module", ["sendrecv_buffer", "sendrecv_indirect"])
 @pytest.mark.parametrize("route", [None, [0, 2, 1], [0, 3, 2, 1]])
 @pytest.mark.parametrize("n", [1, 123457])
-def test_deferred_send_recv_sync(dev, module, route, n):
+@pytest.mark.parametrize("wire", WIRES)
+def test_deferred_send_recv_sync(dev, module, route, n, wire):
     import importlib
     m = importlib.import_module(f"mintccl_amd.{module}")
-    comm = make_comm(4)
+    comm = comm_over(wire, 4)
     src = torch.randn(n, generator=torch.Generator().manual_seed(n)).to(dev)   # fp32 like the reference test
     dst = torch.zeros_like(src)
     with comm.rank(0):
@@ -153,12 +154,13 @@ def test_world_of_one_is_a_no_op(dev):
     assert torch.equal(x, y)
 
 
-def test_launch_is_asynchronous_and_stream_ordered(dev):
+@pytest.mark.parametrize("wire", WIRES)
+def test_launch_is_asynchronous_and_stream_ordered(dev, wire):
     # the operator enqueues on the current stream and returns; a later kernel
     # on the same stream sees the result
     from mintccl_amd.broadcast import broadcast
     world, n = 8, 1 << 22
-    comm = make_comm(world)
+    comm = comm_over(wire, world)
     s = torch.cuda.Stream(device=dev)
     host = uniform(n, -4.0, 4.0, 9)
     with torch.cuda.stream(s):
@@ -224,6 +226,8 @@ def test_device_epoch_wraps_and_clears(dev):
 @pytest.mark.parametrize("knobs", [
     {},
     {"MINTCCL_PROTOCOL": "simple"},
+    {"MINTCCL_PROTOCOL": "simple", "MINTCCL_PLACEMENT": "local"},
+    {"MINTCCL_PLACEMENT": "local"},
     {"MINTCCL_PLACEMENT": "spread", "MINTCCL_CACHE": "agent"},
     {"MINTCCL_TOPOLOGY": "tree", "MINTCCL_ALLGATHER": "temporal"},
     {"MINTCCL_ALLREDUCE": "split", "MINTCCL_NSLOTS": "2", "MINTCCL_BUFFSIZE": "262144"},
@@ -245,17 +249,19 @@ def test_self_tests_over_world_sizes_and_knobs(monkeypatch, capsys, world, knobs
 
 
 @pytest.mark.gpu
-def test_captured_large_collectives_replay(dev):
-    """The same for messages large enough for the tuned launches with compute
-    units set apart for the origins (allgather in both schedules, broadcast,
-    sendrecv over one hop, alltoall): three replays against eager runs."""
+@pytest.mark.parametrize("wire", ["inside", "ll128"])
+def test_captured_large_collectives_replay(dev, wire):
+    """The same for messages large enough, through staging, for the tuned
+    launches with compute units set apart for the origins (allgather in both
+    schedules, broadcast, sendrecv over one hop, alltoall): three replays
+    against eager runs."""
     from mintccl_amd import sendrecv_buffer
     from mintccl_amd.allgather import allgather
     from mintccl_amd.alltoall import alltoall
     from mintccl_amd.broadcast import broadcast
     world, n = 8, (1 << 20) + 40
-    comm = make_comm(world, device_epoch=True)
-    eager = make_comm(world)
+    comm = comm_over(wire, world, device_epoch=True)
+    eager = comm_over(wire, world)
     ins = [torch.zeros(world, n, dtype=torch.float16, device=dev) for _ in range(world)]
 
     def buffers():
@@ -306,7 +312,8 @@ def test_captured_large_collectives_replay(dev):
     assert torch.equal(want[3][6], want[0][2]) and torch.equal(want[3][5], ins[5])
 
 
-def test_captured_collectives_replay(dev):
+@pytest.mark.parametrize("wire", WIRES)
+def test_captured_collectives_replay(dev, wire):
     """A captured sequence of collectives (epoch in device memory) is replayed
     several times, with eager work and fresh inputs in between; every replay
     must equal the eager result."""
@@ -314,8 +321,8 @@ def test_captured_collectives_replay(dev):
     from mintccl_amd.allreduce import allreduce
     from mintccl_amd.broadcast import broadcast
     world, n = 8, 4096 + 24
-    comm = make_comm(world, device_epoch=True)
-    eager = make_comm(world)
+    comm = comm_over(wire, world, device_epoch=True)
+    eager = comm_over(wire, world)
     ins = [torch.zeros(world, n, dtype=torch.float16, device=dev) for _ in range(world)]
     a = [torch.zeros_like(x) for x in ins]
     b = [torch.zeros(world * n, dtype=torch.float16, device=dev) for _ in range(world)]
@@ -362,7 +369,6 @@ def test_local_placement_on_a_stream_confined_to_half_of_the_compute_units(dev):
     import ctypes
     from mintccl_amd import _lib
     from mintccl_amd.allgather import allgather
-    from mintccl_amd.common import VirtualComm
     from mintccl_amd.reducescatter import reducescatter
     hip = ctypes.CDLL("libamdhip64.so")
     words = (ctypes.c_uint32 * 8)(*([0x00FF00FF] * 8))
@@ -370,7 +376,7 @@ def test_local_placement_on_a_stream_confined_to_half_of_the_compute_units(dev):
     assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(handle), 8, words) == 0
     stream = torch.cuda.ExternalStream(handle.value)
     world, n = 8, 100003
-    comm = VirtualComm(world_size=world, device=dev, spin_budget=4000000)
+    comm = comm_over("ll128", world, spin_budget=4000000)
     assert comm.placement == _lib.PLACE_LOCAL
     host = rank_rows(world, n, "f16", 8100)
     bufs = [h.to(dev) for h in host]
@@ -406,10 +412,9 @@ def test_local_placement_beside_another_streams_kernels(dev):
     units have room, in whatever numbers, and still find their seats."""
     from mintccl_amd import _lib
     from mintccl_amd.allgather import allgather
-    from mintccl_amd.common import VirtualComm
     from mintccl_amd.reducescatter import reducescatter
     world, n = 8, 524309
-    comm = VirtualComm(world_size=world, device=dev, spin_budget=4000000)
+    comm = comm_over("ll128", world, spin_budget=4000000)
     assert comm.placement == _lib.PLACE_LOCAL
     host = rank_rows(world, n, "f16", 8200)
     want = ring.reducescatter([as_bytes(h) for h in host], "f16")
@@ -444,7 +449,7 @@ def test_captured_ll128_launch_replayed_after_an_eager_simple_launch(dev):
     from mintccl_amd import _lib
     from mintccl_amd.allgather import allgather
     world, n = 8, 52000
-    comm = make_comm(world, device_epoch=True)
+    comm = comm_over("ll128", world, device_epoch=True)
     ins = [torch.zeros(world, n, dtype=torch.float16, device=dev) for _ in range(world)]
     g = [torch.zeros_like(x) for x in ins]
 

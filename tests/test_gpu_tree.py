@@ -127,8 +127,9 @@ def test_tree_64mib_and_back_to_back_launches(dev):
     staging (the second launch meets the first one's tags under another epoch),
     then a ring reduce on the same communicator."""
     from mintccl_amd.reduce import reduce as ring_reduce
+    from mintccl_amd import _lib
     world, n = 8, 32 << 20
-    comm = make_comm(world)
+    comm = make_comm(world, placement=_lib.PLACE_LOCAL)       # (the ring reduce through staging too)
     g = torch.Generator(device=dev).manual_seed(77)
     src = [torch.empty(n, dtype=torch.float16, device=dev).uniform_(-1, 1, generator=g)
            for _ in range(world)]
