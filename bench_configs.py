@@ -15,11 +15,14 @@ adder folded in ring order).
   next      ring allreduce (the reference's planned 8_allreduce), 64 and 256 MiB fp16;
             alltoall (its planned 9_alltoall), 64 and 256 MiB fp16 per rank
 
-    --staging reference|tuned   only the geometry the configuration names, or
-                                only the library's tuned default (a profile of one
-                                such run has one launch shape per kernel name)
+    --staging reference|tuned|none   only the geometry the configuration names, only
+                                the library's tuned geometry through staging, or
+                                only the operators' default, whose rings run inside
+                                compute units without staging (a profile of one such
+                                run has one launch shape per kernel name)
 
-Algorithmic bytes (`alg_gbps`: what the ring moves, staging included): copy 2S;
+Algorithmic bytes (`alg_gbps`: what the ring moves, staging included; not given
+where there is none): copy 2S;
 sendrecv over h hops (2 + 2h) S; broadcast / allgather (3N - 2) S; reduce /
 reducescatter (3N + 1) S; alltoall 4 N S.  `hbm_gbps` counts only what has to
 cross HBM - inputs read once, results written once: sendrecv 2S, broadcast N S,
@@ -67,32 +70,44 @@ def time_ms(fn, reps: int) -> float:
     return best
 
 
-STAGING = ("reference", "tuned")      # set from --staging
+STAGING = ("reference", "tuned", "none")      # set from --staging
+WIRES = (("ll128", _lib.PROTO_LL128), ("simple", _lib.PROTO_SIMPLE))
 
 
-def geometries(reference_label: str, slots):
-    """(label, slots) pairs to run: the geometry the configuration names and /
-    or the library's tuned default."""
-    out = []
-    if "reference" in STAGING:
-        out.append((reference_label, slots))
-    if "tuned" in STAGING:
-        out.append(("tuned", None))
-    return out
+def runs(reference_label: str | None, slots=None, wires=WIRES):
+    """(protocol's name, its code, label, slots) of every run: through staging at the
+    geometry the configuration names and / or the library's tuned one, by each
+    protocol, and at the operators' default (label "none"), which needs neither."""
+    for name, proto in wires:
+        if "reference" in STAGING and reference_label:
+            yield name, proto, reference_label, slots
+        if "tuned" in STAGING:
+            yield name, proto, "tuned", None
+    if "none" in STAGING:
+        yield None, None, "none", None
 
 
 def emit(**kw) -> None:
+    """One line; ``alg_bytes`` and ``hbm_bytes`` become rates."""
+    t = kw["ms"] if "ms" in kw else kw["us"] / 1e3
+    alg = kw.pop("alg_bytes", None)
+    if alg is not None and kw.get("staging") != "none":
+        kw["alg_gbps"] = round(alg / t / 1e6, 1)
     if "hbm_bytes" in kw:
-        t = kw["ms"] if "ms" in kw else kw["us"] / 1e3
         kw["hbm_gbps"] = round(kw.pop("hbm_bytes") / t / 1e6, 1)
     print(json.dumps(kw), flush=True)
 
 
-def comm_for(world: int, proto: int, slots=None, **kw) -> VirtualComm:
-    """slots = (nslots, slot_bytes) for the geometry the configuration names;
-    None = the library's tuned default."""
+def comm_for(world: int, proto: int | None, label: str = "tuned", slots=None, **kw) -> VirtualComm:
+    """slots = (nslots, slot_bytes) and 512 wave-channels for the geometry the
+    configuration names; "tuned": the library's own through staging (naming the
+    placement asks for it); "none": nothing named."""
+    if label == "none":
+        return VirtualComm(world_size=world, device=DEV, **kw)
     if slots is not None:
-        kw.update(buff_size_=slots[0] * slots[1], nslots=slots[0])
+        kw.update(buff_size_=slots[0] * slots[1], nslots=slots[0], waves_per_rank=512)
+    else:
+        kw.update(placement=_lib.PLACE_LOCAL)
     return VirtualComm(world_size=world, device=DEV, protocol=proto, **kw)
 
 
@@ -125,25 +140,24 @@ def config2(reps: int) -> None:
     src = torch.randn(n, generator=g, device=DEV, dtype=torch.float32).to(torch.float16)
     dst = torch.zeros_like(src)
     S = n * 2
-    for name, proto in (("ll128", 0), ("simple", 1)):
-        for label, slots in geometries("8x512KiB", (8, 512 * 1024)):
-            comm = comm_for(2, proto, slots, waves_per_rank=512 if slots else None)
+    for name, proto, label, slots in runs("8x512KiB", (8, 512 * 1024)):
+        comm = comm_for(2, proto, label, slots)
 
-            def step():
-                with comm.rank(0):
-                    sendrecv_buffer.send(src, 1, comm)
-                with comm.rank(1):
-                    sendrecv_buffer.recv(dst, 0, comm)
-                sendrecv_buffer.sync(comm)
+        def step():
+            with comm.rank(0):
+                sendrecv_buffer.send(src, 1, comm)
+            with comm.rank(1):
+                sendrecv_buffer.recv(dst, 0, comm)
+            sendrecv_buffer.sync(comm)
 
-            dst.zero_()
-            step()
-            comm.check()
-            ok = torch.equal(dst.view(torch.int16), src.view(torch.int16))
-            ms = time_ms(step, reps)
-            emit(config=2, op="sendrecv", protocol=name, staging=label, bytes=S, ms=round(ms, 4),
-                 alg_gbps=round(4 * S / ms / 1e6, 1), hbm_bytes=2 * S,
-                 algbw_gbps=round(S / ms / 1e6, 1), ok=ok, grid=comm.last_grid)
+        dst.zero_()
+        step()
+        comm.check()
+        ok = torch.equal(dst.view(torch.int16), src.view(torch.int16))
+        ms = time_ms(step, reps)
+        emit(config=2, op="sendrecv", protocol=name, staging=label, bytes=S, ms=round(ms, 4),
+             alg_bytes=4 * S, hbm_bytes=2 * S,
+             algbw_gbps=round(S / ms / 1e6, 1), ok=ok, grid=comm.last_grid)
     comm = VirtualComm(world_size=2, device=DEV)
 
     def direct():
@@ -158,7 +172,7 @@ def config2(reps: int) -> None:
     ok = torch.equal(dst.view(torch.int16), src.view(torch.int16))
     ms = time_ms(direct, reps)
     emit(config=2, op="sendrecv_direct", protocol="simple copy", bytes=S, ms=round(ms, 4),
-         alg_gbps=round(2 * S / ms / 1e6, 1), hbm_bytes=2 * S, algbw_gbps=round(S / ms / 1e6, 1), ok=ok)
+         alg_bytes=2 * S, hbm_bytes=2 * S, algbw_gbps=round(S / ms / 1e6, 1), ok=ok)
 
 
 def config3(reps: int) -> None:
@@ -167,22 +181,21 @@ def config3(reps: int) -> None:
     root = (torch.rand(n, generator=g, device=DEV) * 8 - 4).to(torch.float16)
     bufs = [root.clone() if r == 0 else torch.zeros_like(root) for r in range(world)]
     S = n * 2
-    for name, proto in (("ll128", 0), ("simple", 1)):
-        for label, slots in geometries("8x512KiB", (8, 512 * 1024)):
-            comm = comm_for(world, proto, slots, waves_per_rank=512 if slots else None)
-            for b in bufs[1:]:
-                b.zero_()
+    for name, proto, label, slots in runs("8x512KiB", (8, 512 * 1024)):
+        comm = comm_for(world, proto, label, slots)
+        for b in bufs[1:]:
+            b.zero_()
 
-            def step():
-                comm.run(lambda r: broadcast(bufs[r], 0, comm))
+        def step():
+            comm.run(lambda r: broadcast(bufs[r], 0, comm))
 
-            step()
-            comm.check()
-            ok = all(torch.equal(b.view(torch.int16), root.view(torch.int16)) for b in bufs)
-            ms = time_ms(step, reps)
-            emit(config=3, op="broadcast", protocol=name, staging=label, world=world, bytes=S,
-                 ms=round(ms, 4), alg_gbps=round((3 * world - 2) * S / ms / 1e6, 1),
-                 hbm_bytes=world * S, algbw_gbps=round(S / ms / 1e6, 1), ok=ok, grid=comm.last_grid)
+        step()
+        comm.check()
+        ok = all(torch.equal(b.view(torch.int16), root.view(torch.int16)) for b in bufs)
+        ms = time_ms(step, reps)
+        emit(config=3, op="broadcast", protocol=name, staging=label, world=world, bytes=S,
+             ms=round(ms, 4), alg_bytes=(3 * world - 2) * S,
+             hbm_bytes=world * S, algbw_gbps=round(S / ms / 1e6, 1), ok=ok, grid=comm.last_grid)
 
 
 def fold_device(rows: list, order: list[int]) -> torch.Tensor:
@@ -202,8 +215,8 @@ def config4(reps: int) -> None:
             orig.append(torch.randn(world, n, generator=g, device=DEV, dtype=torch.float32)
                         .to(TDT[dt]))
         S = n_total * orig[0].element_size()
-        for label, slots in geometries("8x1MiB", (8, 1 << 20)):
-            comm = comm_for(world, 0, slots, waves_per_rank=512 if slots else None)
+        for _, proto, label, slots in runs("8x1MiB", (8, 1 << 20), WIRES[:1]):
+            comm = comm_for(world, proto, label, slots)
             bufs = [o.clone() for o in orig]
 
             def rs():
@@ -217,7 +230,7 @@ def config4(reps: int) -> None:
                      for c in range(world))
             ms = time_ms(rs, reps)
             emit(config=4, op="reducescatter", dtype=dt, staging=label, world=world, bytes=S,
-                 ms=round(ms, 4), alg_gbps=round((3 * world + 1) * S / ms / 1e6, 1),
+                 ms=round(ms, 4), alg_bytes=(3 * world + 1) * S,
                  hbm_bytes=(world + 1) * S, algbw_gbps=round(S / ms / 1e6, 1), ok=ok, grid=comm.last_grid)
             flat = [o.reshape(-1).clone() for o in orig]
 
@@ -231,91 +244,92 @@ def config4(reps: int) -> None:
                              .view(torch.uint8))
             ms = time_ms(rd, reps)
             emit(config=4, op="reduce", dtype=dt, staging=label, world=world, bytes=S,
-                 ms=round(ms, 4), alg_gbps=round((3 * world + 1) * S / ms / 1e6, 1),
+                 ms=round(ms, 4), alg_bytes=(3 * world + 1) * S,
                  hbm_bytes=(world + 1) * S, algbw_gbps=round(S / ms / 1e6, 1), ok=ok, grid=comm.last_grid)
 
 
 def config5(reps: int, max_log2: int, only_log2=()) -> None:
     world = 8
-    for name, proto in (("ll128", 0), ("simple", 1)):
-        comms = {label: comm_for(world, proto, slots, waves_per_rank=512 if slots else None)
-                 for label, slots in geometries("8x512KiB", (8, 512 * 1024))}
-        for log2 in (only_log2 or range(9, max_log2 + 1)):
-            shard = 1 << log2
-            n = shard // 2
-            bufs = []
-            for r in range(world):
-                g = torch.Generator(device=DEV).manual_seed(4 + r)
-                b = torch.zeros(world, n, device=DEV, dtype=torch.float16)
-                b[r] = (torch.rand(n, generator=g, device=DEV) * 2 - 1).to(torch.float16)
-                bufs.append(b)
-            want = torch.stack([bufs[r][r] for r in range(world)])
-            for label, comm in comms.items():
-                def step():
-                    comm.run(lambda r: allgather(bufs[r], comm))
+    ring = list(range(world)) + [0]
+    comms = [(name, proto, label, comm_for(world, proto, label, slots))
+             for name, proto, label, slots in runs("8x512KiB", (8, 512 * 1024))]
+    for log2 in (only_log2 or range(9, max_log2 + 1)):
+        shard = 1 << log2
+        n = shard // 2
+        S = world * shard
+        many = (reps if log2 < 24 else max(2, reps // 2)) * 4
+        bufs = []
+        for r in range(world):
+            g = torch.Generator(device=DEV).manual_seed(4 + r)
+            b = torch.zeros(world, n, device=DEV, dtype=torch.float16)
+            b[r] = (torch.rand(n, generator=g, device=DEV) * 2 - 1).to(torch.float16)
+            bufs.append(b)
+        want = torch.stack([bufs[r][r] for r in range(world)])
+        ptrs = {r: bufs[r].data_ptr() for r in range(world)}
 
-                step()
+        def right() -> bool:
+            return all(torch.equal(b.view(torch.int16), want.view(torch.int16)) for b in bufs)
+
+        def clear() -> None:
+            for r, b in enumerate(bufs):
+                b.zero_()
+                b[r] = want[r]
+
+        for name, proto, label, comm in comms:
+            clear()
+            comm.run(lambda r: allgather(bufs[r], comm))
+            comm.check()
+            ok = right()
+            # launch straight from a prepared descriptor: leaves out the
+            # per-rank bookkeeping, which would dominate small sizes
+            make = comm.make_cu_op if label == "none" else comm.make_op
+            d = make(_lib.OP_ALLGATHER, _lib.BYTES, shard, ptrs, ptrs, ring, row_stride=shard)
+            ms = time_ms(lambda: comm.launch(d), many)
+            comm.check()
+            emit(config=5, op="allgather", protocol=name, staging=label, world=world,
+                 shard_bytes=shard, us=round(ms * 1e3, 2),
+                 alg_bytes=(3 * world - 2) * S, hbm_bytes=world * S,
+                 busbw_gbps=round(shard * (world - 1) / ms / 1e6, 1), ok=ok)
+            if label == "tuned" and proto == _lib.PROTO_LL128 and log2 in (16, 20, 23, 27):
+                # the temporal schedule (6_allgather.py:25-77): row after row
+                # through one pipeline; same bytes
+                clear()
+                td = comm.make_op(_lib.OP_ALLGATHER_TEMPORAL, _lib.BYTES, shard, ptrs, ptrs, ring,
+                                  row_stride=shard, protocol=_lib.PROTO_LL128)
+                comm.launch(td)
                 comm.check()
-                ok = all(torch.equal(b.view(torch.int16), want.view(torch.int16)) for b in bufs)
-                # launch straight from a prepared descriptor: leaves out the
-                # per-rank Python bookkeeping, which would dominate small sizes
-                ptrs = {r: bufs[r].data_ptr() for r in range(world)}
-                d = comm.make_op(_lib.OP_ALLGATHER, _lib.BYTES, shard, ptrs, ptrs,
-                                 list(range(world)) + [0], row_stride=shard)
-                ms = time_ms(lambda: comm.launch(d), (reps if log2 < 24 else max(2, reps // 2)) * 4)
+                tok = right()
+                tms = time_ms(lambda: comm.launch(td), many)
                 comm.check()
-                S = world * shard
-                emit(config=5, op="allgather", protocol=name, staging=label, world=world,
-                     shard_bytes=shard, us=round(ms * 1e3, 2),
-                     alg_gbps=round((3 * world - 2) * S / ms / 1e6, 1), hbm_bytes=world * S,
-                     busbw_gbps=round(shard * (world - 1) / ms / 1e6, 1), ok=ok)
-                if label == "tuned" and proto == 0 and log2 in (16, 20, 23, 27):
-                    # the temporal schedule (6_allgather.py:25-77): row after row
-                    # through one pipeline; same bytes
-                    for b in bufs:
-                        b.zero_()
-                    for r in range(world):
-                        bufs[r][r] = want[r]
-                    td = comm.make_op(_lib.OP_ALLGATHER_TEMPORAL, _lib.BYTES, shard, ptrs, ptrs,
-                                      list(range(world)) + [0], row_stride=shard,
-                                      protocol=_lib.PROTO_LL128)
-                    comm.launch(td)
-                    comm.check()
-                    tok = all(torch.equal(b.view(torch.int16), want.view(torch.int16)) for b in bufs)
-                    tms = time_ms(lambda: comm.launch(td), (reps if log2 < 24 else max(2, reps // 2)) * 4)
-                    comm.check()
-                    emit(config=5, op="allgather", protocol=name, staging="tuned, temporal",
-                         world=world, shard_bytes=shard, us=round(tms * 1e3, 2),
-                         alg_gbps=round((3 * world - 2) * S / tms / 1e6, 1), hbm_bytes=world * S,
-                         busbw_gbps=round(shard * (world - 1) / tms / 1e6, 1), ok=tok)
-                if label == "tuned" and log2 <= 16 and log2 % 2 == 1:
-                    # the same launch as 20 nodes of a HIP graph (epoch in device
-                    # memory, advanced by a small kernel in front of every launch):
-                    # what the device needs once the host is out of the way
-                    gcomm = VirtualComm(world_size=world, device=DEV, protocol=proto,
-                                        device_epoch=True)
-                    gd = gcomm.make_op(_lib.OP_ALLGATHER, _lib.BYTES, shard, ptrs, ptrs,
-                                       list(range(world)) + [0], row_stride=shard)
-                    side = torch.cuda.Stream(device=DEV)
-                    with torch.cuda.stream(side):
+                emit(config=5, op="allgather", protocol=name, staging="tuned, temporal",
+                     world=world, shard_bytes=shard, us=round(tms * 1e3, 2),
+                     alg_bytes=(3 * world - 2) * S, hbm_bytes=world * S,
+                     busbw_gbps=round(shard * (world - 1) / tms / 1e6, 1), ok=tok)
+            if label == "tuned" and log2 <= 16 and log2 % 2 == 1:
+                # the same launch as 20 nodes of a HIP graph (epoch in device
+                # memory, advanced by a small kernel in front of every launch):
+                # what the device needs once the host is out of the way
+                gcomm = comm_for(world, proto, label, device_epoch=True)
+                gd = gcomm.make_op(_lib.OP_ALLGATHER, _lib.BYTES, shard, ptrs, ptrs, ring, row_stride=shard)
+                side = torch.cuda.Stream(device=DEV)
+                with torch.cuda.stream(side):
+                    gcomm.launch(gd)
+                side.synchronize()
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=side):
+                    for _ in range(20):
                         gcomm.launch(gd)
-                    side.synchronize()
-                    graph = torch.cuda.CUDAGraph()
-                    with torch.cuda.graph(graph, stream=side):
-                        for _ in range(20):
-                            gcomm.launch(gd)
-                    gms = time_ms(graph.replay, reps * 2) / 20
-                    gcomm.check()
-                    gok = all(torch.equal(b.view(torch.int16), want.view(torch.int16)) for b in bufs)
-                    emit(config=5, op="allgather", protocol=name, staging="tuned, graph of 20",
-                         world=world, shard_bytes=shard, us=round(gms * 1e3, 2), ok=gok)
-            del bufs
+                gms = time_ms(graph.replay, reps * 2) / 20
+                gcomm.check()
+                emit(config=5, op="allgather", protocol=name, staging="tuned, graph of 20",
+                     world=world, shard_bytes=shard, us=round(gms * 1e3, 2), ok=right())
+        del bufs
 
 
 def allreduce_bench(reps: int) -> None:
-    """The reference's planned 8_allreduce: 8 ranks x 256 MiB fp16, as a
-    reduce-scatter launch followed by an allgather launch (the default) and as
-    one pass round the ring.  Payload bytes (6N - 4) S for the one pass: per
+    """The reference's planned 8_allreduce: 8 ranks x 64 and 256 MiB fp16, as a
+    reduce-scatter launch followed by an allgather launch (the default through
+    staging) and as one pass round the ring (the default inside compute units).  Payload bytes (6N - 4) S for the one pass: per
     chunk N own-row reads, 2N - 2 staging writes and reads, N result writes;
     the same figure is used for both so that the rates compare."""
     from mintccl_amd.allreduce import allreduce
@@ -327,9 +341,9 @@ def allreduce_bench(reps: int) -> None:
             orig.append(torch.randn(n, generator=g, device=DEV, dtype=torch.float32)
                         .to(torch.float16))
         S = n * 2
-        for name, proto, fused in (("ll128", 0, False), ("ll128", 0, True), ("simple", 1, False),
-                                   ("simple", 1, True)):
-            comm = comm_for(world, proto, None)
+        for name, proto, label, fused in [(name, proto, label, fused) for name, proto, label, _ in runs(None)
+                                          for fused in (False, True)]:
+            comm = comm_for(world, proto, label)
             bufs = [o.clone() for o in orig]
 
             def step():
@@ -346,8 +360,8 @@ def allreduce_bench(reps: int) -> None:
                                             want.view(torch.int16)) for b in bufs)
             ms = time_ms(step, reps)
             emit(config="next", op="allreduce", protocol=name,
-                 mode="one pass" if fused else "reducescatter + allgather", staging="tuned",
-                 world=world, bytes=S, ms=round(ms, 4), alg_gbps=round((6 * world - 4) * S / ms / 1e6, 1),
+                 mode="one pass" if fused else "reducescatter + allgather", staging=label,
+                 world=world, bytes=S, ms=round(ms, 4), alg_bytes=(6 * world - 4) * S,
                  hbm_bytes=2 * world * S, algbw_gbps=round(S / ms / 1e6, 1),
                  busbw_gbps=round(2 * (world - 1) / world * S / ms / 1e6, 1), ok=ok,
                  grid=comm.last_grid)
@@ -369,8 +383,8 @@ def alltoall_bench(reps: int) -> None:
                         .to(torch.float16))
         outs = [torch.zeros_like(b) for b in bufs]
         S = n_total * 2
-        for name, proto in (("ll128", 0), ("simple", 1)):
-            comm = comm_for(world, proto, None)
+        for name, proto, label, _ in runs(None):
+            comm = comm_for(world, proto, label)
 
             def step():
                 comm.run(lambda r: alltoall(bufs[r], outs[r], comm))
@@ -382,8 +396,8 @@ def alltoall_bench(reps: int) -> None:
             ok = all(torch.equal(outs[d][s].view(torch.int16), bufs[s][d].view(torch.int16))
                      for d in range(world) for s in range(world))
             ms = time_ms(step, reps)
-            emit(config="next", op="alltoall", protocol=name, staging="tuned", world=world, bytes=S,
-                 ms=round(ms, 4), alg_gbps=round(4 * world * S / ms / 1e6, 1),
+            emit(config="next", op="alltoall", protocol=name, staging=label, world=world, bytes=S,
+                 ms=round(ms, 4), alg_bytes=4 * world * S,
                  hbm_bytes=2 * world * S, algbw_gbps=round(S / ms / 1e6, 1), ok=ok,
                  grid=comm.last_grid)
         del bufs, outs
@@ -502,7 +516,8 @@ def hypercube_bench(reps: int, log2s=(14, 20, 26)) -> None:
 
 def main() -> int:
     ap = argparse.ArgumentParser()
-    ap.add_argument("--staging", choices=("both", "reference", "tuned"), default="both")
+    ap.add_argument("--staging", choices=("all", "both", "reference", "tuned", "none"), default="all",
+                    help="both: reference and tuned")
     ap.add_argument("--quick", action="store_true", help="fewer repetitions, sweep to 16 MiB")
     ap.add_argument("--only", type=int, default=0,
                     help="run one config (1..5; 8 = allreduce; 9 = alltoall; 10 = tree against ring; "
@@ -515,7 +530,8 @@ def main() -> int:
                     help="config 11: log2 of the message sizes (bytes per rank)")
     args = ap.parse_args()
     global STAGING
-    STAGING = ("reference", "tuned") if args.staging == "both" else (args.staging,)
+    STAGING = {"all": ("reference", "tuned", "none"), "both": ("reference", "tuned")}.get(
+        args.staging, (args.staging,))
     reps = 3 if args.quick else 8
     torch.cuda.set_device(DEV)
     if args.only in (0, 1):
