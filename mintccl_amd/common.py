@@ -294,6 +294,13 @@ class VirtualComm:
     Ranks enter with ``with comm.rank(r):`` and call the reference-named
     operators; the call that completes the set of participants enqueues ONE
     fused launch that runs all ranks' kernels.
+
+    With nothing about the staging named (geometry, placement, cache policy,
+    block size, row fetch, origins: an argument, a knob, or the attribute set
+    later) the operators' rings run inside compute units and use none of it.
+    ``protocol`` alone does not ask for staging: it says how a hop through
+    staging is made safe, and inside a compute unit there is none to make safe -
+    the bytes that arrive are the same either way.
     """
 
     def __init__(self, world_size: int | None = None, device: str | torch.device = "cuda:0",
@@ -319,7 +326,7 @@ class VirtualComm:
         # budget of staging per rank
         self.auto_geometry = (tuned and buff_size_ is None and nslots is None
                               and waves_per_rank is None)
-        # With everything about the wire left to the library the operators' rings
+        # With everything about the staging left to the library the operators' rings
         # run inside compute units; naming a placement, a cache policy, a
         # block size, who fetches the rows or where the origins sit (arguments,
         # MINTCCL_*, or the attribute set later) asks for the rings through

@@ -1,5 +1,5 @@
 """Rings inside compute units (what the operators run when nothing about the
-wire is named): rows around every edge of the walk - less than a lane's 16
+staging is named): rows around every edge of the walk - less than a lane's 16
 bytes, around a wavefront's 1 KiB and a tile's 2, at any byte, in both forms of
 the kernels - bit for bit against the oracle or, for the large rows, against the
 same additions in torch."""

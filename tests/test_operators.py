@@ -117,3 +117,16 @@ def test_naming_the_wire_after_construction_goes_through_staging(make_comm, name
     assert not comm.inside_cu and d.placement != _lib.PLACE_CU and d.nslots
     if name in ("placement", "cache_policy", "row_fetch", "origin_cus", "threads_per_block", "nslots"):
         assert getattr(d, name) == value
+
+
+def test_the_protocol_says_how_a_hop_through_staging_is_made(make_comm, monkeypatch):
+    """It alone does not ask for staging (inside a compute unit there is no hop to
+    make safe); with anything else of the wire named it is the launch's."""
+    assert make_comm(protocol=_lib.PROTO_SIMPLE).inside_cu
+    monkeypatch.setenv("MINTCCL_PROTOCOL", "simple")
+    assert make_comm().inside_cu
+    comm = make_comm(8, placement=_lib.PLACE_LOCAL)
+    assert not comm.inside_cu
+    ptrs = {r: 4096 * (r + 1) for r in range(8)}
+    d = comm.make_op(_lib.OP_ALLGATHER, _lib.BYTES, 4096, ptrs, ptrs, list(range(8)) + [0], row_stride=4096)
+    assert d.protocol == _lib.PROTO_SIMPLE and d.staging[0]
