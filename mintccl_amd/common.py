@@ -283,7 +283,9 @@ _LAUNCH_ATTRIBUTES = frozenset(("inside_cu", "stats", "protocol", "spin_budget",
 _STAGING_ATTRIBUTES = frozenset(("placement", "cache_policy", "row_fetch", "origin_cus", "threads_per_block",
                                  "threads_explicit", "waves_per_rank", "nslots", "slot_bytes", "buff_size",
                                  "auto_geometry"))
-_PASSED_BY = frozenset(("launch", "enqueue", "make_op", "make_cu_op", "Get_rank", "rank"))
+_LAUNCHING = frozenset(("launch", "enqueue", "make_op", "make_cu_op"))
+_PASSED_BY = _LAUNCHING | {"Get_rank", "rank"}
+_ASKED_FOR = _LAUNCH_ATTRIBUTES | _STAGING_ATTRIBUTES | _PASSED_BY
 
 
 class VirtualComm:
@@ -408,24 +410,25 @@ class VirtualComm:
 
     def __setattr__(self, name: str, value) -> None:
         object.__setattr__(self, name, value)
-        if name in _STAGING_ATTRIBUTES and "_board" in self.__dict__:
-            self.inside_cu = False     # as naming it in the constructor
-        if (name in _LAUNCH_ATTRIBUTES or name in _PASSED_BY) and "_board" in self.__dict__:
+        if name in _ASKED_FOR and "_board" in self.__dict__:
+            if name in _STAGING_ATTRIBUTES:
+                self.inside_cu = False     # as naming it in the constructor
             self._board.stale()
 
     def __delattr__(self, name: str) -> None:
         object.__delattr__(self, name)
-        if (name in _LAUNCH_ATTRIBUTES or name in _PASSED_BY) and "_board" in self.__dict__:
+        if name in _ASKED_FOR and "_board" in self.__dict__:
             self._board.stale()
 
-    def _replaced(self, *methods: str) -> bool:
-        """Whether a subclass or this object brings one of ``methods`` itself."""
-        return any(m in self.__dict__ or getattr(type(self), m) is not _METHODS[m] for m in methods)
+    def _replaced(self) -> list[str]:
+        """The methods that a subclass or this object brings itself."""
+        own, cls = self.__dict__, type(self)
+        return [m for m, f in _METHODS.items() if m in own or getattr(cls, m) is not f]
 
     def _runs_inside(self) -> bool:
         """Whether rings run inside compute units (a make_op of one's own
         describes launches through staging)."""
-        return self.inside_cu and self.stats is None and not self._replaced("make_op")
+        return self.inside_cu and self.stats is None and "make_op" not in self._replaced()
 
     def _refresh(self) -> None:
         """Tell the board what launches take from this communicator (it asks
@@ -435,8 +438,9 @@ class VirtualComm:
             ring = ring_of(self)
         except Exception:
             ring = []                  # routes only: a collective will say so
-        self._board.configure(self._runs_inside() and not self._replaced("launch", "enqueue", "make_cu_op"),
-                              self._replaced("Get_rank"), self._replaced("rank"),
+        replaced = self._replaced()
+        self._board.configure(self.inside_cu and self.stats is None and _LAUNCHING.isdisjoint(replaced),
+                              "Get_rank" in replaced, "rank" in replaced,
                               getattr(self, "topology", None) is None, ring, self.protocol,
                               self.spin_budget, self.status.data_ptr())
 
