@@ -8,7 +8,6 @@ import torch
 
 from . import _lib
 from .common import DTYPE_CODE, VirtualComm, get_comm
-from .topology import find_ring, uniform_topology
 
 
 def nbytes(t: torch.Tensor) -> int:
@@ -41,17 +40,8 @@ def front(action: int, go_on=None):
 
 
 def ring_of(comm: VirtualComm) -> list[int]:
-    """The ring of the communicator's topology (searched once per topology
-    object: the search costs more than a small collective)."""
-    topo = getattr(comm, "topology", None)
-    cached = getattr(comm, "_ring_cache", None)
-    if cached is not None and cached[0] is topo:
-        return cached[1]
-    ring = find_ring(topo or uniform_topology(comm.world_size))
-    if len(ring) != comm.world_size + 1:
-        raise RuntimeError("topology has no ring through every rank")
-    comm._ring_cache = (topo, ring)
-    return ring
+    """The ring of the communicator's topology."""
+    return comm._ring()
 
 
 def same_everywhere(posted: dict, field: str, what: str):

@@ -16,6 +16,7 @@ import time
 import torch
 
 from . import _lib
+from .topology import find_ring, find_route, uniform_topology
 
 NULL = 0                       # common.py:71
 WARP_SIZE = 64                 # common.py:104 is 32; a CDNA4 wavefront has 64 lanes
@@ -433,9 +434,8 @@ class VirtualComm:
     def _refresh(self) -> None:
         """Tell the board what launches take from this communicator (it asks
         when it has been told that one of them was set)."""
-        from ._ops import ring_of
         try:
-            ring = ring_of(self)
+            ring = self._ring()
         except Exception:
             ring = []                  # routes only: a collective will say so
         replaced = self._replaced()
@@ -444,8 +444,20 @@ class VirtualComm:
                               getattr(self, "topology", None) is None, ring, self.protocol,
                               self.spin_budget, self.status.data_ptr())
 
+    def _ring(self) -> list[int]:
+        """The ring of the topology (searched once per topology object: the
+        search costs more than a small collective)."""
+        topo = getattr(self, "topology", None)
+        cached = getattr(self, "_ring_cache", None)
+        if cached is not None and cached[0] is topo:
+            return cached[1]
+        ring = find_ring(topo or uniform_topology(self.world_size))
+        if len(ring) != self.world_size + 1:
+            raise RuntimeError("topology has no ring through every rank")
+        self._ring_cache = (topo, ring)
+        return ring
+
     def _find_route(self, src: int, dst: int) -> list[int]:
-        from .topology import find_route, uniform_topology
         return find_route(src, dst, getattr(self, "topology", None) or uniform_topology(self.world_size))
 
     @property
