@@ -6,6 +6,13 @@
 namespace mint {
 namespace {
 
+// `rows`: pipelines, alltoall: destinations
+dim3 grid_of(const Plan& plan, uint32_t rows, uint32_t sources) {
+    const CuRingArgs& a = plan.cu_args;
+    const bool by_row = plan.cu_large || a.shape.part;
+    return dim3(by_row ? a.blocks : rows, by_row ? rows : a.blocks, sources);
+}
+
 template <auto KERNEL, int N, bool SPLIT>
 int launch_as(const Plan& plan, hipStream_t stream) {
     const CuRingArgs& a = plan.cu_args;
@@ -16,10 +23,8 @@ int launch_as(const Plan& plan, hipStream_t stream) {
         if (SPLIT) tables.rank[N + i] = a.output[i];
     }
     tables.status = a.status;
-    const uint32_t x = s.tiles + a.ends;
-    const dim3 grid(plan.cu_large ? x : a.pipes, plan.cu_large ? a.pipes : x);
-    return Launch<KERNEL>::go(grid, (unsigned)plan.threads, (unsigned)plan.cu_lds, stream, s.row_bytes,
-                              s.row_stride, s.short_bytes, s.starts, s.full, s.tiles, tables);
+    return Launch<KERNEL>::go(grid_of(plan, a.pipes, 1), (unsigned)plan.threads, (unsigned)plan.cu_lds, stream,
+                              s.numbers(), s.counts(), tables);
 }
 
 // (in place only in the small form: to the large one the host's time is nothing)
@@ -27,17 +32,21 @@ template <int DT, int N, bool EVERYWHERE>
 int launch_sum(const Plan& plan, hipStream_t stream) {
     if constexpr (N >= kCuStreamRanks && !EVERYWHERE)
         if (plan.cu_stream)
-            return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, true, true, CU_NT>, N, true>(plan, stream);
-    if (plan.cu_large) return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, true, true>, N, true>(plan, stream);
+            return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, CuLargeSumStreamed, true>, N, true>(plan, stream);
+    using Large = std::conditional_t<EVERYWHERE, CuLargeSumEverywhere, CuLargeSum>;
+    using Small = CuSmall<EVERYWHERE>;
+    if (plan.cu_large) return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Large, true>, N, true>(plan, stream);
     if (plan.cu_args.split)
-        return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, false, true>, N, true>(plan, stream);
-    return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, false, false>, N, false>(plan, stream);
+        return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Small, true>, N, true>(plan, stream);
+    return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Small, false>, N, false>(plan, stream);
 }
 template <int N>
 int launch_copy(const Plan& plan, hipStream_t stream) {
-    if (plan.cu_large) return launch_as<&cu_ring_copy_kernel<N, true, true>, N, true>(plan, stream);
-    if (plan.cu_args.split) return launch_as<&cu_ring_copy_kernel<N, false, true>, N, true>(plan, stream);
-    return launch_as<&cu_ring_copy_kernel<N, false, false>, N, false>(plan, stream);
+    using Large = std::conditional_t<(N > 2), CuLargeCopies, CuLargeCopy>;
+    using Small = CuSmall<(N > 2)>;
+    if (plan.cu_large) return launch_as<&cu_ring_copy_kernel<N, Large, true>, N, true>(plan, stream);
+    if (plan.cu_args.split) return launch_as<&cu_ring_copy_kernel<N, Small, true>, N, true>(plan, stream);
+    return launch_as<&cu_ring_copy_kernel<N, Small, false>, N, false>(plan, stream);
 }
 
 template <int N>
@@ -70,17 +79,14 @@ int launch_alltoall(const Plan& plan, hipStream_t stream) {
         near.rank[i] = (uint32_t)(off >> kCuNearShift);
         rest |= off ^ (uint64_t)near.rank[i] << kCuNearShift;
     }
-    const uint32_t x = s.tiles + a.ends;
-    const dim3 grid(plan.cu_large ? x : a.len, plan.cu_large ? a.len : x, a.len);
+    const dim3 grid = grid_of(plan, a.len, a.len);
     const unsigned threads = (unsigned)plan.threads;
+    const u64x4 numbers = {s.row_bytes, s.row_stride, lowest, reinterpret_cast<uint64_t>(a.status)};
     if (plan.cu_large)
-        return Launch<&cu_alltoall_kernel<true, uint64_t>>::go(grid, threads, 0, stream, s.row_bytes, s.row_stride,
-                                                               lowest, a.status, s.tiles, far);
+        return Launch<&cu_alltoall_kernel<CuLargeCopy, uint64_t>>::go(grid, threads, 0, stream, numbers, s.counts(), far);
     if (rest)
-        return Launch<&cu_alltoall_kernel<false, uint64_t>>::go(grid, threads, 0, stream, s.row_bytes, s.row_stride,
-                                                                lowest, a.status, s.tiles, far);
-    return Launch<&cu_alltoall_kernel<false, uint32_t>>::go(grid, threads, 0, stream, s.row_bytes, s.row_stride,
-                                                            lowest, a.status, s.tiles, near);
+        return Launch<&cu_alltoall_kernel<CuSmall<false>, uint64_t>>::go(grid, threads, 0, stream, numbers, s.counts(), far);
+    return Launch<&cu_alltoall_kernel<CuSmall<false>, uint32_t>>::go(grid, threads, 0, stream, numbers, s.counts(), near);
 }
 
 }  // namespace

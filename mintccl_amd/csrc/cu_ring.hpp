@@ -23,26 +23,37 @@
 // reduce-scatter of 256 MiB f16 447 / 470 / 391 / 375 us, allgather of 8 x 128 MiB
 // 1675 / 1660 / 1540 / 1380, allreduce of 64 MiB bf16 205 / 198 / 190 / 165.
 #pragma once
+#include <type_traits>
+
 #include "ring.hpp"
 
 namespace mint {
 
 // One launch.  Grid: tiles of a row, then one block for its ragged ends if it has
-// any, in x (large form) or y; pipelines (alltoall: destinations) in the other;
-// the sources of an alltoall in z.
+// any, and pipelines (alltoall: destinations) in x and y (CuPlace); the sources of an
+// alltoall in z.
 //
 // A block lives for one trip to memory, so what it does before its loads are out
-// counts: the numbers come as kernel arguments of their own, which the compiler
-// has the hardware put into scalar registers before the first instruction
-// (kernarg preload), and one round of scalar loads brings the addresses.
+// counts: the numbers come as the first kernel arguments, which the compiler has the
+// hardware put into scalar registers before the first instruction (kernarg preload;
+// not what is inside a struct, hence the vector), and one round of scalar loads brings
+// the addresses.  Few of them, since each argument costs a launch 10 ns.
+typedef uint64_t u64x4 __attribute__((ext_vector_type(4)));
 struct CuShape {
     uint64_t row_bytes, row_stride;
     uint64_t short_bytes;          // bytes of row `full`; rows behind it are empty
     uint32_t starts;               // bits 3 p: index in the ring of pipeline p's root
     uint32_t full;                 // rows before this one have row_bytes
     uint32_t tiles;                // thread blocks that share the whole vectors of a row
+    uint32_t part;                 // small form: tiles of a row that one XCD takes, or 0 (CuPlace)
+
+    CuShape() = default;
+    __device__ __forceinline__ CuShape(u64x4 numbers, uint64_t counts)
+        : row_bytes(numbers.x), row_stride(numbers.y), short_bytes(numbers.z), starts((uint32_t)numbers.w),
+          full((uint32_t)(numbers.w >> 32)), tiles((uint32_t)counts), part((uint32_t)(counts >> 32)) {}
+    u64x4 numbers() const { return u64x4{row_bytes, row_stride, short_bytes, (uint64_t)full << 32 | starts}; }
+    uint64_t counts() const { return (uint64_t)part << 32 | tiles; }
 };
-#define CU_SHAPE uint64_t row_bytes, uint64_t row_stride, uint64_t short_bytes, uint32_t starts, uint32_t full, uint32_t tiles
 
 // The ranks' buffers in the order of the ring.  One address per rank where they
 // work in place, as the operators do: a launch with up to 112 bytes of arguments
@@ -59,25 +70,10 @@ struct CuRingArgs {
     CuShape shape;
     uint64_t input[kMaxRanks], output[kMaxRanks];
     uint64_t* status;
-    uint32_t op, pipes, len, ends;
+    uint32_t op, pipes, len;
+    uint32_t blocks;               // of the grid for the tiles of a row and its ends
     bool split;
 };
-
-// Two forms of a launch (which: plan_cu in mintccl.hip).
-//
-// LARGE, rows beyond the last-level cache: one wavefront per block and 1 KiB
-// tiles (with several copies two), the pipelines one after the other, as few
-// wavefronts on a compute unit as keep HBM busy (cu_waves).  More of them widen
-// the window over which the loads and stores of 8 or 16 rows are scattered: 8
-// ranks, reduce-scatter of 256 MiB 392 us with 32 to a compute unit, 376 with 9;
-// allreduce of 64 MiB 202 with 20, 158 with 4; allgather of 8 x 64 MiB 89 with 32,
-// 67 with 8.
-//
-// Otherwise: blocks of 128 threads and 2 KiB, dealt to the pipelines in turn,
-// loads through the cache (8 ranks, reduce-scatter of 8 MiB 10.9 us; 15.5 in the
-// large form, 13.0 with one pipeline after the other; blocks of 64 threads lose up
-// to a third where rows are copied once, 512 up to a tenth where they are added).
-constexpr uint32_t cu_threads(bool large, bool copies) { return large && !copies ? 64u : 128u; }
 
 // How rows are loaded: through the caches, or streamed past the last-level one.
 template <bool STREAM>
@@ -93,9 +89,6 @@ __device__ __forceinline__ u32x4 cu_load(const uint8_t* uniform, uint32_t lane) 
 //   large, several:                 allgather of 8 x 64 MiB   - / 73.4 / 94.3 / 67.7
 //   large, one:                     reduce-scatter of 64 MiB 86.9 / 88.6 / 82.1 / 88.0
 enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
-constexpr int cu_stores(bool large, bool several) {
-    return several ? (large ? CU_SC1_NT : CU_SC1) : large ? CU_SC1 : CU_NT;
-}
 // Sums to one place that are far larger than the last-level cache (plan_cu): with
 // many rows to read nt is the faster one, on buffers that have not just been used.
 // Four sets of buffers in turn, reduce-scatter and reduce of f16 and bf16, nt over
@@ -108,6 +101,37 @@ constexpr int cu_stores(bool large, bool several) {
 // The same buffers again and again keep a part of the sums in the cache with sc1:
 // there nt takes 1 - 11 % longer up to 1.5 GiB and is ahead from 2.3 GiB on.
 constexpr int kCuStreamRanks = 6;
+// Two forms of a launch (which: plan_cu in mintccl.hip).
+//
+// LARGE, rows beyond the last-level cache: one wavefront per block and 1 KiB
+// tiles (with several copies two), the pipelines one after the other, as few
+// wavefronts on a compute unit as keep HBM busy (cu_waves).  More of them widen
+// the window over which the loads and stores of 8 or 16 rows are scattered: 8
+// ranks, reduce-scatter of 256 MiB 392 us with 32 to a compute unit, 376 with 9;
+// allreduce of 64 MiB 202 with 20, 158 with 4; allgather of 8 x 64 MiB 89 with 32,
+// 67 with 8.
+//
+// Otherwise: blocks of 128 threads and 2 KiB, loads through the cache, to each XCD
+// consecutive tiles (CuPlace).  8 ranks, reduce-scatter of 8 MiB 10.9 us, 15.5 in the
+// large form.  Blocks of 64 and of 256 threads with 2 KiB and 4 KiB are within 1 % of
+// it, 4 KiB by 64 threads 2 - 4 % slower, 512 threads up to a tenth where rows are added.
+template <int THREADS, int VECTORS, bool LARGE, bool STREAM, int STORES>
+struct CuForm {
+    static constexpr int kThreads = THREADS;       // of a block
+    static constexpr int kVectors = VECTORS;       // of 16 bytes a thread moves, THREADS of them apart
+    static constexpr uint32_t kTile = THREADS * VECTORS * 16;
+    static constexpr bool kLarge = LARGE;
+    static constexpr bool kStream = STREAM;        // rows are loaded past the last-level cache
+    static constexpr int kStores = STORES;
+};
+template <bool SEVERAL>
+using CuSmall = CuForm<128, 1, false, false, SEVERAL ? CU_SC1 : CU_NT>;
+using CuLargeSum = CuForm<64, 1, true, true, CU_SC1>;            // to one place
+using CuLargeSumStreamed = CuForm<64, 1, true, true, CU_NT>;     // (kCuStreamRanks)
+using CuLargeSumEverywhere = CuForm<64, 1, true, true, CU_SC1_NT>;
+using CuLargeCopy = CuForm<64, 1, true, true, CU_SC1>;           // to one place
+using CuLargeCopies = CuForm<128, 1, true, false, CU_SC1_NT>;    // to several
+
 template <int HOW>
 __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 v) {
     if constexpr (HOW == CU_NT)
@@ -116,24 +140,30 @@ __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 
         st128_through<HOW == CU_SC1_NT>(uniform, lane, v);
 }
 
+template <int N>
+struct CuCount {
+    static constexpr int value = N;
+};
+
 // A row cut into vectors of 16 bytes whose stores are aligned: vector i covers
 // the bytes from 16 i - `shift` on.  Vectors that are not wholly inside the row
 // are left out; the bytes they would have brought, fewer than 16 at either end,
 // are moved one element per lane.
+template <typename FORM>
 struct CuRow {
-    uint64_t bytes;
+    // (offsets in a row: the small form's fit into 32 bits)
+    using Bytes = std::conditional_t<FORM::kLarge, uint64_t, uint32_t>;
+    using Offset = std::conditional_t<FORM::kLarge, int64_t, int32_t>;
+    Bytes bytes;
     uint32_t shift;
     __device__ __forceinline__ CuRow(uint64_t row_bytes, uint64_t short_bytes, uint32_t full, uint32_t p,
                                      const uint8_t* stored, uint32_t size) {
-        bytes = p < full ? row_bytes : p == full ? short_bytes : 0u;
+        bytes = p < full ? (Bytes)row_bytes : p == full ? (Bytes)short_bytes : 0u;
         // (whole elements: a row may start at any byte)
         shift = (uint32_t)(uintptr_t)stored & 127u & ~(size - 1u);
     }
-    __device__ __forceinline__ bool whole(int64_t off) const {
-        return off >= 0 && (uint64_t)off + 16u <= bytes;
-    }
     // Element of `size` bytes that this lane (of the first 32) moves, or none.
-    __device__ __forceinline__ bool end_element(uint32_t size, uint64_t& off) const {
+    __device__ __forceinline__ bool end_element(uint32_t size, Bytes& off) const {
         uint32_t head = (0u - shift) & 15u;
         head = bytes < head ? (uint32_t)bytes : head;
         const uint32_t tail = (uint32_t)(bytes - head) & 15u;
@@ -141,6 +171,55 @@ struct CuRow {
         const bool first = threadIdx.x < 16u;
         off = first ? at : bytes - tail + at;
         return threadIdx.x < 32u && at < (first ? head : tail);
+    }
+    // The vectors of a tile: walk(offset of the block's first, how many of them a
+    // lane has), all at once where all are wholly inside the row.
+    template <typename WALK>
+    __device__ __forceinline__ void tile(uint64_t t, const WALK& walk) const {
+        const Offset base = (Offset)((Bytes)t * FORM::kTile) - (Offset)shift;
+        if (__builtin_expect(base >= 0 && (Bytes)base + FORM::kTile <= bytes, 1)) {
+            walk(base, CuCount<FORM::kVectors>{});
+            return;
+        }
+#pragma unroll 1
+        for (Offset off = base; off < base + (Offset)FORM::kTile; off += FORM::kThreads * 16) {
+            const Offset mine = off + (Offset)(threadIdx.x * 16u);
+            if (mine >= 0 && (Bytes)mine + 16u <= bytes) walk(off, CuCount<1>{});
+        }
+    }
+    template <typename WALK>
+    __device__ __forceinline__ void tiles(uint32_t mine, uint32_t all, const WALK& walk) const {
+        if constexpr (FORM::kLarge)
+            for (uint64_t t = mine; t * FORM::kTile < bytes + shift; t += all) tile(t, walk);
+        else
+            tile(mine, walk);
+    }
+};
+
+// Where a block works.  The hardware deals consecutive blocks to the eight XCDs in
+// turn.  Large form: one row after the other, all XCDs next to each other.  Small
+// form: consecutive tiles are one XCD's affair - an eighth of every row (`part` tiles;
+// a row begins on another XCD than the one before it) or, where the pipelines are a
+// multiple of eight, a pipeline.  Against tiles dealt one by one, ranks 2 to 7,
+// geometric means over 24 - 48 MiB / 64 - 96 MiB touched, three sets of buffers in turn:
+// sendrecv 0.90 / 0.94, alltoall 0.94 / 0.96, reduce 0.95 / 0.97, reduce-scatter 0.95 /
+// 0.96, broadcast 0.94 / 0.99, allgather 0.96 / 0.98, allreduce 0.93 / 0.96.  Eight
+// pipelines: an eighth of every row 1.03 (alltoall), 1.00 (reduce-scatter) and 1.02
+// (allgather) of a pipeline to each.
+struct CuPlace {
+    uint32_t tile, pipe;
+    __device__ __forceinline__ CuPlace(bool large, uint32_t part) {
+        const uint32_t x = blockIdx.x, y = blockIdx.y;
+        if (large) {
+            tile = x;
+            pipe = y;
+        } else if (part) {
+            tile = ((x + y + blockIdx.z) & 7u) * part + (x >> 3);
+            pipe = y;
+        } else {
+            tile = y;
+            pipe = x;
+        }
     }
 };
 
@@ -177,12 +256,15 @@ __device__ __forceinline__ void cu_here(P* (&x)[N]) {
 
 // Rings that add: N ranks, the sum goes to the root of the pipeline (reduce,
 // reduce-scatter) or, EVERYWHERE, to all of them (allreduce).
-template <int DT, int N, bool EVERYWHERE, bool LARGE, bool SPLIT, int STORES = cu_stores(LARGE, EVERYWHERE)>
-__global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(CU_SHAPE, const CuTables<N, SPLIT> a) {
-    constexpr uint32_t kSize = DT == DT_F32 ? 4u : 2u, kThreads = cu_threads(LARGE, false), kTile = kThreads * 16u;
-    const uint32_t tile = LARGE ? blockIdx.x : blockIdx.y, p = LARGE ? blockIdx.y : blockIdx.x;
-    const uint32_t root = starts >> (3u * p) & 7u;
-    const uint64_t row_off = (uint64_t)p * row_stride;
+template <int DT, int N, bool EVERYWHERE, typename FORM, bool SPLIT>
+__global__ void __launch_bounds__(FORM::kThreads) cu_ring_sum_kernel(u64x4 numbers, uint64_t counts, const CuTables<N, SPLIT> a) {
+    const CuShape s(numbers, counts);
+    using Row = CuRow<FORM>;
+    constexpr uint32_t kSize = DT == DT_F32 ? 4u : 2u;
+    const CuPlace place(FORM::kLarge, s.part);
+    const uint32_t tile = place.tile, p = place.pipe;
+    const uint32_t root = s.starts >> (3u * p) & 7u;
+    const uint64_t row_off = (uint64_t)p * s.row_stride;
     constexpr int kStored = EVERYWHERE ? N : 1, kOut = SPLIT ? N : 0;
     const uint8_t* from[N];
     uint8_t* to[kStored];
@@ -196,11 +278,11 @@ __global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(C
     for (int i = 0; i < kStored; ++i) to[i] = reinterpret_cast<uint8_t*>(a.rank[kOut + (EVERYWHERE ? (uint32_t)i : root)]);
     cu_here(from);
     cu_here(to);
-    const CuRow row(row_bytes, short_bytes, full, p, to[0] + row_off, kSize);
-    cu_count_if_aborted<kThreads>(a.status);
-    if (__builtin_expect(tile == tiles, 0)) {
-        uint64_t off;
-        if (!row.end_element(kSize, off)) return;
+    const Row row(s.row_bytes, s.short_bytes, s.full, p, to[0] + row_off, kSize);
+    cu_count_if_aborted<FORM::kThreads>(a.status);
+    if (__builtin_expect(tile >= s.tiles, 0)) {
+        typename Row::Bytes off;
+        if (tile > s.tiles || !row.end_element(kSize, off)) return;
         uint32_t v[N];
 #pragma unroll
         for (int h = 0; h < N; ++h) v[h] = cu_load_element<DT>(from[h] + row_off + off);
@@ -212,51 +294,61 @@ __global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_ring_sum_kernel(C
         return;
     }
     const uint32_t lane = threadIdx.x * 16u;
-    for (uint64_t t = tile; t * kTile < row.bytes + row.shift; t += tiles) {
+    row.tiles(tile, s.tiles, [&](typename Row::Offset base, auto count) MINT_INLINE_LAMBDA {
+        constexpr int kCount = decltype(count)::value, kStep = FORM::kThreads * 16;
         // (a uniform part and a lane's: scalar base and 32-bit offset of one instruction)
-        const int64_t base = (int64_t)(t * kTile) - row.shift;
-        if (!row.whole(base + lane)) continue;
-        u32x4 v[N];
+        const int64_t off = (int64_t)row_off + base;
+        u32x4 v[kCount][N];
 #pragma unroll
-        for (int h = 0; h < N; ++h) v[h] = cu_load<LARGE>(from[h] + ((int64_t)row_off + base), lane);
-        u32x4 x = v[0];
+        for (int k = 0; k < kCount; ++k)
 #pragma unroll
-        for (int h = 1; h < N; ++h) x = ll_comp<DT>(v[h], x);
+            for (int h = 0; h < N; ++h) v[k][h] = cu_load<FORM::kStream>(from[h] + off + k * kStep, lane);
 #pragma unroll
-        for (int i = 0; i < kStored; ++i) cu_store<STORES>(to[i] + ((int64_t)row_off + base), lane, x);
-    }
+        for (int k = 0; k < kCount; ++k) {
+            u32x4 x = v[k][0];
+#pragma unroll
+            for (int h = 1; h < N; ++h) x = ll_comp<DT>(v[k][h], x);
+#pragma unroll
+            for (int i = 0; i < kStored; ++i) cu_store<FORM::kStores>(to[i] + off + k * kStep, lane, x);
+        }
+    });
 }
 
 // A row from one place to COPIES others.
-template <int COPIES, bool LARGE>
-__device__ __forceinline__ void cu_copy_row(const CuRow& row, uint32_t tile, uint32_t tiles, const uint8_t* in,
+template <int COPIES, typename FORM>
+__device__ __forceinline__ void cu_copy_row(const CuRow<FORM>& row, uint32_t tile, uint32_t tiles, const uint8_t* in,
                                             uint8_t* const (&out)[COPIES]) {
-    constexpr uint32_t kTile = cu_threads(LARGE, COPIES > 1) * 16u;
-    if (__builtin_expect(tile == tiles, 0)) {
-        uint64_t off;
-        if (!row.end_element(1u, off)) return;
+    using Row = CuRow<FORM>;
+    if (__builtin_expect(tile >= tiles, 0)) {
+        typename Row::Bytes off;
+        if (tile > tiles || !row.end_element(1u, off)) return;
         const uint8_t x = as_global(in)[off];
 #pragma unroll
-        for (int k = 0; k < COPIES; ++k) as_global(out[k])[off] = x;
+        for (int i = 0; i < COPIES; ++i) as_global(out[i])[off] = x;
         return;
     }
     const uint32_t lane = threadIdx.x * 16u;
-    for (uint64_t t = tile; t * kTile < row.bytes + row.shift; t += tiles) {
-        const int64_t base = (int64_t)(t * kTile) - row.shift;
-        if (!row.whole(base + lane)) continue;
-        const u32x4 x = cu_load<LARGE && COPIES == 1>(in + base, lane);
+    row.tiles(tile, tiles, [&](typename Row::Offset base, auto count) MINT_INLINE_LAMBDA {
+        constexpr int kCount = decltype(count)::value, kStep = FORM::kThreads * 16;
+        u32x4 x[kCount];
 #pragma unroll
-        for (int k = 0; k < COPIES; ++k) cu_store<cu_stores(LARGE, (COPIES > 1))>(out[k] + base, lane, x);
-    }
+        for (int k = 0; k < kCount; ++k) x[k] = cu_load<FORM::kStream>(in + base + k * kStep, lane);
+#pragma unroll
+        for (int k = 0; k < kCount; ++k)
+#pragma unroll
+            for (int i = 0; i < COPIES; ++i) cu_store<FORM::kStores>(out[i] + base + k * kStep, lane, x[k]);
+    });
 }
 
 // Rings that copy: N ranks, the root's row to every other one (broadcast,
 // allgather).  A route is a ring of its two ends (sendrecv).
-template <int N, bool LARGE, bool SPLIT>
-__global__ void __launch_bounds__(cu_threads(LARGE, (N > 2))) cu_ring_copy_kernel(CU_SHAPE, const CuTables<N, SPLIT> a) {
-    const uint32_t tile = LARGE ? blockIdx.x : blockIdx.y, p = LARGE ? blockIdx.y : blockIdx.x;
-    const uint32_t root = starts >> (3u * p) & 7u;
-    const uint64_t row_off = (uint64_t)p * row_stride;
+template <int N, typename FORM, bool SPLIT>
+__global__ void __launch_bounds__(FORM::kThreads) cu_ring_copy_kernel(u64x4 numbers, uint64_t counts, const CuTables<N, SPLIT> a) {
+    const CuShape s(numbers, counts);
+    const CuPlace place(FORM::kLarge, s.part);
+    const uint32_t tile = place.tile, p = place.pipe;
+    const uint32_t root = s.starts >> (3u * p) & 7u;
+    const uint64_t row_off = (uint64_t)p * s.row_stride;
     constexpr uint32_t kOut = SPLIT ? N : 0;
     const uint8_t* from[1] = {reinterpret_cast<const uint8_t*>(a.rank[root])};
     uint8_t* to[N - 1];
@@ -268,8 +360,8 @@ __global__ void __launch_bounds__(cu_threads(LARGE, (N > 2))) cu_ring_copy_kerne
     from[0] += row_off;
 #pragma unroll
     for (int k = 0; k < N - 1; ++k) to[k] += row_off;
-    cu_count_if_aborted<cu_threads(LARGE, (N > 2))>(a.status);
-    cu_copy_row<N - 1, LARGE>(CuRow(row_bytes, short_bytes, full, p, to[0], 1u), tile, tiles, from[0], to);
+    cu_count_if_aborted<FORM::kThreads>(a.status);
+    cu_copy_row<N - 1>(CuRow<FORM>(s.row_bytes, s.short_bytes, s.full, p, to[0], 1u), tile, s.tiles, from[0], to);
 }
 
 // The addresses of an alltoall, N to load from and N to store to.  T = uint32_t
@@ -281,24 +373,25 @@ struct CuPairs {
     T rank[2 * kMaxRanks];
 };
 constexpr int kCuNearShift = 8;
-constexpr int cu_near_bytes = 5 * 8 + (int)sizeof(CuPairs<uint32_t>);
-static_assert(cu_near_bytes <= 112, "arguments of an alltoall's launch");
+static_assert(5 * 8 + sizeof(CuPairs<uint32_t>) <= 112, "arguments of an alltoall's launch");
 
 // Row `destination` of the source goes to row `source` of the destination.
-template <bool LARGE, typename T>
-__global__ void __launch_bounds__(cu_threads(LARGE, false)) cu_alltoall_kernel(
-    uint64_t row_bytes, uint64_t row_stride, uint64_t lowest, uint64_t* status, uint32_t tiles, const CuPairs<T> a) {
-    const uint32_t tile = LARGE ? blockIdx.x : blockIdx.y, p = LARGE ? blockIdx.y : blockIdx.x;
+// `numbers`: row_bytes, row_stride, the lowest address, the status block.
+template <typename FORM, typename T>
+__global__ void __launch_bounds__(FORM::kThreads) cu_alltoall_kernel(u64x4 numbers, uint64_t counts, const CuPairs<T> a) {
+    const uint64_t row_bytes = numbers.x, row_stride = numbers.y, lowest = numbers.z;
+    uint64_t* const status = reinterpret_cast<uint64_t*>(numbers.w);
+    const uint32_t tiles = (uint32_t)counts, part = (uint32_t)(counts >> 32);
+    const CuPlace place(FORM::kLarge, part);
+    const uint32_t tile = place.tile, p = place.pipe;
     const uint32_t source = blockIdx.z;
     T load = a.rank[source], store = a.rank[kMaxRanks + p];
     asm volatile("" : "+s"(load), "+s"(store));                 // (see cu_here)
     const auto at = [&](T x) MINT_INLINE_LAMBDA { return sizeof(T) == 4 ? lowest + ((uint64_t)x << kCuNearShift) : (uint64_t)x; };
     const uint8_t* const from = reinterpret_cast<const uint8_t*>(at(load)) + (uint64_t)p * row_stride;
     uint8_t* const to[1] = {reinterpret_cast<uint8_t*>(at(store)) + (uint64_t)source * row_stride};
-    cu_count_if_aborted<cu_threads(LARGE, false)>(status);
-    cu_copy_row<1, LARGE>(CuRow(row_bytes, 0u, kMaxRanks, p, to[0], 1u), tile, tiles, from, to);
+    cu_count_if_aborted<FORM::kThreads>(status);
+    cu_copy_row<1>(CuRow<FORM>(row_bytes, 0u, kMaxRanks, p, to[0], 1u), tile, tiles, from, to);
 }
-
-#undef CU_SHAPE
 
 }  // namespace mint

@@ -100,7 +100,8 @@ int plan_cu(Plan* plan) {
     // line lies where three sets of buffers in turn cross over, 600 MiB (6 ranks) to
     // 740 (8; 640 MiB 110 / 114 us).
     plan->cu_stream = sums && a.op != OP_ALLREDUCE && a.cyc_len >= kCuStreamRanks && touched > (640ull << 20);
-    plan->threads = (int)cu_threads(plan->cu_large, copies);
+    plan->threads = plan->cu_large ? (copies ? CuLargeCopies::kThreads : 64) : CuSmall<true>::kThreads;
+    const uint64_t tile = plan->cu_large ? (copies ? CuLargeCopies::kTile : CuLargeSum::kTile) : CuSmall<true>::kTile;
     // (held to that number by the share of LDS its blocks ask for; LDS is handed
     // out in units of 1280 bytes)
     plan->cu_lds = 0;
@@ -150,14 +151,23 @@ int plan_cu(Plan* plan) {
     }
     stored |= s.row_stride;
     // a row's first tile may start up to 127 bytes before it (CuRow::shift)
-    const uint64_t tile = (uint64_t)plan->threads * 16, slack = stored & 127 ? 127 : 0;
+    const uint64_t slack = stored & 127 ? 127 : 0;
     uint64_t tiles = (a.row_bytes + slack + tile - 1) / tile;
     // (a launch is at most 2^32 - 1 threads; beyond that the blocks take several tiles each)
     const uint64_t most = ((1ull << 31) / plan->threads) / (uint64_t)a.pipes;
     if (tiles > most) tiles = most;
     s.tiles = (uint32_t)tiles;
-    c.ends = ((stored | a.row_bytes | s.short_bytes) & 15) != 0;
-    plan->blocks = (int)(s.tiles + c.ends) * a.pipes;
+    c.blocks = s.tiles + (((stored | a.row_bytes | s.short_bytes) & 15) != 0);
+    // An eighth of every row to each XCD (CuPlace) from 20 MiB touched on: with less, where
+    // a launch is over after one or two rounds of blocks, it takes up to 4 % longer (12 - 16
+    // MiB, geometric mean 1.00), with 24 MiB 5 % less.
+    const int rows = alltoall ? a.cyc_len : a.pipes;
+    s.part = 0;
+    if (!plan->cu_large && rows % kXcds && touched >= (20ull << 20)) {
+        s.part = (c.blocks + kXcds - 1) / kXcds;
+        c.blocks = s.part * kXcds;
+    }
+    plan->blocks = (int)c.blocks * a.pipes;
     plan->lds = false;
     plan->staging_need = 0;
     return MINT_OK;

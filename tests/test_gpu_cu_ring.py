@@ -24,6 +24,15 @@ def make_comm(world, **kw):
     return comm
 
 
+def staged_comm(world):
+    """The same collectives through staging: another path to the same bits."""
+    from mintccl_amd import _lib
+    from mintccl_amd.common import VirtualComm
+    comm = VirtualComm(world_size=world, spin_budget=400000, placement=_lib.PLACE_LOCAL)
+    assert not comm.inside_cu
+    return comm
+
+
 @pytest.mark.parametrize("world,dt", [(8, "f16"), (8, "bf16"), (8, "f32"), (7, "bf16"), (6, "f32"), (5, "f16"),
                                       (4, "bf16"), (3, "f16"), (2, "bf16")])
 def test_reducing_rows(dev, world, dt):
@@ -106,6 +115,69 @@ def test_sums_far_beyond_the_cache(dev, world, dt):
                     x = made[(r + h) % world][row] + x
                 want[row] = x
             assert torch.equal(bufs[r].view(torch.uint8), want.view(torch.uint8)), (op.__name__, r)
+
+
+def added(rows, first):
+    """rows[first] + ... around the ring, one rounding per addition."""
+    x = rows[first]
+    for h in range(1, len(rows)):
+        x = rows[(first + h) % len(rows)] + x
+    return x
+
+
+# MiB touched (bytes of a row times rows times ranks), elements more than that in every row
+@pytest.mark.parametrize("mib,more", [(19, 3), (21, 0), (21, 3), (47, 1021)])
+@pytest.mark.parametrize("world,dt", [(2, "f32"), (3, "f16"), (5, "bf16"), (7, "f16"), (8, "bf16")])
+def test_every_form(dev, world, dt, mib, more):
+    """Sizes on both sides of what a launch's form is chosen by, rows that end in
+    the middle of a vector, a tile and an XCD's part of the tiles."""
+    from mintccl_amd.allgather import allgather
+    from mintccl_amd.allreduce import allreduce
+    from mintccl_amd.alltoall import alltoall
+    from mintccl_amd.broadcast import broadcast
+    from mintccl_amd.reduce import reduce
+    from mintccl_amd.reducescatter import reducescatter
+    dtype = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[dt]
+    comm = make_comm(world)
+    g = torch.Generator(device=dev).manual_seed(100 * world + mib)
+
+    def make(rows, touched):
+        n = (touched << 20) // (rows * world * dtype.itemsize) + more
+        return [torch.randn((rows, n), generator=g, device=dev, dtype=torch.float32).to(dtype) for _ in range(world)]
+
+    def same(got, want, what):
+        comm.check()
+        for r, (x, y) in enumerate(zip(got, want)):
+            assert torch.equal(x.contiguous().view(torch.uint8), y.contiguous().view(torch.uint8)), (what, r)
+
+    made = make(world, mib)
+    bufs = [m.clone() for m in made]
+    comm.run(lambda r: reducescatter(bufs[r], comm))
+    same([b[r] for r, b in enumerate(bufs)], [added([m[r] for m in made], r) for r in range(world)], "reducescatter")
+    for r, (b, m) in enumerate(zip(bufs, made)):
+        keep = [q for q in range(world) if q != r]
+        assert torch.equal(b[keep].view(torch.uint8), m[keep].view(torch.uint8)), ("reducescatter, others' rows", r)
+    bufs = [m.clone() for m in made]
+    comm.run(lambda r: allgather(bufs[r], comm))
+    same(bufs, [torch.stack([made[q][q] for q in range(world)])] * world, "allgather")
+    bufs = [m.clone() for m in made]
+    comm.run(lambda r: allreduce(bufs[r], comm))
+    # (rows of the reduction: the buffer cut into as many as there are ranks, in bytes)
+    flat = [m.view(-1) for m in made]
+    lone = [f.clone() for f in flat]
+    apart = staged_comm(world)
+    apart.run(lambda r: allreduce(lone[r], apart))
+    same([b.view(-1) for b in bufs], lone, "allreduce")
+    made = make(1, mib)
+    bufs = [m.clone() for m in made]
+    comm.run(lambda r: reduce(bufs[r], 1, comm))
+    same(bufs, [added(made, 1) if r == 1 else made[r] for r in range(world)], "reduce")
+    comm.run(lambda r: broadcast(bufs[r], world - 1, comm))
+    same(bufs, [bufs[world - 1]] * world, "broadcast")
+    made = make(world, (mib + 1) // 2 * world // 2)
+    outs = [torch.zeros_like(m) for m in made]
+    comm.run(lambda r: alltoall(made[r], outs[r], comm))
+    same(outs, [torch.stack([made[q][r] for q in range(world)]) for r in range(world)], "alltoall")
 
 
 @pytest.mark.parametrize("shift", [1, 3, 8, 16, 30])
