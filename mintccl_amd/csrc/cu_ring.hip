@@ -31,7 +31,7 @@ int launch_as(const Plan& plan, hipStream_t stream) {
 template <int DT, int N, bool EVERYWHERE>
 int launch_sum(const Plan& plan, hipStream_t stream) {
     if constexpr (N >= kCuStreamRanks && !EVERYWHERE)
-        if (plan.cu_stream)
+        if (plan.cu_far)
             return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, CuLargeSumStreamed, true>, N, true>(plan, stream);
     using Large = std::conditional_t<EVERYWHERE, CuLargeSumEverywhere, CuLargeSum>;
     using Small = CuSmall<EVERYWHERE>;
@@ -42,8 +42,10 @@ int launch_sum(const Plan& plan, hipStream_t stream) {
 }
 template <int N>
 int launch_copy(const Plan& plan, hipStream_t stream) {
-    using Large = std::conditional_t<(N > 2), CuLargeCopies, CuLargeCopy>;
+    using Large = std::conditional_t<(N > 2), CuLargeCopies<N>, CuLargeCopy>;
     using Small = CuSmall<(N > 2)>;
+    if constexpr (N >= kCuVastCopies)
+        if (plan.cu_far) return launch_as<&cu_ring_copy_kernel<N, CuVastCopies, true>, N, true>(plan, stream);
     if (plan.cu_large) return launch_as<&cu_ring_copy_kernel<N, Large, true>, N, true>(plan, stream);
     if (plan.cu_args.split) return launch_as<&cu_ring_copy_kernel<N, Small, true>, N, true>(plan, stream);
     return launch_as<&cu_ring_copy_kernel<N, Small, false>, N, false>(plan, stream);

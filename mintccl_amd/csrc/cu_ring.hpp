@@ -101,15 +101,32 @@ enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
 // The same buffers again and again keep a part of the sums in the cache with sc1:
 // there nt takes 1 - 11 % longer up to 1.5 GiB and is ahead from 2.3 GiB on.
 constexpr int kCuStreamRanks = 6;
+// Rows of six and more ranks to several places (VAST below) from so many MiB touched
+// on.  Over the large form at 0.9 / 1.5 / 3 / 4 GiB touched, three sets of buffers in turn:
+// allgather of 6 ranks 1.01 / 0.98 / 0.95 / 0.94, 7 ranks 0.96 / 0.96 / 0.94 / 0.94, 8 ranks
+// 1.00 / 0.99 / 0.97 / 0.95 (6 and 8 GiB 0.95 / 0.94); 5 ranks 1 - 2 % slower throughout.
+constexpr int kCuVastCopies = 6;
+constexpr int cu_vast_mib(int ranks) { return ranks == 7 ? 700 : ranks == 6 ? 1280 : 2560; }
+
 // Two forms of a launch (which: plan_cu in mintccl.hip).
 //
 // LARGE, rows beyond the last-level cache: one wavefront per block and 1 KiB
-// tiles (with several copies two), the pipelines one after the other, as few
+// tiles that begin at whole KiB, the pipelines one after the other, as few
 // wavefronts on a compute unit as keep HBM busy (cu_waves).  More of them widen
 // the window over which the loads and stores of 8 or 16 rows are scattered: 8
 // ranks, reduce-scatter of 256 MiB 392 us with 32 to a compute unit, 376 with 9;
 // allreduce of 64 MiB 202 with 20, 158 with 4; allgather of 8 x 64 MiB 89 with 32,
-// 67 with 8.
+// 67 with 8.  Rows to several places, over blocks of 128 threads and 2 KiB, three sets
+// of buffers in turn: allgather of 3 / 4 / 5 / 6 / 7 ranks at 0.1 - 2 GiB touched 0.98 /
+// 0.99 / 0.98 / 0.97 / 0.96; eight ranks lose 1 - 5 % by it and keep those.  Tiles at
+// whole KiB rather than lines: ragged rows 1 %.
+//
+// VAST, rows of six and more ranks to several places, far beyond the cache
+// (kCuVastCopies): a wavefront moves 4 KiB, all of it loaded at once and every KiB
+// stored at all places before the next, four or five wavefronts on a compute unit.
+// HBM takes seven streams of rows the better the longer the stretches are that
+// arrive: 8 ranks, allgather of 8 x 128 MiB 1405 -> 1318 us (1473 -> 1331 with rows that
+// are no multiple of a line), 7 ranks and 4 GiB 0.94, 6 ranks 0.96.
 //
 // Otherwise: blocks of 128 threads and 2 KiB, loads through the cache, to each XCD
 // consecutive tiles (CuPlace).  8 ranks, reduce-scatter of 8 MiB 10.9 us, 15.5 in the
@@ -121,6 +138,7 @@ struct CuForm {
     static constexpr int kVectors = VECTORS;       // of 16 bytes a thread moves, THREADS of them apart
     static constexpr uint32_t kTile = THREADS * VECTORS * 16;
     static constexpr bool kLarge = LARGE;
+    static constexpr uint32_t kAlign = LARGE ? 1023 : 127;   // a tile begins at a multiple of kAlign + 1
     static constexpr bool kStream = STREAM;        // rows are loaded past the last-level cache
     static constexpr int kStores = STORES;
 };
@@ -130,7 +148,9 @@ using CuLargeSum = CuForm<64, 1, true, true, CU_SC1>;            // to one place
 using CuLargeSumStreamed = CuForm<64, 1, true, true, CU_NT>;     // (kCuStreamRanks)
 using CuLargeSumEverywhere = CuForm<64, 1, true, true, CU_SC1_NT>;
 using CuLargeCopy = CuForm<64, 1, true, true, CU_SC1>;           // to one place
-using CuLargeCopies = CuForm<128, 1, true, false, CU_SC1_NT>;    // to several
+template <int N>
+using CuLargeCopies = CuForm<N == 8 ? 128 : 64, 1, true, false, CU_SC1_NT>;    // to several
+using CuVastCopies = CuForm<64, 4, true, false, CU_SC1_NT>;
 
 template <int HOW>
 __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 v) {
@@ -160,7 +180,7 @@ struct CuRow {
                                      const uint8_t* stored, uint32_t size) {
         bytes = p < full ? (Bytes)row_bytes : p == full ? (Bytes)short_bytes : 0u;
         // (whole elements: a row may start at any byte)
-        shift = (uint32_t)(uintptr_t)stored & 127u & ~(size - 1u);
+        shift = (uint32_t)(uintptr_t)stored & FORM::kAlign & ~(size - 1u);
     }
     // Element of `size` bytes that this lane (of the first 32) moves, or none.
     __device__ __forceinline__ bool end_element(uint32_t size, Bytes& off) const {

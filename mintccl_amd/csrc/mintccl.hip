@@ -68,18 +68,19 @@ static_assert(MINT_OP_TREE_BROADCAST == OP_TREE_BROADCAST && MINT_OP_TREE_REDUCE
 // and then N results.  Fastest counts on MI355X at 0.5 - 2 GiB, f16 and bf16, for
 // N = 2 / 3 / 4 / 5 / 6 / 7 / 8: reduce-scatter 16 - 18 / 14 / 12 / 10 - 11 / 11 - 12 /
 // 10 / 9, allreduce 14 / 9 / 7 - 8 / 6 - 7 / 5 - 6 / 5 / 4 - 5, allgather - / 18 / 16 /
-// 14 / 12 / 10 / 10 and up; one or two off is 1 - 3 % slower, but twice as many 5 -
-// 20 %.  Rows that are copied from the last-level cache arrive sooner: with 7 and
-// 8 ranks, 8 wavefronts instead of 10 are up to 5 % faster where the same buffers
+// 14 / 12 / 10 / 10 and up (4 KiB each: 5 / 4 / 4 for 6 / 7 / 8); one or two off is 1 - 3 % slower, but
+// twice as many 5 - 20 %.  Rows that are copied from the last-level cache arrive sooner:
+// with 7 and 8 ranks, 8 wavefronts instead of 10 are up to 5 % faster where the same buffers
 // are used again (8 ranks, allgather of 24 MiB in all 27.6 / 29.1 us) and within 1 -
 // 2 % either way on others up to 64 MiB; three sets of buffers in turn, 8 ranks, 8 /
 // 10: 64 MiB 72.7 / 73.0, 72 88.1 / 87.7, 80 97.8 / 97.4, 96 125 / 123, 128 178 / 174,
 // 256 358 / 348.
-int cu_waves(int op, int ranks, uint64_t copied) {
+int cu_waves(int op, int ranks, bool vast, uint64_t copied) {
     if (op == OP_ALLREDUCE) return (26 + ranks - 1) / ranks + 1;
     if (reducing(op)) return (24 + ranks - 1) / ranks + 6;
-    if (ranks >= 7) return copied <= (72ull << 20) ? 8 : 10;
-    return 24 - 2 * ranks;
+    if (vast) return ranks == 6 ? 5 : 4;
+    if (ranks >= 7 && copied <= (72ull << 20)) return 8;
+    return ranks >= 7 ? 10 : 24 - 2 * ranks;
 }
 
 // The grid of a launch inside compute units: a thread block per tile of a row,
@@ -92,21 +93,35 @@ int plan_cu(Plan* plan) {
     // to the next.  Measured with three sets of buffers in turn (8 ranks, small /
     // large, us): allgather 11.5 / 12.0 at 80 MiB, 17.7 / 15.5 at 96; reduce-scatter
     // 17.8 / 19.6 at 96, 28.2 / 25.0 at 128; allreduce 34.9 / 35.3, 52.3 / 46.6; one
-    // copy of a row 19.8 / 20.7 at 128, 45.2 / 41.5 at 256.
+    // copy of a row 20.8 / 22.2 at 140, 24.5 / 25.3 at 160, 29.1 / 27.2 at 175, 45.2 / 41.5 at 256.
     const uint64_t touched = (uint64_t)a.pipes * a.row_bytes *
                              (alltoall || a.op == OP_SENDRECV ? 2u : (uint64_t)a.cyc_len);
-    plan->cu_large = touched > ((uint64_t)(copies ? 88 : sums ? 100 : 192) << 20);
+    // With fewer than 8 ranks the line of the copies lies where the three sets outgrow the
+    // cache (allgather and broadcast of 3 to 7 ranks, large over small: 70 MiB 1.00 - 1.06,
+    // 80 MiB 0.87 - 1.02); with 8 the small form gives a pipeline to each XCD.
+    const uint64_t line = copies ? (a.cyc_len < 8 ? 76 : 88) : sums ? 100 : 168;
+    plan->cu_large = touched > (line << 20);
     // Far beyond it the sums of many ranks are streamed past it (kCuStreamRanks): the
     // line lies where three sets of buffers in turn cross over, 600 MiB (6 ranks) to
-    // 740 (8; 640 MiB 110 / 114 us).
-    plan->cu_stream = sums && a.op != OP_ALLREDUCE && a.cyc_len >= kCuStreamRanks && touched > (640ull << 20);
-    plan->threads = plan->cu_large ? (copies ? CuLargeCopies::kThreads : 64) : CuSmall<true>::kThreads;
-    const uint64_t tile = plan->cu_large ? (copies ? CuLargeCopies::kTile : CuLargeSum::kTile) : CuSmall<true>::kTile;
+    // 740 (8; 640 MiB 110 / 114 us).  Copies of many ranks: kCuVastCopies.
+    plan->cu_far = copies ? a.cyc_len >= kCuVastCopies && touched > (uint64_t)cu_vast_mib(a.cyc_len) << 20
+                          : sums && a.op != OP_ALLREDUCE && a.cyc_len >= kCuStreamRanks && touched > (640ull << 20);
+    // (threads and bytes of a tile)
+    const auto take = [&](auto form, uint64_t* tile) {
+        plan->threads = decltype(form)::kThreads;
+        *tile = decltype(form)::kTile;
+    };
+    uint64_t tile = 0;
+    if (!plan->cu_large) take(CuSmall<true>{}, &tile);
+    else if (!copies) take(CuLargeSum{}, &tile);
+    else if (plan->cu_far) take(CuVastCopies{}, &tile);
+    else if (a.cyc_len == 8) take(CuLargeCopies<8>{}, &tile);
+    else take(CuLargeCopies<3>{}, &tile);
     // (held to that number by the share of LDS its blocks ask for; LDS is handed
     // out in units of 1280 bytes)
     plan->cu_lds = 0;
     if (plan->cu_large && (sums || copies)) {
-        const int blocks = cu_waves(a.op, a.cyc_len, (uint64_t)a.pipes * a.row_bytes) / (plan->threads / 64);
+        const int blocks = cu_waves(a.op, a.cyc_len, plan->cu_far, (uint64_t)a.pipes * a.row_bytes) / (plan->threads / 64);
         if (blocks * (plan->threads / 64) < 32) plan->cu_lds = (160 << 10) / blocks / 1280 * 1280;
     }
     CuRingArgs& c = plan->cu_args;
@@ -150,8 +165,8 @@ int plan_cu(Plan* plan) {
         }
     }
     stored |= s.row_stride;
-    // a row's first tile may start up to 127 bytes before it (CuRow::shift)
-    const uint64_t slack = stored & 127 ? 127 : 0;
+    // a row's first tile may start before it (CuRow::shift)
+    const uint64_t align = plan->cu_large ? CuLargeSum::kAlign : CuSmall<true>::kAlign, slack = stored & align ? align : 0;
     uint64_t tiles = (a.row_bytes + slack + tile - 1) / tile;
     // (a launch is at most 2^32 - 1 threads; beyond that the blocks take several tiles each)
     const uint64_t most = ((1ull << 31) / plan->threads) / (uint64_t)a.pipes;

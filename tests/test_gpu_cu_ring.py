@@ -126,7 +126,7 @@ def added(rows, first):
 
 
 # MiB touched (bytes of a row times rows times ranks), elements more than that in every row
-@pytest.mark.parametrize("mib,more", [(19, 3), (21, 0), (21, 3), (47, 1021)])
+@pytest.mark.parametrize("mib,more", [(19, 3), (21, 0), (21, 3), (47, 1021), (77, 5), (105, 2051)])
 @pytest.mark.parametrize("world,dt", [(2, "f32"), (3, "f16"), (5, "bf16"), (7, "f16"), (8, "bf16")])
 def test_every_form(dev, world, dt, mib, more):
     """Sizes on both sides of what a launch's form is chosen by, rows that end in
@@ -178,6 +178,34 @@ def test_every_form(dev, world, dt, mib, more):
     outs = [torch.zeros_like(m) for m in made]
     comm.run(lambda r: alltoall(made[r], outs[r], comm))
     same(outs, [torch.stack([made[q][r] for q in range(world)]) for r in range(world)], "alltoall")
+
+
+@pytest.mark.parametrize("world", [6, 7, 8])
+def test_copies_far_beyond_the_cache(dev, world):
+    """More than 700 MiB touched, rows that end in the middle of a 4 KiB tile and of
+    a vector; what lies around the rows stays as it was."""
+    from mintccl_amd.allgather import allgather
+    from mintccl_amd.broadcast import broadcast
+    comm = make_comm(world)
+    nbytes = (704 << 20) // (world * world) + 2 * 1024 + 3
+    g = torch.Generator(device=dev).manual_seed(world)
+    rows = [torch.randint(0, 256, (nbytes,), dtype=torch.uint8, generator=g, device=dev) for _ in range(world)]
+    backing = [torch.full((world * nbytes + 64,), 0x5A, dtype=torch.uint8, device=dev) for _ in range(world)]
+    bufs = [b[32: 32 + world * nbytes].view(world, nbytes) for b in backing]
+    for r, b in enumerate(bufs):
+        b[r] = rows[r]
+    comm.run(lambda r: allgather(bufs[r], comm))
+    comm.check()
+    want = torch.stack(rows)
+    for r in range(world):
+        assert torch.equal(bufs[r], want), r
+        assert torch.all(backing[r][:32] == 0x5A) and torch.all(backing[r][32 + world * nbytes:] == 0x5A), r
+    flat = [b[7: 7 + world * nbytes] for b in backing]
+    flat[1].copy_(torch.randint(0, 256, (world * nbytes,), dtype=torch.uint8, generator=g, device=dev))
+    comm.run(lambda r: broadcast(flat[r], 1, comm))
+    comm.check()
+    for r in range(world):
+        assert torch.equal(flat[r], flat[1]), r
 
 
 @pytest.mark.parametrize("shift", [1, 3, 8, 16, 30])
