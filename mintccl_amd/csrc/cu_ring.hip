@@ -33,6 +33,8 @@ int launch_sum(const Plan& plan, hipStream_t stream) {
     if constexpr (N >= kCuStreamRanks && !EVERYWHERE)
         if (plan.cu_far)
             return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, CuLargeSumStreamed, true>, N, true>(plan, stream);
+    if constexpr (N <= kCuMidRanks && !EVERYWHERE)
+        if (plan.cu_mid) return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, CuMidSum<N>, true>, N, true>(plan, stream);
     using Large = std::conditional_t<EVERYWHERE, CuLargeSumEverywhere, CuLargeSum>;
     using Small = CuSmall<EVERYWHERE>;
     if (plan.cu_large) return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Large, true>, N, true>(plan, stream);

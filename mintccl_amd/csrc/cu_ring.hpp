@@ -101,6 +101,17 @@ enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
 // The same buffers again and again keep a part of the sums in the cache with sc1:
 // there nt takes 1 - 11 % longer up to 1.5 GiB and is ahead from 2.3 GiB on.
 constexpr int kCuStreamRanks = 6;
+// Sums to one place of two to six ranks, rows up to cu_mid_mib touched: the places of
+// the small form, rows streamed past the last-level cache, results left in it (the rows
+// of three sets of buffers are beyond it, their results are not).  Over the large form,
+// reduce-scatter and reduce of f16 / of bf16 (f32 as f16), at 110, 128, 150, 180, 220, 270 MiB
+// touched: 2 ranks 0.91 0.91 0.91 0.90 1.01 / 0.90 0.90 0.90 0.90; 3 ranks 0.89 0.89 0.88 0.88 0.90
+// 0.95 / 0.91 0.89 0.88 0.90 0.91 0.93; 4 ranks 0.94 0.93 0.94 0.93 0.95 0.95 / 0.95 0.96 0.98 0.98 0.99
+// 1.02; 5 and 6 ranks (blocks of 64 threads, 14 wavefronts on a compute unit) 0.95 0.94 0.95 1.00
+// 1.00 0.99 / 0.97 0.95 0.97 1.02 1.00 1.01; 7 and 8 ranks 0.92 - 1.10.
+constexpr int kCuMidRanks = 6;
+constexpr int cu_mid_mib(int ranks) { return ranks == 3 ? 264 : ranks == 4 ? 208 : 176; }
+
 // Rows of six and more ranks to several places (VAST below) from so many MiB touched
 // on.  Over the large form at 0.9 / 1.5 / 3 / 4 GiB touched, three sets of buffers in turn:
 // allgather of 6 ranks 1.01 / 0.98 / 0.95 / 0.94, 7 ranks 0.96 / 0.96 / 0.94 / 0.94, 8 ranks
@@ -144,6 +155,8 @@ struct CuForm {
 };
 template <bool SEVERAL>
 using CuSmall = CuForm<128, 1, false, false, SEVERAL ? CU_SC1 : CU_NT>;
+template <int N>
+using CuMidSum = CuForm<N <= 4 ? 128 : 64, 1, false, true, CU_SC1>;   // (kCuMidRanks)
 using CuLargeSum = CuForm<64, 1, true, true, CU_SC1>;            // to one place
 using CuLargeSumStreamed = CuForm<64, 1, true, true, CU_NT>;     // (kCuStreamRanks)
 using CuLargeSumEverywhere = CuForm<64, 1, true, true, CU_SC1_NT>;

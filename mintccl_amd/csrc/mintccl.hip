@@ -99,8 +99,12 @@ int plan_cu(Plan* plan) {
     // With fewer than 8 ranks the line of the copies lies where the three sets outgrow the
     // cache (allgather and broadcast of 3 to 7 ranks, large over small: 70 MiB 1.00 - 1.06,
     // 80 MiB 0.87 - 1.02); with 8 the small form gives a pipeline to each XCD.
-    const uint64_t line = copies ? (a.cyc_len < 8 ? 76 : 88) : sums ? 100 : 168;
-    plan->cu_large = touched > (line << 20);
+    // (sums of two ranks, which take the form between the two, small over that: 85 MiB 1.07,
+    // 96 MiB 1.02)
+    const uint64_t line = copies ? (a.cyc_len < 8 ? 76 : 88) : sums ? (a.cyc_len == 2 && a.op != OP_ALLREDUCE ? 80 : 100) : 168;
+    plan->cu_mid = sums && a.op != OP_ALLREDUCE && a.cyc_len <= kCuMidRanks && touched > (line << 20) &&
+                   touched <= (uint64_t)cu_mid_mib(a.cyc_len) << 20;
+    plan->cu_large = touched > (line << 20) && !plan->cu_mid;
     // Far beyond it the sums of many ranks are streamed past it (kCuStreamRanks): the
     // line lies where three sets of buffers in turn cross over, 600 MiB (6 ranks) to
     // 740 (8; 640 MiB 110 / 114 us).  Copies of many ranks: kCuVastCopies.
@@ -112,16 +116,21 @@ int plan_cu(Plan* plan) {
         *tile = decltype(form)::kTile;
     };
     uint64_t tile = 0;
-    if (!plan->cu_large) take(CuSmall<true>{}, &tile);
-    else if (!copies) take(CuLargeSum{}, &tile);
+    if (plan->cu_mid && a.cyc_len <= 4) take(CuMidSum<4>{}, &tile);
+    else if (plan->cu_mid) take(CuMidSum<5>{}, &tile);
+    else if (!plan->cu_large) take(CuSmall<true>{}, &tile);
+    else if (sums) take(CuLargeSum{}, &tile);
+    else if (!copies) take(CuLargeCopy{}, &tile);
     else if (plan->cu_far) take(CuVastCopies{}, &tile);
     else if (a.cyc_len == 8) take(CuLargeCopies<8>{}, &tile);
     else take(CuLargeCopies<3>{}, &tile);
     // (held to that number by the share of LDS its blocks ask for; LDS is handed
     // out in units of 1280 bytes)
     plan->cu_lds = 0;
-    if (plan->cu_large && (sums || copies)) {
-        const int blocks = cu_waves(a.op, a.cyc_len, plan->cu_far, (uint64_t)a.pipes * a.row_bytes) / (plan->threads / 64);
+    if ((plan->cu_large && (sums || copies)) || plan->cu_mid) {
+        const int waves = plan->cu_mid ? (a.cyc_len <= 4 ? 32 : 14)
+                                       : cu_waves(a.op, a.cyc_len, plan->cu_far, (uint64_t)a.pipes * a.row_bytes);
+        const int blocks = waves / (plan->threads / 64);
         if (blocks * (plan->threads / 64) < 32) plan->cu_lds = (160 << 10) / blocks / 1280 * 1280;
     }
     CuRingArgs& c = plan->cu_args;

@@ -24,6 +24,7 @@ struct Plan {
     bool cu;                  // rings inside compute units: `cu_args` instead of `args`
     CuRingArgs cu_args;
     bool cu_large;            // which form of the kernels
+    bool cu_mid;              // neither: CuMidSum
     bool cu_far;              // far beyond the last-level cache: CuLargeSumStreamed, CuVastCopies
     int cu_lds;               // bytes of LDS per block, to bound how many a compute unit holds
 };

@@ -126,7 +126,7 @@ def added(rows, first):
 
 
 # MiB touched (bytes of a row times rows times ranks), elements more than that in every row
-@pytest.mark.parametrize("mib,more", [(19, 3), (21, 0), (21, 3), (47, 1021), (77, 5), (105, 2051)])
+@pytest.mark.parametrize("mib,more", [(19, 3), (21, 0), (21, 3), (47, 1021), (77, 5), (85, 3), (105, 2051), (170, 9), (270, 1)])
 @pytest.mark.parametrize("world,dt", [(2, "f32"), (3, "f16"), (5, "bf16"), (7, "f16"), (8, "bf16")])
 def test_every_form(dev, world, dt, mib, more):
     """Sizes on both sides of what a launch's form is chosen by, rows that end in
