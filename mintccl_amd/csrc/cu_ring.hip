@@ -23,8 +23,10 @@ int launch_as(const Plan& plan, hipStream_t stream) {
         if (SPLIT) tables.rank[N + i] = a.output[i];
     }
     tables.status = a.status;
+    u64x4 numbers;
+    s.numbers(numbers);
     return Launch<KERNEL>::go(grid_of(plan, a.pipes, 1), (unsigned)plan.threads, (unsigned)plan.cu_lds, stream,
-                              s.numbers(), s.counts(), tables);
+                              numbers, s.counts(), tables);
 }
 
 // (in place only in the small form: to the large one the host's time is nothing)

@@ -38,7 +38,6 @@ namespace mint {
 // hardware put into scalar registers before the first instruction (kernarg preload;
 // not what is inside a struct, hence the vector), and one round of scalar loads brings
 // the addresses.  Few of them, since each argument costs a launch 10 ns.
-typedef uint64_t u64x4 __attribute__((ext_vector_type(4)));
 struct CuShape {
     uint64_t row_bytes, row_stride;
     uint64_t short_bytes;          // bytes of row `full`; rows behind it are empty
@@ -51,7 +50,7 @@ struct CuShape {
     __device__ __forceinline__ CuShape(u64x4 numbers, uint64_t counts)
         : row_bytes(numbers.x), row_stride(numbers.y), short_bytes(numbers.z), starts((uint32_t)numbers.w),
           full((uint32_t)(numbers.w >> 32)), tiles((uint32_t)counts), part((uint32_t)(counts >> 32)) {}
-    u64x4 numbers() const { return u64x4{row_bytes, row_stride, short_bytes, (uint64_t)full << 32 | starts}; }
+    void numbers(u64x4& x) const { x = u64x4{row_bytes, row_stride, short_bytes, (uint64_t)full << 32 | starts}; }
     uint64_t counts() const { return (uint64_t)part << 32 | tiles; }
 };
 

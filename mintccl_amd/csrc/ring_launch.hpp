@@ -50,7 +50,7 @@ template <auto KERNEL>
 struct Launch;
 template <typename... P, void (*KERNEL)(P...)>
 struct Launch<KERNEL> {
-    static int go(dim3 grid, unsigned threads, unsigned lds_bytes, hipStream_t stream, P... args) {
+    static int go(dim3 grid, unsigned threads, unsigned lds_bytes, hipStream_t stream, const P&... args) {
         static std::atomic<hipFunction_t> known[kDevices];
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess) return MINT_ERR_HIP;

@@ -249,3 +249,23 @@ def test_step_mix_saves_what_it_loads_from_staging(dev):
     primitive.step_mix(rows, staging, waves, iters, what=2 | 4 | 16)       # only has to run
     torch.cuda.synchronize()
 
+
+@pytest.mark.parametrize("nbytes", [(4 << 20) - 1, 4 << 20, (4 << 20) + 961, 15 * 960 * 1024 + 7, (60 << 20) - 3, (60 << 20) + 2])
+def test_order_of_the_blocks_changes_nothing(dev, nbytes):
+    """Messages whose blocks are dealt to the XCDs in stretches: every block as it
+    is in a message of its own, nothing behind the last one, every flag found."""
+    from mintccl_amd import protocol
+    g = torch.Generator(device=dev).manual_seed(nbytes)
+    raw = torch.randint(0, 256, (nbytes,), dtype=torch.uint8, generator=g, device=dev)
+    need = protocol.packed_bytes(nbytes)
+    msg = torch.full((need + 1024,), 0x5A, dtype=torch.uint8, device=dev)
+    protocol.pack(raw, flag_base=7, flag_stride=3, out=msg)
+    assert torch.all(msg[need:] == 0x5A)
+    step = 4000 * 960                                         # below 4 MiB: dealt one by one
+    for i, at in enumerate(range(0, nbytes, step)):
+        piece = protocol.pack(raw[at: at + step].clone(), flag_base=7 + 3 * 8 * 4000 * i, flag_stride=3)
+        assert torch.equal(msg[4000 * 1024 * i: 4000 * 1024 * i + piece.numel()], piece), at
+    back = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device=dev)
+    bad = torch.zeros(1, dtype=torch.int64, device=dev)
+    protocol.unpack(msg, back[:nbytes], flag_base=7, flag_stride=3, bad_flags=bad)
+    assert torch.equal(back[:nbytes], raw) and torch.all(back[nbytes:] == 0xA5) and bad.item() == 0
