@@ -26,7 +26,7 @@ int launch_as(const Plan& plan, hipStream_t stream) {
     u64x4 numbers;
     s.numbers(numbers);
     return Launch<KERNEL>::go(grid_of(plan, a.pipes, 1), (unsigned)plan.threads, (unsigned)plan.cu_lds, stream,
-                              numbers, s.counts(), tables);
+                              numbers, u32x2{s.tiles, s.part}, tables);
 }
 
 // (in place only in the small form: to the large one the host's time is nothing)
@@ -87,12 +87,13 @@ int launch_alltoall(const Plan& plan, hipStream_t stream) {
     }
     const dim3 grid = grid_of(plan, a.len, a.len);
     const unsigned threads = (unsigned)plan.threads;
+    const u32x2 counts = {s.tiles, s.part};
     const u64x4 numbers = {s.row_bytes, s.row_stride, lowest, reinterpret_cast<uint64_t>(a.status)};
     if (plan.cu_large)
-        return Launch<&cu_alltoall_kernel<CuLargeCopy, uint64_t>>::go(grid, threads, 0, stream, numbers, s.counts(), far);
+        return Launch<&cu_alltoall_kernel<CuLargeCopy, uint64_t>>::go(grid, threads, 0, stream, numbers, counts, far);
     if (rest)
-        return Launch<&cu_alltoall_kernel<CuSmall<false>, uint64_t>>::go(grid, threads, 0, stream, numbers, s.counts(), far);
-    return Launch<&cu_alltoall_kernel<CuSmall<false>, uint32_t>>::go(grid, threads, 0, stream, numbers, s.counts(), near);
+        return Launch<&cu_alltoall_kernel<CuSmall<false>, uint64_t>>::go(grid, threads, 0, stream, numbers, counts, far);
+    return Launch<&cu_alltoall_kernel<CuSmall<false>, uint32_t>>::go(grid, threads, 0, stream, numbers, counts, near);
 }
 
 }  // namespace

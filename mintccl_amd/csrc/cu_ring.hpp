@@ -47,11 +47,10 @@ struct CuShape {
     uint32_t part;                 // small form: tiles of a row that one XCD takes, or 0 (CuPlace)
 
     CuShape() = default;
-    __device__ __forceinline__ CuShape(u64x4 numbers, uint64_t counts)
+    __device__ __forceinline__ CuShape(u64x4 numbers, u32x2 counts)
         : row_bytes(numbers.x), row_stride(numbers.y), short_bytes(numbers.z), starts((uint32_t)numbers.w),
-          full((uint32_t)(numbers.w >> 32)), tiles((uint32_t)counts), part((uint32_t)(counts >> 32)) {}
+          full((uint32_t)(numbers.w >> 32)), tiles(counts.x), part(counts.y) {}
     void numbers(u64x4& x) const { x = u64x4{row_bytes, row_stride, short_bytes, (uint64_t)full << 32 | starts}; }
-    uint64_t counts() const { return (uint64_t)part << 32 | tiles; }
 };
 
 // The ranks' buffers in the order of the ring.  One address per rank where they
@@ -209,13 +208,15 @@ struct CuRow {
     template <typename WALK>
     __device__ __forceinline__ void tile(uint64_t t, const WALK& walk) const {
         const Offset base = (Offset)((Bytes)t * FORM::kTile) - (Offset)shift;
-        if (__builtin_expect(base >= 0 && (Bytes)base + FORM::kTile <= bytes, 1)) {
-            walk(base, CuCount<FORM::kVectors>{});
-            return;
-        }
+        if constexpr (FORM::kVectors > 1)
+            if (base >= 0 && (Bytes)base + FORM::kTile <= bytes) {
+                walk(base, CuCount<FORM::kVectors>{});
+                return;
+            }
+        // (lane by lane: a compute unit has one scalar unit for all its wavefronts)
 #pragma unroll 1
-        for (Offset off = base; off < base + (Offset)FORM::kTile; off += FORM::kThreads * 16) {
-            const Offset mine = off + (Offset)(threadIdx.x * 16u);
+        for (int i = 0; i < FORM::kVectors; ++i) {
+            const Offset off = base + i * FORM::kThreads * 16, mine = off + (Offset)(threadIdx.x * 16u);
             if (mine >= 0 && (Bytes)mine + 16u <= bytes) walk(off, CuCount<1>{});
         }
     }
@@ -285,11 +286,23 @@ __device__ __forceinline__ void cu_here(P* (&x)[N]) {
 #pragma unroll
     for (int i = 0; i < N; ++i) asm volatile("" : "+s"(x[i]));
 }
+// The addresses of a table from `root` on around the ring (by their bytes' distance from
+// its start, which one scalar load takes as it is).
+template <int N>
+__device__ __forceinline__ void cu_around(const uint64_t* table, uint32_t root, const uint8_t* (&x)[N]) {
+    uint32_t at = root * 8u;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        x[i] = *reinterpret_cast<const uint8_t* const*>(reinterpret_cast<const uint8_t*>(table) + at);
+        at = at == 8u * (N - 1) ? 0u : at + 8u;
+    }
+    cu_here(x);
+}
 
 // Rings that add: N ranks, the sum goes to the root of the pipeline (reduce,
 // reduce-scatter) or, EVERYWHERE, to all of them (allreduce).
 template <int DT, int N, bool EVERYWHERE, typename FORM, bool SPLIT>
-__global__ void __launch_bounds__(FORM::kThreads) cu_ring_sum_kernel(u64x4 numbers, uint64_t counts, const CuTables<N, SPLIT> a) {
+__global__ void __launch_bounds__(FORM::kThreads) cu_ring_sum_kernel(u64x4 numbers, u32x2 counts, const CuTables<N, SPLIT> a) {
     const CuShape s(numbers, counts);
     using Row = CuRow<FORM>;
     constexpr uint32_t kSize = DT == DT_F32 ? 4u : 2u;
@@ -300,16 +313,13 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_ring_sum_kernel(u64x4 numbe
     constexpr int kStored = EVERYWHERE ? N : 1, kOut = SPLIT ? N : 0;
     const uint8_t* from[N];
     uint8_t* to[kStored];
-    uint32_t idx = root;
+    if constexpr (EVERYWHERE || SPLIT) {
 #pragma unroll
-    for (int h = 0; h < N; ++h) {
-        from[h] = reinterpret_cast<const uint8_t*>(a.rank[idx]);
-        idx = idx + 1u == (uint32_t)N ? 0u : idx + 1u;
+        for (int i = 0; i < kStored; ++i) to[i] = reinterpret_cast<uint8_t*>(a.rank[kOut + (EVERYWHERE ? (uint32_t)i : root)]);
+        cu_here(to);
     }
-#pragma unroll
-    for (int i = 0; i < kStored; ++i) to[i] = reinterpret_cast<uint8_t*>(a.rank[kOut + (EVERYWHERE ? (uint32_t)i : root)]);
-    cu_here(from);
-    cu_here(to);
+    cu_around(a.rank, root, from);
+    if constexpr (!EVERYWHERE && !SPLIT) to[0] = const_cast<uint8_t*>(from[0]);
     const Row row(s.row_bytes, s.short_bytes, s.full, p, to[0] + row_off, kSize);
     cu_count_if_aborted<FORM::kThreads>(a.status);
     if (__builtin_expect(tile >= s.tiles, 0)) {
@@ -375,7 +385,7 @@ __device__ __forceinline__ void cu_copy_row(const CuRow<FORM>& row, uint32_t til
 // Rings that copy: N ranks, the root's row to every other one (broadcast,
 // allgather).  A route is a ring of its two ends (sendrecv).
 template <int N, typename FORM, bool SPLIT>
-__global__ void __launch_bounds__(FORM::kThreads) cu_ring_copy_kernel(u64x4 numbers, uint64_t counts, const CuTables<N, SPLIT> a) {
+__global__ void __launch_bounds__(FORM::kThreads) cu_ring_copy_kernel(u64x4 numbers, u32x2 counts, const CuTables<N, SPLIT> a) {
     const CuShape s(numbers, counts);
     const CuPlace place(FORM::kLarge, s.part);
     const uint32_t tile = place.tile, p = place.pipe;
@@ -383,12 +393,14 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_ring_copy_kernel(u64x4 numb
     const uint64_t row_off = (uint64_t)p * s.row_stride;
     constexpr uint32_t kOut = SPLIT ? N : 0;
     const uint8_t* from[1] = {reinterpret_cast<const uint8_t*>(a.rank[root])};
+    uint8_t* all[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) all[k] = reinterpret_cast<uint8_t*>(a.rank[kOut + k]);
+    cu_here(from);
+    cu_here(all);
     uint8_t* to[N - 1];
 #pragma unroll
-    for (int k = 0; k < N - 1; ++k)
-        to[k] = reinterpret_cast<uint8_t*>((uint32_t)k < root ? a.rank[kOut + k] : a.rank[kOut + k + 1]);
-    cu_here(from);
-    cu_here(to);
+    for (int k = 0; k < N - 1; ++k) to[k] = (uint32_t)k < root ? all[k] : all[k + 1];
     from[0] += row_off;
 #pragma unroll
     for (int k = 0; k < N - 1; ++k) to[k] += row_off;
@@ -410,10 +422,10 @@ static_assert(5 * 8 + sizeof(CuPairs<uint32_t>) <= 112, "arguments of an alltoal
 // Row `destination` of the source goes to row `source` of the destination.
 // `numbers`: row_bytes, row_stride, the lowest address, the status block.
 template <typename FORM, typename T>
-__global__ void __launch_bounds__(FORM::kThreads) cu_alltoall_kernel(u64x4 numbers, uint64_t counts, const CuPairs<T> a) {
+__global__ void __launch_bounds__(FORM::kThreads) cu_alltoall_kernel(u64x4 numbers, u32x2 counts, const CuPairs<T> a) {
     const uint64_t row_bytes = numbers.x, row_stride = numbers.y, lowest = numbers.z;
     uint64_t* const status = reinterpret_cast<uint64_t*>(numbers.w);
-    const uint32_t tiles = (uint32_t)counts, part = (uint32_t)(counts >> 32);
+    const uint32_t tiles = counts.x, part = counts.y;
     const CuPlace place(FORM::kLarge, part);
     const uint32_t tile = place.tile, p = place.pipe;
     const uint32_t source = blockIdx.z;
