@@ -38,7 +38,7 @@ int launch_sum(const Plan& plan, hipStream_t stream) {
     if constexpr (N <= kCuMidRanks && !EVERYWHERE)
         if (plan.cu_mid) return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, CuMidSum<N>, true>, N, true>(plan, stream);
     using Large = std::conditional_t<EVERYWHERE, CuLargeSumEverywhere, CuLargeSum>;
-    using Small = CuSmall<EVERYWHERE>;
+    using Small = CuSmallSum<N, EVERYWHERE>;
     if (plan.cu_large) return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Large, true>, N, true>(plan, stream);
     if (plan.cu_args.split)
         return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Small, true>, N, true>(plan, stream);

@@ -153,6 +153,12 @@ struct CuForm {
 };
 template <bool SEVERAL>
 using CuSmall = CuForm<128, 1, false, false, SEVERAL ? CU_SC1 : CU_NT>;
+// (Sums of two and three ranks to one place: reduce and reduce-scatter of all types, CU_SC1
+// over CU_NT, 6 - 12 / 12 - 20 / 20 - 80 MiB touched, three sets of buffers in turn, 2 ranks 0.99 /
+// 0.81 / 0.97, 16 MiB 5.0 -> 3.8 us; 3 ranks 0.99 / 0.91 / 1.00; 4 and 5 ranks 0.99 / 0.93 - 1.01 /
+// 1.00 - 1.02.)
+template <int N, bool EVERYWHERE>
+using CuSmallSum = CuForm<128, 1, false, false, EVERYWHERE || N <= 3 ? CU_SC1 : CU_NT>;
 template <int N>
 using CuMidSum = CuForm<N <= 4 ? 128 : 64, 1, false, true, CU_SC1>;   // (kCuMidRanks)
 using CuLargeSum = CuForm<64, 1, true, true, CU_SC1>;            // to one place
