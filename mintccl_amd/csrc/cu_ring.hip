@@ -38,21 +38,29 @@ int launch_sum(const Plan& plan, hipStream_t stream) {
     if constexpr (N <= kCuMidRanks && !EVERYWHERE)
         if (plan.cu_mid) return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, CuMidSum<N>, true>, N, true>(plan, stream);
     using Large = std::conditional_t<EVERYWHERE, CuLargeSumEverywhere, CuLargeSum>;
-    using Small = CuSmallSum<N, EVERYWHERE>;
     if (plan.cu_large) return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Large, true>, N, true>(plan, stream);
-    if (plan.cu_args.split)
-        return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Small, true>, N, true>(plan, stream);
-    return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Small, false>, N, false>(plan, stream);
+    const auto small = [&](auto form) {
+        using Small = decltype(form);
+        if (plan.cu_args.split)
+            return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Small, true>, N, true>(plan, stream);
+        return launch_as<&cu_ring_sum_kernel<DT, N, EVERYWHERE, Small, false>, N, false>(plan, stream);
+    };
+    if constexpr (EVERYWHERE || N <= kCuThroughRanks) return small(CuSmall<true>{});
+    else return plan.cu_through ? small(CuSmallSum<true>{}) : small(CuSmallSum<false>{});
 }
 template <int N>
 int launch_copy(const Plan& plan, hipStream_t stream) {
     using Large = std::conditional_t<(N > 2), CuLargeCopies<N>, CuLargeCopy>;
-    using Small = CuSmall<(N > 2)>;
     if constexpr (N >= kCuVastCopies)
         if (plan.cu_far) return launch_as<&cu_ring_copy_kernel<N, CuVastCopies, true>, N, true>(plan, stream);
     if (plan.cu_large) return launch_as<&cu_ring_copy_kernel<N, Large, true>, N, true>(plan, stream);
-    if (plan.cu_args.split) return launch_as<&cu_ring_copy_kernel<N, Small, true>, N, true>(plan, stream);
-    return launch_as<&cu_ring_copy_kernel<N, Small, false>, N, false>(plan, stream);
+    const auto small = [&](auto form) {
+        using Small = decltype(form);
+        if (plan.cu_args.split) return launch_as<&cu_ring_copy_kernel<N, Small, true>, N, true>(plan, stream);
+        return launch_as<&cu_ring_copy_kernel<N, Small, false>, N, false>(plan, stream);
+    };
+    if constexpr (N > 2) return small(CuSmall<true>{});
+    else return plan.cu_through ? small(CuSmall<true>{}) : small(CuSmall<false>{});
 }
 
 template <int N>
@@ -91,9 +99,12 @@ int launch_alltoall(const Plan& plan, hipStream_t stream) {
     const u64x4 numbers = {s.row_bytes, s.row_stride, lowest, reinterpret_cast<uint64_t>(a.status)};
     if (plan.cu_large)
         return Launch<&cu_alltoall_kernel<CuLargeCopy, uint64_t>>::go(grid, threads, 0, stream, numbers, counts, far);
-    if (rest)
-        return Launch<&cu_alltoall_kernel<CuSmall<false>, uint64_t>>::go(grid, threads, 0, stream, numbers, counts, far);
-    return Launch<&cu_alltoall_kernel<CuSmall<false>, uint32_t>>::go(grid, threads, 0, stream, numbers, counts, near);
+    const auto small = [&](auto form) {
+        using Small = decltype(form);
+        if (rest) return Launch<&cu_alltoall_kernel<Small, uint64_t>>::go(grid, threads, 0, stream, numbers, counts, far);
+        return Launch<&cu_alltoall_kernel<Small, uint32_t>>::go(grid, threads, 0, stream, numbers, counts, near);
+    };
+    return plan.cu_through ? small(CuSmall<true>{}) : small(CuSmall<false>{});
 }
 
 }  // namespace

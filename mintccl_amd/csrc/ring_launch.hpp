@@ -25,6 +25,7 @@ struct Plan {
     CuRingArgs cu_args;
     bool cu_large;            // which form of the kernels
     bool cu_mid;              // neither: CuMidSum
+    bool cu_through;          // small, what is touched fits into the L2s: cu_through_mib
     bool cu_far;              // far beyond the last-level cache: CuLargeSumStreamed, CuVastCopies
     int cu_lds;               // bytes of LDS per block, to bound how many a compute unit holds
 };
