@@ -88,16 +88,17 @@ __device__ __forceinline__ u32x4 cu_load(const uint8_t* uniform, uint32_t lane) 
 //   large, one:                     reduce-scatter of 64 MiB 86.9 / 88.6 / 82.1 / 88.0
 enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
 // One place, less than the eight L2s hold (cu_through_mib touched): sc1 too; a call is over
-// in 3 - 5 us and would end with a wait for stores on their way past the caches.  sc1
+// in 3 - 6 us and would end with a wait for stores on their way past the caches.  sc1
 // over nt at 6 - 12 / 13 - 20 / 21 - 24 / 25 - 40 MiB touched, three sets of buffers in turn:
 // sendrecv, alltoall and the copies of two ranks 1.00 / 0.98 / 0.95 / 1.00 (19 MiB 4.4 -> 3.9
 // us; larger ones as above); sums of four and more ranks, rows streamed as well, f32 0.99 /
-// 0.96, bf16 0.99 / 0.91 (15 MiB 4.9 -> 4.2 us), from 21 MiB on 0.97 - 1.06.  Sums of two and
-// three ranks, rows through the caches, at every size: 6 - 12 / 12 - 20 / 20 - 80 MiB 2 ranks 0.99 /
-// 0.81 / 0.97, 16 MiB 5.0 -> 3.8 us; 3 ranks 0.99 / 0.91 / 1.00 (4 and 5 ranks so 0.99 / 0.93 -
-// 1.01 / 1.00 - 1.02).
+// 0.96, bf16 0.99 / 0.91 (15 MiB 4.9 -> 4.2 us), at 21 - 32 MiB 4 to 6 ranks 0.98, 7 ranks 0.97
+// (reduce) and 1.00 (reduce-scatter, up to 1.09), 8 ranks 1.01 and 1.05.  Sums of two and
+// three ranks, rows through the caches, at every size: 6 - 12 / 12 - 20 / 20 - 80 MiB 2 ranks
+// 0.99 / 0.81 / 0.97, 16 MiB 5.0 -> 3.8 us; 3 ranks 0.99 / 0.91 / 1.00 (4 and 5 ranks so 0.99 /
+// 0.93 - 1.01 / 1.00 - 1.02).
 constexpr int kCuThroughRanks = 3;
-constexpr int cu_through_mib(bool sums) { return sums ? 20 : 24; }
+constexpr int cu_through_mib(bool sums, int ranks) { return !sums ? 24 : ranks > 6 ? 20 : 32; }
 // Sums to one place that are far larger than the last-level cache (plan_cu): with
 // many rows to read nt is the faster one, on buffers that have not just been used.
 // Four sets of buffers in turn, reduce-scatter and reduce of f16 and bf16, nt over

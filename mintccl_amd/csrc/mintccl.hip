@@ -105,7 +105,7 @@ int plan_cu(Plan* plan) {
     plan->cu_mid = sums && a.op != OP_ALLREDUCE && a.cyc_len <= kCuMidRanks && touched > (line << 20) &&
                    touched <= (uint64_t)cu_mid_mib(a.cyc_len) << 20;
     plan->cu_large = touched > (line << 20) && !plan->cu_mid;
-    plan->cu_through = touched <= (uint64_t)cu_through_mib(sums) << 20;
+    plan->cu_through = touched <= (uint64_t)cu_through_mib(sums, a.cyc_len) << 20;
     // Far beyond it the sums of many ranks are streamed past it (kCuStreamRanks): the
     // line lies where three sets of buffers in turn cross over, 600 MiB (6 ranks) to
     // 740 (8; 640 MiB 110 / 114 us).  Copies of many ranks: kCuVastCopies.
