@@ -44,7 +44,7 @@ PROTO_LL128, PROTO_SIMPLE = 0, 1
 KINDS = ("broadcast", "reduce", "allgather", "reducescatter", "allreduce", "alltoall")
 (KIND_BROADCAST, KIND_REDUCE, KIND_ALLGATHER, KIND_REDUCESCATTER, KIND_ALLREDUCE,
  KIND_ALLTOALL) = range(6)
-SEND, RECV, SYNC = range(6, 9)       # ... and the other calls a front takes
+SEND, RECV, SYNC, PACK, UNPACK = range(6, 11)   # ... and the other calls a front takes
 PLACE_SPREAD, PLACE_LOCAL, PLACE_CU = 0, 1, 2
 FETCH_INLINE, FETCH_LDS = 0, 1
 
@@ -304,8 +304,8 @@ def host():
                                "g.build()'` in the repository root. There is no Python fallback.")
         from . import _host as module
         if (module.DESCRIPTOR_BYTES != ctypes.sizeof(RingOp) or
-                any(getattr(module, k.upper()) != i for i, k in enumerate(
-                    KINDS + ("send", "recv", "sync")))):
+                any(getattr(module, k.upper(), None) != i for i, k in enumerate(
+                    KINDS + ("send", "recv", "sync", "pack", "unpack")))):
             raise RuntimeError(f"{HOST_PATH} was built for another descriptor: rebuild it")
         module.bind(*[ctypes.cast(getattr(L, name), ctypes.c_void_p).value
                       for name in ("mint_ring_launch", "mint_ring_grid_blocks", "mint_ll128_pack",

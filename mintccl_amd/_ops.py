@@ -35,7 +35,9 @@ def front(action: int, go_on=None):
         except ImportError:
             return op
         made = getattr(_host, "Front", None)
-        return op if made is None else functools.update_wrapper(made(op, action, go_on), op)
+        if made is None or action >= getattr(_host, "ACTIONS", 0):      # an older build
+            return op
+        return functools.update_wrapper(made(op, action, go_on), op)
     return wrap
 
 

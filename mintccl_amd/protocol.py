@@ -10,6 +10,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+from ._ops import front
 from .common import VECTORIZED_BYTES, WARP_SIZE
 
 PAYLOAD_WORK_THREAD = 16      # protocol.py:42
@@ -29,12 +30,14 @@ def packed_bytes(nbytes: int, layout: int = LAYOUT_WAVE64) -> int:
     return _lib.lib().mint_ll128_packed_bytes(nbytes, layout)
 
 
+@front(_lib.PACK)
 def pack(raw: torch.Tensor, flag_base: int = 1, layout: int = LAYOUT_WAVE64,
          flag_stride: int = 1, out: torch.Tensor | None = None) -> torch.Tensor:
     """Device tensor (any dtype, contiguous) -> uint8 tensor of LL128 lines."""
     return _lib.host().pack(raw, flag_base, layout, flag_stride, out)
 
 
+@front(_lib.UNPACK)
 def unpack(msg: torch.Tensor, out: torch.Tensor, flag_base: int = 1,
            layout: int = LAYOUT_WAVE64, flag_stride: int = 1,
            bad_flags: torch.Tensor | None = None) -> torch.Tensor:

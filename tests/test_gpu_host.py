@@ -139,6 +139,39 @@ def test_codec_refuses_what_it_cannot_take(dev):
     assert e.value.code == _lib.ERR_ALIGN
 
 
+def test_codec_takes_its_arguments_in_every_form(dev):
+    """Positional, by name, defaults, a name made at run time; what does not fit is
+    the function's own TypeError, before the library is bound as after."""
+    import inspect
+    import pickle
+
+    from mintccl_amd import _lib, protocol
+    raw = torch.arange(2001, dtype=torch.int32, device=dev)
+    bad = torch.zeros(1, dtype=torch.int64, device=dev)
+    wave, pair = _lib.LAYOUT_WAVE64, _lib.LAYOUT_PAIR
+    want = {(base, layout, stride): protocol.pack.__wrapped__(raw, base, layout, stride)
+            for base, layout, stride in ((1, wave, 1), (9, pair, 1), (9, wave, 3), (2**64 - 1, wave, 1))}
+    into = torch.zeros_like(want[1, wave, 1])
+    assert protocol.pack(raw, out=into) is into
+    for msg, kept in ((into, (1, wave, 1)), (protocol.pack(raw), (1, wave, 1)), (protocol.pack(raw=raw), (1, wave, 1)),
+                      (protocol.pack(raw, 9, pair), (9, pair, 1)), (protocol.pack(raw, layout=pair, flag_base=9), (9, pair, 1)),
+                      (protocol.pack(raw, 9, flag_stride=3), (9, wave, 3)), (protocol.pack(raw, **{"flag" + "_base": -1}), (2**64 - 1, wave, 1))):
+        base, layout, stride = kept
+        assert torch.equal(msg, want[kept])
+        for form in (lambda o: protocol.unpack(msg, o, base, layout, stride, bad),
+                     lambda o: protocol.unpack(out=o, msg=msg, flag_stride=stride, bad_flags=bad, flag_base=base, layout=layout)):
+            back = torch.zeros_like(raw)
+            assert form(back) is back and torch.equal(back, raw)
+    assert int(bad) == 0
+    for call in (lambda: protocol.pack(), lambda: protocol.pack(raw, raws=1), lambda: protocol.pack(raw, raw=raw),
+                 lambda: protocol.pack(raw, 1, wave, 1, None, 5), lambda: protocol.unpack(into),
+                 lambda: protocol.pack(raw, "1"), lambda: protocol.unpack(into, raw, bad_flags=3)):
+        with pytest.raises(TypeError):
+            call()
+    assert list(inspect.signature(protocol.unpack).parameters) == ["msg", "out", "flag_base", "layout", "flag_stride", "bad_flags"]
+    assert pickle.loads(pickle.dumps(protocol.pack)) is protocol.pack
+
+
 def test_operators_take_their_arguments_in_every_form(dev, monkeypatch):
     """Positional, by name, the default communicator; what does not fit is the
     operator's own TypeError; MINTCCL_TOPOLOGY still reaches the other modules."""
