@@ -98,10 +98,11 @@ int plan_cu(Plan* plan) {
                              (alltoall || a.op == OP_SENDRECV ? 2u : (uint64_t)a.cyc_len);
     // With fewer than 8 ranks the line of the copies lies where the three sets outgrow the
     // cache (allgather and broadcast of 3 to 7 ranks, large over small: 70 MiB 1.00 - 1.06,
-    // 80 MiB 0.87 - 1.02); with 8 the small form gives a pipeline to each XCD.
+    // 80 MiB 0.87 - 1.02; 73 - 76 MiB, allgather / broadcast of 6 ranks 1.00 / 0.95, 7 ranks 0.97 /
+    // 0.95); with 8 the small form gives a pipeline to each XCD.
     // (sums of two ranks, which take the form between the two, small over that: 85 MiB 1.07,
     // 96 MiB 1.02)
-    const uint64_t line = copies ? (a.cyc_len < 8 ? 76 : 88) : sums ? (a.cyc_len == 2 && a.op != OP_ALLREDUCE ? 80 : 100) : 168;
+    const uint64_t line = copies ? (a.cyc_len < 6 ? 76 : a.cyc_len < 8 ? 73 : 88) : sums ? (a.cyc_len == 2 && a.op != OP_ALLREDUCE ? 80 : 100) : 168;
     plan->cu_mid = sums && a.op != OP_ALLREDUCE && a.cyc_len <= kCuMidRanks && touched > (line << 20) &&
                    touched <= (uint64_t)cu_mid_mib(a.cyc_len) << 20;
     plan->cu_large = touched > (line << 20) && !plan->cu_mid;
