@@ -19,9 +19,10 @@
 // consecutive bytes per row that moves through memory.  Wavefronts that stay
 // resident and stride through the rows drift apart and lose a tenth of the rate.
 // 8 ranks: one ring per resident thread block, hops through LDS / one lane and
-// resident / a block per tile / and the wavefronts held down (cu_threads):
+// resident / a block per tile / and the wavefronts held down (cu_waves):
 // reduce-scatter of 256 MiB f16 447 / 470 / 391 / 375 us, allgather of 8 x 128 MiB
-// 1675 / 1660 / 1540 / 1380, allreduce of 64 MiB bf16 205 / 198 / 190 / 165.
+// 1675 / 1660 / 1540 / 1380 (4 KiB to a wavefront 1318), allreduce of 64 MiB bf16 205 / 198 /
+// 190 / 161.
 #pragma once
 #include <type_traits>
 
@@ -129,7 +130,7 @@ constexpr int cu_mid_mib(int ranks) { return ranks == 3 ? 264 : ranks == 4 ? 208
 constexpr int kCuVastCopies = 6;
 constexpr int cu_vast_mib(int ranks) { return ranks == 7 ? 700 : ranks == 6 ? 1280 : 2560; }
 
-// Two forms of a launch (which: plan_cu in mintccl.hip).
+// The forms of a launch (which: plan_cu in mintccl.hip).
 //
 // LARGE, rows beyond the last-level cache: one wavefront per block and 1 KiB
 // tiles that begin at whole KiB, the pipelines one after the other, as few
