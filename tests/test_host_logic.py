@@ -80,6 +80,44 @@ def test_tuned_geometry_is_always_launchable(op, world, row_blocks):
     assert _lib.lib().mint_ring_grid_blocks(d) * (threads // 64) <= budget
 
 
+@pytest.mark.parametrize("world", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("op", [_lib.OP_SENDRECV, _lib.OP_BROADCAST, _lib.OP_REDUCE, _lib.OP_ALLGATHER,
+                                _lib.OP_REDUCESCATTER, _lib.OP_ALLREDUCE, _lib.OP_ALLTOALL])
+def test_every_tile_of_a_row_has_its_block_inside_compute_units(op, world):
+    """Small rings inside compute units: the grid has a thread block for every 2 KiB
+    tile of a row and one for its ragged ends, and where the XCDs take an eighth of a
+    row each, the blocks of a row are dealt to its tiles one to one."""
+    from tests.test_abi import make_op
+    reducing = op in (_lib.OP_REDUCE, _lib.OP_REDUCESCATTER, _lib.OP_ALLREDUCE)
+    alltoall, one = op == _lib.OP_ALLTOALL, op in (_lib.OP_SENDRECV, _lib.OP_BROADCAST, _lib.OP_REDUCE)
+    pipes, rows = (world * world, world) if alltoall else (1, 1) if one else (world, world)
+    touching = 2 if alltoall or op == _lib.OP_SENDRECV else world
+    for mib in (1, 19, 20, 21, 33, 50, 72):
+        for more in (0, 1, 15, 2047, 2048):
+            row = (mib << 20) // (pipes * touching) // 2048 * 2048 + more * 2
+            d = make_op(op=op, world=world, placement=_lib.PLACE_CU, dtype=_lib.F16 if reducing else _lib.BYTES,
+                        count_bytes=row * (world if op == _lib.OP_ALLREDUCE else 1), row_stride=0 if one or op == _lib.OP_ALLREDUCE else row,
+                        route_len=2 if op == _lib.OP_SENDRECV else 0)
+            for i in range(9):
+                d.ring[i] = i % world if i <= world else 0
+            for r in range(8):
+                d.input[r] = d.output[r] = 0x1000000000 + r * 0x10000000 if r < world else 0
+                if alltoall and r < world:
+                    d.output[r] += 0x800000000
+            blocks = _lib.lib().mint_ring_grid_blocks(d)
+            assert blocks > 0 and blocks % pipes == 0, (mib, more, blocks)
+            blocks //= pipes
+            held = -(-row // 16) * 16 if op == _lib.OP_ALLREDUCE else row       # (cut in whole vectors)
+            slack = 127 if not one and held % 128 else 0
+            assert blocks >= -(-(held + slack) // 2048) + (d.count_bytes % 16 != 0), (mib, more, blocks)
+            touched = pipes * row * touching
+            if rows % 8 and touched >= 20 << 20:
+                assert blocks % 8 == 0
+                for y in range(rows):
+                    for z in range(world if alltoall else 1):
+                        assert sorted(((x + y + z) % 8) * (blocks // 8) + x // 8 for x in range(blocks)) == list(range(blocks))
+
+
 def test_headline_geometry():
     assert common.tuned_geometry(_lib.OP_REDUCESCATTER, 8, 0, 128, 3) == (448 * 1024, 3, 56)
     assert common.tuned_geometry(_lib.OP_ALLREDUCE, 8, 0, 128, 3) == (512 * 1024, 3, 32)
