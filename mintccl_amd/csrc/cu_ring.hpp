@@ -166,8 +166,12 @@ struct CuForm {
 };
 template <bool THROUGH>
 using CuSmall = CuForm<128, 1, false, false, THROUGH ? CU_SC1 : CU_NT>;
+// (of more than kCuThroughRanks.  Those through the L2s by 64 threads, over 128: 4 to 8 ranks,
+// three types, 12 - 16 / 16 - 20 / 20 - 32 MiB touched, reduce 0.99 / 0.96 / 0.985, reduce-scatter
+// 1.00 / 0.98 / 0.985, 20 MiB 5.0 -> 4.8 us; copies, alltoall and sums of two ranks take 1.1 - 1.5
+// of the time at 14 - 20 MiB with twice the blocks)
 template <bool THROUGH>
-using CuSmallSum = CuForm<128, 1, false, THROUGH, THROUGH ? CU_SC1 : CU_NT>;   // of more than kCuThroughRanks
+using CuSmallSum = CuForm<THROUGH ? 64 : 128, 1, false, THROUGH, THROUGH ? CU_SC1 : CU_NT>;
 template <int N>
 using CuMidSum = CuForm<N <= 4 ? 128 : 64, 1, false, true, CU_SC1>;   // (kCuMidRanks)
 using CuLargeSum = CuForm<64, 1, true, true, CU_SC1>;            // to one place

@@ -120,6 +120,8 @@ int plan_cu(Plan* plan) {
     uint64_t tile = 0;
     if (plan->cu_mid && a.cyc_len <= 4) take(CuMidSum<4>{}, &tile);
     else if (plan->cu_mid) take(CuMidSum<5>{}, &tile);
+    else if (!plan->cu_large && plan->cu_through && sums && a.op != OP_ALLREDUCE && a.cyc_len > kCuThroughRanks)
+        take(CuSmallSum<true>{}, &tile);
     else if (!plan->cu_large) take(CuSmall<true>{}, &tile);
     else if (sums) take(CuLargeSum{}, &tile);
     else if (!copies) take(CuLargeCopy{}, &tile);
