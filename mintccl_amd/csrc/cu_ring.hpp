@@ -88,18 +88,21 @@ __device__ __forceinline__ u32x4 cu_load(const uint8_t* uniform, uint32_t lane) 
 //   large, several:                 allgather of 8 x 64 MiB   - / 73.4 / 94.3 / 67.7
 //   large, one:                     reduce-scatter of 64 MiB 86.9 / 88.6 / 82.1 / 88.0
 enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
-// One place, less than the eight L2s hold (cu_through_mib touched): sc1 too; a call is over
+// One place, about what the eight L2s hold (cu_through_mib touched): sc1 too; a call is over
 // in 3 - 6 us and would end with a wait for stores on their way past the caches.  sc1
 // over nt at 6 - 12 / 13 - 20 / 21 - 24 / 25 - 40 MiB touched, three sets of buffers in turn:
 // sendrecv, alltoall and the copies of two ranks 1.00 / 0.98 / 0.95 / 1.00 (19 MiB 4.4 -> 3.9
 // us; larger ones as above); sums of four and more ranks, rows streamed as well, f32 0.99 /
-// 0.96, bf16 0.99 / 0.91 (15 MiB 4.9 -> 4.2 us), at 21 - 32 MiB 4 to 6 ranks 0.98, 7 ranks 0.97
-// (reduce) and 1.00 (reduce-scatter, up to 1.09), 8 ranks 1.01 and 1.05.  Sums of two and
+// 0.96, bf16 0.99 / 0.91 (15 MiB 4.9 -> 4.2 us).  At 20 - 26 / 26 - 32 / 32 - 38 / 38 - 45 / 45 - 65 MiB,
+// three types, in blocks of 64 threads: reduce of 4 to 6 ranks 0.98 / 0.98 / 0.99 / 0.99 / 1.03, 7
+// ranks 0.95 / 0.97 / 0.97 / 1.00 / 1.01, 8 ranks 0.94 / 0.96 / 0.99 / 1.00 / 1.02, reduce-scatter of
+// 4 to 6 ranks 0.98 / 0.98 / 0.99 / 0.99 / 1.02, 7 ranks 0.98 / 0.97 / 0.97 / 1.00 / 1.01, 8 ranks
+// 0.97 / 0.98 / 1.03 (up to 1.18) / 1.02 / 1.05; beyond, as above.  Sums of two and
 // three ranks, rows through the caches, at every size: 6 - 12 / 12 - 20 / 20 - 80 MiB 2 ranks
 // 0.99 / 0.81 / 0.97, 16 MiB 5.0 -> 3.8 us; 3 ranks 0.99 / 0.91 / 1.00 (4 and 5 ranks so 0.99 /
 // 0.93 - 1.01 / 1.00 - 1.02).
 constexpr int kCuThroughRanks = 3;
-constexpr int cu_through_mib(bool sums, int ranks) { return !sums ? 24 : ranks > 6 ? 20 : 32; }
+constexpr int cu_through_mib(bool sums, int ranks) { return !sums ? 24 : ranks == 8 ? 32 : 40; }
 // Sums to one place that are far larger than the last-level cache (plan_cu): with
 // many rows to read nt is the faster one, on buffers that have not just been used.
 // Four sets of buffers in turn, reduce-scatter and reduce of f16 and bf16, nt over
