@@ -185,6 +185,72 @@ template <int N>
 using CuLargeCopies = CuForm<N == 8 ? 128 : 64, 1, true, false, CU_SC1_NT>;    // to several
 using CuVastCopies = CuForm<64, 4, true, false, CU_SC1_NT>;
 
+// What plan_cu decides by the sizes of a launch, and the form that this makes of it: the
+// one place where a form is named, for the grid that plan_cu counts and for the kernel that
+// is launched alike.
+struct CuChoice {
+    bool large, far;          // rows beyond the last-level cache, far beyond it
+    bool mid;                 // neither: CuMidSum
+    bool through;             // small, about what the L2s hold: cu_through_mib
+};
+// (IN_PLACE: ranks that work in place are given by one address each; to a launch beyond the
+// small form the host's time is nothing)
+template <typename FORM, bool IN_PLACE = !FORM::kLarge>
+struct CuFormIs {
+    using type = FORM;
+    static constexpr bool in_place = IN_PLACE;
+};
+// use(CuFormIs<form>{}), sums of N ranks
+template <int N, bool EVERYWHERE, typename USE>
+auto cu_sum_form(const CuChoice& c, const USE& use) {
+    if constexpr (EVERYWHERE) {
+        return c.large ? use(CuFormIs<CuLargeSumEverywhere>{}) : use(CuFormIs<CuSmall<true>>{});
+    } else {
+        if constexpr (N >= kCuStreamRanks)
+            if (c.far) return use(CuFormIs<CuLargeSumStreamed>{});
+        if constexpr (N <= kCuMidRanks)
+            if (c.mid) return use(CuFormIs<CuMidSum<N>, false>{});
+        if (c.large) return use(CuFormIs<CuLargeSum>{});
+        if constexpr (N <= kCuThroughRanks) return use(CuFormIs<CuSmall<true>>{});
+        else return c.through ? use(CuFormIs<CuSmallSum<true>>{}) : use(CuFormIs<CuSmallSum<false>>{});
+    }
+}
+// a row copied to one place (sendrecv, alltoall, two ranks)
+template <typename USE>
+auto cu_move_form(const CuChoice& c, const USE& use) {
+    if (c.large) return use(CuFormIs<CuLargeCopy>{});
+    return c.through ? use(CuFormIs<CuSmall<true>>{}) : use(CuFormIs<CuSmall<false>>{});
+}
+// a row of N ranks copied to the others
+template <int N, typename USE>
+auto cu_copy_form(const CuChoice& c, const USE& use) {
+    if constexpr (N == 2) {
+        return cu_move_form(c, use);
+    } else {
+        if constexpr (N >= kCuVastCopies)
+            if (c.far) return use(CuFormIs<CuVastCopies>{});
+        return c.large ? use(CuFormIs<CuLargeCopies<N>>{}) : use(CuFormIs<CuSmall<true>>{});
+    }
+}
+// use(CuCount<ranks>{}), or MINT_ERR_ARG
+template <int N>
+struct CuCount {
+    static constexpr int value = N;
+};
+template <typename USE>
+int cu_with_ranks(int ranks, const USE& use) {
+    switch (ranks) {
+        case 2: return use(CuCount<2>{});
+        case 3: return use(CuCount<3>{});
+        case 4: return use(CuCount<4>{});
+        case 5: return use(CuCount<5>{});
+        case 6: return use(CuCount<6>{});
+        case 7: return use(CuCount<7>{});
+        case 8: return use(CuCount<8>{});
+        default: return MINT_ERR_ARG;
+    }
+}
+
 template <int HOW>
 __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 v) {
     if constexpr (HOW == CU_NT)
@@ -192,11 +258,6 @@ __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 
     else
         st128_through<HOW == CU_SC1_NT>(uniform, lane, v);
 }
-
-template <int N>
-struct CuCount {
-    static constexpr int value = N;
-};
 
 // A row cut into vectors of 16 bytes whose stores are aligned: vector i covers
 // the bytes from 16 i - `shift` on.  Vectors that are not wholly inside the row

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "kernels.hpp"
@@ -83,70 +84,76 @@ int cu_waves(int op, int ranks, bool vast, uint64_t copied) {
     return ranks >= 7 ? 10 : 24 - 2 * ranks;
 }
 
-// The grid of a launch inside compute units: a thread block per tile of a row,
-// one 16-byte vector per thread.
-int plan_cu(Plan* plan) {
-    const RingArgs& a = plan->args;
-    const bool sums = reducing(a.op), alltoall = a.op == OP_ALLTOALL;
-    const bool copies = (a.op == OP_BROADCAST || a.op == OP_ALLGATHER) && a.cyc_len > 2;
-    // Large: the last-level cache (256 MiB) would not hold the rows from one use
-    // to the next.  Measured with three sets of buffers in turn (8 ranks, small /
-    // large, us): allgather 11.5 / 12.0 at 80 MiB, 17.7 / 15.5 at 96; reduce-scatter
-    // 17.8 / 19.6 at 96, 28.2 / 25.0 at 128; allreduce 34.9 / 35.3, 52.3 / 46.6; one
-    // copy of a row 20.8 / 22.2 at 140, 24.5 / 25.3 at 160, 29.1 / 27.2 at 175, 45.2 / 41.5 at 256.
-    const uint64_t touched = (uint64_t)a.pipes * a.row_bytes *
-                             (alltoall || a.op == OP_SENDRECV ? 2u : (uint64_t)a.cyc_len);
+// MiB touched beyond which the last-level cache (256 MiB) would not hold the rows from one
+// use to the next.  Measured with three sets of buffers in turn (8 ranks, small / large, us):
+// allgather 11.5 / 12.0 at 80 MiB, 17.7 / 15.5 at 96; reduce-scatter 17.8 / 19.6 at 96, 28.2 /
+// 25.0 at 128; allreduce 34.9 / 35.3, 52.3 / 46.6; one copy of a row 20.8 / 22.2 at 140, 24.5 /
+// 25.3 at 160, 29.1 / 27.2 at 175, 45.2 / 41.5 at 256.
+uint64_t cu_large_mib(bool sums, bool everywhere, bool copies, int ranks) {
     // With fewer than 8 ranks the line of the copies lies where the three sets outgrow the
     // cache (allgather and broadcast of 3 to 7 ranks, large over small: 70 MiB 1.00 - 1.06,
     // 80 MiB 0.87 - 1.02; 73 - 76 MiB, allgather / broadcast of 6 ranks 1.00 / 0.95, 7 ranks 0.97 /
     // 0.95); with 8 the small form gives a pipeline to each XCD.
+    if (copies) return ranks < 6 ? 76 : ranks < 8 ? 73 : 88;
+    if (!sums) return 168;
     // (sums of two ranks, which take the form between the two, small over that: 85 MiB 1.07,
     // 96 MiB 1.02)
-    const uint64_t line = copies ? (a.cyc_len < 6 ? 76 : a.cyc_len < 8 ? 73 : 88) : sums ? (a.cyc_len == 2 && a.op != OP_ALLREDUCE ? 80 : 100) : 168;
-    plan->cu_mid = sums && a.op != OP_ALLREDUCE && a.cyc_len <= kCuMidRanks && touched > (line << 20) &&
-                   touched <= (uint64_t)cu_mid_mib(a.cyc_len) << 20;
-    plan->cu_large = touched > (line << 20) && !plan->cu_mid;
-    plan->cu_through = touched <= (uint64_t)cu_through_mib(sums, a.cyc_len) << 20;
+    return ranks == 2 && !everywhere ? 80 : 100;
+}
+
+// The grid of a launch inside compute units: a thread block per tile of a row.
+int plan_cu(Plan* plan) {
+    const RingArgs& a = plan->args;
+    const bool sums = reducing(a.op), alltoall = a.op == OP_ALLTOALL;
+    const bool copies = (a.op == OP_BROADCAST || a.op == OP_ALLGATHER) && a.cyc_len > 2;
+    const uint64_t touched = (uint64_t)a.pipes * a.row_bytes *
+                             (alltoall || a.op == OP_SENDRECV ? 2u : (uint64_t)a.cyc_len);
+    const bool everywhere = a.op == OP_ALLREDUCE;
+    const int ranks = a.op == OP_SENDRECV ? 2 : a.cyc_len;
+    const auto beyond = [&](uint64_t mib) { return touched > mib << 20; };
+    const uint64_t line = cu_large_mib(sums, everywhere, copies, ranks);
+    CuChoice& choice = plan->cu_choice;
+    choice.mid = sums && !everywhere && ranks <= kCuMidRanks && beyond(line) && !beyond(cu_mid_mib(ranks));
+    choice.large = beyond(line) && !choice.mid;
+    choice.through = !beyond(cu_through_mib(sums, ranks));
     // Far beyond it the sums of many ranks are streamed past it (kCuStreamRanks): the
     // line lies where three sets of buffers in turn cross over, 600 MiB (6 ranks) to
     // 740 (8; 640 MiB 110 / 114 us).  Copies of many ranks: kCuVastCopies.
-    plan->cu_far = copies ? a.cyc_len >= kCuVastCopies && touched > (uint64_t)cu_vast_mib(a.cyc_len) << 20
-                          : sums && a.op != OP_ALLREDUCE && a.cyc_len >= kCuStreamRanks && touched > (640ull << 20);
-    // (threads and bytes of a tile)
-    const auto take = [&](auto form, uint64_t* tile) {
-        plan->threads = decltype(form)::kThreads;
-        *tile = decltype(form)::kTile;
+    choice.far = copies ? ranks >= kCuVastCopies && beyond(cu_vast_mib(ranks))
+                        : sums && !everywhere && ranks >= kCuStreamRanks && beyond(640);
+    uint64_t tile = 0, align = 0;
+    const auto take = [&](auto form) {
+        using Form = typename decltype(form)::type;
+        plan->threads = Form::kThreads;
+        tile = Form::kTile;
+        align = Form::kAlign;
+        return MINT_OK;
     };
-    uint64_t tile = 0;
-    if (plan->cu_mid && a.cyc_len <= 4) take(CuMidSum<4>{}, &tile);
-    else if (plan->cu_mid) take(CuMidSum<5>{}, &tile);
-    else if (!plan->cu_large && plan->cu_through && sums && a.op != OP_ALLREDUCE && a.cyc_len > kCuThroughRanks)
-        take(CuSmallSum<true>{}, &tile);
-    else if (!plan->cu_large) take(CuSmall<true>{}, &tile);
-    else if (sums) take(CuLargeSum{}, &tile);
-    else if (!copies) take(CuLargeCopy{}, &tile);
-    else if (plan->cu_far) take(CuVastCopies{}, &tile);
-    else if (a.cyc_len == 8) take(CuLargeCopies<8>{}, &tile);
-    else take(CuLargeCopies<3>{}, &tile);
+    // (a rank alone launches nothing)
+    const int known = alltoall ? cu_move_form(choice, take)
+                               : cu_with_ranks(std::max(ranks, 2), [&](auto n) {
+                                     constexpr int N = decltype(n)::value;
+                                     if (!sums) return cu_copy_form<N>(choice, take);
+                                     return everywhere ? cu_sum_form<N, true>(choice, take) : cu_sum_form<N, false>(choice, take);
+                                 });
+    if (known != MINT_OK) return known;
     // (held to that number by the share of LDS its blocks ask for; LDS is handed
     // out in units of 1280 bytes)
     plan->cu_lds = 0;
-    if ((plan->cu_large && (sums || copies)) || plan->cu_mid) {
-        const int waves = plan->cu_mid ? (a.cyc_len <= 4 ? 32 : 14)
-                                       : cu_waves(a.op, a.cyc_len, plan->cu_far, (uint64_t)a.pipes * a.row_bytes);
+    if ((choice.large && (sums || copies)) || choice.mid) {
+        const int waves = choice.mid ? (ranks <= 4 ? 32 : 14) : cu_waves(a.op, ranks, choice.far, (uint64_t)a.pipes * a.row_bytes);
         const int blocks = waves / (plan->threads / 64);
         if (blocks * (plan->threads / 64) < 32) plan->cu_lds = (160 << 10) / blocks / 1280 * 1280;
     }
     CuRingArgs& c = plan->cu_args;
     c.op = (uint32_t)a.op;
     c.pipes = (uint32_t)a.pipes;
-    c.len = (uint32_t)a.cyc_len;
+    c.len = (uint32_t)ranks;
     c.split = alltoall;
     c.status = a.status;
     uint64_t stored = 0;           // what the stored rows' addresses have in their low bits
     if (a.op == OP_SENDRECV) {
         // a route: only its ends touch the caller's buffers
-        c.len = 2;
         c.input[0] = a.input[a.cyc[0]];
         c.output[0] = c.input[1] = 0;
         stored = c.output[1] = a.output[a.cyc[a.cyc_len - 1]];
@@ -179,7 +186,7 @@ int plan_cu(Plan* plan) {
     }
     stored |= s.row_stride;
     // a row's first tile may start before it (CuRow::shift)
-    const uint64_t align = plan->cu_large ? CuLargeSum::kAlign : CuSmall<true>::kAlign, slack = stored & align ? align : 0;
+    const uint64_t slack = stored & align ? align : 0;
     uint64_t tiles = (a.row_bytes + slack + tile - 1) / tile;
     // (a launch is at most 2^32 - 1 threads; beyond that the blocks take several tiles each)
     const uint64_t most = ((1ull << 31) / plan->threads) / (uint64_t)a.pipes;
@@ -191,7 +198,7 @@ int plan_cu(Plan* plan) {
     // MiB, geometric mean 1.00), with 24 MiB 5 % less.
     const int rows = alltoall ? a.cyc_len : a.pipes;
     s.part = 0;
-    if (!plan->cu_large && rows % kXcds && touched >= (20ull << 20)) {
+    if (!choice.large && rows % kXcds && touched >= (20ull << 20)) {
         s.part = (c.blocks + kXcds - 1) / kXcds;
         c.blocks = s.part * kXcds;
     }

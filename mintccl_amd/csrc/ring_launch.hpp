@@ -23,10 +23,7 @@ struct Plan {
                               // threads only, the launch adds the fetcher wavefront
     bool cu;                  // rings inside compute units: `cu_args` instead of `args`
     CuRingArgs cu_args;
-    bool cu_large;            // which form of the kernels
-    bool cu_mid;              // neither: CuMidSum
-    bool cu_through;          // small, what is touched fits into the L2s: cu_through_mib
-    bool cu_far;              // far beyond the last-level cache: CuLargeSumStreamed, CuVastCopies
+    CuChoice cu_choice;       // ... and the form of their kernels
     int cu_lds;               // bytes of LDS per block, to bound how many a compute unit holds
 };
 
