@@ -88,11 +88,22 @@ __device__ __forceinline__ u32x4 cu_load(const uint8_t* uniform, uint32_t lane) 
 //   large, several:                 allgather of 8 x 64 MiB   - / 73.4 / 94.3 / 67.7
 //   large, one:                     reduce-scatter of 64 MiB 86.9 / 88.6 / 82.1 / 88.0
 enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
-// One place, about what the eight L2s hold (cu_through_mib touched): sc1 too; a call is over
+// A copy to one place in the small form: both (with eight pipelines, a pipeline to each XCD, nt).
+// A choice that holds whatever the caches hold; nt or sc1 alone does not.  Alltoall of 2 to 7
+// ranks, over nt in tiles dealt one by one, the same buffers again / three sets in turn / buffers
+// that 700 MiB lie between two uses of, in tiles dealt by the eighth (CuPlace) from 20 MiB on:
+//   touched MiB       9 - 19                  22 - 25                33 - 60                 85 - 145
+//   nt           1.00  / 0.97 / 1.00    0.85 / 0.93 / 1.03    0.85 / 0.96 / 1.02    0.99 / 0.98 / 1.00
+//   sc1          0.94  / 0.96 / 1.03    0.86 / 0.91 / 1.07    0.81 / 0.96 / 1.05
+//   sc1 nt       0.94  / 0.96 / 0.99    0.88 / 0.93 / 1.01    0.83 / 0.96 / 0.99    0.96 / 0.96 / 0.97
+// sendrecv and the copies of two ranks alike (19 MiB, beyond: sc1 1.08, sc1 nt 0.99; sendrecv of
+// 24 MiB 5.1 -> 4.7 / 5.9 -> 5.4 / 7.4 -> 7.1 us).  Eight ranks and odd rows: sc1 1.00 / 0.98 / 1.16 at
+// 16 - 21 MiB, sc1 nt 1.00 / 1.06 / 1.06 up to 33.
+//
+// A sum to one place, about what the eight L2s hold (cu_through_mib touched): sc1 too; a call is over
 // in 3 - 6 us and would end with a wait for stores on their way past the caches.  sc1
-// over nt at 6 - 12 / 13 - 20 / 21 - 24 / 25 - 40 MiB touched, three sets of buffers in turn:
-// sendrecv, alltoall and the copies of two ranks 1.00 / 0.98 / 0.95 / 1.00 (19 MiB 4.4 -> 3.9
-// us; larger ones as above); sums of four and more ranks, rows streamed as well, f32 0.99 /
+// over nt at 6 - 12 / 13 - 20 MiB touched, three sets of buffers in turn: sums of four and more
+// ranks, rows streamed as well, f32 0.99 /
 // 0.96, bf16 0.99 / 0.91 (15 MiB 4.9 -> 4.2 us).  At 20 - 26 / 26 - 32 / 32 - 38 / 38 - 45 / 45 - 65 MiB,
 // three types, in blocks of 64 threads: reduce of 4 to 6 ranks 0.98 / 0.98 / 0.99 / 0.99 / 1.03, 7
 // ranks 0.95 / 0.97 / 0.97 / 1.00 / 1.01, 8 ranks 0.94 / 0.96 / 0.99 / 1.00 / 1.02, reduce-scatter of
@@ -102,7 +113,7 @@ enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
 // 0.99 / 0.81 / 0.97, 16 MiB 5.0 -> 3.8 us; 3 ranks 0.99 / 0.91 / 1.00 (4 and 5 ranks so 0.99 /
 // 0.93 - 1.01 / 1.00 - 1.02).
 constexpr int kCuThroughRanks = 3;
-constexpr int cu_through_mib(bool sums, int ranks) { return !sums ? 24 : ranks == 8 ? 32 : 40; }
+constexpr int cu_through_mib(int ranks) { return ranks == 8 ? 32 : 40; }
 // Sums to one place that are far larger than the last-level cache (plan_cu): with
 // many rows to read nt is the faster one, on buffers that have not just been used.
 // Four sets of buffers in turn, reduce-scatter and reduce of f16 and bf16, nt over
@@ -167,8 +178,8 @@ struct CuForm {
     static constexpr bool kStream = STREAM;        // rows are loaded past the last-level cache
     static constexpr int kStores = STORES;
 };
-template <bool THROUGH>
-using CuSmall = CuForm<128, 1, false, false, THROUGH ? CU_SC1 : CU_NT>;
+template <int STORES>
+using CuSmall = CuForm<128, 1, false, false, STORES>;
 // (of more than kCuThroughRanks.  Those through the L2s by 64 threads, over 128: 4 to 8 ranks,
 // three types, 12 - 16 / 16 - 20 / 20 - 32 MiB touched, reduce 0.99 / 0.96 / 0.985, reduce-scatter
 // 1.00 / 0.98 / 0.985, 20 MiB 5.0 -> 4.8 us; copies, alltoall and sums of two ranks take 1.1 - 1.5
@@ -191,7 +202,8 @@ using CuVastCopies = CuForm<64, 4, true, false, CU_SC1_NT>;
 struct CuChoice {
     bool large, far;          // rows beyond the last-level cache, far beyond it
     bool mid;                 // neither: CuMidSum
-    bool through;             // small, about what the L2s hold: cu_through_mib
+    bool through;             // small sums, about what the L2s hold: cu_through_mib
+    bool pipe_each;           // small: each XCD takes a pipeline (CuPlace)
 };
 // (IN_PLACE: ranks that work in place are given by one address each; to a launch beyond the
 // small form the host's time is nothing)
@@ -204,14 +216,14 @@ struct CuFormIs {
 template <int N, bool EVERYWHERE, typename USE>
 auto cu_sum_form(const CuChoice& c, const USE& use) {
     if constexpr (EVERYWHERE) {
-        return c.large ? use(CuFormIs<CuLargeSumEverywhere>{}) : use(CuFormIs<CuSmall<true>>{});
+        return c.large ? use(CuFormIs<CuLargeSumEverywhere>{}) : use(CuFormIs<CuSmall<CU_SC1>>{});
     } else {
         if constexpr (N >= kCuStreamRanks)
             if (c.far) return use(CuFormIs<CuLargeSumStreamed>{});
         if constexpr (N <= kCuMidRanks)
             if (c.mid) return use(CuFormIs<CuMidSum<N>, false>{});
         if (c.large) return use(CuFormIs<CuLargeSum>{});
-        if constexpr (N <= kCuThroughRanks) return use(CuFormIs<CuSmall<true>>{});
+        if constexpr (N <= kCuThroughRanks) return use(CuFormIs<CuSmall<CU_SC1>>{});
         else return c.through ? use(CuFormIs<CuSmallSum<true>>{}) : use(CuFormIs<CuSmallSum<false>>{});
     }
 }
@@ -219,7 +231,7 @@ auto cu_sum_form(const CuChoice& c, const USE& use) {
 template <typename USE>
 auto cu_move_form(const CuChoice& c, const USE& use) {
     if (c.large) return use(CuFormIs<CuLargeCopy>{});
-    return c.through ? use(CuFormIs<CuSmall<true>>{}) : use(CuFormIs<CuSmall<false>>{});
+    return c.pipe_each ? use(CuFormIs<CuSmall<CU_NT>>{}) : use(CuFormIs<CuSmall<CU_SC1_NT>>{});
 }
 // a row of N ranks copied to the others
 template <int N, typename USE>
@@ -229,7 +241,7 @@ auto cu_copy_form(const CuChoice& c, const USE& use) {
     } else {
         if constexpr (N >= kCuVastCopies)
             if (c.far) return use(CuFormIs<CuVastCopies>{});
-        return c.large ? use(CuFormIs<CuLargeCopies<N>>{}) : use(CuFormIs<CuSmall<true>>{});
+        return c.large ? use(CuFormIs<CuLargeCopies<N>>{}) : use(CuFormIs<CuSmall<CU_SC1>>{});
     }
 }
 // use(CuCount<ranks>{}), or MINT_ERR_ARG

@@ -115,7 +115,8 @@ int plan_cu(Plan* plan) {
     CuChoice& choice = plan->cu_choice;
     choice.mid = sums && !everywhere && ranks <= kCuMidRanks && beyond(line) && !beyond(cu_mid_mib(ranks));
     choice.large = beyond(line) && !choice.mid;
-    choice.through = !beyond(cu_through_mib(sums, ranks));
+    choice.through = !beyond(cu_through_mib(ranks));
+    choice.pipe_each = (alltoall ? ranks : a.pipes) % kXcds == 0;
     // Far beyond it the sums of many ranks are streamed past it (kCuStreamRanks): the
     // line lies where three sets of buffers in turn cross over, 600 MiB (6 ranks) to
     // 740 (8; 640 MiB 110 / 114 us).  Copies of many ranks: kCuVastCopies.
@@ -196,9 +197,8 @@ int plan_cu(Plan* plan) {
     // An eighth of every row to each XCD (CuPlace) from 20 MiB touched on: with less, where
     // a launch is over after one or two rounds of blocks, it takes up to 4 % longer (12 - 16
     // MiB, geometric mean 1.00), with 24 MiB 5 % less.
-    const int rows = alltoall ? a.cyc_len : a.pipes;
     s.part = 0;
-    if (!choice.large && rows % kXcds && touched >= (20ull << 20)) {
+    if (!choice.large && !choice.pipe_each && touched >= (20ull << 20)) {
         s.part = (c.blocks + kXcds - 1) / kXcds;
         c.blocks = s.part * kXcds;
     }
