@@ -80,30 +80,60 @@ def test_tuned_geometry_is_always_launchable(op, world, row_blocks):
     assert _lib.lib().mint_ring_grid_blocks(d) * (threads // 64) <= budget
 
 
+CU_OPS = [_lib.OP_SENDRECV, _lib.OP_BROADCAST, _lib.OP_REDUCE, _lib.OP_ALLGATHER, _lib.OP_REDUCESCATTER,
+          _lib.OP_ALLREDUCE, _lib.OP_ALLTOALL]
+CU_SUMS = (_lib.OP_REDUCE, _lib.OP_REDUCESCATTER, _lib.OP_ALLREDUCE)
+
+
+def inside_compute_units(op, world, row):
+    """Descriptor of a collective inside compute units, rows of `row` bytes."""
+    from tests.test_abi import make_op
+    alltoall, one = op == _lib.OP_ALLTOALL, op in (_lib.OP_SENDRECV, _lib.OP_BROADCAST, _lib.OP_REDUCE)
+    d = make_op(op=op, world=world, placement=_lib.PLACE_CU, dtype=_lib.F16 if op in CU_SUMS else _lib.BYTES,
+                count_bytes=row * (world if op == _lib.OP_ALLREDUCE else 1),
+                row_stride=0 if one or op == _lib.OP_ALLREDUCE else row, route_len=2 if op == _lib.OP_SENDRECV else 0)
+    for i in range(9):
+        d.ring[i] = i % world if i <= world else 0
+    for r in range(8):
+        d.input[r] = d.output[r] = 0x100000000000 + r * 0x4000000000 if r < world else 0
+        if alltoall and r < world:
+            d.output[r] += 0x200000000000
+    return d
+
+
+def cu_grid(op, world, mib):
+    """Thread blocks per row, and the bytes of a row, of a collective inside compute
+    units whose ranks touch `mib` MiB in all; rows in whole 4 KiB."""
+    pipes = world * world if op == _lib.OP_ALLTOALL else 1 if op in CU_OPS[:3] else world
+    touching = 2 if op in (_lib.OP_ALLTOALL, _lib.OP_SENDRECV) else world
+    row = int(mib * 2**20) // (pipes * touching) // 4096 * 4096
+    blocks = _lib.lib().mint_ring_grid_blocks(inside_compute_units(op, world, row))
+    assert blocks > 0 and blocks % pipes == 0
+    return blocks // pipes, row
+
+
+@pytest.mark.parametrize("op,world", [(_lib.OP_SENDRECV, 2), (_lib.OP_SENDRECV, 8), (_lib.OP_BROADCAST, 2),
+                                      (_lib.OP_ALLGATHER, 2)] + [(_lib.OP_ALLTOALL, w) for w in range(2, 9)])
+def test_a_row_copied_once_moves_in_small_tiles_up_to_192_mib(op, world):
+    """Where the same buffers are used again the large form costs 2 - 12 % there."""
+    for mib, tile in ((150, 2048), (167, 2048), (172, 2048), (190, 2048), (193, 1024), (300, 1024)):
+        blocks, row = cu_grid(op, world, mib)
+        assert 0 <= blocks - -(-row // tile) < 8, (mib, blocks, row)
+
+
 @pytest.mark.parametrize("world", [2, 3, 4, 5, 6, 7, 8])
-@pytest.mark.parametrize("op", [_lib.OP_SENDRECV, _lib.OP_BROADCAST, _lib.OP_REDUCE, _lib.OP_ALLGATHER,
-                                _lib.OP_REDUCESCATTER, _lib.OP_ALLREDUCE, _lib.OP_ALLTOALL])
+@pytest.mark.parametrize("op", CU_OPS)
 def test_every_tile_of_a_row_has_its_block_inside_compute_units(op, world):
     """Small rings inside compute units: the grid has a thread block for every 2 KiB
     tile of a row and one for its ragged ends, and where the XCDs take an eighth of a
     row each, the blocks of a row are dealt to its tiles one to one."""
-    from tests.test_abi import make_op
-    reducing = op in (_lib.OP_REDUCE, _lib.OP_REDUCESCATTER, _lib.OP_ALLREDUCE)
     alltoall, one = op == _lib.OP_ALLTOALL, op in (_lib.OP_SENDRECV, _lib.OP_BROADCAST, _lib.OP_REDUCE)
     pipes, rows = (world * world, world) if alltoall else (1, 1) if one else (world, world)
     touching = 2 if alltoall or op == _lib.OP_SENDRECV else world
     for mib in (1, 19, 20, 21, 33, 50, 72):
         for more in (0, 1, 15, 2047, 2048):
             row = (mib << 20) // (pipes * touching) // 2048 * 2048 + more * 2
-            d = make_op(op=op, world=world, placement=_lib.PLACE_CU, dtype=_lib.F16 if reducing else _lib.BYTES,
-                        count_bytes=row * (world if op == _lib.OP_ALLREDUCE else 1), row_stride=0 if one or op == _lib.OP_ALLREDUCE else row,
-                        route_len=2 if op == _lib.OP_SENDRECV else 0)
-            for i in range(9):
-                d.ring[i] = i % world if i <= world else 0
-            for r in range(8):
-                d.input[r] = d.output[r] = 0x1000000000 + r * 0x10000000 if r < world else 0
-                if alltoall and r < world:
-                    d.output[r] += 0x800000000
+            d = inside_compute_units(op, world, row)
             blocks = _lib.lib().mint_ring_grid_blocks(d)
             assert blocks > 0 and blocks % pipes == 0, (mib, more, blocks)
             blocks //= pipes
