@@ -100,18 +100,14 @@ enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
 // 24 MiB 5.1 -> 4.7 / 5.9 -> 5.4 / 7.4 -> 7.1 us).  Eight ranks and odd rows: sc1 1.00 / 0.98 / 1.16 at
 // 16 - 21 MiB, sc1 nt 1.00 / 1.06 / 1.06 up to 33.
 //
-// A sum to one place, about what the eight L2s hold (cu_through_mib touched): sc1 too; a call is over
-// in 3 - 6 us and would end with a wait for stores on their way past the caches.  sc1
-// over nt at 6 - 12 / 13 - 20 MiB touched, three sets of buffers in turn: sums of four and more
-// ranks, rows streamed as well, f32 0.99 /
-// 0.96, bf16 0.99 / 0.91 (15 MiB 4.9 -> 4.2 us).  At 20 - 26 / 26 - 32 / 32 - 38 / 38 - 45 / 45 - 65 MiB,
-// three types, in blocks of 64 threads: reduce of 4 to 6 ranks 0.98 / 0.98 / 0.99 / 0.99 / 1.03, 7
-// ranks 0.95 / 0.97 / 0.97 / 1.00 / 1.01, 8 ranks 0.94 / 0.96 / 0.99 / 1.00 / 1.02, reduce-scatter of
-// 4 to 6 ranks 0.98 / 0.98 / 0.99 / 0.99 / 1.02, 7 ranks 0.98 / 0.97 / 0.97 / 1.00 / 1.01, 8 ranks
-// 0.97 / 0.98 / 1.03 (up to 1.18) / 1.02 / 1.05; beyond, as above.  Sums of two and
-// three ranks, rows through the caches, at every size: 6 - 12 / 12 - 20 / 20 - 80 MiB 2 ranks
-// 0.99 / 0.81 / 0.97, 16 MiB 5.0 -> 3.8 us; 3 ranks 0.99 / 0.91 / 1.00 (4 and 5 ranks so 0.99 /
-// 0.93 - 1.01 / 1.00 - 1.02).
+// A sum to one place in the small form, two and three ranks: sc1 (over nt at 6 - 12 / 12 - 20 /
+// 20 - 80 MiB touched, three sets in turn, 2 ranks 0.99 / 0.81 / 0.97, 16 MiB 5.0 -> 3.8 us; 3 ranks
+// 0.99 / 0.91 / 1.00).  Four and more: sc1 up to cu_through_mib touched, about what the eight L2s hold
+// (over nt alone 0.97 - 1.02; the kernel that reads the sum next takes 0.5 - 1.5 us less).
+// Not taken for either: rows streamed.  The call alone is then 0.85 - 0.95 of that at 12 - 40 MiB, but
+// streamed rows do not stay in any cache.  A kernel that reads the buffers again next takes 8 - 13 us
+// longer (multiplied in place, four ranks of 22 MiB in all 17 -> 25 us), and the same call on the same
+// buffers again up to 1.3 at 20 - 32 MiB.
 constexpr int kCuThroughRanks = 3;
 constexpr int cu_through_mib(int ranks) { return ranks == 8 ? 32 : 40; }
 // Sums to one place that are far larger than the last-level cache (plan_cu): with
@@ -180,12 +176,6 @@ struct CuForm {
 };
 template <int STORES>
 using CuSmall = CuForm<128, 1, false, false, STORES>;
-// (of more than kCuThroughRanks.  Those through the L2s by 64 threads, over 128: 4 to 8 ranks,
-// three types, 12 - 16 / 16 - 20 / 20 - 32 MiB touched, reduce 0.99 / 0.96 / 0.985, reduce-scatter
-// 1.00 / 0.98 / 0.985, 20 MiB 5.0 -> 4.8 us; copies, alltoall and sums of two ranks take 1.1 - 1.5
-// of the time at 14 - 20 MiB with twice the blocks)
-template <bool THROUGH>
-using CuSmallSum = CuForm<THROUGH ? 64 : 128, 1, false, THROUGH, THROUGH ? CU_SC1 : CU_NT>;
 template <int N>
 using CuMidSum = CuForm<N <= 4 ? 128 : 64, 1, false, true, CU_SC1>;   // (kCuMidRanks)
 using CuLargeSum = CuForm<64, 1, true, true, CU_SC1>;            // to one place
@@ -202,7 +192,7 @@ using CuVastCopies = CuForm<64, 4, true, false, CU_SC1_NT>;
 struct CuChoice {
     bool large, far;          // rows beyond the last-level cache, far beyond it
     bool mid;                 // neither: CuMidSum
-    bool through;             // small sums, about what the L2s hold: cu_through_mib
+    bool through;             // small sums of many ranks: cu_through_mib
     bool pipe_each;           // small: each XCD takes a pipeline (CuPlace)
 };
 // (IN_PLACE: ranks that work in place are given by one address each; to a launch beyond the
@@ -223,8 +213,9 @@ auto cu_sum_form(const CuChoice& c, const USE& use) {
         if constexpr (N <= kCuMidRanks)
             if (c.mid) return use(CuFormIs<CuMidSum<N>, false>{});
         if (c.large) return use(CuFormIs<CuLargeSum>{});
-        if constexpr (N <= kCuThroughRanks) return use(CuFormIs<CuSmall<CU_SC1>>{});
-        else return c.through ? use(CuFormIs<CuSmallSum<true>>{}) : use(CuFormIs<CuSmallSum<false>>{});
+        if constexpr (N > kCuThroughRanks)
+            if (!c.through) return use(CuFormIs<CuSmall<CU_NT>>{});
+        return use(CuFormIs<CuSmall<CU_SC1>>{});
     }
 }
 // a row copied to one place (sendrecv, alltoall, two ranks)

@@ -121,6 +121,16 @@ def test_a_row_copied_once_moves_in_small_tiles_up_to_192_mib(op, world):
         assert 0 <= blocks - -(-row // tile) < 8, (mib, blocks, row)
 
 
+@pytest.mark.parametrize("op", [_lib.OP_REDUCE, _lib.OP_REDUCESCATTER])
+@pytest.mark.parametrize("world", [2, 3, 4, 5, 6, 7, 8])
+def test_small_sums_do_not_stream_their_rows(op, world):
+    """A form that streams its rows moves them in tiles of one wavefront.  Rows of a few MiB
+    would leave the caches that the next kernel finds them in."""
+    for mib in (1, 8, 12, 16, 19, 22, 28, 31, 33, 39, 41, 60, 75):
+        blocks, row = cu_grid(op, world, mib)
+        assert 0 <= blocks - -(-row // 2048) < 8, (mib, blocks, row)
+
+
 @pytest.mark.parametrize("world", [2, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("op", CU_OPS)
 def test_every_tile_of_a_row_has_its_block_inside_compute_units(op, world):
