@@ -88,17 +88,17 @@ __device__ __forceinline__ u32x4 cu_load(const uint8_t* uniform, uint32_t lane) 
 //   large, several:                 allgather of 8 x 64 MiB   - / 73.4 / 94.3 / 67.7
 //   large, one:                     reduce-scatter of 64 MiB 86.9 / 88.6 / 82.1 / 88.0
 enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
-// A copy to one place in the small form: both (with eight pipelines, a pipeline to each XCD, nt).
-// A choice that holds whatever the caches hold; nt or sc1 alone does not.  Alltoall of 2 to 7
-// ranks, over nt in tiles dealt one by one, the same buffers again / three sets in turn / buffers
-// that 700 MiB lie between two uses of, in tiles dealt by the eighth (CuPlace) from 20 MiB on:
-//   touched MiB       9 - 19                  22 - 25                33 - 60                 85 - 145
-//   nt           1.00  / 0.97 / 1.00    0.85 / 0.93 / 1.03    0.85 / 0.96 / 1.02    0.99 / 0.98 / 1.00
-//   sc1          0.94  / 0.96 / 1.03    0.86 / 0.91 / 1.07    0.81 / 0.96 / 1.05
-//   sc1 nt       0.94  / 0.96 / 0.99    0.88 / 0.93 / 1.01    0.83 / 0.96 / 0.99    0.96 / 0.96 / 0.97
-// sendrecv and the copies of two ranks alike (19 MiB, beyond: sc1 1.08, sc1 nt 0.99; sendrecv of
-// 24 MiB 5.1 -> 4.7 / 5.9 -> 5.4 / 7.4 -> 7.1 us).  Eight ranks and odd rows: sc1 1.00 / 0.98 / 1.16 at
-// 16 - 21 MiB, sc1 nt 1.00 / 1.06 / 1.06 up to 33.
+// A copy to one place in the small form, up to 24 MiB touched (cu_through_mib): sc1.  The results stay
+// in the L2s, and the kernel that reads them next takes 6 - 20 us less than behind nt or sc1 nt
+// (multiplied in place, buffers of 3 - 6 MiB 27 -> 7 us and 13 -> 7); alone the call takes 0.94 / 0.96 / 1.03 -
+// 1.07 of nt (the same buffers again / three sets in turn / buffers that 700 MiB lie between two uses of).
+// Beyond: sc1 nt, a choice that holds whatever the caches hold, nt alone does not (with eight pipelines,
+// a pipeline to each XCD, it does: odd rows 1.00 / 1.06 / 1.06 by sc1 nt).  Alltoall of 2 to 7 ranks, over
+// nt in tiles dealt one by one, tiles dealt by the eighth (CuPlace):
+//   touched MiB       25 - 30               30 - 64               65 - 160
+//   nt         0.83 / 0.94 / 1.03    0.81 / 0.94 / 1.02    0.96 / 0.95 / 0.99
+//   sc1 nt     0.86 / 0.94 / 1.00    0.80 / 0.94 / 0.98    0.93 / 0.94 / 0.96
+// sendrecv and the copies of two ranks alike (65 - 160 MiB nt 0.97 / 0.98 / 1.02, sc1 nt 0.97 / 0.97 / 1.00).
 //
 // A sum to one place in the small form, two and three ranks: sc1 (over nt at 6 - 12 / 12 - 20 /
 // 20 - 80 MiB touched, three sets in turn, 2 ranks 0.99 / 0.81 / 0.97, 16 MiB 5.0 -> 3.8 us; 3 ranks
@@ -109,7 +109,7 @@ enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
 // longer (multiplied in place, four ranks of 22 MiB in all 17 -> 25 us), and the same call on the same
 // buffers again up to 1.3 at 20 - 32 MiB.
 constexpr int kCuThroughRanks = 3;
-constexpr int cu_through_mib(int ranks) { return ranks == 8 ? 32 : 40; }
+constexpr int cu_through_mib(bool sums, int ranks) { return !sums ? 24 : ranks == 8 ? 32 : 40; }
 // Sums to one place that are far larger than the last-level cache (plan_cu): with
 // many rows to read nt is the faster one, on buffers that have not just been used.
 // Four sets of buffers in turn, reduce-scatter and reduce of f16 and bf16, nt over
@@ -192,7 +192,7 @@ using CuVastCopies = CuForm<64, 4, true, false, CU_SC1_NT>;
 struct CuChoice {
     bool large, far;          // rows beyond the last-level cache, far beyond it
     bool mid;                 // neither: CuMidSum
-    bool through;             // small sums of many ranks: cu_through_mib
+    bool through;             // small: cu_through_mib
     bool pipe_each;           // small: each XCD takes a pipeline (CuPlace)
 };
 // (IN_PLACE: ranks that work in place are given by one address each; to a launch beyond the
@@ -222,6 +222,7 @@ auto cu_sum_form(const CuChoice& c, const USE& use) {
 template <typename USE>
 auto cu_move_form(const CuChoice& c, const USE& use) {
     if (c.large) return use(CuFormIs<CuLargeCopy>{});
+    if (c.through) return use(CuFormIs<CuSmall<CU_SC1>>{});
     return c.pipe_each ? use(CuFormIs<CuSmall<CU_NT>>{}) : use(CuFormIs<CuSmall<CU_SC1_NT>>{});
 }
 // a row of N ranks copied to the others

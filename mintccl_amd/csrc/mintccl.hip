@@ -117,7 +117,7 @@ int plan_cu(Plan* plan) {
     CuChoice& choice = plan->cu_choice;
     choice.mid = sums && !everywhere && ranks <= kCuMidRanks && beyond(line) && !beyond(cu_mid_mib(ranks));
     choice.large = beyond(line) && !choice.mid;
-    choice.through = !beyond(cu_through_mib(ranks));
+    choice.through = !beyond(cu_through_mib(sums, ranks));
     choice.pipe_each = (alltoall ? ranks : a.pipes) % kXcds == 0;
     // Far beyond it the sums of many ranks are streamed past it (kCuStreamRanks): the
     // line lies where three sets of buffers in turn cross over, 600 MiB (6 ranks) to
