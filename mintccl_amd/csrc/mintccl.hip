@@ -89,11 +89,11 @@ int cu_waves(int op, int ranks, bool vast, uint64_t copied) {
 // allgather 11.5 / 12.0 at 80 MiB, 17.7 / 15.5 at 96; reduce-scatter 17.8 / 19.6 at 96, 28.2 /
 // 25.0 at 128; allreduce 34.9 / 35.3, 52.3 / 46.6; one copy of a row 45.2 / 41.5 at 256.
 uint64_t cu_large_mib(bool sums, bool everywhere, bool copies, int ranks) {
-    // With fewer than 8 ranks the line of the copies lies where the three sets outgrow the
-    // cache (allgather and broadcast of 3 to 7 ranks, large over small: 70 MiB 1.00 - 1.06,
-    // 80 MiB 0.87 - 1.02; 73 - 76 MiB, allgather / broadcast of 6 ranks 1.00 / 0.95, 7 ranks 0.97 /
-    // 0.95); with 8 the small form gives a pipeline to each XCD.
-    if (copies) return ranks < 6 ? 76 : ranks < 8 ? 73 : 88;
+    // (copies to several places, 3 to 7 ranks, large over small at 74 - 87 MiB alone: the same buffers
+    // again 1.06, three sets in turn 0.93, buffers that 700 MiB lie between two uses of 0.84.  But the
+    // results are not in the cache then: with a kernel before the call that reads its inputs and one
+    // behind it that reads its results, 40 us in all, 24 - 33 us more, up to 78)
+    if (copies) return 88;
     // (one copy, large over small at 169 - 190 MiB, the same buffers again / three sets in turn /
     // buffers that 700 MiB lie between two uses of: alltoall of 2 to 8 ranks 1.10 (up to 1.16) / 1.02 /
     // 1.00, sendrecv 1.03 / 1.00 / 0.93, allgather of two ranks 1.05 / 1.00 / 0.93)

@@ -131,6 +131,17 @@ def test_small_sums_do_not_stream_their_rows(op, world):
         assert 0 <= blocks - -(-row // 2048) < 8, (mib, blocks, row)
 
 
+@pytest.mark.parametrize("op", [_lib.OP_BROADCAST, _lib.OP_ALLGATHER])
+@pytest.mark.parametrize("world", [3, 4, 5, 6, 7, 8])
+def test_rows_copied_to_several_places_stay_in_the_cache_up_to_88_mib(op, world):
+    """The large form (tiles of 1 KiB, of eight ranks 2 KiB at whole KiB) stores past the
+    last-level cache; a kernel that reads the results next misses them there."""
+    for mib in (70, 72.5, 73.5, 75.5, 76.5, 80, 87.5, 88.5, 100):
+        blocks, row = cu_grid(op, world, mib)
+        tile = 2048 if mib < 88 or world == 8 else 1024
+        assert 0 <= blocks - -(-row // tile) < 8, (mib, blocks, row)
+
+
 @pytest.mark.parametrize("world", [2, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("op", CU_OPS)
 def test_every_tile_of_a_row_has_its_block_inside_compute_units(op, world):
