@@ -88,7 +88,7 @@ int cu_waves(int op, int ranks, bool vast, uint64_t copied) {
 // use to the next.  Measured with three sets of buffers in turn (8 ranks, small / large, us):
 // allgather 11.5 / 12.0 at 80 MiB, 17.7 / 15.5 at 96; reduce-scatter 17.8 / 19.6 at 96, 28.2 /
 // 25.0 at 128; allreduce 34.9 / 35.3, 52.3 / 46.6; one copy of a row 45.2 / 41.5 at 256.
-uint64_t cu_large_mib(bool sums, bool everywhere, bool copies, int ranks) {
+uint64_t cu_large_mib(bool sums, bool copies) {
     // (copies to several places, 3 to 7 ranks, large over small at 74 - 87 MiB alone: the same buffers
     // again 1.06, three sets in turn 0.93, buffers that 700 MiB lie between two uses of 0.84.  But the
     // results are not in the cache then: with a kernel before the call that reads its inputs and one
@@ -98,9 +98,11 @@ uint64_t cu_large_mib(bool sums, bool everywhere, bool copies, int ranks) {
     // buffers that 700 MiB lie between two uses of: alltoall of 2 to 8 ranks 1.10 (up to 1.16) / 1.02 /
     // 1.00, sendrecv 1.03 / 1.00 / 0.93, allgather of two ranks 1.05 / 1.00 / 0.93)
     if (!sums) return 192;
-    // (sums of two ranks, which take the form between the two, small over that: 85 MiB 1.07,
-    // 96 MiB 1.02)
-    return ranks == 2 && !everywhere ? 80 : 100;
+    // (sums of two ranks, the form between the two over small at 82 - 99 MiB alone: the same buffers
+    // again 0.92, three sets in turn 0.98, buffers that 700 MiB lie between two uses of 0.91.  But its
+    // rows are in no cache then: a kernel that reads them again, on one set of buffers, takes 12 - 25 us
+    // more)
+    return 100;
 }
 
 // The grid of a launch inside compute units: a thread block per tile of a row.
@@ -113,7 +115,7 @@ int plan_cu(Plan* plan) {
     const bool everywhere = a.op == OP_ALLREDUCE;
     const int ranks = a.op == OP_SENDRECV ? 2 : a.cyc_len;
     const auto beyond = [&](uint64_t mib) { return touched > mib << 20; };
-    const uint64_t line = cu_large_mib(sums, everywhere, copies, ranks);
+    const uint64_t line = cu_large_mib(sums, copies);
     CuChoice& choice = plan->cu_choice;
     choice.mid = sums && !everywhere && ranks <= kCuMidRanks && beyond(line) && !beyond(cu_mid_mib(ranks));
     choice.large = beyond(line) && !choice.mid;
