@@ -105,6 +105,16 @@ uint64_t cu_large_mib(bool sums, bool copies) {
     return 100;
 }
 
+// Whether each XCD takes an eighth of every row (CuPlace) in the small form.
+bool cu_by_eighths(uint64_t touched, bool copies) {
+    // With less than 20 MiB touched a launch is over after one or two rounds of blocks and takes up to 4
+    // % longer so (12 - 16 MiB, geometric mean 1.00), with 24 MiB 5 % less. 
+    // Copies to several places up to 73 MiB: beyond, three sets of buffers meet the edge of the
+    // last-level cache (74 - 88 MiB, over tiles dealt one by one, three sets in turn: broadcast 1.01, up to
+    // 1.14; with a kernel around that reads inputs and results 2 us more).
+    return touched >= (20ull << 20) && !(copies && touched > (73ull << 20));
+}
+
 // The grid of a launch inside compute units: a thread block per tile of a row.
 int plan_cu(Plan* plan) {
     const RingArgs& a = plan->args;
@@ -198,11 +208,8 @@ int plan_cu(Plan* plan) {
     if (tiles > most) tiles = most;
     s.tiles = (uint32_t)tiles;
     c.blocks = s.tiles + (((stored | a.row_bytes | s.short_bytes) & 15) != 0);
-    // An eighth of every row to each XCD (CuPlace) from 20 MiB touched on: with less, where
-    // a launch is over after one or two rounds of blocks, it takes up to 4 % longer (12 - 16
-    // MiB, geometric mean 1.00), with 24 MiB 5 % less.
     s.part = 0;
-    if (!choice.large && !choice.pipe_each && touched >= (20ull << 20)) {
+    if (!choice.large && !choice.pipe_each && cu_by_eighths(touched, copies)) {
         s.part = (c.blocks + kXcds - 1) / kXcds;
         c.blocks = s.part * kXcds;
     }

@@ -142,6 +142,21 @@ def test_rows_copied_to_several_places_stay_in_the_cache_up_to_88_mib(op, world)
         assert 0 <= blocks - -(-row // tile) < 8, (mib, blocks, row)
 
 
+@pytest.mark.parametrize("op,world,least,most", [
+    (_lib.OP_REDUCE, 5, 20, 100), (_lib.OP_BROADCAST, 3, 20, 73), (_lib.OP_BROADCAST, 8, 20, 73),
+    (_lib.OP_ALLGATHER, 4, 20, 73), (_lib.OP_ALLGATHER, 8, 99, 0), (_lib.OP_SENDRECV, 2, 20, 192)])
+def test_where_an_xcd_takes_an_eighth_of_every_row(op, world, least, most):
+    """Then a row has a multiple of eight thread blocks, else one per tile."""
+    for mib in (11, 13, 17, 19, 21, 30, 45, 59, 71, 72.9, 73.1, 80, 87):
+        row = int(mib * 2**20) // (2 if op == _lib.OP_SENDRECV else world) // (world if op == _lib.OP_ALLGATHER else 1)
+        row = row // 16384 * 16384 + 2048 * 3                     # tiles: 3 more than a multiple of 8
+        blocks = _lib.lib().mint_ring_grid_blocks(inside_compute_units(op, world, row))
+        tiles = row // 2048 * (world if op == _lib.OP_ALLGATHER else 1)
+        if op == _lib.OP_ALLGATHER:
+            blocks, tiles = blocks // world, tiles // world
+        assert blocks == (tiles + 5 if least <= mib <= most else tiles), (mib, blocks, tiles)
+
+
 @pytest.mark.parametrize("world", [2, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("op", CU_OPS)
 def test_every_tile_of_a_row_has_its_block_inside_compute_units(op, world):
