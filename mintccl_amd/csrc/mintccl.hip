@@ -106,13 +106,17 @@ uint64_t cu_large_mib(bool sums, bool copies) {
 }
 
 // Whether each XCD takes an eighth of every row (CuPlace) in the small form.
-bool cu_by_eighths(uint64_t touched, bool copies) {
+bool cu_by_eighths(uint64_t touched, int ranks, int pipes, bool sums, bool copies) {
     // With less than 20 MiB touched a launch is over after one or two rounds of blocks and takes up to 4
-    // % longer so (12 - 16 MiB, geometric mean 1.00), with 24 MiB 5 % less. 
+    // % longer so (12 - 16 MiB, geometric mean 1.00), with 24 MiB 5 % less.  A reduce of two ranks from 12
+    // MiB on: 13 - 18 MiB, dealt one by one / by the eighth, over nt stores and dealt one by one: the same
+    // buffers again 0.92 / 0.89, three sets in turn 0.82 / 0.77, buffers that 700 MiB lie between two uses
+    // of 1.08 (up to 1.15) / 1.00.
+    const uint64_t least = sums && ranks == 2 && pipes == 1 ? 12 : 20;
     // Copies to several places up to 73 MiB: beyond, three sets of buffers meet the edge of the
     // last-level cache (74 - 88 MiB, over tiles dealt one by one, three sets in turn: broadcast 1.01, up to
     // 1.14; with a kernel around that reads inputs and results 2 us more).
-    return touched >= (20ull << 20) && !(copies && touched > (73ull << 20));
+    return touched >= least << 20 && !(copies && touched > (73ull << 20));
 }
 
 // The grid of a launch inside compute units: a thread block per tile of a row.
@@ -209,7 +213,7 @@ int plan_cu(Plan* plan) {
     s.tiles = (uint32_t)tiles;
     c.blocks = s.tiles + (((stored | a.row_bytes | s.short_bytes) & 15) != 0);
     s.part = 0;
-    if (!choice.large && !choice.pipe_each && cu_by_eighths(touched, copies)) {
+    if (!choice.large && !choice.pipe_each && cu_by_eighths(touched, ranks, a.pipes, sums, copies)) {
         s.part = (c.blocks + kXcds - 1) / kXcds;
         c.blocks = s.part * kXcds;
     }

@@ -143,7 +143,7 @@ def test_rows_copied_to_several_places_stay_in_the_cache_up_to_88_mib(op, world)
 
 
 @pytest.mark.parametrize("op,world,least,most", [
-    (_lib.OP_REDUCE, 5, 20, 100), (_lib.OP_BROADCAST, 3, 20, 73), (_lib.OP_BROADCAST, 8, 20, 73),
+    (_lib.OP_REDUCE, 2, 12, 100), (_lib.OP_REDUCE, 5, 20, 100), (_lib.OP_BROADCAST, 3, 20, 73), (_lib.OP_BROADCAST, 8, 20, 73),
     (_lib.OP_ALLGATHER, 4, 20, 73), (_lib.OP_ALLGATHER, 8, 99, 0), (_lib.OP_SENDRECV, 2, 20, 192)])
 def test_where_an_xcd_takes_an_eighth_of_every_row(op, world, least, most):
     """Then a row has a multiple of eight thread blocks, else one per tile."""
