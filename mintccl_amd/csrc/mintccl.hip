@@ -133,8 +133,12 @@ int plan_cu(Plan* plan) {
     CuChoice& choice = plan->cu_choice;
     choice.mid = sums && !everywhere && ranks <= kCuMidRanks && beyond(line) && !beyond(cu_mid_mib(ranks));
     choice.large = beyond(line) && !choice.mid;
-    choice.through = !beyond(cu_through_mib(sums, ranks));
     choice.pipe_each = (alltoall ? ranks : a.pipes) % kXcds == 0;
+    // (a pipeline to each XCD leaves a whole row of results in one XCD's L2: short ones, which few blocks
+    // read next, are sooner there from the last-level cache.  Eight ranks, multiplied in place behind the
+    // call, sc1 / nt: reduce-scatter of 4 MiB 4 us more, 8 MiB 9, 10 MiB 0; alltoall of 2 MiB 4 more, 2.5 MiB
+    // 6 less)
+    choice.through = !beyond(cu_through_mib(sums, ranks)) && !(choice.pipe_each && !beyond(sums ? 9 : 2));
     // Far beyond it the sums of many ranks are streamed past it (kCuStreamRanks): the
     // line lies where three sets of buffers in turn cross over, 600 MiB (6 ranks) to
     // 740 (8; 640 MiB 110 / 114 us).  Copies of many ranks: kCuVastCopies.
