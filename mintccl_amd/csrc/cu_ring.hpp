@@ -326,6 +326,24 @@ struct CuRow {
 // 0.96, broadcast 0.94 / 0.99, allgather 0.96 / 0.98, allreduce 0.93 / 0.96.  Eight
 // pipelines: an eighth of every row 1.03 (alltoall), 1.00 (reduce-scatter) and 1.02
 // (allgather) of a pipeline to each.
+//
+// The tile of block x of a row whose first tiles are XCD `turn`'s (mod 8), `part` tiles to each XCD:
+__host__ __device__ constexpr uint32_t dealt_tile(uint32_t x, uint32_t turn, uint32_t part) {
+    return ((x + turn) & 7u) * part + (x >> 3);
+}
+// (8 part blocks have as many tiles, each once)
+constexpr bool dealt_once(uint32_t part) {
+    for (uint32_t turn = 0; turn < 2 * 8; ++turn) {
+        bool taken[64] = {};
+        for (uint32_t x = 0; x < 8 * part; ++x) {
+            const uint32_t tile = dealt_tile(x, turn, part);
+            if (tile >= 8 * part || taken[tile]) return false;
+            taken[tile] = true;
+        }
+    }
+    return true;
+}
+static_assert(dealt_once(1) && dealt_once(2) && dealt_once(3) && dealt_once(5) && dealt_once(8), "one block per tile");
 struct CuPlace {
     uint32_t tile, pipe;
     __device__ __forceinline__ CuPlace(bool large, uint32_t part) {
@@ -334,7 +352,7 @@ struct CuPlace {
             tile = x;
             pipe = y;
         } else if (part) {
-            tile = ((x + y + blockIdx.z) & 7u) * part + (x >> 3);
+            tile = dealt_tile(x, y + blockIdx.z, part);
             pipe = y;
         } else {
             tile = y;

@@ -157,31 +157,52 @@ def test_where_an_xcd_takes_an_eighth_of_every_row(op, world, least, most):
         assert blocks == (tiles + 5 if least <= mib <= most else tiles), (mib, blocks, tiles)
 
 
+def cu_tile(op, world, touched):
+    """Bytes of a tile inside compute units, and of what it begins at whole ones."""
+    mib = touched / 2**20
+    if op in CU_SUMS:
+        if mib <= 100:
+            return 2048, 128
+        if op != _lib.OP_ALLREDUCE and mib <= {2: 176, 3: 264, 4: 208, 5: 176, 6: 176}.get(world, 0):
+            return (2048 if world <= 4 else 1024), 128
+        return 1024, 1024
+    if op in (_lib.OP_SENDRECV, _lib.OP_ALLTOALL) or world == 2:
+        return (2048, 128) if mib <= 192 else (1024, 1024)
+    if mib <= 88:
+        return 2048, 128
+    if mib > {6: 1280, 7: 700, 8: 2560}.get(world, 1 << 30):
+        return 4096, 1024
+    return (2048 if world == 8 else 1024), 1024
+
+
 @pytest.mark.parametrize("world", [2, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("op", CU_OPS)
 def test_every_tile_of_a_row_has_its_block_inside_compute_units(op, world):
-    """Small rings inside compute units: the grid has a thread block for every 2 KiB
-    tile of a row and one for its ragged ends, and where the XCDs take an eighth of a
-    row each, the blocks of a row are dealt to its tiles one to one."""
-    alltoall, one = op == _lib.OP_ALLTOALL, op in (_lib.OP_SENDRECV, _lib.OP_BROADCAST, _lib.OP_REDUCE)
+    """The grid has a thread block for every tile of a row and one for its ragged ends, and
+    no others but what makes a row's a multiple of eight where the XCDs take an eighth of it
+    each; on both sides of every line between the forms."""
+    alltoall, one = op == _lib.OP_ALLTOALL, op in CU_OPS[:3]
+    copies = op in (_lib.OP_BROADCAST, _lib.OP_ALLGATHER) and world > 2
     pipes, rows = (world * world, world) if alltoall else (1, 1) if one else (world, world)
     touching = 2 if alltoall or op == _lib.OP_SENDRECV else world
-    for mib in (1, 19, 20, 21, 33, 50, 72):
-        for more in (0, 1, 15, 2047, 2048):
-            row = (mib << 20) // (pipes * touching) // 2048 * 2048 + more * 2
+    for mib in (1, 8, 11, 13, 19, 21, 23, 33, 41, 50, 72, 74, 87, 89, 99, 101, 150, 175, 177, 191, 193, 207, 209, 263, 265,
+                639, 641, 699, 701, 1279, 1281, 2559, 2561):
+        for more in (0, 2, 30, 1022, 2046, 4094, 4096):
+            row = (mib << 20) // (pipes * touching) // 4096 * 4096 + more
             d = inside_compute_units(op, world, row)
             blocks = _lib.lib().mint_ring_grid_blocks(d)
             assert blocks > 0 and blocks % pipes == 0, (mib, more, blocks)
-            blocks //= pipes
             held = -(-row // 16) * 16 if op == _lib.OP_ALLREDUCE else row       # (cut in whole vectors)
-            slack = 127 if not one and held % 128 else 0
-            assert blocks >= -(-(held + slack) // 2048) + (d.count_bytes % 16 != 0), (mib, more, blocks)
-            touched = pipes * row * touching
-            if rows % 8 and touched >= 20 << 20:
-                assert blocks % 8 == 0
-                for y in range(rows):
-                    for z in range(world if alltoall else 1):
-                        assert sorted(((x + y + z) % 8) * (blocks // 8) + x // 8 for x in range(blocks)) == list(range(blocks))
+            touched = pipes * held * touching
+            tile, align = cu_tile(op, world, touched)
+            slack = align - 1 if not one and held % align else 0
+            # (the last row of an allreduce is what the others leave of the buffer)
+            last = d.count_bytes - (world - 1) * held if op == _lib.OP_ALLREDUCE else row
+            want = -(-(held + slack) // tile) + (last % 16 != 0 or held % 16 != 0)
+            least = 12 if op == _lib.OP_REDUCE and world == 2 else 20
+            if rows % 8 and align == 128 and touched >= least << 20 and not (copies and touched > 73 << 20):
+                want = -(-want // 8) * 8
+            assert blocks // pipes == want, (mib, more, blocks // pipes, want)
 
 
 def test_headline_geometry():
