@@ -125,9 +125,11 @@ def added(rows, first):
     return x
 
 
-# MiB touched (bytes of a row times rows times ranks), elements more than that in every row
-@pytest.mark.parametrize("mib,more", [(19, 3), (21, 0), (21, 3), (47, 1021), (77, 5), (85, 3), (105, 2051), (170, 9), (270, 1)])
-@pytest.mark.parametrize("world,dt", [(2, "f32"), (3, "f16"), (5, "bf16"), (7, "f16"), (8, "bf16")])
+# MiB touched (bytes loaded and stored, sums: loaded), elements more than that in every row
+@pytest.mark.parametrize("mib,more", [(1, 5), (8, 1), (11, 3), (19, 3), (21, 0), (21, 3), (25, 9), (31, 2), (33, 3), (41, 7),
+                                      (47, 1021), (72, 6), (74, 1), (85, 3), (89, 5), (105, 2051), (170, 9), (178, 3),
+                                      (194, 7), (206, 1), (210, 3), (262, 1), (270, 1)])
+@pytest.mark.parametrize("world,dt", [(2, "f32"), (3, "f16"), (4, "f16"), (5, "bf16"), (6, "f32"), (7, "f16"), (8, "bf16")])
 def test_every_form(dev, world, dt, mib, more):
     """Sizes on both sides of what a launch's form is chosen by, rows that end in
     the middle of a vector, a tile and an XCD's part of the tiles."""
@@ -142,7 +144,7 @@ def test_every_form(dev, world, dt, mib, more):
     g = torch.Generator(device=dev).manual_seed(100 * world + mib)
 
     def make(rows, touched):
-        n = (touched << 20) // (rows * world * dtype.itemsize) + more
+        n = int(touched * 2**20) // (rows * world * dtype.itemsize) + more
         return [torch.randn((rows, n), generator=g, device=dev, dtype=torch.float32).to(dtype) for _ in range(world)]
 
     def same(got, want, what):
@@ -174,20 +176,24 @@ def test_every_form(dev, world, dt, mib, more):
     same(bufs, [added(made, 1) if r == 1 else made[r] for r in range(world)], "reduce")
     comm.run(lambda r: broadcast(bufs[r], world - 1, comm))
     same(bufs, [bufs[world - 1]] * world, "broadcast")
-    made = make(world, (mib + 1) // 2 * world // 2)
+    made = make(world, mib / 2)                       # (as much again is stored)
     outs = [torch.zeros_like(m) for m in made]
     comm.run(lambda r: alltoall(made[r], outs[r], comm))
     same(outs, [torch.stack([made[q][r] for q in range(world)]) for r in range(world)], "alltoall")
 
 
-@pytest.mark.parametrize("world", [6, 7, 8])
-def test_copies_far_beyond_the_cache(dev, world):
-    """More than 700 MiB touched, rows that end in the middle of a 4 KiB tile and of
-    a vector; what lies around the rows stays as it was."""
+@pytest.mark.parametrize("world,mib", [(6, 1284), (7, 704), (8, 2564)])
+def test_copies_far_beyond_the_cache(dev, world, mib):
+    """Just beyond where a wavefront moves 4 KiB, rows that end in the middle of such a
+    tile and of a vector; what lies around the rows stays as it was."""
     from mintccl_amd.allgather import allgather
     from mintccl_amd.broadcast import broadcast
     comm = make_comm(world)
-    nbytes = (704 << 20) // (world * world) + 2 * 1024 + 3
+    nbytes = (mib << 20) // (world * world) + 2 * 1024 + 3
+
+    def blocks(row):                       # (a row's first tile may begin up to 1023 bytes before it; one block for the ends)
+        return -(-(row + 1023) // 4096) + 1
+
     g = torch.Generator(device=dev).manual_seed(world)
     rows = [torch.randint(0, 256, (nbytes,), dtype=torch.uint8, generator=g, device=dev) for _ in range(world)]
     backing = [torch.full((world * nbytes + 64,), 0x5A, dtype=torch.uint8, device=dev) for _ in range(world)]
@@ -196,6 +202,7 @@ def test_copies_far_beyond_the_cache(dev, world):
         b[r] = rows[r]
     comm.run(lambda r: allgather(bufs[r], comm))
     comm.check()
+    assert comm.last_grid == world * blocks(nbytes)
     want = torch.stack(rows)
     for r in range(world):
         assert torch.equal(bufs[r], want), r
@@ -204,6 +211,7 @@ def test_copies_far_beyond_the_cache(dev, world):
     flat[1].copy_(torch.randint(0, 256, (world * nbytes,), dtype=torch.uint8, generator=g, device=dev))
     comm.run(lambda r: broadcast(flat[r], 1, comm))
     comm.check()
+    assert comm.last_grid == blocks(world * nbytes)
     for r in range(world):
         assert torch.equal(flat[r], flat[1]), r
 
@@ -247,7 +255,8 @@ def test_rows_at_any_byte_touch_nothing_else(dev, shift):
 
 @pytest.mark.parametrize("world,dt", [(8, "bf16"), (7, "f16"), (5, "f32"), (3, "f16"), (2, "f32")])
 def test_rows_beyond_the_cache(dev, world, dt):
-    """The large form (more than 96 MiB touched), buffers that start 6 or 12 bytes
+    """Just beyond 100 MiB touched (the large form; sums of two to six ranks to one place the
+    form between, small copies of two ranks), buffers that start 6 or 12 bytes
     behind a 16-byte boundary and rows that end in the middle of a vector."""
     from mintccl_amd.allgather import allgather
     from mintccl_amd.allreduce import allreduce
