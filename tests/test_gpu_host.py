@@ -141,7 +141,7 @@ def test_codec_refuses_what_it_cannot_take(dev):
 
 def test_codec_takes_its_arguments_in_every_form(dev):
     """Positional, by name, defaults, a name made at run time; what does not fit is
-    the function's own TypeError, before the library is bound as after."""
+    the function's own TypeError."""
     import inspect
     import pickle
 
@@ -153,9 +153,11 @@ def test_codec_takes_its_arguments_in_every_form(dev):
             for base, layout, stride in ((1, wave, 1), (9, pair, 1), (9, wave, 3), (2**64 - 1, wave, 1))}
     into = torch.zeros_like(want[1, wave, 1])
     assert protocol.pack(raw, out=into) is into
+    made = "".join(["flag", "_", "base"])              # (another object than the name in the code)
+    assert made is not inspect.signature(protocol.pack.__wrapped__).parameters["flag_base"].name
     for msg, kept in ((into, (1, wave, 1)), (protocol.pack(raw), (1, wave, 1)), (protocol.pack(raw=raw), (1, wave, 1)),
                       (protocol.pack(raw, 9, pair), (9, pair, 1)), (protocol.pack(raw, layout=pair, flag_base=9), (9, pair, 1)),
-                      (protocol.pack(raw, 9, flag_stride=3), (9, wave, 3)), (protocol.pack(raw, **{"flag" + "_base": -1}), (2**64 - 1, wave, 1))):
+                      (protocol.pack(raw, 9, flag_stride=3), (9, wave, 3)), (protocol.pack(raw, **{made: -1}), (2**64 - 1, wave, 1))):
         base, layout, stride = kept
         assert torch.equal(msg, want[kept])
         for form in (lambda o: protocol.unpack(msg, o, base, layout, stride, bad),

@@ -1,7 +1,13 @@
 """Host-side logic that needs no GPU: knobs and wave-count selection."""
+import os
+import subprocess
+import sys
+
 import pytest
 
 from mintccl_amd import _lib, common, protocol
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def test_reference_constants():
@@ -229,3 +235,24 @@ def test_headline_geometry():
     assert common.tuned_geometry(_lib.OP_BROADCAST, 8, 0, 256, 3, row_blocks=5) == (32 * 1024, 3, 32)
     assert common.tuned_geometry(_lib.OP_TREE_REDUCE, 8, 0, 256, 3, row_blocks=5) == (2 * 32 * 1024, 3, 32)
     assert common.tuned_geometry(_lib.OP_TREE_REDUCE, 8, 0, 256, 3) == (2 * 512 * 1024, 3, 512)
+
+
+def test_codec_front_before_the_library_is_bound():
+    """A call goes to the function as it came, one that does not fit included."""
+    code = """if True:
+        from mintccl_amd import _host
+        def pack(raw, flag_base=1, layout=2, flag_stride=3, out=None):
+            return raw, flag_base, layout, flag_stride, out
+        front = _host.Front(pack, _host.PACK, None)
+        assert front(5) == (5, 1, 2, 3, None) and front(out=4, raw=5) == (5, 1, 2, 3, 4)
+        assert front(5, 6, 7, 8, 9) == (5, 6, 7, 8, 9)
+        for args, names in (((), {}), ((1, 2, 3, 4, 5, 6), {}), ((5,), {"raw": 5}), ((5,), {"raws": 5})):
+            try:
+                front(*args, **names)
+            except TypeError as e:
+                assert "pack()" in str(e)
+            else:
+                raise AssertionError(args)
+        print("DONE")
+    """
+    assert "DONE" in subprocess.check_output([sys.executable, "-c", code], cwd=ROOT).decode()
