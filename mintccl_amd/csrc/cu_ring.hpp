@@ -88,10 +88,13 @@ __device__ __forceinline__ u32x4 cu_load(const uint8_t* uniform, uint32_t lane) 
 //   large, several:                 allgather of 8 x 64 MiB   - / 73.4 / 94.3 / 67.7
 //   large, one:                     reduce-scatter of 64 MiB 86.9 / 88.6 / 82.1 / 88.0
 enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
-// A copy to one place in the small form, up to 24 MiB touched (cu_through_mib): sc1.  The results stay
+// A copy to one place in the small form, up to 24 MiB touched: sc1.  The results stay
 // in the L2s, and the kernel that reads them next takes 6 - 20 us less than behind nt or sc1 nt
 // (multiplied in place, buffers of 3 - 6 MiB 27 -> 7 us and 13 -> 7); alone the call takes 0.94 / 0.96 / 1.03 -
 // 1.07 of nt (the same buffers again / three sets in turn / buffers that 700 MiB lie between two uses of).
+// (a pipeline to each XCD leaves a whole row of results in one XCD's L2: short ones, which few blocks
+// read next, are sooner there from the last-level cache.  Alltoall of eight ranks, multiplied in place
+// behind the call, sc1 / nt: 2 MiB 4 us more, 2.5 MiB 6 less)
 // Beyond: sc1 nt, a choice that holds whatever the caches hold, nt alone does not (with eight pipelines,
 // a pipeline to each XCD, it does: odd rows 1.00 / 1.06 / 1.06 by sc1 nt).  Alltoall of 2 to 7 ranks, over
 // nt in tiles dealt one by one, tiles dealt by the eighth (CuPlace):
@@ -100,16 +103,35 @@ enum { CU_NT = 0, CU_SC1 = 1, CU_SC1_NT = 2 };
 //   sc1 nt     0.86 / 0.94 / 1.00    0.80 / 0.94 / 0.98    0.93 / 0.94 / 0.96
 // sendrecv and the copies of two ranks alike (65 - 160 MiB nt 0.97 / 0.98 / 1.02, sc1 nt 0.97 / 0.97 / 1.00).
 //
-// A sum to one place in the small form, two and three ranks: sc1 (over nt at 6 - 12 / 12 - 20 /
-// 20 - 80 MiB touched, three sets in turn, 2 ranks 0.99 / 0.81 / 0.97, 16 MiB 5.0 -> 3.8 us; 3 ranks
-// 0.99 / 0.91 / 1.00).  Four and more: sc1 up to cu_through_mib touched, about what the eight L2s hold
-// (over nt alone 0.97 - 1.02; the kernel that reads the sum next takes 0.5 - 1.5 us less).
+// A sum to one place in the small form: sc1 in the bands below (cu_through_mib), nt elsewhere.  Time over
+// that of nt in tiles dealt one by one, reduce and reduce-scatter in three types, the same buffers again /
+// three sets in turn / 700 MiB between two uses, geometric means (largest):
+//   touched MiB              sc1                                        nt
+//   2 ranks   4 - 6   0.98 (1.05) / 1.01 (1.09) / 1.02 (1.06)    0.96 (1.01) / 0.98 (1.02) / 0.99 (0.99)
+//             6 - 20  0.89 (1.02) / 0.87 (1.02) / 1.00 (1.05)    0.96 (1.00) / 0.99 (1.09) / 1.00 (1.07)
+//            32 - 56  0.73 (0.89) / 0.94 (0.97) / 0.99 (1.05)    1.00 (1.13) / 0.98 (1.02) / 1.02 (1.09)
+//   3 ranks   6 - 12  0.98 (1.03) / 0.93 (1.03) / 1.08 (1.51)    0.97 (1.00) / 0.98 (1.02) / 0.99 (1.00)
+//            12 - 20  0.91 (0.98) / 0.87 (1.01) / 0.99 (1.02)    0.98 (1.00) / 0.99 (0.99) / 0.99 (1.00)
+//            32 - 56  0.77 (1.01) / 0.93 (0.99) / 0.97 (1.03)    0.97 (1.08) / 0.94 (1.00) / 0.99 (1.05)
+//   4 - 8     4 - 20  0.98 (1.11) / 0.97 (1.05) / 1.00 (1.32)    0.97 (1.02) / 0.98 (1.03) / 0.99 (1.02)
+//   4 - 7    20 - 32  0.90 (1.11) / 0.96 (1.03) / 0.98 (1.05)    0.88 (1.07) / 0.95 (1.01) / 0.98 (1.05)
+//            32 - 56  0.87 (1.13) / 0.96 (1.04) / 0.97 (1.05)    0.97 (1.31) / 0.95 (1.03) / 0.98 (1.09)
+// sc1 takes longest on rows of 2 - 3 MiB that lie 4 MiB apart and are in no cache: 3 ranks 3.6 -> 5.9
+// us, 4 ranks 4.3 -> 5.8.  With a pipeline to each XCD it is 1.08 / 1.01 / 1.00 at 20 - 32 MiB.
+//
 // Not taken for either: rows streamed.  The call alone is then 0.85 - 0.95 of that at 12 - 40 MiB, but
 // streamed rows do not stay in any cache.  A kernel that reads the buffers again next takes 8 - 13 us
 // longer (multiplied in place, four ranks of 22 MiB in all 17 -> 25 us), and the same call on the same
 // buffers again up to 1.3 at 20 - 32 MiB.
-constexpr int kCuThroughRanks = 3;
-constexpr int cu_through_mib(bool sums, int ranks) { return !sums ? 24 : ranks == 8 ? 32 : 40; }
+struct CuBand {
+    int above, most;          // MiB touched
+};
+constexpr CuBand cu_through_mib(bool sums, int ranks, int pipes, bool pipe_each) {
+    if (!sums) return {pipe_each ? 2 : 0, 24};
+    if (ranks <= 3) return {ranks == 2 ? 6 : 12, 1 << 20};
+    if (pipe_each || (ranks >= 7 && pipes == 1)) return {0, 0};      // (cu_by_eighths)
+    return {32, 56};
+}
 // Sums to one place that are far larger than the last-level cache (plan_cu): with
 // many rows to read nt is the faster one, on buffers that have not just been used.
 // Four sets of buffers in turn, reduce-scatter and reduce of f16 and bf16, nt over
@@ -213,9 +235,7 @@ auto cu_sum_form(const CuChoice& c, const USE& use) {
         if constexpr (N <= kCuMidRanks)
             if (c.mid) return use(CuFormIs<CuMidSum<N>, false>{});
         if (c.large) return use(CuFormIs<CuLargeSum>{});
-        if constexpr (N > kCuThroughRanks)
-            if (!c.through) return use(CuFormIs<CuSmall<CU_NT>>{});
-        return use(CuFormIs<CuSmall<CU_SC1>>{});
+        return c.through ? use(CuFormIs<CuSmall<CU_SC1>>{}) : use(CuFormIs<CuSmall<CU_NT>>{});
     }
 }
 // a row copied to one place (sendrecv, alltoall, two ranks)

@@ -116,6 +116,11 @@ bool cu_by_eighths(uint64_t touched, int ranks, int pipes, bool sums, bool copie
     // Copies to several places up to 73 MiB: beyond, three sets of buffers meet the edge of the
     // last-level cache (74 - 88 MiB, over tiles dealt one by one, three sets in turn: broadcast 1.01, up to
     // 1.14; with a kernel around that reads inputs and results 2 us more).
+    // Not a reduce of seven and eight ranks that just outgrows the L2s: by the eighth none of the rows
+    // stay in them from one use to the next, dealt one by one a part does.  33 - 56 MiB, the same buffers
+    // again / three sets in turn / buffers that 700 MiB lie between two uses of: 7 ranks 1.03 (up to
+    // 1.35) / 0.96 / 0.98, 8 ranks 1.18 (up to 1.71) / 0.95 / 0.96.
+    if (sums && ranks >= 7 && pipes == 1 && touched > (32ull << 20) && touched <= (56ull << 20)) return false;
     return touched >= least << 20 && !(copies && touched > (73ull << 20));
 }
 
@@ -134,11 +139,8 @@ int plan_cu(Plan* plan) {
     choice.mid = sums && !everywhere && ranks <= kCuMidRanks && beyond(line) && !beyond(cu_mid_mib(ranks));
     choice.large = beyond(line) && !choice.mid;
     choice.pipe_each = (alltoall ? ranks : a.pipes) % kXcds == 0;
-    // (a pipeline to each XCD leaves a whole row of results in one XCD's L2: short ones, which few blocks
-    // read next, are sooner there from the last-level cache.  Eight ranks, multiplied in place behind the
-    // call, sc1 / nt: reduce-scatter of 4 MiB 4 us more, 8 MiB 9, 10 MiB 0; alltoall of 2 MiB 4 more, 2.5 MiB
-    // 6 less)
-    choice.through = !beyond(cu_through_mib(sums, ranks)) && !(choice.pipe_each && !beyond(sums ? 9 : 2));
+    const CuBand through = cu_through_mib(sums, ranks, a.pipes, choice.pipe_each);
+    choice.through = beyond(through.above) && !beyond(through.most);
     // Far beyond it the sums of many ranks are streamed past it (kCuStreamRanks): the
     // line lies where three sets of buffers in turn cross over, 600 MiB (6 ranks) to
     // 740 (8; 640 MiB 110 / 114 us).  Copies of many ranks: kCuVastCopies.

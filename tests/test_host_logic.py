@@ -149,18 +149,20 @@ def test_rows_copied_to_several_places_stay_in_the_cache_up_to_88_mib(op, world)
 
 
 @pytest.mark.parametrize("op,world,least,most", [
-    (_lib.OP_REDUCE, 2, 12, 100), (_lib.OP_REDUCE, 5, 20, 100), (_lib.OP_BROADCAST, 3, 20, 73), (_lib.OP_BROADCAST, 8, 20, 73),
+    (_lib.OP_REDUCE, 2, 12, 100), (_lib.OP_REDUCE, 6, 20, 100), (_lib.OP_REDUCE, 7, 20, 100), (_lib.OP_REDUCE, 8, 20, 100), (_lib.OP_BROADCAST, 3, 20, 73), (_lib.OP_BROADCAST, 8, 20, 73),
     (_lib.OP_ALLGATHER, 4, 20, 73), (_lib.OP_ALLGATHER, 8, 99, 0), (_lib.OP_SENDRECV, 2, 20, 192)])
 def test_where_an_xcd_takes_an_eighth_of_every_row(op, world, least, most):
-    """Then a row has a multiple of eight thread blocks, else one per tile."""
-    for mib in (11, 13, 17, 19, 21, 30, 45, 59, 71, 72.9, 73.1, 80, 87):
+    """Then a row has a multiple of eight thread blocks, else one per tile.  Not where a reduce
+    of seven or eight ranks just outgrows the L2s: the same buffers again up to 1.7 of the time."""
+    for mib in (11, 13, 17, 19, 21, 30, 31.5, 33, 45, 55.5, 57, 59, 71, 72.9, 73.1, 80, 87):
         row = int(mib * 2**20) // (2 if op == _lib.OP_SENDRECV else world) // (world if op == _lib.OP_ALLGATHER else 1)
         row = row // 16384 * 16384 + 2048 * 3                     # tiles: 3 more than a multiple of 8
         blocks = _lib.lib().mint_ring_grid_blocks(inside_compute_units(op, world, row))
         tiles = row // 2048 * (world if op == _lib.OP_ALLGATHER else 1)
         if op == _lib.OP_ALLGATHER:
             blocks, tiles = blocks // world, tiles // world
-        assert blocks == (tiles + 5 if least <= mib <= most else tiles), (mib, blocks, tiles)
+        outgrows = op == _lib.OP_REDUCE and world >= 7 and 32 < mib < 56
+        assert blocks == (tiles + 5 if least <= mib <= most and not outgrows else tiles), (mib, blocks, tiles)
 
 
 def cu_tile(op, world, touched):
@@ -206,7 +208,8 @@ def test_every_tile_of_a_row_has_its_block_inside_compute_units(op, world):
             last = d.count_bytes - (world - 1) * held if op == _lib.OP_ALLREDUCE else row
             want = -(-(held + slack) // tile) + (last % 16 != 0 or held % 16 != 0)
             least = 12 if op == _lib.OP_REDUCE and world == 2 else 20
-            if rows % 8 and align == 128 and touched >= least << 20 and not (copies and touched > 73 << 20):
+            outgrows = op == _lib.OP_REDUCE and world >= 7 and 32 << 20 < touched <= 56 << 20
+            if rows % 8 and align == 128 and touched >= least << 20 and not (copies and touched > 73 << 20) and not outgrows:
                 want = -(-want // 8) * 8
             assert blocks // pipes == want, (mib, more, blocks // pipes, want)
 
