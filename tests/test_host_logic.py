@@ -171,7 +171,7 @@ def cu_tile(op, world, touched):
     if op in CU_SUMS:
         if mib <= 100:
             return 2048, 128
-        if op != _lib.OP_ALLREDUCE and mib <= {2: 176, 3: 264, 4: 208, 5: 176, 6: 176}.get(world, 0):
+        if op != _lib.OP_ALLREDUCE and mib <= {2: 196, 3: 264, 4: 208, 5: 176, 6: 160}.get(world, 0):
             return (2048 if world <= 4 else 1024), 128
         return 1024, 1024
     if op in (_lib.OP_SENDRECV, _lib.OP_ALLTOALL) or world == 2:
@@ -193,7 +193,7 @@ def test_every_tile_of_a_row_has_its_block_inside_compute_units(op, world):
     copies = op in (_lib.OP_BROADCAST, _lib.OP_ALLGATHER) and world > 2
     pipes, rows = (world * world, world) if alltoall else (1, 1) if one else (world, world)
     touching = 2 if alltoall or op == _lib.OP_SENDRECV else world
-    for mib in (1, 8, 11, 13, 19, 21, 23, 33, 41, 50, 72, 74, 87, 89, 99, 101, 150, 175, 177, 191, 193, 207, 209, 263, 265,
+    for mib in (1, 8, 11, 13, 19, 21, 23, 33, 41, 50, 72, 74, 87, 89, 99, 101, 150, 159, 161, 175, 177, 191, 193, 195, 197, 207, 209, 263, 265,
                 639, 641, 699, 701, 1279, 1281, 2559, 2561):
         for more in (0, 2, 30, 1022, 2046, 4094, 4096):
             row = (mib << 20) // (pipes * touching) // 4096 * 4096 + more
