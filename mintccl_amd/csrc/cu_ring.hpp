@@ -189,10 +189,11 @@ constexpr int cu_vast_mib(int ranks) { return ranks == 7 ? 700 : ranks == 6 ? 12
 // arrive: 8 ranks, allgather of 8 x 128 MiB 1405 -> 1318 us (1473 -> 1331 with rows that
 // are no multiple of a line), 7 ranks and 4 GiB 0.94, 6 ranks 0.96.
 //
-// Otherwise: blocks of 128 threads and 2 KiB, loads through the cache, to each XCD
+// SMALL, otherwise: blocks of 128 threads and 2 KiB, loads through the cache, to each XCD
 // consecutive tiles (CuPlace).  8 ranks, reduce-scatter of 8 MiB 10.9 us, 15.5 in the
 // large form.  Blocks of 64 and of 256 threads with 2 KiB and 4 KiB are within 1 % of
 // it, 4 KiB by 64 threads 2 - 4 % slower, 512 threads up to a tenth where rows are added.
+// CuMidSum (kCuMidRanks) is the small form in its places, with the large one's loads.
 template <int THREADS, int VECTORS, bool LARGE, bool STREAM, int STORES>
 struct CuForm {
     static constexpr int kThreads = THREADS;       // of a block

@@ -626,11 +626,12 @@ uint32_t codec_blocks(uint64_t lines, int layout) {
     return (uint32_t)(cap && blocks > cap ? cap : blocks);
 }
 
-// A launch of the wave64 codec.  From 4 MiB on, up to where raw bytes and message no longer
-// stay in the last-level cache, an XCD takes consecutive thread blocks.  pack + unpack, three
-// sets of buffers in turn, dealt one by one / so, us: 4 MiB 7.9 / 7.9, 6 MiB 7.5 / 7.3, 8 MiB
-// 8.0 / 7.6, 16 MiB 12.8 / 12.3, 32 MiB 22.4 / 21.1, 48 MiB 32.0 / 30.3, 56 MiB 36.4 / 35.5, 64 MiB
-// 41.2 / 42.1.
+// A launch of the wave64 codec.  An XCD takes consecutive thread blocks between the sizes where
+// that is measured to be faster.  pack + unpack, dealt one by one (and with eight launch arguments) / so, us,
+// the same buffers again, three sets in turn, 750 MiB between two uses: 4 MiB 6.4 / 6.1, 6.4 / 6.2, 7.0 / 6.7; 8 MiB 7.4 / 7.2, 8.4 / 8.2, 9.6 /
+// 9.6; 16 MiB 12.2 / 11.0, 12.9 / 12.4, 14.7 / 14.6; 32 MiB 22.1 / 21.2, 22.0 / 21.1, 24.5 / 24.8; 48 MiB 31.1 /
+// 30.3, 32.6 / 32.2, 34.0 / 33.4; 59 MiB 37.4 / 36.5, 39.6 / 38.5, 40.5 / 39.8; at 64 MiB, three sets, 41.2 /
+// 42.1.
 template <auto KERNEL>
 int codec_wave64(const void* from, void* to, uint64_t nbytes, uint64_t lines, uint64_t flag_base, uint64_t flag_stride,
                  void* bad, void* stream) {
