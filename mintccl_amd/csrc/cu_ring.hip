@@ -30,10 +30,26 @@ int launch_as(const Plan& plan, hipStream_t stream) {
                               u32x2{s.tiles, s.part}, tables);
 }
 
+template <typename FORM, auto KERNEL>
+int launch_near(const Plan& plan, hipStream_t stream) {
+    const CuRingArgs& a = plan.cu_args;
+    const CuShape& s = a.shape;
+    uint32_t at[kMaxRanks] = {};
+    for (uint32_t i = 0; i < a.len; ++i) at[i] = (uint32_t)((a.input[i] ? a.input[i] : a.output[i]) - a.lowest);
+    const bool cut = s.full < a.pipes;
+    const u32x8 rows = {(uint32_t)a.lowest, (uint32_t)(a.lowest >> 32), (uint32_t)s.row_bytes,
+                        (uint32_t)(cut ? s.short_bytes : s.row_stride), at[0], at[1], at[2], at[3]};
+    const u32x4 high = {at[4], at[5], at[6], at[7]};
+    const u32x2 counts = {s.starts | s.full << 24 | (cut ? kCuNearCut : 0u), FORM::kLarge ? s.tiles : s.tiles | s.part << 16};
+    return Launch<KERNEL>::go(grid_of<FORM>(plan, a.pipes, 1), FORM::kThreads, (unsigned)plan.cu_lds, stream, rows, high, counts,
+                              a.status);
+}
+
 template <int DT, int N, bool EVERYWHERE>
 int launch_sum(const Plan& plan, hipStream_t stream) {
     return cu_sum_form<N, EVERYWHERE>(plan.cu_choice, [&](auto form) {
         using Form = typename decltype(form)::type;
+        if (plan.cu_args.near) return launch_near<Form, &cu_near_sum_kernel<DT, N, EVERYWHERE, Form>>(plan, stream);
         if constexpr (decltype(form)::in_place)
             if (!plan.cu_args.split)
                 return launch_as<Form, &cu_ring_sum_kernel<DT, N, EVERYWHERE, Form, false>, N, false>(plan, stream);
@@ -44,6 +60,7 @@ template <int N>
 int launch_copy(const Plan& plan, hipStream_t stream) {
     return cu_copy_form<N>(plan.cu_choice, [&](auto form) {
         using Form = typename decltype(form)::type;
+        if (plan.cu_args.near) return launch_near<Form, &cu_near_copy_kernel<N, Form>>(plan, stream);
         if constexpr (decltype(form)::in_place)
             if (!plan.cu_args.split) return launch_as<Form, &cu_ring_copy_kernel<N, Form, false>, N, false>(plan, stream);
         return launch_as<Form, &cu_ring_copy_kernel<N, Form, true>, N, true>(plan, stream);

@@ -25,6 +25,7 @@
 // 190 / 161.
 #pragma once
 #include <type_traits>
+#include <utility>
 
 #include "ring.hpp"
 
@@ -64,6 +65,32 @@ struct CuTables {
     uint64_t* status;
 };
 static_assert(sizeof(CuShape) + sizeof(CuTables<kMaxRanks, false>) <= 112, "arguments of a launch in place");
+
+// The ranks' buffers where ranks work in place and all rows lie within 4 GiB (`near` in
+// CuRingArgs): the lowest address and every rank's distance from it, in bytes.  With numbers
+// of 32 bits all that the loads wait for fits into the 14 words that a launch can bring in
+// registers; behind them only the status block's address is read from memory, by the one
+// wavefront that looks there.  A table in memory costs each block a round trip before its
+// loads, and its compute unit's first blocks a long one: the runtime has just written it across the bus.
+// Over launches by tables, us, trains of calls over three sets of buffers in turn:
+//   touched      10 MiB        25 MiB        64 MiB        110 MiB        400 MiB
+//   8 ranks, allgather       2.95 / 2.67   4.65 / 4.23   9.38 / 8.85   17.0 / 16.8    57.9 / 57.3
+//            reduce-scatter  2.74 / 2.53   5.49 / 5.25   11.2 / 10.9   23.7 / 22.7    68.7 / 68.2
+//            allreduce       4.19 / 3.93   8.49 / 8.06   18.8 / 18.8   40.6 / 40.6    130 / 129
+//   3 ranks, broadcast       2.57 / 2.51   3.79 / 3.60   10.2 / 10.1   16.9 / 16.8    63.2 / 62.1
+//            reduce          3.44 / 3.45   6.13 / 6.07   13.2 / 13.1   22.3 / 22.1    85.6 / 83.6
+// Below 4 MiB the host's 2.7 us per launch hide it.
+//   rows    lowest address (two words), row_bytes, row_stride; where rows are cut (kCuNearCut),
+//           which follow each other without gaps then, short_bytes in its place; distances of
+//           ranks 0 - 3
+//   high    those of ranks 4 - 7
+//   counts  starts | full << 24 | kCuNearCut, tiles | part << 16 (large form: tiles)
+constexpr uint32_t kCuNearCut = 1u << 31;
+// At most: bytes from the lowest address to the end of the last row, of a row (offsets have a
+// sign), tiles of a row in the small form.
+constexpr uint64_t kCuNearSpan = 0xffffffffull, kCuNearRow = 1ull << 30;
+constexpr uint32_t kCuNearTiles = 0xffff;
+
 // (host side: the whole of a launch)
 struct CuRingArgs {
     CuShape shape;
@@ -72,6 +99,8 @@ struct CuRingArgs {
     uint32_t op, pipes, len;
     uint32_t blocks;               // of the grid for the tiles of a row and its ends
     bool split;
+    uint64_t lowest;               // of the ranks' addresses
+    bool near;
 };
 
 // How rows are loaded: through the caches, or streamed past the last-level one.
@@ -295,11 +324,11 @@ __device__ __forceinline__ void cu_store(uint8_t* uniform, uint32_t lane, u32x4 
 // the bytes from 16 i - `shift` on.  Vectors that are not wholly inside the row
 // are left out; the bytes they would have brought, fewer than 16 at either end,
 // are moved one element per lane.
-template <typename FORM>
+// WIDE: offsets in a row may need more than 31 bits, and tiles more blocks than a grid has.
+template <typename FORM, bool WIDE = FORM::kLarge>
 struct CuRow {
-    // (offsets in a row: the small form's fit into 32 bits)
-    using Bytes = std::conditional_t<FORM::kLarge, uint64_t, uint32_t>;
-    using Offset = std::conditional_t<FORM::kLarge, int64_t, int32_t>;
+    using Bytes = std::conditional_t<WIDE, uint64_t, uint32_t>;
+    using Offset = std::conditional_t<WIDE, int64_t, int32_t>;
     Bytes bytes;
     uint32_t shift;
     __device__ __forceinline__ CuRow(uint64_t row_bytes, uint64_t short_bytes, uint32_t full, uint32_t p,
@@ -337,10 +366,28 @@ struct CuRow {
     }
     template <typename WALK>
     __device__ __forceinline__ void tiles(uint32_t mine, uint32_t all, const WALK& walk) const {
-        if constexpr (FORM::kLarge)
+        if constexpr (WIDE)
             for (uint64_t t = mine; t * FORM::kTile < bytes + shift; t += all) tile(t, walk);
         else
             tile(mine, walk);
+    }
+};
+
+// (device side of a launch by distances)
+struct CuNear {
+    uint8_t* lowest;
+    uint32_t row_bytes, row_stride, short_bytes;
+    u32x8 rank;
+    uint32_t starts, full, tiles, part;
+    __device__ __forceinline__ CuNear(u32x8 rows, u32x4 high, u32x2 counts, bool large)
+        : lowest(reinterpret_cast<uint8_t*>((uint64_t)rows[1] << 32 | rows[0])), row_bytes(rows[2]),
+          row_stride(counts.x & kCuNearCut ? rows[2] : rows[3]), short_bytes(rows[3]),
+          rank{rows[4], rows[5], rows[6], rows[7], high.x, high.y, high.z, high.w}, starts(counts.x),
+          full(counts.x >> 24 & 15u), tiles(large ? counts.y : counts.y & kCuNearTiles), part(large ? 0u : counts.y >> 16) {}
+    __device__ __forceinline__ uint32_t root(uint32_t p) const { return starts >> (3u * p) & 7u; }
+    template <typename FORM>
+    __device__ __forceinline__ CuRow<FORM, false> row(uint32_t p, const uint8_t* stored, uint32_t size) const {
+        return CuRow<FORM, false>(row_bytes, short_bytes, full, p, stored, size);
     }
 };
 
@@ -395,7 +442,7 @@ struct CuPlace {
 // small that this load would show.
 template <uint32_t THREADS>
 __device__ __forceinline__ void cu_count_if_aborted(uint64_t* status) {
-    if (blockIdx.x == 0u && blockIdx.y == 0u && blockIdx.z == 0u && threadIdx.x >= THREADS - 64u)
+    if (__builtin_expect((blockIdx.x | blockIdx.y | blockIdx.z) == 0u, 0) && threadIdx.x >= THREADS - 64u)
         count_launch_if_aborted(status, 0);
 }
 
@@ -403,12 +450,14 @@ typedef uint32_t u32_unaligned __attribute__((aligned(1)));
 typedef uint16_t u16_unaligned __attribute__((aligned(1)));
 template <int DT>
 __device__ __forceinline__ uint32_t cu_load_element(const uint8_t* p) {
-    if constexpr (DT == DT_F32) return *(MINT_GLOBAL const u32_unaligned*)p;
+    if constexpr (DT == DT_BYTES) return *as_global(p);
+    else if constexpr (DT == DT_F32) return *(MINT_GLOBAL const u32_unaligned*)p;
     else return *(MINT_GLOBAL const u16_unaligned*)p;
 }
 template <int DT>
 __device__ __forceinline__ void cu_store_element(uint8_t* p, uint32_t v) {
-    if constexpr (DT == DT_F32) *(MINT_GLOBAL u32_unaligned*)p = v;
+    if constexpr (DT == DT_BYTES) *as_global(p) = (uint8_t)v;
+    else if constexpr (DT == DT_F32) *(MINT_GLOBAL u32_unaligned*)p = v;
     else *(MINT_GLOBAL u16_unaligned*)p = (uint16_t)v;
 }
 
@@ -432,87 +481,165 @@ __device__ __forceinline__ void cu_around(const uint64_t* table, uint32_t root, 
     cu_here(x);
 }
 
+// Where a block finds the ranks' rows: ranks as they follow each other around the ring, the
+// pipeline's root first; an offset in a row is a part that all lanes share and a lane's.
+//
+// By their addresses.  STORED: places that are stored to, the root's first.
+template <int N, int STORED>
+struct CuByTable {
+    const uint8_t* from[N];
+    uint8_t* to[STORED];
+    uint64_t row_off;
+    // (a uniform part and a lane's: scalar base and 32-bit offset of one instruction)
+    template <bool STREAM>
+    __device__ __forceinline__ u32x4 load(int h, int64_t off, uint32_t lane) const {
+        return cu_load<STREAM>(from[h] + ((int64_t)row_off + off), lane);
+    }
+    template <int HOW>
+    __device__ __forceinline__ void store(int i, int64_t off, uint32_t lane, u32x4 v) const {
+        cu_store<HOW>(to[i] + ((int64_t)row_off + off), lane, v);
+    }
+    template <int DT>
+    __device__ __forceinline__ uint32_t load_element(int h, uint64_t off) const { return cu_load_element<DT>(from[h] + row_off + off); }
+    template <int DT>
+    __device__ __forceinline__ void store_element(int i, uint64_t off, uint32_t v) const { cu_store_element<DT>(to[i] + row_off + off, v); }
+};
+// By their distances from the lowest of them (CuNear).
+// FIRST: the first rank that is stored to.
+template <int N, int FIRST>
+struct CuByDistance {
+    // (a vector, not an array: of that the compiler would make LDS for an index it finds in
+    // the selects)
+    typedef uint32_t Ranks __attribute__((ext_vector_type(N)));
+    uint8_t* lowest;
+    Ranks rank;
+    uint32_t row_off;
+    template <int BY, int... I>
+    static __device__ __forceinline__ Ranks turned(Ranks x, std::integer_sequence<int, I...>) {
+        return __builtin_shufflevector(x, x, (I + BY) % N...);
+    }
+    // turned by the bits of `root`: one select of two scalars per rank and bit
+    template <int BY = 1>
+    static __device__ __forceinline__ Ranks around(Ranks x, uint32_t root) {
+        if constexpr (BY >= N) return x;
+        else return around<2 * BY>(root & BY ? turned<BY>(x, std::make_integer_sequence<int, N>{}) : x, root);
+    }
+    __device__ __forceinline__ CuByDistance(const CuNear& a, uint32_t root, uint32_t row_off_) : lowest(a.lowest), row_off(row_off_) {
+        Ranks x;
+#pragma unroll
+        for (int i = 0; i < N; ++i) x[i] = a.rank[i];
+        rank = around(x, root);
+    }
+    __device__ __forceinline__ const uint8_t* stored() const { return lowest + rank[FIRST] + row_off; }
+    template <bool STREAM>
+    __device__ __forceinline__ u32x4 load(int h, int32_t off, uint32_t lane) const {
+        return cu_load<STREAM>(lowest, rank[h] + (row_off + (uint32_t)off + lane));
+    }
+    template <int HOW>
+    __device__ __forceinline__ void store(int i, int32_t off, uint32_t lane, u32x4 v) const {
+        cu_store<HOW>(lowest, rank[FIRST + i] + (row_off + (uint32_t)off + lane), v);
+    }
+    template <int DT>
+    __device__ __forceinline__ uint32_t load_element(int h, uint32_t off) const {
+        return cu_load_element<DT>(lowest + (rank[h] + (row_off + off)));
+    }
+    template <int DT>
+    __device__ __forceinline__ void store_element(int i, uint32_t off, uint32_t v) const {
+        cu_store_element<DT>(lowest + (rank[FIRST + i] + (row_off + off)), v);
+    }
+};
+
 // Rings that add: N ranks, the sum goes to the root of the pipeline (reduce,
-// reduce-scatter) or, EVERYWHERE, to all of them (allreduce).
+// reduce-scatter) or to all of them (allreduce): to STORED places.
+template <int DT, int N, int STORED, typename FORM, bool WIDE, typename PLACES>
+__device__ __forceinline__ void cu_sum_row(const CuRow<FORM, WIDE>& row, uint32_t tile, uint32_t tiles, const PLACES& at) {
+    using Row = CuRow<FORM, WIDE>;
+    if (__builtin_expect(tile < tiles, 1)) {
+        const uint32_t lane = threadIdx.x * 16u;
+        row.tiles(tile, tiles, [&](typename Row::Offset base, auto count) MINT_INLINE_LAMBDA {
+            constexpr int kCount = decltype(count)::value, kStep = FORM::kThreads * 16;
+            u32x4 v[kCount][N];
+#pragma unroll
+            for (int k = 0; k < kCount; ++k)
+#pragma unroll
+                for (int h = 0; h < N; ++h) v[k][h] = at.template load<FORM::kStream>(h, base + k * kStep, lane);
+#pragma unroll
+            for (int k = 0; k < kCount; ++k) {
+                u32x4 x = v[k][0];
+#pragma unroll
+                for (int h = 1; h < N; ++h) x = ll_comp<DT>(v[k][h], x);
+#pragma unroll
+                for (int i = 0; i < STORED; ++i) at.template store<FORM::kStores>(i, base + k * kStep, lane, x);
+            }
+        });
+        return;
+    }
+    typename Row::Bytes off;
+    if (tile > tiles || !row.end_element(DT == DT_F32 ? 4u : 2u, off)) return;
+    uint32_t v[N];
+#pragma unroll
+    for (int h = 0; h < N; ++h) v[h] = at.template load_element<DT>(h, off);
+    uint32_t x = v[0];
+#pragma unroll
+    for (int h = 1; h < N; ++h) x = add_rn<DT>(v[h], x);
+#pragma unroll
+    for (int i = 0; i < STORED; ++i) at.template store_element<DT>(i, off, x);
+}
 template <int DT, int N, bool EVERYWHERE, typename FORM, bool SPLIT>
 __global__ void __launch_bounds__(FORM::kThreads) cu_ring_sum_kernel(u64x4 numbers, u32x2 counts, const CuTables<N, SPLIT> a) {
     const CuShape s(numbers, counts);
-    using Row = CuRow<FORM>;
     constexpr uint32_t kSize = DT == DT_F32 ? 4u : 2u;
     const CuPlace place(FORM::kLarge, s.part);
     const uint32_t tile = place.tile, p = place.pipe;
     const uint32_t root = s.starts >> (3u * p) & 7u;
-    const uint64_t row_off = (uint64_t)p * s.row_stride;
     constexpr int kStored = EVERYWHERE ? N : 1, kOut = SPLIT ? N : 0;
-    const uint8_t* from[N];
-    uint8_t* to[kStored];
+    CuByTable<N, kStored> at;
+    at.row_off = (uint64_t)p * s.row_stride;
     // (all of them asked for before the first is waited for: large sums to one place, whose
     // few wavefronts do not hide a second wait: 8 ranks, 0.99 at 110 - 180 MiB touched)
 #pragma unroll
-    for (int i = 0; i < kStored; ++i) to[i] = reinterpret_cast<uint8_t*>(a.rank[kOut + (EVERYWHERE ? (uint32_t)i : root)]);
-    cu_around(a.rank, root, from);
-    if constexpr (EVERYWHERE || SPLIT) cu_here(to);
-    else to[0] = const_cast<uint8_t*>(from[0]);
-    const Row row(s.row_bytes, s.short_bytes, s.full, p, to[0] + row_off, kSize);
+    for (int i = 0; i < kStored; ++i) at.to[i] = reinterpret_cast<uint8_t*>(a.rank[kOut + (EVERYWHERE ? (uint32_t)i : root)]);
+    cu_around(a.rank, root, at.from);
+    if constexpr (EVERYWHERE || SPLIT) cu_here(at.to);
+    else at.to[0] = const_cast<uint8_t*>(at.from[0]);
+    const CuRow<FORM> row(s.row_bytes, s.short_bytes, s.full, p, at.to[0] + at.row_off, kSize);
     cu_count_if_aborted<FORM::kThreads>(a.status);
-    if (__builtin_expect(tile >= s.tiles, 0)) {
-        typename Row::Bytes off;
-        if (tile > s.tiles || !row.end_element(kSize, off)) return;
-        uint32_t v[N];
-#pragma unroll
-        for (int h = 0; h < N; ++h) v[h] = cu_load_element<DT>(from[h] + row_off + off);
-        uint32_t x = v[0];
-#pragma unroll
-        for (int h = 1; h < N; ++h) x = add_rn<DT>(v[h], x);
-#pragma unroll
-        for (int i = 0; i < kStored; ++i) cu_store_element<DT>(to[i] + row_off + off, x);
-        return;
-    }
-    const uint32_t lane = threadIdx.x * 16u;
-    row.tiles(tile, s.tiles, [&](typename Row::Offset base, auto count) MINT_INLINE_LAMBDA {
-        constexpr int kCount = decltype(count)::value, kStep = FORM::kThreads * 16;
-        // (a uniform part and a lane's: scalar base and 32-bit offset of one instruction)
-        const int64_t off = (int64_t)row_off + base;
-        u32x4 v[kCount][N];
-#pragma unroll
-        for (int k = 0; k < kCount; ++k)
-#pragma unroll
-            for (int h = 0; h < N; ++h) v[k][h] = cu_load<FORM::kStream>(from[h] + off + k * kStep, lane);
-#pragma unroll
-        for (int k = 0; k < kCount; ++k) {
-            u32x4 x = v[k][0];
-#pragma unroll
-            for (int h = 1; h < N; ++h) x = ll_comp<DT>(v[k][h], x);
-#pragma unroll
-            for (int i = 0; i < kStored; ++i) cu_store<FORM::kStores>(to[i] + off + k * kStep, lane, x);
-        }
-    });
+    cu_sum_row<DT, N, kStored>(row, tile, s.tiles, at);
+}
+template <int DT, int N, bool EVERYWHERE, typename FORM>
+__global__ void __launch_bounds__(FORM::kThreads) cu_near_sum_kernel(u32x8 rows, u32x4 high, u32x2 counts, uint64_t* status) {
+    const CuNear a(rows, high, counts, FORM::kLarge);
+    const CuPlace place(FORM::kLarge, a.part);
+    const uint32_t p = place.pipe;
+    const CuByDistance<N, 0> at(a, a.root(p), p * a.row_stride);
+    const auto row = a.template row<FORM>(p, at.stored(), DT == DT_F32 ? 4u : 2u);
+    cu_count_if_aborted<FORM::kThreads>(status);
+    cu_sum_row<DT, N, EVERYWHERE ? N : 1>(row, place.tile, a.tiles, at);
 }
 
 // A row from one place to COPIES others.
-template <int COPIES, typename FORM>
-__device__ __forceinline__ void cu_copy_row(const CuRow<FORM>& row, uint32_t tile, uint32_t tiles, const uint8_t* in,
-                                            uint8_t* const (&out)[COPIES]) {
-    using Row = CuRow<FORM>;
-    if (__builtin_expect(tile >= tiles, 0)) {
-        typename Row::Bytes off;
-        if (tile > tiles || !row.end_element(1u, off)) return;
-        const uint8_t x = as_global(in)[off];
+template <int COPIES, typename FORM, bool WIDE, typename PLACES>
+__device__ __forceinline__ void cu_copy_row(const CuRow<FORM, WIDE>& row, uint32_t tile, uint32_t tiles, const PLACES& at) {
+    using Row = CuRow<FORM, WIDE>;
+    if (__builtin_expect(tile < tiles, 1)) {
+        const uint32_t lane = threadIdx.x * 16u;
+        row.tiles(tile, tiles, [&](typename Row::Offset base, auto count) MINT_INLINE_LAMBDA {
+            constexpr int kCount = decltype(count)::value, kStep = FORM::kThreads * 16;
+            u32x4 x[kCount];
 #pragma unroll
-        for (int i = 0; i < COPIES; ++i) as_global(out[i])[off] = x;
+            for (int k = 0; k < kCount; ++k) x[k] = at.template load<FORM::kStream>(0, base + k * kStep, lane);
+#pragma unroll
+            for (int k = 0; k < kCount; ++k)
+#pragma unroll
+                for (int i = 0; i < COPIES; ++i) at.template store<FORM::kStores>(i, base + k * kStep, lane, x[k]);
+        });
         return;
     }
-    const uint32_t lane = threadIdx.x * 16u;
-    row.tiles(tile, tiles, [&](typename Row::Offset base, auto count) MINT_INLINE_LAMBDA {
-        constexpr int kCount = decltype(count)::value, kStep = FORM::kThreads * 16;
-        u32x4 x[kCount];
+    typename Row::Bytes off;
+    if (tile > tiles || !row.end_element(1u, off)) return;
+    const uint32_t x = at.template load_element<DT_BYTES>(0, off);
 #pragma unroll
-        for (int k = 0; k < kCount; ++k) x[k] = cu_load<FORM::kStream>(in + base + k * kStep, lane);
-#pragma unroll
-        for (int k = 0; k < kCount; ++k)
-#pragma unroll
-            for (int i = 0; i < COPIES; ++i) cu_store<FORM::kStores>(out[i] + base + k * kStep, lane, x[k]);
-    });
+    for (int i = 0; i < COPIES; ++i) at.template store_element<DT_BYTES>(i, off, x);
 }
 
 // Rings that copy: N ranks, the root's row to every other one (broadcast,
@@ -521,24 +648,32 @@ template <int N, typename FORM, bool SPLIT>
 __global__ void __launch_bounds__(FORM::kThreads) cu_ring_copy_kernel(u64x4 numbers, u32x2 counts, const CuTables<N, SPLIT> a) {
     const CuShape s(numbers, counts);
     const CuPlace place(FORM::kLarge, s.part);
-    const uint32_t tile = place.tile, p = place.pipe;
+    const uint32_t p = place.pipe;
     const uint32_t root = s.starts >> (3u * p) & 7u;
-    const uint64_t row_off = (uint64_t)p * s.row_stride;
     constexpr uint32_t kOut = SPLIT ? N : 0;
-    const uint8_t* from[1] = {reinterpret_cast<const uint8_t*>(a.rank[root])};
+    CuByTable<1, N - 1> at;
+    at.row_off = (uint64_t)p * s.row_stride;
+    at.from[0] = reinterpret_cast<const uint8_t*>(a.rank[root]);
     uint8_t* all[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) all[k] = reinterpret_cast<uint8_t*>(a.rank[kOut + k]);
-    cu_here(from);
+    cu_here(at.from);
     cu_here(all);
-    uint8_t* to[N - 1];
 #pragma unroll
-    for (int k = 0; k < N - 1; ++k) to[k] = (uint32_t)k < root ? all[k] : all[k + 1];
-    from[0] += row_off;
-#pragma unroll
-    for (int k = 0; k < N - 1; ++k) to[k] += row_off;
+    for (int k = 0; k < N - 1; ++k) at.to[k] = (uint32_t)k < root ? all[k] : all[k + 1];
+    const CuRow<FORM> row(s.row_bytes, s.short_bytes, s.full, p, at.to[0] + at.row_off, 1u);
     cu_count_if_aborted<FORM::kThreads>(a.status);
-    cu_copy_row<N - 1>(CuRow<FORM>(s.row_bytes, s.short_bytes, s.full, p, to[0], 1u), tile, s.tiles, from[0], to);
+    cu_copy_row<N - 1>(row, place.tile, s.tiles, at);
+}
+template <int N, typename FORM>
+__global__ void __launch_bounds__(FORM::kThreads) cu_near_copy_kernel(u32x8 rows, u32x4 high, u32x2 counts, uint64_t* status) {
+    const CuNear a(rows, high, counts, FORM::kLarge);
+    const CuPlace place(FORM::kLarge, a.part);
+    const uint32_t p = place.pipe;
+    const CuByDistance<N, 1> at(a, a.root(p), p * a.row_stride);
+    const auto row = a.template row<FORM>(p, at.stored(), 1u);
+    cu_count_if_aborted<FORM::kThreads>(status);
+    cu_copy_row<N - 1>(row, place.tile, a.tiles, at);
 }
 
 // The addresses of an alltoall, N to load from and N to store to.  T = uint32_t
@@ -565,10 +700,12 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_alltoall_kernel(u64x4 numbe
     T load = a.rank[source], store = a.rank[kMaxRanks + p];
     asm volatile("" : "+s"(load), "+s"(store));                 // (see cu_here)
     const auto at = [&](T x) MINT_INLINE_LAMBDA { return sizeof(T) == 4 ? lowest + ((uint64_t)x << kCuNearShift) : (uint64_t)x; };
-    const uint8_t* const from = reinterpret_cast<const uint8_t*>(at(load)) + (uint64_t)p * row_stride;
-    uint8_t* const to[1] = {reinterpret_cast<uint8_t*>(at(store)) + (uint64_t)source * row_stride};
+    CuByTable<1, 1> places;
+    places.from[0] = reinterpret_cast<const uint8_t*>(at(load)) + (uint64_t)p * row_stride;
+    places.to[0] = reinterpret_cast<uint8_t*>(at(store)) + (uint64_t)source * row_stride;
+    places.row_off = 0;
     cu_count_if_aborted<FORM::kThreads>(status);
-    cu_copy_row<1>(CuRow<FORM>(row_bytes, 0u, kMaxRanks, p, to[0], 1u), tile, tiles, from, to);
+    cu_copy_row<1>(CuRow<FORM>(row_bytes, 0u, kMaxRanks, p, places.to[0], 1u), tile, tiles, places);
 }
 
 }  // namespace mint

@@ -66,21 +66,25 @@ static_assert(MINT_OP_TREE_BROADCAST == OP_TREE_BROADCAST && MINT_OP_TREE_REDUCE
 // of rows on their way to or from a compute unit keep HBM busy: fewer
 // wavefronts leave it idle, more only scatter its accesses.  Each holds a KiB of
 // N rows to be added, of a row that goes to N - 1 others, or (allreduce) of N rows
-// and then N results.  Fastest counts on MI355X at 0.5 - 2 GiB, f16 and bf16, for
-// N = 2 / 3 / 4 / 5 / 6 / 7 / 8: reduce-scatter 16 - 18 / 14 / 12 / 10 - 11 / 11 - 12 /
-// 10 / 9, allreduce 14 / 9 / 7 - 8 / 6 - 7 / 5 - 6 / 5 / 4 - 5, allgather - / 18 / 16 /
-// 14 / 12 / 10 / 10 and up (4 KiB each: 5 / 4 / 4 for 6 / 7 / 8); one or two off is 1 - 3 % slower, but
-// twice as many 5 - 20 %.  Rows that are copied from the last-level cache arrive sooner:
-// with 7 and 8 ranks, 8 wavefronts instead of 10 are up to 5 % faster where the same buffers
-// are used again (8 ranks, allgather of 24 MiB in all 27.6 / 29.1 us) and within 1 -
-// 2 % either way on others up to 64 MiB; three sets of buffers in turn, 8 ranks, 8 /
-// 10: 64 MiB 72.7 / 73.0, 72 88.1 / 87.7, 80 97.8 / 97.4, 96 125 / 123, 128 178 / 174,
-// 256 358 / 348.
+// and then N results.  One or two off is 1 - 3 % slower, twice as many 5 - 20 %.
+// Launches by distances (CuNear), whose wavefronts are sooner at their loads, over
+// the number that launches by tables want, three sets of buffers in turn (in no cache alike):
+//   sums, one fewer: 4 ranks 0.98 from 530 MiB on (290 1.02, 430 0.99); 5 ranks 1.02 at 290 - 430, 0.99
+//     beyond; 7 ranks 0.985 - 0.99 throughout; 6 and 8 ranks 1.00 - 1.04
+//   copies: 8 ranks, 6 for 8, 0.99; 7 ranks, 5 for 8, 0.97 up to 450 MiB (the same buffers again 0.96);
+//     6 ranks, 9 for 12, 0.99 (0.96), beyond 600 MiB 1.07
+//   allreduce of 8 ranks, 6 for 5: 105 - 130 MiB 0.99 (0.95), 180 and more 1.02; of fewer one off 0.99 - 1.1
+// Copies of seven and eight ranks beyond 72 MiB copied: 10 (72 MiB 88.1 with 8, 87.7 with 10; 128 MiB 178 / 174).
 int cu_waves(int op, int ranks, bool vast, uint64_t copied) {
-    if (op == OP_ALLREDUCE) return (26 + ranks - 1) / ranks + 1;
-    if (reducing(op)) return (24 + ranks - 1) / ranks + 6;
+    const uint64_t touched = copied * (uint64_t)ranks;
+    if (op == OP_ALLREDUCE) return (26 + ranks - 1) / ranks + 1 + (ranks == 8 && touched <= (150ull << 20));
+    if (reducing(op)) {
+        if (ranks == 4) return touched <= (320ull << 20) ? 12 : 11;
+        if (ranks == 5) return touched <= (480ull << 20) ? 11 : 10;
+        return ranks == 6 ? 10 : 24 / ranks + 6;
+    }
     if (vast) return ranks == 6 ? 5 : 4;
-    if (ranks >= 7 && copied <= (72ull << 20)) return 8;
+    if (copied <= (72ull << 20)) return ranks == 8 ? 6 : ranks == 7 ? 5 : ranks == 6 ? 9 : 24 - 2 * ranks;
     return ranks >= 7 ? 10 : 24 - 2 * ranks;
 }
 
@@ -222,6 +226,22 @@ int plan_cu(Plan* plan) {
     if (!choice.large && !choice.pipe_each && cu_by_eighths(touched, ranks, a.pipes, sums, copies)) {
         s.part = (c.blocks + kXcds - 1) / kXcds;
         c.blocks = s.part * kXcds;
+    }
+    // By distances, where the ranks work in place and all rows lie within 4 GiB: not the sums of eight
+    // ranks far beyond the cache, where the nine wavefronts of a compute unit are a little too
+    // many if they are sooner at their loads (0.7 - 2 GiB touched 1.00 - 1.01 of the launch by tables).
+    c.near = false;
+    if (!c.split && !(sums && choice.far && ranks == 8)) {
+        uint64_t highest = 0;
+        c.lowest = ~0ull;
+        for (uint32_t i = 0; i < c.len; ++i) {
+            const uint64_t at = c.input[i] ? c.input[i] : c.output[i];
+            c.lowest = std::min(c.lowest, at);
+            highest = std::max(highest, at);
+        }
+        const uint64_t span = highest - c.lowest + (uint64_t)(a.pipes - 1) * s.row_stride + s.row_bytes;
+        c.near = s.row_stride <= kCuNearSpan && span <= kCuNearSpan && s.row_bytes <= kCuNearRow &&
+                 (choice.large || s.tiles <= kCuNearTiles) && (s.full == c.pipes || s.row_stride == s.row_bytes);
     }
     plan->blocks = (int)c.blocks * a.pipes;
     plan->lds = false;

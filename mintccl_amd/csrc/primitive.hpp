@@ -24,6 +24,7 @@ namespace mint {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint64_t u64x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 enum : int { DT_F16 = 0, DT_BF16 = 1, DT_F32 = 2, DT_BYTES = 3 };

@@ -125,6 +125,99 @@ def added(rows, first):
     return x
 
 
+@pytest.fixture(scope="module")
+def wide(dev):
+    """One allocation of somewhat more than 4 GiB, in which buffers lie wherever a test wants them."""
+    return torch.empty((4 << 30) + (64 << 20), dtype=torch.uint8, device=dev)
+
+
+# span: bytes from the lowest buffer to the end of the last row.  Up to 2^32 - 1 a launch
+# in place names its buffers by their distances, beyond by their addresses.
+@pytest.mark.parametrize("shift", [0, 6])
+@pytest.mark.parametrize("world", range(2, 9))
+def test_buffers_near_and_far(dev, wide, world, shift):
+    """The same collective on buffers that lie together, as far apart as 32 bits reach, and one
+    byte further: the same bytes, those between the buffers included.  The ring is not in the order of the ranks, rows are
+    cut, or have gaps between them, and every rank is the lowest once."""
+    from mintccl_amd import _lib
+    comm = make_comm(world)
+    order = list(range(1, world, 2)) + list(range(0, world, 2))
+    cycle = order + order[:1]
+    row = 4096 + 66                                             # of f16, three tiles, a ragged end
+    room = 64 << 10
+    ops = [("reduce", _lib.OP_REDUCE, dict(root=world - 1)), ("broadcast", _lib.OP_BROADCAST, dict(root=world // 2)),
+           ("allreduce", _lib.OP_ALLREDUCE, {}), ("allgather", _lib.OP_ALLGATHER, dict(row_stride=row)),
+           ("reducescatter", _lib.OP_REDUCESCATTER, dict(row_stride=row)),
+           ("reducescatter, gaps", _lib.OP_REDUCESCATTER, dict(row_stride=row + 190)),
+           ("allgather, cut", _lib.OP_ALLGATHER, dict(row_stride=row, total_bytes=(world - 1) * row - 34)),
+           ("reducescatter, cut", _lib.OP_REDUCESCATTER, dict(row_stride=row, total_bytes=(world - 1) * row - 34)),
+           ("reducescatter, gaps and cut", _lib.OP_REDUCESCATTER, dict(row_stride=row + 190, total_bytes=world * row - 38))]
+    g = torch.Generator(device=dev).manual_seed(world)
+    made = torch.randn((world, room // 2), generator=g, device=dev).to(torch.float16).view(torch.uint8)
+    for i, (name, op, kw) in enumerate(ops):
+        rows = world if "row_stride" in kw else 1
+        need = (rows - 1) * kw.get("row_stride", 0) + row
+        at = [(r + i) % world * room + shift for r in range(world)]           # from the lowest
+        lowest, highest = at.index(min(at)), at.index(max(at))
+        results = []
+        for span in (None, (1 << 32) - 2, 1 << 32):
+            place = list(at)
+            if span is not None:
+                place[highest] = at[lowest] + span - need
+            bufs = [wide[x: x + room - shift] for x in place]
+            for b, m in zip(bufs, made):
+                b.copy_(m[:room - shift])
+            ptrs = {r: b.data_ptr() for r, b in enumerate(bufs)}
+            dtype = _lib.BYTES if op in (_lib.OP_BROADCAST, _lib.OP_ALLGATHER) else _lib.F16
+            comm.enqueue(op, dtype, row, ptrs, ptrs, cycle, **kw)
+            comm.check()
+            results.append([b.clone() for b in bufs])
+        for got in results[1:]:
+            assert all(torch.equal(x, y) for x, y in zip(got, results[0])), name
+        if op == _lib.OP_REDUCESCATTER and "cut" not in name:                # against the additions themselves
+            for r in range(world):
+                part = slice(r * kw["row_stride"], r * kw["row_stride"] + row)
+                want = added([made[q][part].view(torch.float16) for q in order], order.index(r))
+                assert torch.equal(results[0][r][part], want.view(torch.uint8)), (name, r)
+
+
+# MiB touched: in the small form, between, large, far beyond the cache
+@pytest.mark.parametrize("mib", [30, 150, 300, 660])
+@pytest.mark.parametrize("world,dt", [(2, "f32"), (4, "bf16"), (5, "f32"), (6, "f16"), (7, "bf16"), (8, "f16")])
+def test_every_form_near_and_far(dev, wide, world, dt, mib):
+    from mintccl_amd.allreduce import allreduce
+    from mintccl_amd.broadcast import broadcast
+    from mintccl_amd.reduce import reduce
+    dtype = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[dt]
+    comm = make_comm(world)
+    n = (mib << 20) // (world * dtype.itemsize) + 5
+    g = torch.Generator(device=dev).manual_seed(world + mib)
+    made = [torch.randn(n, generator=g, device=dev).to(dtype) for _ in range(world)]
+    nbytes = n * dtype.itemsize
+    step = -(-nbytes // 4096) * 4096 + 16
+    total = wide.numel() - 64
+    summed = added(made, 1)
+    for far in (False, True):
+        places = [r * step for r in range(world - 1)] + [(total - nbytes) // 16 * 16 if far else (world - 1) * step]
+        bufs = [wide[x: x + nbytes].view(dtype) for x in places]
+        for op, want in ((lambda r: reduce(bufs[r], 1, comm), lambda r: summed if r == 1 else made[r]),
+                         (lambda r: broadcast(bufs[r], 1, comm), lambda r: made[1]),
+                         (lambda r: allreduce(bufs[r], comm), None)):
+            for b, m in zip(bufs, made):
+                b.copy_(m)
+            comm.run(op)
+            comm.check()
+            for r in range(world):
+                if want:
+                    assert torch.equal(bufs[r].view(torch.uint8), want(r).view(torch.uint8)), (far, r)
+                elif far or r:
+                    assert torch.equal(bufs[r].view(torch.uint8), same.view(torch.uint8)), (far, r)
+                else:
+                    same = bufs[0].clone()
+    per = (-(-nbytes // world) + 15) // 16 * 16 // dtype.itemsize
+    assert torch.equal(same[:per].view(torch.uint8), added([m[:per] for m in made], 0).view(torch.uint8))
+
+
 # MiB touched (bytes loaded and stored, sums: loaded), elements more than that in every row
 @pytest.mark.parametrize("mib,more", [(1, 5), (8, 1), (11, 3), (19, 3), (21, 0), (21, 3), (25, 9), (31, 2), (33, 3), (41, 7),
                                       (47, 1021), (72, 6), (74, 1), (85, 3), (89, 5), (105, 2051), (158, 9), (170, 9), (178, 3),
