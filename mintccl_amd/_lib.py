@@ -19,6 +19,7 @@ SO_PATH = os.getenv("MINTCCL_LIBRARY") or os.path.join(_PKG, "libmintccl.so")
 _CSRC = os.path.join(_PKG, "csrc")
 SRC = os.path.join(_CSRC, "mintccl.hip")
 CU_SRC = os.path.join(_CSRC, "cu_ring.hip")
+CODEC_SRC = os.path.join(_CSRC, "codec.hip")
 FAMILY_SRC = os.path.join(_CSRC, "ring_family.hip")     # compiled once per element type
 HOST_SRC = os.path.join(_CSRC, "host.cpp")              # the extension module _host
 HOST_PATH = os.path.join(_PKG, "_host.so")
@@ -57,8 +58,8 @@ HIPCC_FLAGS = [
     # refuses a kernel that uses scratch (see there)
     "-Rpass-analysis=kernel-resource-usage",
 ]
-# the first ten words of a launch's arguments (CuShape) arrive in registers
-CU_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=10"]
+# the first 14 words of a launch's arguments, of up to ten arguments, arrive in registers
+PRELOAD_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=10"]
 
 
 class RingOp(ctypes.Structure):
@@ -175,7 +176,7 @@ def host_command(out: str) -> list[str]:
 def build(verbose: bool = False, defines: tuple[str, ...] = (), so_path: str | None = None) -> str:
     """Compile the HIP sources for gfx950 into ``libmintccl.so`` (in-tree).
 
-    The ring kernels are one translation unit per element type; the six
+    The ring kernels are one translation unit per element type; the seven
     compilations run side by side and are linked at the end.  ``defines``
     (``-DMINT_RING_STATS``: wait accounting per ring position,
     ``-DMINT_ROW_NOLOAD``: whole blocks of own rows are not loaded - wrong
@@ -186,7 +187,8 @@ def build(verbose: bool = False, defines: tuple[str, ...] = (), so_path: str | N
     build_dir = BUILD_DIR if so_path is None else out + ".objs"
     os.makedirs(build_dir, exist_ok=True)
     units = [(SRC, list(defines), os.path.join(build_dir, "mintccl.o")),
-             (CU_SRC, [*CU_FLAGS, *defines], os.path.join(build_dir, "cu_ring.o"))]
+             (CU_SRC, [*PRELOAD_FLAGS, *defines], os.path.join(build_dir, "cu_ring.o")),
+             (CODEC_SRC, [*PRELOAD_FLAGS, *defines], os.path.join(build_dir, "codec.o"))]
     for dt in range(4):
         units.append((FAMILY_SRC, [f"-DMINT_FAMILY_DT={dt}", *defines],
                       os.path.join(build_dir, f"ring_family_{dt}.o")))

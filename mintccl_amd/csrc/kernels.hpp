@@ -1,4 +1,4 @@
-// Stand-alone kernels: simple-protocol copy, LL128 codec, element sum,
+// Stand-alone kernels: simple-protocol copy, LL128 codec (pair layout; wave64: codec.hip), element sum,
 // torn-line probe, block -> XCD map.
 #pragma once
 #include "protocol.hpp"
@@ -262,77 +262,6 @@ __global__ void __launch_bounds__(256) step_mix_deep_kernel(const uint8_t* rows,
     }
     if (!(WHAT & 4) && acc.x == 0x9E3779B9u && acc.y == 0x85EBCA6Bu && acc.z == 0xC2B2AE35u)
         sink[0] = acc.w;     // keeps the loads alive; practically never taken
-}
-
-// ---- LL128 codec, wave64 layout: one wavefront per block -------------------
-// Bound by memory from some MiB on.  A wavefront moves one block and ends (the
-// loop is for messages beyond 2^31 threads), so that what is in flight is one
-// window that moves through memory; the lines go through the L2 into the last-level
-// cache for whoever unpacks them, the raw bytes that unpack leaves past it.
-// pack + unpack, resident wavefronts that stride / a wavefront per block and plain
-// stores / this: 16 MiB 14.1 / 13.7 / 13.0 us, 32 MiB 25.6 / 22.8 / 22.2, 48 MiB 36.7 /
-// 34.7 / 32.4, 64 MiB 47.0 / 45.4 / 42.4 (blocks of 256 threads 1 - 3 % slower, of 64 within
-// 1 %); which thread blocks an XCD takes: codec_wave64 in mintccl.hip.
-constexpr uint32_t kCodecThreads = 128;
-// `a`: where from, where to, raw bytes, blocks of the message | part << 32 (CodecWaves);
-// `b`: flag base, flag stride, wavefronts of the launch, the counter of bad flags.  (Two
-// arguments: each costs a launch 10 ns.)
-// The blocks of the message that a wavefront moves: every `waves`-th, or, `part` > 0,
-// one, an XCD `part` thread blocks' worth of consecutive ones (see CuPlace: the
-// hardware deals thread blocks to the eight XCDs in turn).
-struct CodecWaves {
-    uint32_t first, blocks, waves;
-    __device__ __forceinline__ CodecWaves(uint64_t counts, uint64_t all) {
-        const uint32_t part = (uint32_t)(counts >> 32), x = blockIdx.x;
-        const uint32_t at = part ? (x & 7u) * part + (x >> 3) : x;
-        first = __builtin_amdgcn_readfirstlane(at * (kCodecThreads / 64u) + (uint32_t)wave_in_block());
-        blocks = (uint32_t)counts;
-        waves = (uint32_t)all;
-    }
-};
-__global__ void __launch_bounds__(kCodecThreads) pack_wave64_kernel(u64x4 a, u64x4 b) {
-    const uint8_t* const raw = reinterpret_cast<const uint8_t*>(a.x);
-    uint8_t* const msg = reinterpret_cast<uint8_t*>(a.y);
-    const uint64_t nbytes = a.z, flag_base = b.x, flag_stride = b.y;
-    const CodecWaves w(a.w, b.z);
-    const LaneMap m;
-    const uint32_t lane_off = m.flag_lane ? m.raw_off - 4u : m.raw_off;
-    for (uint32_t g = w.first; g < w.blocks; g += w.waves) {
-        const uint64_t base = (uint64_t)g * kBlockRawLL;
-        const bool full = base + kBlockRawLL <= nbytes;
-        u32x4 v = full ? *(MINT_GLOBAL const u32x4_a1*)(as_global(raw + base) + lane_off)
-                       : load_guarded(raw, base + m.raw_off, m.raw_len, nbytes);
-        v = ll_arrange(v, full, m);
-        // line = two sectors; both carry the low 32 bits of the line's flag
-        const uint64_t flag = flag_base + ((uint64_t)g * 8u + (m.sector >> 1)) * flag_stride;
-        if (m.flag_lane) v.w = (uint32_t)flag;
-        st128_through<false>(msg + (uint64_t)g * kBlockMsg, m.lane * 16u, v);
-    }
-}
-__global__ void __launch_bounds__(kCodecThreads) unpack_wave64_kernel(u64x4 a, u64x4 b) {
-    const uint8_t* const msg = reinterpret_cast<const uint8_t*>(a.x);
-    uint8_t* const raw = reinterpret_cast<uint8_t*>(a.y);
-    const uint64_t nbytes = a.z, flag_base = b.x, flag_stride = b.y;
-    unsigned long long* const bad_flags = reinterpret_cast<unsigned long long*>(b.w);
-    const CodecWaves w(a.w, b.z);
-    const LaneMap m;
-    uint32_t bad = 0;
-    for (uint32_t g = w.first; g < w.blocks; g += w.waves) {
-        const u32x4 v = *(MINT_GLOBAL const u32x4*)(as_global(msg + (uint64_t)g * kBlockMsg) + m.lane * 16u);
-        if (bad_flags) {
-            const uint64_t flag = flag_base + ((uint64_t)g * 8u + (m.sector >> 1)) * flag_stride;
-            // a line is bad if either of its two sector tags is (flag lanes 3 and
-            // 7 of every 8); count it once
-            uint64_t wrong = __ballot(m.flag_lane && v.w != (uint32_t)flag);
-            wrong |= wrong << 4;
-            bad += (uint32_t)__popcll(wrong & 0x8080808080808080ull);
-        }
-        const uint64_t base = (uint64_t)g * kBlockRawLL;
-        if (base + kBlockRawLL > nbytes) store_guarded(raw, base + m.raw_off, m.raw_len, nbytes, v);
-        else if (m.flag_lane) st96_through<true>(raw + base, m.raw_off, u32x3{v.x, v.y, v.z});
-        else st128_through<true>(raw + base, m.raw_off, v);
-    }
-    if (bad && lane_id() == 0) atomicAdd(bad_flags, (unsigned long long)bad);
 }
 
 // ---- LL128 codec, reference pair layout: one thread per 16-byte message

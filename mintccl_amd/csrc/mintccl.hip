@@ -635,35 +635,13 @@ int list_schedule(const RingArgs& a, uint32_t raw_per_block, int pipeline, int p
 }  // namespace
 
 namespace {
-// Thread blocks of the codec: one wavefront per block of the message, but no
-// more threads than a launch may have; pair layout: 8 blocks per compute unit.
+// Thread blocks of the codec in pair layout: a thread per 16 bytes of the message, 8 blocks per compute unit.
 constexpr uint32_t kPairThreads = 256;
-uint32_t codec_blocks(uint64_t lines, int layout) {
-    const bool wave64 = layout == MINT_LAYOUT_WAVE64;
-    const uint64_t threads = wave64 ? kCodecThreads : kPairThreads, work = lines * 8;     // (one thread each)
-    const uint64_t cap = wave64 ? (1ull << 31) / threads : (uint64_t)device_cus() * 8;
-    const uint64_t blocks = (work + threads - 1) / threads;
+uint32_t pair_blocks(uint64_t lines) {
+    const uint64_t cap = (uint64_t)device_cus() * 8, blocks = (lines * 8 + kPairThreads - 1) / kPairThreads;
     return (uint32_t)(cap && blocks > cap ? cap : blocks);
 }
 
-// A launch of the wave64 codec.  An XCD takes consecutive thread blocks between the sizes where
-// that is measured to be faster.  pack + unpack, dealt one by one (and with eight launch arguments) / so, us,
-// the same buffers again, three sets in turn, 750 MiB between two uses: 4 MiB 6.4 / 6.1, 6.4 / 6.2, 7.0 / 6.7; 8 MiB 7.4 / 7.2, 8.4 / 8.2, 9.6 /
-// 9.6; 16 MiB 12.2 / 11.0, 12.9 / 12.4, 14.7 / 14.6; 32 MiB 22.1 / 21.2, 22.0 / 21.1, 24.5 / 24.8; 48 MiB 31.1 /
-// 30.3, 32.6 / 32.2, 34.0 / 33.4; 59 MiB 37.4 / 36.5, 39.6 / 38.5, 40.5 / 39.8; at 64 MiB, three sets, 41.2 /
-// 42.1.
-template <auto KERNEL>
-int codec_wave64(const void* from, void* to, uint64_t nbytes, uint64_t lines, uint64_t flag_base, uint64_t flag_stride,
-                 void* bad, void* stream) {
-    uint32_t blocks = codec_blocks(lines, MINT_LAYOUT_WAVE64), part = 0;
-    if (nbytes >= (4ull << 20) && nbytes <= (60ull << 20)) {
-        part = (blocks + kXcds - 1) / kXcds;
-        blocks = part * kXcds;
-    }
-    const u64x4 a = {reinterpret_cast<uint64_t>(from), reinterpret_cast<uint64_t>(to), nbytes, (uint64_t)part << 32 | lines / 8};
-    const u64x4 b = {flag_base, flag_stride, (uint64_t)blocks * (kCodecThreads / 64), reinterpret_cast<uint64_t>(bad)};
-    return Launch<KERNEL>::go(blocks, kCodecThreads, 0, as_stream(stream), a, b);
-}
 }  // namespace
 
 extern "C" {
@@ -856,10 +834,10 @@ int mint_ll128_pack(const void* raw, void* msg, size_t nbytes, uint64_t flag_bas
     const uint64_t lines = mint_ll128_packed_bytes(nbytes, layout) / 128;
     if (lines >= (1ull << 31)) return MINT_ERR_TOO_LARGE;
     if (layout == MINT_LAYOUT_WAVE64)
-        return codec_wave64<&pack_wave64_kernel>(raw, msg, nbytes, lines, flag_base, flag_stride, nullptr, stream);
+        return launch_pack_wave64(raw, msg, nbytes, lines, flag_base, flag_stride, as_stream(stream));
     const uint8_t* from = static_cast<const uint8_t*>(raw);
     uint8_t* to = static_cast<uint8_t*>(msg);
-    return Launch<&pack_pair_kernel>::go(codec_blocks(lines, layout), kPairThreads, 0, as_stream(stream), from, to, nbytes, lines,
+    return Launch<&pack_pair_kernel>::go(pair_blocks(lines), kPairThreads, 0, as_stream(stream), from, to, nbytes, lines,
                                          flag_base, flag_stride);
 }
 
@@ -872,11 +850,11 @@ int mint_ll128_unpack(const void* msg, void* raw, size_t nbytes, uint64_t flag_b
     const uint64_t lines = mint_ll128_packed_bytes(nbytes, layout) / 128;
     if (lines >= (1ull << 31)) return MINT_ERR_TOO_LARGE;
     if (layout == MINT_LAYOUT_WAVE64)
-        return codec_wave64<&unpack_wave64_kernel>(msg, raw, nbytes, lines, flag_base, flag_stride, bad_flags, stream);
+        return launch_unpack_wave64(msg, raw, nbytes, lines, flag_base, flag_stride, bad_flags, as_stream(stream));
     const uint8_t* from = static_cast<const uint8_t*>(msg);
     uint8_t* to = static_cast<uint8_t*>(raw);
     unsigned long long* bad = static_cast<unsigned long long*>(bad_flags);
-    return Launch<&unpack_pair_kernel>::go(codec_blocks(lines, layout), kPairThreads, 0, as_stream(stream), from, to, nbytes, lines,
+    return Launch<&unpack_pair_kernel>::go(pair_blocks(lines), kPairThreads, 0, as_stream(stream), from, to, nbytes, lines,
                                            flag_base, flag_stride, bad);
 }
 

@@ -81,5 +81,10 @@ int launch_ring_family_bf16(const Plan& plan, int protocol, int cache_policy, hi
 int launch_ring_family_f32(const Plan& plan, int protocol, int cache_policy, hipStream_t stream);
 int launch_ring_family_bytes(const Plan& plan, int protocol, int cache_policy, hipStream_t stream);
 int launch_cu_ring(const Plan& plan, int dtype, hipStream_t stream);
+// the codec, wave64 layout (codec.hip): `lines` of the message, whole blocks of eight
+int launch_pack_wave64(const void* raw, void* msg, uint64_t nbytes, uint64_t lines, uint64_t flag_base, uint64_t flag_stride,
+                       hipStream_t stream);
+int launch_unpack_wave64(const void* msg, void* raw, uint64_t nbytes, uint64_t lines, uint64_t flag_base, uint64_t flag_stride,
+                         void* bad_flags, hipStream_t stream);
 
 }  // namespace mint

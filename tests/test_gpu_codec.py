@@ -269,3 +269,45 @@ def test_order_of_the_blocks_changes_nothing(dev, nbytes):
     bad = torch.zeros(1, dtype=torch.int64, device=dev)
     protocol.unpack(msg, back[:nbytes], flag_base=7, flag_stride=3, bad_flags=bad)
     assert torch.equal(back[:nbytes], raw) and torch.all(back[nbytes:] == 0xA5) and bad.item() == 0
+
+
+@pytest.mark.parametrize("nbytes", [1, 959, 960, 961, 2 * 960, 8 * 1920 - 1, 8 * 1920 + 1, (4 << 20) + 1])
+@pytest.mark.parametrize("base,stride", [(2**32 - 3, 1), ((5 << 32) + 9, (3 << 32) + 7)])
+def test_flags_beyond_32_bits(dev, nbytes, base, stride):
+    """A sector's tag is the low half of its line's flag; lines without payload behind the last raw
+    byte have theirs too, and every wrong one is counted."""
+    from mintccl_amd import protocol
+    raw = np.random.default_rng(nbytes).integers(0, 256, nbytes, dtype=np.uint8)
+    msg = protocol.pack(dev_bytes(raw, dev), base, flag_stride=stride)
+    tags = msg.cpu().numpy().view(np.uint32).reshape(-1, 32)[:, [15, 31]]
+    want = (base + stride * np.arange(len(tags), dtype=object)) % 2**32
+    assert (tags == want.astype(np.uint32)[:, None]).all()
+    for flag, wrong in ((base, 0), (base + 1, len(tags))):
+        out = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device=dev)
+        bad = torch.zeros(1, dtype=torch.int64, device=dev)
+        protocol.unpack(msg, out[:nbytes], flag, flag_stride=stride, bad_flags=bad)
+        assert (out.cpu().numpy()[:nbytes] == raw).all() and torch.all(out[nbytes:] == 0xA5) and bad.item() == wrong
+
+
+def test_more_blocks_than_a_launch_has_wavefronts(dev):
+    """2^25 wavefronts and a few blocks more, the last one ragged: 32 GB of raw bytes."""
+    from mintccl_amd import protocol
+    most = 2**25
+    nbytes = (most + 5) * 960 + 7
+    need = protocol.packed_bytes(nbytes)
+    if torch.cuda.mem_get_info(dev)[0] < 2 * nbytes + need + (8 << 30):
+        pytest.skip("not enough memory")
+    g = torch.Generator(device=dev).manual_seed(1)
+    raw = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
+    for at in (0, most * 960 - 5000):                       # around the first and the last wavefronts' blocks
+        raw[at: at + 16 * 960].copy_(torch.randint(0, 256, raw[at: at + 16 * 960].shape, dtype=torch.uint8, generator=g, device=dev))
+    msg = protocol.pack(raw, flag_base=3)
+    for first in (0, most - 8, most):                       # (blocks of 8 lines)
+        piece = protocol.pack(raw[first * 960: (first + 8) * 960].clone(), flag_base=3 + 8 * first)
+        assert torch.equal(msg[first * 1024: first * 1024 + piece.numel()], piece), first
+    raw_end = raw[most * 960 - 100000:].clone()
+    back = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device=dev)
+    bad = torch.zeros(1, dtype=torch.int64, device=dev)
+    protocol.unpack(msg, back[:nbytes], flag_base=3, bad_flags=bad)
+    assert bad.item() == 0 and torch.equal(back[nbytes - raw_end.numel(): nbytes], raw_end)
+    assert torch.equal(back[: 1 << 20], raw[: 1 << 20]) and torch.all(back[nbytes:] == 0xA5)
