@@ -34,13 +34,16 @@ template <typename FORM, auto KERNEL>
 int launch_near(const Plan& plan, hipStream_t stream) {
     const CuRingArgs& a = plan.cu_args;
     const CuShape& s = a.shape;
+    // (one pipeline: from its root on, so that the kernel has nothing to turn)
     uint32_t at[kMaxRanks] = {};
-    for (uint32_t i = 0; i < a.len; ++i) at[i] = (uint32_t)((a.input[i] ? a.input[i] : a.output[i]) - a.lowest);
+    const uint32_t first = a.pipes == 1 ? s.starts : 0u;
+    for (uint32_t i = 0, from = first; i < a.len; ++i, from = from + 1 == a.len ? 0 : from + 1)
+        at[i] = (uint32_t)((a.input[from] ? a.input[from] : a.output[from]) - a.lowest);
     const bool cut = s.full < a.pipes;
     const u32x8 rows = {(uint32_t)a.lowest, (uint32_t)(a.lowest >> 32), (uint32_t)s.row_bytes,
                         (uint32_t)(cut ? s.short_bytes : s.row_stride), at[0], at[1], at[2], at[3]};
     const u32x4 high = {at[4], at[5], at[6], at[7]};
-    const u32x2 counts = {s.starts | s.full << 24 | (cut ? kCuNearCut : 0u), FORM::kLarge ? s.tiles : s.tiles | s.part << 16};
+    const u32x2 counts = {(a.pipes == 1 ? 0u : s.starts) | s.full << 24 | (cut ? kCuNearCut : 0u), FORM::kLarge ? s.tiles : s.tiles | s.part << 16};
     return Launch<KERNEL>::go(grid_of<FORM>(plan, a.pipes, 1), FORM::kThreads, (unsigned)plan.cu_lds, stream, rows, high, counts,
                               a.status);
 }

@@ -528,7 +528,13 @@ struct CuByDistance {
         Ranks x;
 #pragma unroll
         for (int i = 0; i < N; ++i) x[i] = a.rank[i];
-        rank = around(x, root);
+        if (root) {
+            // (a branch: the one row of a reduce or a broadcast is named from its root on.  8 ranks, reduce and
+            // broadcast of 6 - 25 MiB touched 0.98 - 0.99, beyond and allgather 1.00)
+            asm volatile("");
+            x = around(x, root);
+        }
+        rank = x;
     }
     __device__ __forceinline__ const uint8_t* stored() const { return lowest + rank[FIRST] + row_off; }
     template <bool STREAM>
