@@ -30,29 +30,46 @@ int launch_as(const Plan& plan, hipStream_t stream) {
                               u32x2{s.tiles, s.part}, tables);
 }
 
-template <typename FORM, auto KERNEL>
+// use(what follows the rows and four words among the arguments of a launch by distances)
+template <int N, typename USE>
+int cu_near_more(const USE& use) {
+    if constexpr (N <= 4) return use();
+    else if constexpr (N <= 6) return use((uint64_t*)nullptr);
+    else return use(u32x2{}, (uint64_t*)nullptr);
+}
+template <typename FORM, int N, auto KERNEL>
 int launch_near(const Plan& plan, hipStream_t stream) {
     const CuRingArgs& a = plan.cu_args;
     const CuShape& s = a.shape;
+    const dim3 grid = grid_of<FORM>(plan, a.pipes, 1);
     // (one pipeline: from its root on, so that the kernel has nothing to turn)
-    uint32_t at[kMaxRanks] = {};
-    const uint32_t first = a.pipes == 1 ? s.starts : 0u;
-    for (uint32_t i = 0, from = first; i < a.len; ++i, from = from + 1 == a.len ? 0 : from + 1)
+    const bool one = a.pipes == 1;
+    uint32_t at[kMaxRanks] = {}, from = one ? s.starts : 0u;
+    for (int i = 0; i < N; ++i) {
         at[i] = (uint32_t)((a.input[from] ? a.input[from] : a.output[from]) - a.lowest);
+        from = from + 1 == N ? 0 : from + 1;
+    }
     const bool cut = s.full < a.pipes;
     const u32x8 rows = {(uint32_t)a.lowest, (uint32_t)(a.lowest >> 32), (uint32_t)s.row_bytes,
                         (uint32_t)(cut ? s.short_bytes : s.row_stride), at[0], at[1], at[2], at[3]};
-    const u32x4 high = {at[4], at[5], at[6], at[7]};
-    const u32x2 counts = {(a.pipes == 1 ? 0u : s.starts) | s.full << 24 | (cut ? kCuNearCut : 0u), FORM::kLarge ? s.tiles : s.tiles | s.part << 16};
-    return Launch<KERNEL>::go(grid_of<FORM>(plan, a.pipes, 1), FORM::kThreads, (unsigned)plan.cu_lds, stream, rows, high, counts,
-                              a.status);
+    const u32x2 counts = {(one ? 0u : s.starts) | s.full << 24 | (cut ? kCuNearCut : 0u), FORM::kLarge ? s.tiles : s.tiles | s.part << 16};
+    const auto go = [&](const auto&... words) {
+        return Launch<KERNEL>::go(grid, FORM::kThreads, (unsigned)plan.cu_lds, stream, rows, words...);
+    };
+    const uint64_t status = reinterpret_cast<uint64_t>(a.status);
+    if constexpr (N <= 4) return go(u32x4{counts.x, counts.y, (uint32_t)status, (uint32_t)(status >> 32)});
+    else if constexpr (N <= 6) return go(u32x4{at[4], at[5], counts.x, counts.y}, a.status);
+    else return go(u32x4{at[4], at[5], at[6], at[7]}, counts, a.status);
 }
 
 template <int DT, int N, bool EVERYWHERE>
 int launch_sum(const Plan& plan, hipStream_t stream) {
     return cu_sum_form<N, EVERYWHERE>(plan.cu_choice, [&](auto form) {
         using Form = typename decltype(form)::type;
-        if (plan.cu_args.near) return launch_near<Form, &cu_near_sum_kernel<DT, N, EVERYWHERE, Form>>(plan, stream);
+        if (plan.cu_args.near)
+            return cu_near_more<N>([&](auto... more) {
+                return launch_near<Form, N, &cu_near_sum_kernel<DT, N, EVERYWHERE, Form, decltype(more)...>>(plan, stream);
+            });
         if constexpr (decltype(form)::in_place)
             if (!plan.cu_args.split)
                 return launch_as<Form, &cu_ring_sum_kernel<DT, N, EVERYWHERE, Form, false>, N, false>(plan, stream);
@@ -63,7 +80,10 @@ template <int N>
 int launch_copy(const Plan& plan, hipStream_t stream) {
     return cu_copy_form<N>(plan.cu_choice, [&](auto form) {
         using Form = typename decltype(form)::type;
-        if (plan.cu_args.near) return launch_near<Form, &cu_near_copy_kernel<N, Form>>(plan, stream);
+        if (plan.cu_args.near)
+            return cu_near_more<N>([&](auto... more) {
+                return launch_near<Form, N, &cu_near_copy_kernel<N, Form, decltype(more)...>>(plan, stream);
+            });
         if constexpr (decltype(form)::in_place)
             if (!plan.cu_args.split) return launch_as<Form, &cu_ring_copy_kernel<N, Form, false>, N, false>(plan, stream);
         return launch_as<Form, &cu_ring_copy_kernel<N, Form, true>, N, true>(plan, stream);

@@ -83,8 +83,12 @@ static_assert(sizeof(CuShape) + sizeof(CuTables<kMaxRanks, false>) <= 112, "argu
 //   rows    lowest address (two words), row_bytes, row_stride; where rows are cut (kCuNearCut),
 //           which follow each other without gaps then, short_bytes in its place; distances of
 //           ranks 0 - 3
-//   high    those of ranks 4 - 7
+//   high    those of the ranks from 4 on
 //   counts  starts | full << 24 | kCuNearCut, tiles | part << 16 (large form: tiles)
+//   status
+// Each argument costs a launch 10 ns, so what follows the rows shares one where it fits
+// (cu_near_more): up to four ranks {counts, status}; five and six {high, counts}, status; seven
+// and eight high, counts, status.
 constexpr uint32_t kCuNearCut = 1u << 31;
 // At most: bytes from the lowest address to the end of the last row, of a row (offsets have a
 // sign), tiles of a row in the small form.
@@ -379,11 +383,16 @@ struct CuNear {
     uint32_t row_bytes, row_stride, short_bytes;
     u32x8 rank;
     uint32_t starts, full, tiles, part;
-    __device__ __forceinline__ CuNear(u32x8 rows, u32x4 high, u32x2 counts, bool large)
+    uint64_t* status;
+    __device__ __forceinline__ CuNear(bool large, u32x8 rows, u32x4 high, u32x2 counts, uint64_t* status_)
         : lowest(reinterpret_cast<uint8_t*>((uint64_t)rows[1] << 32 | rows[0])), row_bytes(rows[2]),
           row_stride(counts.x & kCuNearCut ? rows[2] : rows[3]), short_bytes(rows[3]),
           rank{rows[4], rows[5], rows[6], rows[7], high.x, high.y, high.z, high.w}, starts(counts.x),
-          full(counts.x >> 24 & 15u), tiles(large ? counts.y : counts.y & kCuNearTiles), part(large ? 0u : counts.y >> 16) {}
+          full(counts.x >> 24 & 15u), tiles(large ? counts.y : counts.y & kCuNearTiles), part(large ? 0u : counts.y >> 16), status(status_) {}
+    __device__ __forceinline__ CuNear(bool large, u32x8 rows, u32x4 words, uint64_t* status_)
+        : CuNear(large, rows, u32x4{words.x, words.y, 0u, 0u}, u32x2{words.z, words.w}, status_) {}
+    __device__ __forceinline__ CuNear(bool large, u32x8 rows, u32x4 words)
+        : CuNear(large, rows, u32x4{}, u32x2{words.x, words.y}, reinterpret_cast<uint64_t*>((uint64_t)words.w << 32 | words.z)) {}
     __device__ __forceinline__ uint32_t root(uint32_t p) const { return starts >> (3u * p) & 7u; }
     template <typename FORM>
     __device__ __forceinline__ CuRow<FORM, false> row(uint32_t p, const uint8_t* stored, uint32_t size) const {
@@ -612,14 +621,14 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_ring_sum_kernel(u64x4 numbe
     cu_count_if_aborted<FORM::kThreads>(a.status);
     cu_sum_row<DT, N, kStored>(row, tile, s.tiles, at);
 }
-template <int DT, int N, bool EVERYWHERE, typename FORM>
-__global__ void __launch_bounds__(FORM::kThreads) cu_near_sum_kernel(u32x8 rows, u32x4 high, u32x2 counts, uint64_t* status) {
-    const CuNear a(rows, high, counts, FORM::kLarge);
+template <int DT, int N, bool EVERYWHERE, typename FORM, typename... MORE>
+__global__ void __launch_bounds__(FORM::kThreads) cu_near_sum_kernel(u32x8 rows, u32x4 words, MORE... more) {
+    const CuNear a(FORM::kLarge, rows, words, more...);
     const CuPlace place(FORM::kLarge, a.part);
     const uint32_t p = place.pipe;
     const CuByDistance<N, 0> at(a, a.root(p), p * a.row_stride);
     const auto row = a.template row<FORM>(p, at.stored(), DT == DT_F32 ? 4u : 2u);
-    cu_count_if_aborted<FORM::kThreads>(status);
+    cu_count_if_aborted<FORM::kThreads>(a.status);
     cu_sum_row<DT, N, EVERYWHERE ? N : 1>(row, place.tile, a.tiles, at);
 }
 
@@ -671,14 +680,14 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_ring_copy_kernel(u64x4 numb
     cu_count_if_aborted<FORM::kThreads>(a.status);
     cu_copy_row<N - 1>(row, place.tile, s.tiles, at);
 }
-template <int N, typename FORM>
-__global__ void __launch_bounds__(FORM::kThreads) cu_near_copy_kernel(u32x8 rows, u32x4 high, u32x2 counts, uint64_t* status) {
-    const CuNear a(rows, high, counts, FORM::kLarge);
+template <int N, typename FORM, typename... MORE>
+__global__ void __launch_bounds__(FORM::kThreads) cu_near_copy_kernel(u32x8 rows, u32x4 words, MORE... more) {
+    const CuNear a(FORM::kLarge, rows, words, more...);
     const CuPlace place(FORM::kLarge, a.part);
     const uint32_t p = place.pipe;
     const CuByDistance<N, 1> at(a, a.root(p), p * a.row_stride);
     const auto row = a.template row<FORM>(p, at.stored(), 1u);
-    cu_count_if_aborted<FORM::kThreads>(status);
+    cu_count_if_aborted<FORM::kThreads>(a.status);
     cu_copy_row<N - 1>(row, place.tile, a.tiles, at);
 }
 

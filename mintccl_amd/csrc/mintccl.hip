@@ -181,20 +181,24 @@ int plan_cu(Plan* plan) {
     c.split = alltoall;
     c.status = a.status;
     uint64_t stored = 0;           // what the stored rows' addresses have in their low bits
+    uint64_t highest = 0;          // of the ranks' addresses where they work in place
+    c.lowest = ~0ull;
+    const auto rank_at = [&](int i, uint64_t input, uint64_t output) {
+        c.input[i] = input;
+        c.output[i] = output;
+        stored |= output;
+        const uint64_t at = input ? input : output;
+        c.split |= output && at != output;
+        c.lowest = std::min(c.lowest, at);
+        highest = std::max(highest, at);
+    };
     if (a.op == OP_SENDRECV) {
         // a route: only its ends touch the caller's buffers
-        c.input[0] = a.input[a.cyc[0]];
-        c.output[0] = c.input[1] = 0;
-        stored = c.output[1] = a.output[a.cyc[a.cyc_len - 1]];
+        rank_at(0, a.input[a.cyc[0]], 0);
+        rank_at(1, 0, a.output[a.cyc[a.cyc_len - 1]]);
     } else {
-        for (int i = 0; i < a.cyc_len; ++i) {
-            // (alltoall names ranks, not places on a ring)
-            const int rank = alltoall ? i : a.cyc[i];
-            c.input[i] = a.input[rank];
-            c.output[i] = a.output[rank];
-            c.split |= a.input[rank] && a.output[rank] && a.input[rank] != a.output[rank];
-            stored |= a.output[rank];
-        }
+        // (alltoall names ranks, not places on a ring)
+        for (int i = 0; i < a.cyc_len; ++i) rank_at(i, a.input[alltoall ? i : a.cyc[i]], a.output[alltoall ? i : a.cyc[i]]);
     }
     CuShape& s = c.shape;
     s.starts = 0;
@@ -232,13 +236,6 @@ int plan_cu(Plan* plan) {
     // many if they are sooner at their loads (0.7 - 2 GiB touched 1.00 - 1.01 of the launch by tables).
     c.near = false;
     if (!c.split && !(sums && choice.far && ranks == 8)) {
-        uint64_t highest = 0;
-        c.lowest = ~0ull;
-        for (uint32_t i = 0; i < c.len; ++i) {
-            const uint64_t at = c.input[i] ? c.input[i] : c.output[i];
-            c.lowest = std::min(c.lowest, at);
-            highest = std::max(highest, at);
-        }
         const uint64_t span = highest - c.lowest + (uint64_t)(a.pipes - 1) * s.row_stride + s.row_bytes;
         c.near = s.row_stride <= kCuNearSpan && span <= kCuNearSpan && s.row_bytes <= kCuNearRow &&
                  (choice.large || s.tiles <= kCuNearTiles) && (s.full == c.pipes || s.row_stride == s.row_bytes);
@@ -312,6 +309,7 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
 
     // ring / route
     bool seen[MINT_MAX_RANKS] = {};
+    uint8_t index_of[MINT_MAX_RANKS] = {};
     if (op->op == MINT_OP_SENDRECV) {
         if (op->route_len < 1 || op->route_len > op->world) return MINT_ERR_ARG;
         a.cyc_len = op->route_len;
@@ -326,11 +324,8 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
         if (r < 0 || r >= op->world || seen[r]) return MINT_ERR_ARG;
         seen[r] = true;
         a.cyc[i] = (uint8_t)r;
+        index_of[r] = (uint8_t)i;
     }
-    auto index_of = [&](int rank) {
-        for (int i = 0; i < a.cyc_len; ++i) if (a.cyc[i] == rank) return i;
-        return -1;
-    };
     switch (op->op) {
         case MINT_OP_SENDRECV:  a.hops = a.cyc_len - 1; a.start[0] = 0; break;
         case MINT_OP_BROADCAST:
@@ -340,7 +335,7 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
             if (op->root < 0 || op->root >= op->world) return MINT_ERR_ARG;
             // (a tree has one position per node)
             a.hops = op->op == MINT_OP_REDUCE ? op->world : op->world - 1;
-            a.start[0] = (uint8_t)index_of(op->root);
+            a.start[0] = index_of[op->root];
             break;
         }
         case MINT_OP_ALLTOALL: a.hops = 1; break;
@@ -348,7 +343,7 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
             a.hops = op->op == MINT_OP_ALLGATHER || temporal || hyper ? op->world - 1
                      : allreduce                             ? 2 * op->world - 2
                                                              : op->world;
-            for (int p = 0; p < op->world; ++p) a.start[p] = (uint8_t)index_of(p);
+            for (int p = 0; p < op->world; ++p) a.start[p] = index_of[p];
     }
 
     const int dt_size = op->dtype == MINT_F32 ? 4 : (op->dtype == MINT_BYTES ? 1 : 2);
