@@ -580,9 +580,12 @@ __device__ __forceinline__ void cu_sum_row(const CuRow<FORM, WIDE>& row, uint32_
                 for (int h = 0; h < N; ++h) v[k][h] = at.template load<FORM::kStream>(h, base + k * kStep, lane);
 #pragma unroll
             for (int k = 0; k < kCount; ++k) {
-                u32x4 x = v[k][0];
+                // (three ranks of bf16 in the large form, 300 MiB touched: 60.9 us, with the shorter additions
+                // 62.9; 500 MiB and more 0.99 - 1.00)
+                Sum<DT, FORM::kLarge && N == 3 && STORED == 1> sum(v[k][0]);
 #pragma unroll
-                for (int h = 1; h < N; ++h) x = ll_comp<DT>(v[k][h], x);
+                for (int h = 1; h < N; ++h) sum.add(v[k][h]);
+                const u32x4 x = sum.value();
 #pragma unroll
                 for (int i = 0; i < STORED; ++i) at.template store<FORM::kStores>(i, base + k * kStep, lane, x);
             }

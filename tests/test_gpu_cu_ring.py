@@ -125,6 +125,30 @@ def added(rows, first):
     return x
 
 
+@pytest.mark.parametrize("world", [2, 3, 8])
+def test_every_bf16_pattern_in_a_sum(dev, world):
+    """Each of the 65536 patterns on the first, the second and the last rank that is added, the
+    others with zeros, subnormals, the largest values, infinities and NaNs of every kind: bit for bit, a
+    NaN as the canonical one, wherever on the ring it came in."""
+    from mintccl_amd.allreduce import allreduce
+    from mintccl_amd.reduce import reduce
+    comm = make_comm(world)
+    special = np.array([0x0000, 0x8000, 0x0001, 0x807F, 0x3F80, 0xBF80, 0x7F7F, 0xFF7F, 0x7F80, 0xFF80, 0x7F81, 0xFF81,
+                        0x7FBF, 0x7FC0, 0xFFC0, 0x7FFF, 0xFFFF], dtype=np.uint16)
+    for at in sorted({0, 1, world - 1}):
+        pick = np.random.default_rng(world + at)
+        host = [pick.choice(special, 65536) if pick.random() < 0.7 or r == (at + 1) % world
+                else (pick.standard_normal(65536).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16) for r in range(world)]
+        host[at] = np.arange(65536, dtype=np.uint16)
+        for op, want in ((lambda b: reduce(b, 0, comm), ring.reduce(host, 0, "bf16")[:1]),
+                         (lambda b: allreduce(b, comm), ring.allreduce(host, "bf16"))):
+            bufs = [torch.from_numpy(h.view(np.int16).copy()).to(dev).view(torch.bfloat16) for h in host]
+            comm.run(lambda r: op(bufs[r]))
+            comm.check()
+            for r, w in enumerate(want):
+                assert np.array_equal(as_bytes(bufs[r]), w.view(np.uint8)), (at, r)
+
+
 @pytest.fixture(scope="module")
 def wide(dev):
     """One allocation of somewhat more than 4 GiB, in which buffers lie wherever a test wants them."""
