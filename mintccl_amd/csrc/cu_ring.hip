@@ -52,7 +52,7 @@ int launch_near(const Plan& plan, hipStream_t stream) {
     const bool cut = s.full < a.pipes;
     const u32x8 rows = {(uint32_t)a.lowest, (uint32_t)(a.lowest >> 32), (uint32_t)s.row_bytes,
                         (uint32_t)(cut ? s.short_bytes : s.row_stride), at[0], at[1], at[2], at[3]};
-    const u32x2 counts = {(one ? 0u : s.starts) | s.full << 24 | (cut ? kCuNearCut : 0u), FORM::kLarge ? s.tiles : s.tiles | s.part << 16};
+    const u32x2 counts = {(one ? 0u : s.starts) | s.full << 24 | (cut ? kCuNearCut : 0u), s.tiles | s.part << cu_near_part_bit(FORM::kLarge)};
     const auto go = [&](const auto&... words) {
         return Launch<KERNEL>::go(grid, FORM::kThreads, (unsigned)plan.cu_lds, stream, rows, words...);
     };

@@ -46,7 +46,8 @@ struct CuShape {
     uint32_t starts;               // bits 3 p: index in the ring of pipeline p's root
     uint32_t full;                 // rows before this one have row_bytes
     uint32_t tiles;                // thread blocks that share the whole vectors of a row
-    uint32_t part;                 // small form: tiles of a row that one XCD takes, or 0 (CuPlace)
+    uint32_t part;                 // small form: tiles of a row that one XCD takes, or 0 (CuPlace);
+                                   // large form: cu_pause of a wavefront before it stores
 
     CuShape() = default;
     __device__ __forceinline__ CuShape(u64x4 numbers, u32x2 counts)
@@ -84,7 +85,7 @@ static_assert(sizeof(CuShape) + sizeof(CuTables<kMaxRanks, false>) <= 112, "argu
 //           which follow each other without gaps then, short_bytes in its place; distances of
 //           ranks 0 - 3
 //   high    those of the ranks from 4 on
-//   counts  starts | full << 24 | kCuNearCut, tiles | part << 16 (large form: tiles)
+//   counts  starts | full << 24 | kCuNearCut, tiles | part << 16 (large form: << 24)
 //   status
 // Each argument costs a launch 10 ns, so what follows the rows shares one where it fits
 // (cu_near_more): up to four ranks {counts, status}; five and six {high, counts}, status; seven
@@ -94,6 +95,8 @@ constexpr uint32_t kCuNearCut = 1u << 31;
 // sign), tiles of a row in the small form.
 constexpr uint64_t kCuNearSpan = 0xffffffffull, kCuNearRow = 1ull << 30;
 constexpr uint32_t kCuNearTiles = 0xffff;
+constexpr uint32_t cu_near_part_bit(bool large) { return large ? 24u : 16u; }
+static_assert(kCuNearRow / 1024 + 1 < 1u << cu_near_part_bit(true), "tiles of a KiB in the large form");
 
 // (host side: the whole of a launch)
 struct CuRingArgs {
@@ -388,7 +391,8 @@ struct CuNear {
         : lowest(reinterpret_cast<uint8_t*>((uint64_t)rows[1] << 32 | rows[0])), row_bytes(rows[2]),
           row_stride(counts.x & kCuNearCut ? rows[2] : rows[3]), short_bytes(rows[3]),
           rank{rows[4], rows[5], rows[6], rows[7], high.x, high.y, high.z, high.w}, starts(counts.x),
-          full(counts.x >> 24 & 15u), tiles(large ? counts.y : counts.y & kCuNearTiles), part(large ? 0u : counts.y >> 16), status(status_) {}
+          full(counts.x >> 24 & 15u), tiles(counts.y & ((1u << cu_near_part_bit(large)) - 1u)), part(counts.y >> cu_near_part_bit(large)),
+          status(status_) {}
     __device__ __forceinline__ CuNear(bool large, u32x8 rows, u32x4 words, uint64_t* status_)
         : CuNear(large, rows, u32x4{words.x, words.y, 0u, 0u}, u32x2{words.z, words.w}, status_) {}
     __device__ __forceinline__ CuNear(bool large, u32x8 rows, u32x4 words)
@@ -564,10 +568,17 @@ struct CuByDistance {
     }
 };
 
+// A wavefront of the large form that has its rows waits `times` 256 clocks before it stores
+// (cu_pauses in mintccl.hip: how often, and what it is worth).
+__device__ __forceinline__ void cu_pause(uint32_t times, u32x4& arrived) {
+#pragma unroll 1
+    for (; times; --times) asm volatile("s_sleep 4" : "+v"(arrived));
+}
+
 // Rings that add: N ranks, the sum goes to the root of the pipeline (reduce,
 // reduce-scatter) or to all of them (allreduce): to STORED places.
 template <int DT, int N, int STORED, typename FORM, bool WIDE, typename PLACES>
-__device__ __forceinline__ void cu_sum_row(const CuRow<FORM, WIDE>& row, uint32_t tile, uint32_t tiles, const PLACES& at) {
+__device__ __forceinline__ void cu_sum_row(const CuRow<FORM, WIDE>& row, uint32_t tile, uint32_t tiles, uint32_t pauses, const PLACES& at) {
     using Row = CuRow<FORM, WIDE>;
     if (__builtin_expect(tile < tiles, 1)) {
         const uint32_t lane = threadIdx.x * 16u;
@@ -581,11 +592,12 @@ __device__ __forceinline__ void cu_sum_row(const CuRow<FORM, WIDE>& row, uint32_
 #pragma unroll
             for (int k = 0; k < kCount; ++k) {
                 // (three ranks of bf16 in the large form, 300 MiB touched: 60.9 us, with the shorter additions
-                // 62.9; 500 MiB and more 0.99 - 1.00)
+                // 62.9, and no wait (cu_pause) in their place brings it back; 500 MiB and more 0.99 - 1.00)
                 Sum<DT, FORM::kLarge && N == 3 && STORED == 1> sum(v[k][0]);
 #pragma unroll
                 for (int h = 1; h < N; ++h) sum.add(v[k][h]);
-                const u32x4 x = sum.value();
+                u32x4 x = sum.value();
+                if constexpr (FORM::kLarge) cu_pause(pauses, x);
 #pragma unroll
                 for (int i = 0; i < STORED; ++i) at.template store<FORM::kStores>(i, base + k * kStep, lane, x);
             }
@@ -622,7 +634,7 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_ring_sum_kernel(u64x4 numbe
     else at.to[0] = const_cast<uint8_t*>(at.from[0]);
     const CuRow<FORM> row(s.row_bytes, s.short_bytes, s.full, p, at.to[0] + at.row_off, kSize);
     cu_count_if_aborted<FORM::kThreads>(a.status);
-    cu_sum_row<DT, N, kStored>(row, tile, s.tiles, at);
+    cu_sum_row<DT, N, kStored>(row, tile, s.tiles, s.part, at);
 }
 template <int DT, int N, bool EVERYWHERE, typename FORM, typename... MORE>
 __global__ void __launch_bounds__(FORM::kThreads) cu_near_sum_kernel(u32x8 rows, u32x4 words, MORE... more) {
@@ -632,12 +644,12 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_near_sum_kernel(u32x8 rows,
     const CuByDistance<N, 0> at(a, a.root(p), p * a.row_stride);
     const auto row = a.template row<FORM>(p, at.stored(), DT == DT_F32 ? 4u : 2u);
     cu_count_if_aborted<FORM::kThreads>(a.status);
-    cu_sum_row<DT, N, EVERYWHERE ? N : 1>(row, place.tile, a.tiles, at);
+    cu_sum_row<DT, N, EVERYWHERE ? N : 1>(row, place.tile, a.tiles, a.part, at);
 }
 
 // A row from one place to COPIES others.
 template <int COPIES, typename FORM, bool WIDE, typename PLACES>
-__device__ __forceinline__ void cu_copy_row(const CuRow<FORM, WIDE>& row, uint32_t tile, uint32_t tiles, const PLACES& at) {
+__device__ __forceinline__ void cu_copy_row(const CuRow<FORM, WIDE>& row, uint32_t tile, uint32_t tiles, uint32_t pauses, const PLACES& at) {
     using Row = CuRow<FORM, WIDE>;
     if (__builtin_expect(tile < tiles, 1)) {
         const uint32_t lane = threadIdx.x * 16u;
@@ -646,6 +658,7 @@ __device__ __forceinline__ void cu_copy_row(const CuRow<FORM, WIDE>& row, uint32
             u32x4 x[kCount];
 #pragma unroll
             for (int k = 0; k < kCount; ++k) x[k] = at.template load<FORM::kStream>(0, base + k * kStep, lane);
+            if constexpr (FORM::kLarge && COPIES == 1) cu_pause(pauses, x[0]);
 #pragma unroll
             for (int k = 0; k < kCount; ++k)
 #pragma unroll
@@ -681,7 +694,7 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_ring_copy_kernel(u64x4 numb
     for (int k = 0; k < N - 1; ++k) at.to[k] = (uint32_t)k < root ? all[k] : all[k + 1];
     const CuRow<FORM> row(s.row_bytes, s.short_bytes, s.full, p, at.to[0] + at.row_off, 1u);
     cu_count_if_aborted<FORM::kThreads>(a.status);
-    cu_copy_row<N - 1>(row, place.tile, s.tiles, at);
+    cu_copy_row<N - 1>(row, place.tile, s.tiles, s.part, at);
 }
 template <int N, typename FORM, typename... MORE>
 __global__ void __launch_bounds__(FORM::kThreads) cu_near_copy_kernel(u32x8 rows, u32x4 words, MORE... more) {
@@ -691,7 +704,7 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_near_copy_kernel(u32x8 rows
     const CuByDistance<N, 1> at(a, a.root(p), p * a.row_stride);
     const auto row = a.template row<FORM>(p, at.stored(), 1u);
     cu_count_if_aborted<FORM::kThreads>(a.status);
-    cu_copy_row<N - 1>(row, place.tile, a.tiles, at);
+    cu_copy_row<N - 1>(row, place.tile, a.tiles, a.part, at);
 }
 
 // The addresses of an alltoall, N to load from and N to store to.  T = uint32_t
@@ -723,7 +736,7 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_alltoall_kernel(u64x4 numbe
     places.to[0] = reinterpret_cast<uint8_t*>(at(store)) + (uint64_t)source * row_stride;
     places.row_off = 0;
     cu_count_if_aborted<FORM::kThreads>(status);
-    cu_copy_row<1>(CuRow<FORM>(row_bytes, 0u, kMaxRanks, p, places.to[0], 1u), tile, tiles, places);
+    cu_copy_row<1>(CuRow<FORM>(row_bytes, 0u, kMaxRanks, p, places.to[0], 1u), tile, tiles, part, places);
 }
 
 }  // namespace mint

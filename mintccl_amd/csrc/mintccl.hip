@@ -73,12 +73,13 @@ static_assert(MINT_OP_TREE_BROADCAST == OP_TREE_BROADCAST && MINT_OP_TREE_REDUCE
 //     beyond; 7 ranks 0.985 - 0.99 throughout; 6 and 8 ranks 1.00 - 1.04
 //   copies: 8 ranks, 6 for 8, 0.99; 7 ranks, 5 for 8, 0.97 up to 450 MiB (the same buffers again 0.96);
 //     6 ranks, 9 for 12, 0.99 (0.96), beyond 600 MiB 1.07
-//   allreduce of 8 ranks, 6 for 5: 105 - 130 MiB 0.99 (0.95), 180 and more 1.02; of fewer one off 0.99 - 1.1
+//   (a sum of two ranks, 20 for 18, and an allreduce of four, 9 for 8, by cu_pauses: see there)
 // Copies of seven and eight ranks beyond 72 MiB copied: 10 (72 MiB 88.1 with 8, 87.7 with 10; 128 MiB 178 / 174).
-int cu_waves(int op, int ranks, bool vast, uint64_t copied) {
+int cu_waves(int op, int dtype, int ranks, bool vast, uint64_t copied) {
     const uint64_t touched = copied * (uint64_t)ranks;
-    if (op == OP_ALLREDUCE) return (26 + ranks - 1) / ranks + 1 + (ranks == 8 && touched <= (150ull << 20));
+    if (op == OP_ALLREDUCE) return (26 + ranks - 1) / ranks + 1 + (ranks == 4 && dtype != MINT_BF16);
     if (reducing(op)) {
+        if (ranks == 2) return 20;
         if (ranks == 4) return touched <= (320ull << 20) ? 12 : 11;
         if (ranks == 5) return touched <= (480ull << 20) ? 11 : 10;
         return ranks == 6 ? 10 : 24 / ranks + 6;
@@ -86,6 +87,48 @@ int cu_waves(int op, int ranks, bool vast, uint64_t copied) {
     if (vast) return ranks == 6 ? 5 : 4;
     if (copied <= (72ull << 20)) return ranks == 8 ? 6 : ranks == 7 ? 5 : ranks == 6 ? 9 : 24 - 2 * ranks;
     return ranks >= 7 ? 10 : 24 - 2 * ranks;
+}
+
+// Times 256 clocks that a wavefront of the large form, its rows there and added, waits
+// before it stores (cu_pause).  It is the spread of the accesses that this holds down, like a wavefront less on
+// the compute unit does (cu_waves) but in smaller steps, and the stores: as far as can be told, HBM loses time where
+// they come one by one between the loads.  Additions of bf16, which are conversions too, are a part of the wait.  Time over
+// that without, in thousandths, f16 and f32 / bf16, reduce-scatter and reduce, up to 200 MiB the same buffers again
+// and three sets in turn, beyond three sets:
+//   touched MiB       180 - 200          300          500 - 700         1000            2000
+//   2 ranks (20 wf.)      -           968 / 987      965 / 988       968 / 978       971 / 985
+//   3                     -           971 / -        976 / -         976 / -         967 / -
+//   4                     -           957 / -        981 / -         988 / -         956 / -
+//   5                938 - 972 / 987  963 / 991      973 / 992       979 / 986       976 / 988
+//   6                961 - 984 / 993  973 / 984      977 / 990       995 / 1003      993 / 997
+//   7                962 - 989 / 992  981 / 1000     982 / 993      1004 / 1005     1013 / 1006
+//   8                990 - 1037 / 1010  984 / 1000   977 / 980       976 / 975      1003 / 996
+// Two more are 1 - 5 % slower.  Allreduce, geometric means of 110 - 1000 MiB on 15 sets of buffers (largest): 8 ranks (five
+// wavefronts throughout) 989 (1002) / 986 (1006), 7 ranks 997 (1004) / 1000, 6 ranks 996 (1001) / 1000, 5 ranks 994
+// (1004) / 1000, 4 ranks (nine wavefronts) 992 (1003) / 999; 2 and 3 ranks lose by it.
+// One copy: sendrecv 954 - 997 from 200 MiB on, alltoall 1000 - 1009 at 200 - 300, 991 at 1000, 985 at 2000.
+// Several copies of a row lose 3 % and more: their stores are most of what there is.
+uint32_t cu_pauses(int op, int dtype, int ranks, uint64_t touched) {
+    const auto upto = [&](uint64_t mib) { return touched <= mib << 20; };
+    const bool bf16 = dtype == MINT_BF16;
+    if (op == OP_ALLREDUCE) {
+        if (ranks == 8) return bf16 ? 3 : 4;
+        if (ranks == 7) return bf16 && !upto(150) ? 0 : 2;
+        return ranks < 4 || bf16 ? 0 : ranks == 4 ? 3 : 2;
+    }
+    if (reducing(op)) {
+        switch (ranks) {
+            case 8: return bf16 ? (upto(400) ? 0 : 3) : upto(240) || !upto(1500) ? 0 : 4;
+            case 7: return upto(160) || !upto(800) ? 0 : bf16 ? 1 : 3;
+            case 6:
+            case 5: return bf16 ? 1 : 3;
+            case 4:
+            case 3: return bf16 ? 0 : 2;
+            default: return 3;
+        }
+    }
+    if (op == OP_ALLTOALL) return upto(400) ? 0 : 2;
+    return ranks == 2 ? 2 : 0;
 }
 
 // MiB touched beyond which the last-level cache (256 MiB) would not hold the rows from one
@@ -129,7 +172,7 @@ bool cu_by_eighths(uint64_t touched, int ranks, int pipes, bool sums, bool copie
 }
 
 // The grid of a launch inside compute units: a thread block per tile of a row.
-int plan_cu(Plan* plan) {
+int plan_cu(Plan* plan, int dtype) {
     const RingArgs& a = plan->args;
     const bool sums = reducing(a.op), alltoall = a.op == OP_ALLTOALL;
     const bool copies = (a.op == OP_BROADCAST || a.op == OP_ALLGATHER) && a.cyc_len > 2;
@@ -170,7 +213,7 @@ int plan_cu(Plan* plan) {
     // out in units of 1280 bytes)
     plan->cu_lds = 0;
     if ((choice.large && (sums || copies)) || choice.mid) {
-        const int waves = choice.mid ? (ranks <= 4 ? 32 : 14) : cu_waves(a.op, ranks, choice.far, (uint64_t)a.pipes * a.row_bytes);
+        const int waves = choice.mid ? (ranks <= 4 ? 32 : 14) : cu_waves(a.op, dtype, ranks, choice.far, (uint64_t)a.pipes * a.row_bytes);
         const int blocks = waves / (plan->threads / 64);
         if (blocks * (plan->threads / 64) < 32) plan->cu_lds = (160 << 10) / blocks / 1280 * 1280;
     }
@@ -231,6 +274,7 @@ int plan_cu(Plan* plan) {
         s.part = (c.blocks + kXcds - 1) / kXcds;
         c.blocks = s.part * kXcds;
     }
+    if (choice.large) s.part = cu_pauses(a.op, dtype, ranks, touched);
     // By distances, where the ranks work in place and all rows lie within 4 GiB: not the sums of eight
     // ranks far beyond the cache, where the nine wavefronts of a compute unit are a little too
     // many if they are sooner at their loads (0.7 - 2 GiB touched 1.00 - 1.01 of the launch by tables).
@@ -433,7 +477,7 @@ int make_plan(const mint_ring_op* op, Plan* plan, bool for_launch = false,
     plan->cu = cu;
     if (cu) {
         if (dbg && (dbg->skip_origin || dbg->stats)) return MINT_ERR_ARG;
-        return plan_cu(plan);
+        return plan_cu(plan, op->dtype);
     }
 
     // geometry

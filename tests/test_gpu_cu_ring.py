@@ -299,6 +299,35 @@ def test_every_form(dev, world, dt, mib, more):
     same(outs, [torch.stack([made[q][r] for q in range(world)]) for r in range(world)], "alltoall")
 
 
+@pytest.mark.parametrize("world,mib", [(2, 402), (5, 398), (5, 402), (8, 402)])
+def test_a_row_to_one_place_far_beyond_the_cache(dev, world, mib):
+    """Both sides of where the wavefronts of an alltoall wait before they store, and a transfer
+    between two ranks, which wait throughout: rows that end in the middle of a vector."""
+    from mintccl_amd import sendrecv_buffer
+    from mintccl_amd.alltoall import alltoall
+    comm = make_comm(world)
+    n = (mib << 20) // (2 * world * world) + 1029
+    g = torch.Generator(device=dev).manual_seed(world + mib)
+    bufs = [torch.randint(0, 256, (world, n), dtype=torch.uint8, generator=g, device=dev) for _ in range(world)]
+    taken = [torch.full((world * n + 64,), 0x5A, dtype=torch.uint8, device=dev) for _ in range(world)]
+    outs = [t[32: 32 + world * n].view(world, n) for t in taken]
+    comm.run(lambda r: alltoall(bufs[r], outs[r], comm))
+    comm.check()
+    for r in range(world):
+        assert torch.equal(outs[r], torch.stack([b[r] for b in bufs])), r
+        assert torch.all(taken[r][:32] == 0x5A) and torch.all(taken[r][32 + world * n:] == 0x5A), r
+    sent = torch.cat([b.view(-1) for b in bufs])[: (mib << 19) + 1029]
+    backing = torch.full((sent.numel() + 64,), 0x5A, dtype=torch.uint8, device=dev)
+    with comm.rank(0):
+        sendrecv_buffer.send(sent, 1, comm)
+    with comm.rank(1):
+        sendrecv_buffer.recv(backing[32: 32 + sent.numel()], 0, comm)
+    comm.run(lambda r: sendrecv_buffer.sync(comm))
+    comm.check()
+    assert torch.equal(backing[32: 32 + sent.numel()], sent)
+    assert torch.all(backing[:32] == 0x5A) and torch.all(backing[32 + sent.numel():] == 0x5A)
+
+
 @pytest.mark.parametrize("world,mib", [(6, 1284), (7, 704), (8, 2564)])
 def test_copies_far_beyond_the_cache(dev, world, mib):
     """Just beyond where a wavefront moves 4 KiB, rows that end in the middle of such a
