@@ -182,19 +182,21 @@ constexpr CuBand cu_through_mib(bool sums, int ranks, int pipes, bool pipe_each)
 constexpr int kCuStreamRanks = 6;
 // Sums to one place of two to six ranks, rows up to cu_mid_mib touched: the places of
 // the small form, rows streamed past the last-level cache, results left in it (the rows
-// of three sets of buffers are beyond it, their results are not).  Over the large form with its waits
-// (cu_pauses), reduce and reduce-scatter of f16 and bf16, the same buffers again / three sets in turn / 700 MiB
+// of three sets of buffers are beyond it, their results are not).  Over the large form,
+// reduce and reduce-scatter in three types, the same buffers again / three sets in turn / 700 MiB
 // between two uses:
-//   touched MiB     110              130              150              180              200 - 210
-//   2 ranks          -                -        0.98 / 0.97 / 1.04  0.98 / 0.96 / 1.04  0.97 / 1.06 / 1.05
-//   3                -                -        0.96 / 0.96 / 1.03  1.01 / 0.98 / 1.02  0.97 / 0.97 / 1.05
-//   4                -        0.92 / 1.00 / 1.00  0.99 / 1.01 / 1.02  1.04 / 1.02 / 1.02  1.07 / 1.03 / 1.04
-//   5        0.96 / 0.99 / 0.99  0.96 / 1.00 / 1.00  0.97 / 1.00 / 1.01  (170 MiB 1.04 / 1.03 / 1.02)
-//   6        0.97 / 1.03 / 1.02  0.94 / 1.02 / 1.02  1.00 / 1.03 / 1.03  (155 MiB 1.03 / 1.04 / 1.04)
-// (3 ranks at 240 - 270 MiB 0.98 / 0.99 / 1.06; 7 and 8 ranks 0.92 - 1.10 without the waits.  5 and 6 ranks in
-// blocks of 64 threads, 14 wavefronts on a compute unit.)
+//   touched MiB   100 - 130           130 - 160           160 - 176           176 - 196           196 - 208
+//   2 ranks  0.89 / 0.92 / 0.99  0.91 / 0.92 / 1.00  0.92 / 0.91 / 1.00  0.91 / 0.93 / 0.99  0.92 / 1.00 / 1.01
+//   3        0.87 / 0.87 / 0.97  0.88 / 0.88 / 1.00  0.90 / 0.89 / 1.03  0.89 / 0.88 / 1.03  0.88 / 0.88 / 1.04
+//   4        0.84 / 0.92 / 0.93  0.90 / 0.95 / 0.97  0.96 / 0.96 / 0.98  0.97 / 0.97 / 1.00  0.98 / 0.97 / 0.99
+//   5        0.89 / 0.93 / 0.93  0.91 / 0.96 / 0.96  0.97 / 0.97 / 0.97    (180 MiB, three sets 1.01)
+//   6        0.89 / 0.95 / 0.95  0.90 / 0.97 / 0.97  0.97 / 1.01 / 1.00, a reduce at 171 MiB 1.10 in each
+// (3 ranks at 235 - 264 MiB 0.89 / 0.91 / 1.04; 4 ranks at 270 MiB, three sets, f16 0.95, bf16 1.02; 7 and 8
+// ranks 0.92 - 1.10.  5 and 6 ranks in blocks of 64 threads, 14 wavefronts on a compute unit.)
 constexpr int kCuMidRanks = 6;
-constexpr int cu_mid_mib(int ranks) { return ranks == 2 ? 196 : ranks == 3 ? 264 : ranks <= 5 ? 150 : 144; }
+constexpr int cu_mid_mib(int ranks) {
+    return ranks == 2 ? 196 : ranks == 3 ? 264 : ranks == 4 ? 208 : ranks == 5 ? 176 : 160;
+}
 
 // Rows of six and more ranks to several places (VAST below) from so many MiB touched
 // on.  Over the large form at 0.9 / 1.5 / 3 / 4 GiB touched, three sets of buffers in turn:
