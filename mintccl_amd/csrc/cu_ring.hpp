@@ -193,6 +193,8 @@ constexpr int kCuStreamRanks = 6;
 //   6        0.89 / 0.95 / 0.95  0.90 / 0.97 / 0.97  0.97 / 1.01 / 1.00, a reduce at 171 MiB 1.10 in each
 // (3 ranks at 235 - 264 MiB 0.89 / 0.91 / 1.04; 4 ranks at 270 MiB, three sets, f16 0.95, bf16 1.02; 7 and 8
 // ranks 0.92 - 1.10.  5 and 6 ranks in blocks of 64 threads, 14 wavefronts on a compute unit.)
+// Since the large form's wavefronts wait before they store (cu_pauses) it is ahead by 1 - 4 % from 150 MiB on with 4
+// and 5 ranks and from 144 on with 6 (the same buffers again up to 9 % behind at 125 - 140 MiB).
 constexpr int kCuMidRanks = 6;
 constexpr int cu_mid_mib(int ranks) {
     return ranks == 2 ? 196 : ranks == 3 ? 264 : ranks == 4 ? 208 : ranks == 5 ? 176 : 160;

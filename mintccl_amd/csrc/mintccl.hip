@@ -82,6 +82,9 @@ int cu_waves(int op, int dtype, int ranks, bool vast, uint64_t copied) {
         if (ranks == 2) return 20;
         if (ranks == 4) return touched <= (320ull << 20) ? 12 : 11;
         if (ranks == 5) return touched <= (480ull << 20) ? 11 : 10;
+        // (7 ranks, 10 for 9, the same buffers again / three sets in turn / 700 MiB between two uses: 104 MiB 0.97 / 0.985 / 0.985,
+        // 130 MiB 0.975 / 0.995 / 0.995, 150 MiB 0.98 / 0.995 / 0.995, 180 MiB 0.985 / 1.005 / 1.01)
+        if (ranks == 7 && touched <= (160ull << 20)) return 10;
         return ranks == 6 ? 10 : 24 / ranks + 6;
     }
     if (vast) return ranks == 6 ? 5 : 4;
