@@ -92,6 +92,22 @@ int cu_waves(int op, int dtype, int ranks, bool vast, uint64_t copied) {
     return ranks >= 7 ? 10 : 24 - 2 * ranks;
 }
 
+// ... and of the small form of an allreduce, which stores as many rows as it loads, once it touches about as much as the L2s hold.
+// Over all 32, f16 and bf16, the same buffers again / three sets in turn / 700 MiB between two uses:
+//   touched MiB        26                 36                 48                 60                 72                 98
+//   2 ranks, 20  0.97 / 0.97 / 0.97  0.98 / 0.98 / 0.96  0.99 / 0.99 / 0.97  0.99 / 0.99 / 0.96  0.99 / 0.99 / 0.97  0.99 / 0.99 / 0.97
+//   3, 16        0.98 / 0.98 / 0.98  1.00 / 1.00 / 0.99  0.99 / 0.99 / 0.98  1.00 / 0.99 / 0.97  0.99 / 0.99 / 0.97  0.98 / 0.97 / 0.97
+//   4, 12        0.99 / 0.98 / 0.97  0.97 / 0.97 / 0.99  0.98 / 0.98 / 0.97  0.98 / 0.98 / 0.98  0.98 / 0.98 / 0.98  0.98 / 0.99 / 0.97
+//   5, 8         0.98 / 0.98 / 0.97  0.98 / 0.97 / 0.98  0.98 / 0.98 / 0.97  0.98 / 0.97 / 0.97  0.98 / 0.98 / 0.97  0.98 / 1.00 / 0.98
+//   6, 8         1.01 / 1.01 / 0.99  0.98 / 0.98 / 0.99  0.98 / 0.98 / 0.98  0.98 / 0.98 / 0.98  0.98 / 0.98 / 0.99  0.98 / 1.00 / 0.99
+//   7, 8         1.00 / 0.99 / 1.00  0.99 / 0.99 / 0.98  0.99 / 0.99 / 0.98  0.99 / 0.99 / 0.98  0.99 / 0.96 / 0.99  1.00 / 1.00 / 0.99
+// (3 and 4 ranks of bf16 at 25 MiB 1.01 - 1.03 / 1.00 - 1.01 / 0.98.)  Up to 20 MiB as fast or slower; 8 ranks 1.00 - 1.05. Sums to one place 1.00 - 1.1, copies 0.96 - 1.08 by their size.
+int cu_small_waves(int op, int ranks, uint64_t touched) {
+    const uint64_t least = ranks == 2 || ranks == 5 ? 24 : ranks <= 4 ? 28 : 32;
+    if (op != OP_ALLREDUCE || ranks == 8 || touched < least << 20) return 32;
+    return ranks == 2 ? 20 : ranks == 3 ? 16 : ranks == 4 ? 12 : 8;
+}
+
 // Times 256 clocks that a wavefront of the large form, its rows there and added, waits
 // before it stores (cu_pause).  It is the spread of the accesses that this holds down, like a wavefront less on
 // the compute unit does (cu_waves) but in smaller steps, and the stores: as far as can be told, HBM loses time where
@@ -215,11 +231,11 @@ int plan_cu(Plan* plan, int dtype) {
     // (held to that number by the share of LDS its blocks ask for; LDS is handed
     // out in units of 1280 bytes)
     plan->cu_lds = 0;
-    if ((choice.large && (sums || copies)) || choice.mid) {
-        const int waves = choice.mid ? (ranks <= 4 ? 32 : 14) : cu_waves(a.op, dtype, ranks, choice.far, (uint64_t)a.pipes * a.row_bytes);
-        const int blocks = waves / (plan->threads / 64);
-        if (blocks * (plan->threads / 64) < 32) plan->cu_lds = (160 << 10) / blocks / 1280 * 1280;
-    }
+    const int waves = choice.mid       ? (ranks <= 4 ? 32 : 14)
+                      : !choice.large  ? cu_small_waves(a.op, ranks, touched)
+                      : sums || copies ? cu_waves(a.op, dtype, ranks, choice.far, (uint64_t)a.pipes * a.row_bytes)
+                                       : 32;
+    if (waves < 32) plan->cu_lds = (160 << 10) / (waves * 64 / plan->threads) / 1280 * 1280;
     CuRingArgs& c = plan->cu_args;
     c.op = (uint32_t)a.op;
     c.pipes = (uint32_t)a.pipes;
