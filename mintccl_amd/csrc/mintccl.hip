@@ -72,7 +72,8 @@ static_assert(MINT_OP_TREE_BROADCAST == OP_TREE_BROADCAST && MINT_OP_TREE_REDUCE
 //   sums, one fewer: 4 ranks 0.98 from 530 MiB on (290 1.02, 430 0.99); 5 ranks 1.02 at 290 - 430, 0.99
 //     beyond; 7 ranks 0.985 - 0.99 throughout; 6 and 8 ranks 1.00 - 1.04
 //   copies: 8 ranks, 6 for 8, 0.99; 7 ranks, 5 for 8, 0.97 up to 450 MiB (the same buffers again 0.96);
-//     6 ranks, 9 for 12, 0.99 (0.96), beyond 600 MiB 1.07
+//     6 ranks, 9 for 12, 0.99 (0.96), beyond 600 MiB 1.07, 8 for 9 0.995 (0.98); 5 ranks, 8 for 14, 90 - 150 MiB 0.985
+//     (0.92), 250 - 350 MiB 0.98 (0.99), 450 and more 1.16
 //   (a sum of two ranks, 20 for 18, and an allreduce of four, 9 for 8, by cu_pauses: see there)
 // Copies of seven and eight ranks beyond 72 MiB copied: 10 (72 MiB 88.1 with 8, 87.7 with 10; 128 MiB 178 / 174).
 int cu_waves(int op, int dtype, int ranks, bool vast, uint64_t copied) {
@@ -88,8 +89,16 @@ int cu_waves(int op, int dtype, int ranks, bool vast, uint64_t copied) {
         return ranks == 6 ? 10 : 24 / ranks + 6;
     }
     if (vast) return ranks == 6 ? 5 : 4;
-    if (copied <= (72ull << 20)) return ranks == 8 ? 6 : ranks == 7 ? 5 : ranks == 6 ? 9 : 24 - 2 * ranks;
+    if (copied <= (72ull << 20)) return ranks == 8 ? 6 : ranks == 7 ? 5 : ranks >= 5 ? 8 : 24 - 2 * ranks;
     return ranks >= 7 ? 10 : 24 - 2 * ranks;
+}
+
+// ... of the form between.  4 ranks, over 32, the same buffers again / three sets in turn / 700 MiB between two uses: 105 - 125 MiB 18
+// 1.00 / 0.985 / 0.98 (16: 1.02 / 0.975 / 0.975), 150 MiB 22 0.99 / 0.995 / 0.99 (18: 1.03 / 0.99 / 0.99), 170 - 205 MiB 16
+// 0.975 / 0.97 / 0.97 (18: 0.99); 2 ranks 24 1.02 - 1.05; 3 ranks 24 0.99 - 1.00.  5 and 6 ranks: kCuMidRanks.
+int cu_mid_waves(int ranks, uint64_t touched) {
+    if (ranks == 4) return touched <= (130ull << 20) ? 18 : touched <= (165ull << 20) ? 22 : 16;
+    return ranks < 4 ? 32 : 14;
 }
 
 // ... and of the small form of an allreduce, which stores as many rows as it loads, once it touches about as much as the L2s hold.
@@ -231,7 +240,7 @@ int plan_cu(Plan* plan, int dtype) {
     // (held to that number by the share of LDS its blocks ask for; LDS is handed
     // out in units of 1280 bytes)
     plan->cu_lds = 0;
-    const int waves = choice.mid       ? (ranks <= 4 ? 32 : 14)
+    const int waves = choice.mid       ? cu_mid_waves(ranks, touched)
                       : !choice.large  ? cu_small_waves(a.op, ranks, touched)
                       : sums || copies ? cu_waves(a.op, dtype, ranks, choice.far, (uint64_t)a.pipes * a.row_bytes)
                                        : 32;
