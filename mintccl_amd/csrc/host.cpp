@@ -55,11 +55,16 @@ PyObject* checked(int code, const char* where) {
 }
 
 // The current device is `device` for as long as this lives (a launch goes to
-// the current device's context).
+// the current device's context).  Where there is only one it is that: nothing to
+// ask (53 ns, a small collective takes 4 us and the codec's two calls 6).
 struct OnDevice {
     int before, device;
-    explicit OnDevice(int d) : before(c10::hip::current_device()), device(d) {
+    explicit OnDevice(int d) : before(only() ? d : (int)c10::hip::current_device()), device(d) {
         if (before != device) c10::hip::set_device((c10::DeviceIndex)device);
+    }
+    static bool only() {
+        static const bool one = c10::hip::device_count() == 1;
+        return one;
     }
     ~OnDevice() {
         if (before != device) c10::hip::set_device((c10::DeviceIndex)before);
