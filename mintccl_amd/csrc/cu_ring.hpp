@@ -13,7 +13,7 @@
 // once; there is no staging, no epoch, no seat to claim and nobody to wait for,
 // and both protocols (which say how a hop is made safe) are the same.
 //
-// Bound by HBM (6.4 - 6.8 TB/s of rows read and written).  A thread block moves
+// Bound by HBM (6.4 - 7.0 TB/s of rows read and written).  A thread block moves
 // one tile and ends, and the tiles of a pipeline follow each other in the order
 // the blocks are dealt: what is in flight over the device is one window of
 // consecutive bytes per row that moves through memory.  Wavefronts that stay
