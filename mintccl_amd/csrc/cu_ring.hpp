@@ -721,24 +721,51 @@ constexpr int kCuNearShift = 8;
 static_assert(5 * 8 + sizeof(CuPairs<uint32_t>) <= 112, "arguments of an alltoall's launch");
 
 // Row `destination` of the source goes to row `source` of the destination.
+template <typename FORM>
+__device__ __forceinline__ void cu_alltoall_row(uint64_t from, uint64_t to, uint64_t row_bytes, uint64_t row_stride, uint32_t tiles,
+                                                uint32_t part, const CuPlace& place, uint64_t* status) {
+    CuByTable<1, 1> places;
+    places.from[0] = reinterpret_cast<const uint8_t*>(from) + (uint64_t)place.pipe * row_stride;
+    places.to[0] = reinterpret_cast<uint8_t*>(to) + (uint64_t)blockIdx.z * row_stride;
+    places.row_off = 0;
+    cu_count_if_aborted<FORM::kThreads>(status);
+    cu_copy_row<1>(CuRow<FORM>(row_bytes, 0u, kMaxRanks, place.pipe, places.to[0], 1u), place.tile, tiles, part, places);
+}
 // `numbers`: row_bytes, row_stride, the lowest address, the status block.
 template <typename FORM, typename T>
 __global__ void __launch_bounds__(FORM::kThreads) cu_alltoall_kernel(u64x4 numbers, u32x2 counts, const CuPairs<T> a) {
-    const uint64_t row_bytes = numbers.x, row_stride = numbers.y, lowest = numbers.z;
-    uint64_t* const status = reinterpret_cast<uint64_t*>(numbers.w);
-    const uint32_t tiles = counts.x, part = counts.y;
-    const CuPlace place(FORM::kLarge, part);
-    const uint32_t tile = place.tile, p = place.pipe;
-    const uint32_t source = blockIdx.z;
-    T load = a.rank[source], store = a.rank[kMaxRanks + p];
+    const uint64_t lowest = numbers.z;
+    const CuPlace place(FORM::kLarge, counts.y);
+    T load = a.rank[blockIdx.z], store = a.rank[kMaxRanks + place.pipe];
     asm volatile("" : "+s"(load), "+s"(store));                 // (see cu_here)
     const auto at = [&](T x) MINT_INLINE_LAMBDA { return sizeof(T) == 4 ? lowest + ((uint64_t)x << kCuNearShift) : (uint64_t)x; };
-    CuByTable<1, 1> places;
-    places.from[0] = reinterpret_cast<const uint8_t*>(at(load)) + (uint64_t)p * row_stride;
-    places.to[0] = reinterpret_cast<uint8_t*>(at(store)) + (uint64_t)source * row_stride;
-    places.row_off = 0;
-    cu_count_if_aborted<FORM::kThreads>(status);
-    cu_copy_row<1>(CuRow<FORM>(row_bytes, 0u, kMaxRanks, p, places.to[0], 1u), tile, tiles, part, places);
+    cu_alltoall_row<FORM>(at(load), at(store), numbers.x, numbers.y, counts.x, counts.y, place, reinterpret_cast<uint64_t*>(numbers.w));
+}
+// Up to four ranks, whose rows follow each other without gaps: all that the loads wait for in the
+// 14 words that come in registers (CuNear); the selects of a block's two distances take no longer than one to a
+// table's entry. Over tables, the same buffers again / three sets in turn:
+//   touched MiB      20             30             45             64             90            150
+//   2 ranks     0.985 / 0.99   0.97 / 0.97    1.02 / 0.99    0.98 / 0.985   0.98 / 0.98   0.99 / 0.99
+//   3           0.98 / 0.97    0.99 / 0.96    0.95 / 0.97    0.97 / 0.98    0.98 / 0.98   0.99 / 0.99
+//   4           0.99 / 0.98    0.95 / 0.95    0.98 / 0.975   0.97 / 0.99    0.98 / 0.98   0.99 / 0.99
+// (4 ranks of 30 MiB, three sets, 5.50 -> 5.24 us, 6.0 TB/s; 64 MiB 10.27 -> 10.18; 90 MiB 13.9 -> 13.6), below the host's 3.4 us and
+// from 200 MiB on 1.00.  More ranks: 16 distances of 20 bits, in halves and fours, fit as well, but finding two of them takes
+// about what the table does (5 and 6 ranks 0.98 - 1.02, 7 and 8 ranks 0.98 - 1.01).
+//   rows    lowest address (two words), row_bytes, tiles | part << cu_near_part_bit; what ranks 0 - 3 load from
+//   stored  what they store to
+constexpr uint32_t kCuNearPairs = 4;
+template <typename FORM>
+__global__ void __launch_bounds__(FORM::kThreads) cu_near_alltoall_kernel(u32x8 rows, u32x4 stored, uint64_t* status) {
+    constexpr uint32_t kBit = cu_near_part_bit(FORM::kLarge);
+    const uint64_t lowest = (uint64_t)rows[1] << 32 | rows[0];
+    const uint32_t tiles = rows[3] & ((1u << kBit) - 1u), part = rows[3] >> kBit;
+    const CuPlace place(FORM::kLarge, part);
+    const auto at = [&](uint32_t r, uint32_t a, uint32_t b, uint32_t c, uint32_t d) MINT_INLINE_LAMBDA {
+        const uint32_t low = r & 1u ? b : a, high = r & 1u ? d : c;
+        return lowest + ((uint64_t)(r & 2u ? high : low) << kCuNearShift);
+    };
+    cu_alltoall_row<FORM>(at(blockIdx.z, rows[4], rows[5], rows[6], rows[7]), at(place.pipe, stored.x, stored.y, stored.z, stored.w),
+                          rows[2], rows[2], tiles, part, place, status);
 }
 
 }  // namespace mint

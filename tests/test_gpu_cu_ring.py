@@ -205,6 +205,42 @@ def test_buffers_near_and_far(dev, wide, world, shift):
                 assert torch.equal(results[0][r][part], want.view(torch.uint8)), (name, r)
 
 
+# row: one tile and less, ragged, an eighth of the row to each XCD, in the large form
+@pytest.mark.parametrize("row", [2, 2048, 3 * 2048 + 50, (1 << 20) + 16, (1 << 20) + 18, (7 << 20) + 6])
+@pytest.mark.parametrize("world", [2, 3, 4, 5])
+def test_alltoall_by_distances_and_by_addresses(dev, wide, world, row):
+    """An alltoall of up to four ranks names its buffers by their distances in units of 256 bytes, others by
+    tables of distances or of addresses: whole units apart (in three orders, as far apart as the
+    allocation lets them), 16 and 6 bytes off a unit, and with gaps between the rows, the same bytes and nothing beside them."""
+    from mintccl_amd import _lib
+    comm = make_comm(world)
+    g = torch.Generator(device=dev).manual_seed(world + row)
+    cycle = list(range(world)) + [0]
+    for turn, far, shift, gap in [(0, False, 0, 0), (1, True, 0, 0), (world, False, 0, 0), (0, True, 16, 0), (1, False, 6, 0),
+                                  (0, False, 0, 190)]:
+        step = -(-(world * (row + gap) + 64) // 256) * 256
+        # inputs and outputs by turns around each other; the last of them far away
+        at = [(i + turn) % (2 * world) * step + shift * (i % 2) for i in range(2 * world)]
+        if far:
+            at[at.index(max(at))] += (wide.numel() - 2 * world * step) // 256 * 256 - 256
+        views = [wide[x: x + world * (row + gap) + 32] for x in at]
+        for v in views:
+            v.fill_(0x5A)
+        made = torch.randint(0, 256, (world, world, row), dtype=torch.uint8, generator=g, device=dev)
+        rows = [v[: world * (row + gap)].view(world, row + gap) for v in views]
+        for r in range(world):
+            rows[r][:, :row] = made[r]
+        ins = {r: views[r].data_ptr() for r in range(world)}
+        outs = {r: views[world + r].data_ptr() for r in range(world)}
+        comm.enqueue(_lib.OP_ALLTOALL, _lib.BYTES, row, ins, outs, cycle, row_stride=row + gap)
+        comm.check()
+        for r in range(world):
+            assert torch.equal(rows[world + r][:, :row], made[:, r]), (turn, far, shift, gap, r)
+            assert torch.equal(rows[r][:, :row], made[r])
+        for v, x in zip(views, rows):
+            assert torch.all(v[world * (row + gap):] == 0x5A) and torch.all(x[:, row:] == 0x5A)
+
+
 # MiB touched: in the small form, between, large, far beyond the cache
 @pytest.mark.parametrize("mib", [30, 150, 300, 660])
 @pytest.mark.parametrize("world,dt", [(2, "f32"), (4, "bf16"), (5, "f32"), (6, "f16"), (7, "bf16"), (8, "f16")])
