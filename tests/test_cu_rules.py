@@ -1,0 +1,62 @@
+"""The rules that say how many wavefronts of a launch inside compute units a compute unit
+holds (csrc/cu_rules.hpp), compiled by the host's compiler alone."""
+import os
+import subprocess
+
+import pytest
+
+from mintccl_amd import _lib
+
+CSRC = os.path.join(os.path.dirname(_lib.__file__), "csrc")
+OPS = {"broadcast": _lib.OP_BROADCAST, "allgather": _lib.OP_ALLGATHER, "reduce": _lib.OP_REDUCE,
+       "reducescatter": _lib.OP_REDUCESCATTER, "allreduce": _lib.OP_ALLREDUCE}
+TYPES = {"f16": _lib.F16, "bf16": _lib.BF16, "f32": _lib.F32, "bytes": _lib.BYTES}
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    """rule(expression) -> its value as a whole number."""
+    where = tmp_path_factory.mktemp("rules")
+    known = {}
+
+    def evaluate(*expressions):
+        new = [e for e in expressions if e not in known]
+        if new:
+            source, program = str(where / "rules.cpp"), str(where / "rules")
+            with open(source, "w") as f:
+                f.write('#include "cu_rules.hpp"\n#include <cstdio>\nusing namespace mint;\nint main() {\n')
+                f.writelines(f'    printf("%lld\\n", (long long)({e}));\n' for e in new)
+                f.write("}\n")
+            subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, source, "-o", program], check=True)
+            known.update(zip(new, map(int, subprocess.check_output([program]).split())))
+        return [known[e] for e in expressions]
+    return evaluate
+
+
+def waves(op, dtype, ranks, mib, vast=False):
+    """The large form's count for `mib` MiB touched."""
+    return f"cu_waves({OPS[op]}, {TYPES[dtype]}, {ranks}, {str(vast).lower()}, {(mib << 20) // ranks}ull)"
+
+
+def test_a_block_at_least(rule):
+    """However few wavefronts a rule names, a compute unit holds a block of them, and no less LDS
+    than that leaves is asked for."""
+    lds, unit = rule("kCuLds", "kCuLdsUnit")
+    cases = [(w, t) for t in (64, 128, 256) for w in range(1, 33)]
+    for (w, t), share in zip(cases, rule(*(f"cu_lds_share({w}, {t})" for w, t in cases))):
+        blocks = max(1, w * 64 // t)
+        if w == 32:
+            assert share == 0
+        else:
+            assert share % unit == 0 and share * blocks <= lds < (share + unit) * blocks, (w, t, share)
+
+
+def test_every_rule_names_whole_blocks(rule):
+    """No form has more than two wavefronts to a block."""
+    sizes = (1, 20, 24, 25, 28, 30, 32, 40, 90, 101, 129, 131, 150, 164, 166, 210, 300, 330, 470, 490, 700, 3000)
+    asked = [e for r in range(2, 9) for m in sizes for e in (
+        [waves(op, dt, r, m) for op in ("reduce", "reducescatter", "allreduce") for dt in ("f16", "bf16", "f32")] +
+        [waves(op, "bytes", r, m, vast) for op in ("broadcast", "allgather") for vast in (False, True)] +
+        [f"cu_mid_waves({r}, {m << 20}ull)"] + [f"cu_small_waves({op}, {r}, {m << 20}ull)" for op in OPS.values()])]
+    for e, value in zip(asked, rule(*asked)):
+        assert 2 <= value <= 32, e
