@@ -30,11 +30,18 @@ constexpr bool cu_adds(int op) { return op == MINT_OP_REDUCE || op == MINT_OP_RE
 // the number that launches by tables want, three sets of buffers in turn (in no cache alike):
 //   sums, one fewer: 4 ranks 0.98 from 530 MiB on (290 1.02, 430 0.99); 5 ranks 1.02 at 290 - 430, 0.99
 //     beyond; 7 ranks 0.985 - 0.99 throughout; 6 and 8 ranks 1.00 - 1.04
-//   copies: 8 ranks, 6 for 8, 0.99; 7 ranks, 5 for 8, 0.97 up to 450 MiB (the same buffers again 0.96);
-//     6 ranks, 9 for 12, 0.99 (0.96), beyond 600 MiB 1.07, 8 for 9 0.995 (0.98); 5 ranks, 8 for 14, 90 - 150 MiB 0.985
-//     (0.92), 250 - 350 MiB 0.98 (0.99), 450 and more 1.16
+
 //   (a sum of two ranks, 20 for 18, and an allreduce of four, 9 for 8, by cu_pauses: see there)
 // Copies of seven and eight ranks beyond 72 MiB copied: 10 (72 MiB 88.1 with 8, 87.7 with 10; 128 MiB 178 / 174).
+// Copies with fewer wavefronts than these (8 / 8 / 5 / 6 of 5 / 6 / 7 / 8 ranks up to 72 MiB copied) are ahead on
+// buffers that have just been used and behind where 1.3 GB and more lie between two uses, as with first uses:
+// an access waits for its address's translation too then, and more of them have to be under
+// way.  Over these, geometric means, the same buffers again / three sets in turn / 3.5 GB between two uses:
+//   touched MiB      90 - 150               180 - 260              310 - 570
+//   5 ranks    0.92 / 0.98 / 1.18    0.99 / 0.98 / 1.19    0.98 / 0.98 / 1.20
+//   6          0.93 / 0.98 / 1.10    0.96 / 0.97 / 1.11    0.99 / 0.98 / 1.12
+//   7          0.95 / 0.99 / 1.20    0.96 / 0.97 / 1.21    0.97 / 0.98 / 1.22
+//   8          1.00 / 1.01 / 1.07    0.97 / 1.00 / 1.08    1.00 / 1.00 / 1.10
 constexpr int cu_waves(int op, int dtype, int ranks, bool vast, uint64_t copied) {
     const uint64_t touched = copied * (uint64_t)ranks;
     if (op == MINT_OP_ALLREDUCE) return (26 + ranks - 1) / ranks + 1 + (ranks == 4 && dtype != MINT_BF16);
@@ -48,8 +55,7 @@ constexpr int cu_waves(int op, int dtype, int ranks, bool vast, uint64_t copied)
         return ranks == 6 ? 10 : 24 / ranks + 6;
     }
     if (vast) return ranks == 6 ? 5 : 4;
-    if (copied <= (72ull << 20)) return ranks == 8 ? 6 : ranks == 7 ? 5 : ranks >= 5 ? 8 : 24 - 2 * ranks;
-    return ranks >= 7 ? 10 : 24 - 2 * ranks;
+    return ranks < 7 ? 24 - 2 * ranks : copied <= (72ull << 20) ? 8 : 10;
 }
 
 // ... of the form between.  4 ranks, over 32, the same buffers again / three sets in turn / 700 MiB between two uses: 105 - 125 MiB 18

@@ -60,3 +60,14 @@ def test_every_rule_names_whole_blocks(rule):
         [f"cu_mid_waves({r}, {m << 20}ull)"] + [f"cu_small_waves({op}, {r}, {m << 20}ull)" for op in OPS.values()])]
     for e, value in zip(asked, rule(*asked)):
         assert 2 <= value <= 32, e
+
+
+@pytest.mark.parametrize("op", ["broadcast", "allgather"])
+def test_copies_of_rows_that_no_translation_is_at_hand_for(rule, op):
+    """On buffers that 1.3 GB and more lie between two uses of, every access waits for its address to be
+    translated too, and fewer wavefronts than these leave HBM idle: five to eight ranks with 8, 8, 5 and 6
+    of them up to 72 MiB copied took 1.02 - 1.2 of the time."""
+    for ranks, least in ((3, 18), (4, 16), (5, 14), (6, 12), (7, 8), (8, 8)):
+        sizes = (89, 120, 200, 72 * ranks - 1, 72 * ranks, 72 * ranks + ranks, 640)
+        for mib, value in zip(sizes, rule(*(waves(op, "bytes", ranks, m) for m in sizes))):
+            assert value == (10 if ranks >= 7 and mib > 72 * ranks else least), (ranks, mib, value)
