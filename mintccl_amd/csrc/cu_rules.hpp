@@ -96,9 +96,10 @@ constexpr int cu_small_waves(int op, int ranks, uint64_t touched) {
 //   6                961 - 984 / 993  973 / 984      977 / 990       995 / 1003      993 / 997
 //   7                962 - 989 / 992  981 / 1000     982 / 993      1004 / 1005     1013 / 1006
 //   8                990 - 1037 / 1010  984 / 1000   977 / 980       976 / 975      1003 / 996
-// Two more are 1 - 5 % slower.  Allreduce, geometric means of 110 - 1000 MiB on 15 sets of buffers (largest): 8 ranks (five
-// wavefronts throughout) 989 (1002) / 986 (1006), 7 ranks 997 (1004) / 1000, 6 ranks 996 (1001) / 1000, 5 ranks 994
-// (1004) / 1000, 4 ranks (nine wavefronts) 992 (1003) / 999; 2 and 3 ranks lose by it.
+// Two more are 1 - 5 % slower.  Allreduce, f16 and f32, geometric means of 102 - 2500 MiB (largest), the same buffers again / three
+// sets in turn / 3.5 GB between two uses: 8 ranks (bf16 too) 993 (1006) / 992 (1006) / 991 (1003), 7 ranks 996 (1007) / 995 (1003) / 993, 6 ranks
+// 998 (1010) / 994 / 990, 5 ranks 997 (1010) / 996 (1005) / 992, 4 ranks (nine wavefronts) 991 / 992 / 989; the same build on both
+// sides 996 - 1003.  bf16 of 7 ranks up to 150 MiB, 512 clocks: 1002 (1010) / 1001 (1007) / 998, no gain; 2 and 3 ranks lose by it.
 // One copy: sendrecv 954 - 997 from 200 MiB on, alltoall 1000 - 1009 at 200 - 300, 991 at 1000, 985 at 2000.
 // Several copies of a row lose 3 % and more: their stores are most of what there is.
 constexpr uint32_t cu_pauses(int op, int dtype, int ranks, uint64_t touched) {
@@ -106,7 +107,6 @@ constexpr uint32_t cu_pauses(int op, int dtype, int ranks, uint64_t touched) {
     const bool bf16 = dtype == MINT_BF16;
     if (op == MINT_OP_ALLREDUCE) {
         if (ranks == 8) return bf16 ? 3 : 4;
-        if (ranks == 7) return bf16 && !upto(150) ? 0 : 2;
         return ranks < 4 || bf16 ? 0 : ranks == 4 ? 3 : 2;
     }
     if (cu_adds(op)) {

@@ -71,3 +71,11 @@ def test_copies_of_rows_that_no_translation_is_at_hand_for(rule, op):
         sizes = (89, 120, 200, 72 * ranks - 1, 72 * ranks, 72 * ranks + ranks, 640)
         for mib, value in zip(sizes, rule(*(waves(op, "bytes", ranks, m) for m in sizes))):
             assert value == (10 if ranks >= 7 and mib > 72 * ranks else least), (ranks, mib, value)
+
+
+def test_no_wait_where_none_was_worth_it(rule):
+    """An allreduce of bf16 and fewer than eight ranks: its additions are the wait (seven ranks with
+    512 clocks more: 1.002 of the time, the same buffers again up to 1.010)."""
+    sizes = (101, 113, 130, 149, 151, 700)
+    asked = [f"cu_pauses({_lib.OP_ALLREDUCE}, {_lib.BF16}, {r}, {m << 20}ull)" for r in range(2, 8) for m in sizes]
+    assert rule(*asked) == [0] * len(asked)
