@@ -126,11 +126,10 @@ int launch_alltoall(const Plan& plan, hipStream_t stream) {
         using Form = typename decltype(form)::type;
         const dim3 grid = grid_of<Form>(plan, a.len, a.len);
         if constexpr (decltype(form)::in_place) {
-            if (!rest && a.len <= kCuNearPairs && s.row_stride == s.row_bytes && s.row_bytes <= UINT32_MAX &&
-                (Form::kLarge || s.tiles <= kCuNearTiles)) {
+            if (!rest && a.len <= kCuNearPairs && s.row_stride == s.row_bytes && s.tiles <= kCuNearTiles) {
                 const uint32_t *from = near.rank, *to = near.rank + kMaxRanks;
                 const u32x8 rows = {(uint32_t)lowest, (uint32_t)(lowest >> 32), (uint32_t)s.row_bytes,
-                                    s.tiles | s.part << cu_near_part_bit(Form::kLarge), from[0], from[1], from[2], from[3]};
+                                    s.tiles | s.part << cu_near_part_bit(false), from[0], from[1], from[2], from[3]};
                 return Launch<&cu_near_alltoall_kernel<Form>>::go(grid, Form::kThreads, 0, stream, rows, u32x4{to[0], to[1], to[2], to[3]},
                                                                   a.status);
             }

@@ -70,8 +70,8 @@ static_assert(sizeof(CuShape) + sizeof(CuTables<kMaxRanks, false>) <= 112, "argu
 // The ranks' buffers where ranks work in place and all rows lie within 4 GiB (`near` in
 // CuRingArgs): the lowest address and every rank's distance from it, in bytes.  With numbers
 // of 32 bits all that the loads wait for fits into the 14 words that a launch can bring in
-// registers; behind them only the status block's address is read from memory, by the one
-// wavefront that looks there.  A table in memory costs each block a round trip before its
+// registers (of seven and eight ranks the status block's address comes behind them and is read from memory, by the one
+// wavefront that looks there).  A table in memory costs each block a round trip before its
 // loads, and its compute unit's first blocks a long one: the runtime has just written it across the bus.
 // Over launches by tables, us, trains of calls over three sets of buffers in turn:
 //   touched      10 MiB        25 MiB        64 MiB        110 MiB        400 MiB
@@ -756,10 +756,11 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_alltoall_kernel(u64x4 numbe
 constexpr uint32_t kCuNearPairs = 4;
 template <typename FORM>
 __global__ void __launch_bounds__(FORM::kThreads) cu_near_alltoall_kernel(u32x8 rows, u32x4 stored, uint64_t* status) {
-    constexpr uint32_t kBit = cu_near_part_bit(FORM::kLarge);
+    static_assert(!FORM::kLarge, "rows of 32 bits, tiles and their part in a word");
+    constexpr uint32_t kBit = cu_near_part_bit(false);
     const uint64_t lowest = (uint64_t)rows[1] << 32 | rows[0];
     const uint32_t tiles = rows[3] & ((1u << kBit) - 1u), part = rows[3] >> kBit;
-    const CuPlace place(FORM::kLarge, part);
+    const CuPlace place(false, part);
     const auto at = [&](uint32_t r, uint32_t a, uint32_t b, uint32_t c, uint32_t d) MINT_INLINE_LAMBDA {
         const uint32_t low = r & 1u ? b : a, high = r & 1u ? d : c;
         return lowest + ((uint64_t)(r & 2u ? high : low) << kCuNearShift);
