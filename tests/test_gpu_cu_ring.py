@@ -278,6 +278,91 @@ def test_every_form_near_and_far(dev, wide, world, dt, mib):
     assert torch.equal(same[:per].view(torch.uint8), added([m[:per] for m in made], 0).view(torch.uint8))
 
 
+# MiB touched: in the small form, between, large, streamed far beyond the cache
+@pytest.mark.parametrize("world,mib", [(2, 30), (2, 150), (2, 300), (3, 150), (3, 300), (3, 400), (5, 150), (5, 300), (6, 660), (7, 300),
+                                       (8, 30), (8, 300), (8, 660)])
+def test_bf16_specials_in_every_form(dev, world, mib):
+    """NaNs of several payloads, infinities of both signs, the largest values and subnormals scattered over rows of normal ones:
+    the sums bit for bit, a NaN as the canonical one."""
+    from mintccl_amd.allreduce import allreduce
+    from mintccl_amd.reduce import reduce
+    from mintccl_amd.reducescatter import reducescatter
+    comm = make_comm(world)
+    special = torch.tensor([0x7F80, 0xFF80, 0x7F81, 0xFFA3, 0x7FC0, 0xFFC1, 0x7FFF, 0xFFFF, 0x7F7F, 0xFF7F, 0x0001, 0x8000],
+                           dtype=torch.int32, device=dev).to(torch.int16)
+    n = ((mib << 20) // (2 * world * world) // 8 * 8) * world + world             # rows of whole elements, ragged
+    g = torch.Generator(device=dev).manual_seed(world * mib)
+    made = []
+    for _ in range(world):
+        m = torch.randn(n, generator=g, device=dev).to(torch.bfloat16).view(torch.int16)
+        at = torch.randint(0, n, (n // 8,), generator=g, device=dev)
+        m[at] = special[torch.randint(0, len(special), (n // 8,), generator=g, device=dev)]
+        made.append(m)
+
+    def want(first, part=slice(None)):
+        x = added([m[part].view(torch.bfloat16) for m in made], first)
+        return torch.where(torch.isnan(x), torch.tensor(0x7FC0, dtype=torch.int16, device=dev), x.view(torch.int16))
+
+    def run(call):
+        bufs = [m.clone() for m in made]
+        comm.run(lambda r: call(bufs[r].view(torch.bfloat16)))
+        comm.check()
+        return bufs
+
+    got = run(lambda b: reduce(b, 1, comm))
+    assert torch.equal(got[1], want(1)) and torch.equal(got[0], made[0])
+    got = run(lambda b: reducescatter(b.view(world, -1), comm))
+    row = n // world
+    for r in range(world):
+        part = slice(r * row, r * row + row)
+        assert torch.equal(got[r][part], want(r, part)), r
+    got = run(lambda b: allreduce(b, comm))
+    row = (-(-2 * n // world) + 15) // 16 * 8                                      # (cut in whole vectors)
+    for p in range(world):
+        part = slice(p * row, min(n, p * row + row))
+        result = want(p, part)
+        assert all(torch.equal(b[part], result) for b in got), p
+
+
+# What a launch by distances reaches: rows up to 2^30 bytes, the last one's end up to 2^32 - 1 from the lowest
+# address; here both sides of each.
+@pytest.mark.parametrize("end", [(1 << 32) - 2, 1 << 32])
+@pytest.mark.parametrize("row", [(1 << 30) - 6, 1 << 30, (1 << 30) + 2])
+@pytest.mark.parametrize("world", [2, 3])
+def test_the_longest_rows_by_distances(dev, wide, world, row, end):
+    """A broadcast and a reduce of rows that begin at any byte and lie as far apart as they may: whole
+    rows, and the bytes around them."""
+    from mintccl_amd import _lib
+    comm = make_comm(world)
+    cycle = list(range(world)) + [0]
+    guard = 64
+    # (the ranks' order is not that of the addresses)
+    at = [guard + 6 + x for x in ([end - row, 0] if world == 2 else [end - row, 0, (end - row) // 2 // 16 * 16 + 10])]
+    g = torch.Generator(device=dev).manual_seed(row % 1000 + world)
+    made = [torch.randint(0, 2048, (row // 2,), generator=g, device=dev, dtype=torch.int32).to(torch.float16).view(torch.uint8)
+            for _ in range(world)]
+
+    def fresh():
+        for x, m in zip(at, made):
+            wide[x - guard: x + row + guard].fill_(0x5A)
+            wide[x: x + row].copy_(m)
+
+    def same(wanted, what):
+        comm.check()
+        for r, (x, w) in enumerate(zip(at, wanted)):
+            assert torch.equal(wide[x: x + row], w), (what, r)
+            assert torch.all(wide[x - guard: x] == 0x5A) and torch.all(wide[x + row: x + row + guard] == 0x5A), (what, r)
+
+    pointers = {r: wide.data_ptr() + x for r, x in enumerate(at)}
+    fresh()
+    comm.enqueue(_lib.OP_BROADCAST, _lib.BYTES, row, pointers, pointers, cycle, root=1)
+    same([made[1]] * world, "broadcast")
+    fresh()
+    comm.enqueue(_lib.OP_REDUCE, _lib.F16, row, pointers, {0: pointers[0]}, cycle, root=0)
+    summed = added([m.view(torch.float16) for m in made], 0).view(torch.uint8)
+    same([summed] + made[1:], "reduce")
+
+
 # MiB touched (bytes loaded and stored, sums: loaded), elements more than that in every row
 @pytest.mark.parametrize("mib,more", [(1, 5), (8, 1), (11, 3), (19, 3), (21, 0), (21, 3), (25, 9), (31, 2), (33, 3), (41, 7),
                                       (47, 1021), (72, 6), (74, 1), (85, 3), (89, 5), (105, 2051), (158, 9), (170, 9), (178, 3),
