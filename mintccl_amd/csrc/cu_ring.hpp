@@ -182,19 +182,18 @@ constexpr CuBand cu_through_mib(bool sums, int ranks, int pipes, bool pipe_each)
 constexpr int kCuStreamRanks = 6;
 // Sums to one place of two to six ranks, rows up to cu_mid_mib touched: the places of
 // the small form, rows streamed past the last-level cache, results left in it (the rows
-// of three sets of buffers are beyond it, their results are not).  Over the large form,
-// reduce and reduce-scatter in three types, the same buffers again / three sets in turn / 700 MiB
-// between two uses:
-//   touched MiB   100 - 130           130 - 160           160 - 176           176 - 196           196 - 208
-//   2 ranks  0.89 / 0.92 / 0.99  0.91 / 0.92 / 1.00  0.92 / 0.91 / 1.00  0.91 / 0.93 / 0.99  0.92 / 1.00 / 1.01
-//   3        0.87 / 0.87 / 0.97  0.88 / 0.88 / 1.00  0.90 / 0.89 / 1.03  0.89 / 0.88 / 1.03  0.88 / 0.88 / 1.04
-//   4        0.84 / 0.92 / 0.93  0.90 / 0.95 / 0.97  0.96 / 0.96 / 0.98  0.97 / 0.97 / 1.00  0.98 / 0.97 / 0.99
-//   5        0.89 / 0.93 / 0.93  0.91 / 0.96 / 0.96  0.97 / 0.97 / 0.97    (180 MiB, three sets 1.01)
-//   6        0.89 / 0.95 / 0.95  0.90 / 0.97 / 0.97  0.97 / 1.01 / 1.00, a reduce at 171 MiB 1.10 in each
-// (3 ranks at 235 - 264 MiB 0.89 / 0.91 / 1.04; 4 ranks at 270 MiB, three sets, f16 0.95, bf16 1.02; 7 and 8
-// ranks 0.92 - 1.10.  5 and 6 ranks in blocks of 64 threads, 14 wavefronts on a compute unit.)
-// Since the large form's wavefronts wait before they store (cu_pauses) it is ahead by 1 - 4 % from 150 MiB on with 4
-// and 5 ranks and from 144 on with 6 (the same buffers again up to 9 % behind at 125 - 140 MiB).
+// of three sets of buffers are beyond it, their results are not).  5 and 6 ranks in blocks of 64 threads, 14
+// wavefronts on a compute unit; 4 ranks: cu_mid_waves.  Over the large form with its waits (cu_pauses), reduce and
+// reduce-scatter in three types, geometric means, the same buffers again / three sets in turn / 700 MiB between two uses /
+// 3.5 GB between two uses:
+//   touched MiB     100 - 120                  120 - 145                  145 - 165                  165 - 190                  190 - 264
+//   2 ranks  0.96 / 0.96 / 1.04 / 1.04  0.97 / 0.98 / 1.03 / 1.03  0.99 / 0.98 / 1.04 / 1.04  0.99 / 0.98 / 1.04 / 1.05  1.01 / 1.03 / 1.03 / 1.04
+//   3        0.93 / 0.96 / 1.00 / 1.03  0.94 / 0.97 / 1.06 / 1.07  0.98 / 0.97 / 1.04 / 1.05  1.01 / 0.98 / 1.06 / 1.07  1.00 / 0.99 / 1.07 / 1.08
+//   4        0.92 / 0.98 / 0.98 / 1.02  0.93 / 1.01 / 1.01 / 1.03  1.01 / 1.00 / 1.01 / 1.05  1.02 / 0.99 / 1.00 / 1.05  1.04 / 0.99 / 1.00 / 1.05
+//   5        0.96 / 0.98 / 0.98 / 1.01  0.98 / 1.02 / 1.00 / 1.05  0.99 / 1.02 / 1.00 / 1.04  1.06 / 1.02 / 1.00 / 1.04
+//   6        0.95 / 1.00 / 0.99 / 1.02  0.97 / 1.01 / 1.00 / 1.03  1.02 / 1.02 / 1.01 / 1.05
+// The lines stand where the form crossed the large one without waits (at 176 MiB 0.97 throughout): with them it is ahead up to
+// about 140 MiB, and on distant uses nowhere.
 constexpr int kCuMidRanks = 6;
 constexpr int cu_mid_mib(int ranks) {
     return ranks == 2 ? 196 : ranks == 3 ? 264 : ranks == 4 ? 208 : ranks == 5 ? 176 : 160;
@@ -593,8 +592,9 @@ __device__ __forceinline__ void cu_sum_row(const CuRow<FORM, WIDE>& row, uint32_
                 for (int h = 0; h < N; ++h) v[k][h] = at.template load<FORM::kStream>(h, base + k * kStep, lane);
 #pragma unroll
             for (int k = 0; k < kCount; ++k) {
-                // (three ranks of bf16 in the large form, 300 MiB touched: 60.9 us, with the shorter additions
-                // 62.9, and no wait (cu_pause) in their place brings it back; 500 MiB and more 0.99 - 1.00)
+                // (three ranks of bf16 in the large form: the longer additions are a part of the wait before the stores
+                // (cu_pauses), 0.990 - 0.995 of the shorter ones at 270 - 700 MiB touched, 0.998 at 1000, and no wait of
+                // whole 256 clocks in their place does it)
                 Sum<DT, FORM::kLarge && N == 3 && STORED == 1> sum(v[k][0]);
 #pragma unroll
                 for (int h = 1; h < N; ++h) sum.add(v[k][h]);
@@ -745,11 +745,12 @@ __global__ void __launch_bounds__(FORM::kThreads) cu_alltoall_kernel(u64x4 numbe
 // 14 words that come in registers (CuNear); the selects of a block's two distances take no longer than one to a
 // table's entry. Over tables, the same buffers again / three sets in turn:
 //   touched MiB      20             30             45             64             90            150
-//   2 ranks     0.985 / 0.99   0.97 / 0.97    1.02 / 0.99    0.98 / 0.985   0.98 / 0.98   0.99 / 0.99
-//   3           0.98 / 0.97    0.99 / 0.96    0.95 / 0.97    0.97 / 0.98    0.98 / 0.98   0.99 / 0.99
-//   4           0.99 / 0.98    0.95 / 0.95    0.98 / 0.975   0.97 / 0.99    0.98 / 0.98   0.99 / 0.99
-// (4 ranks of 30 MiB, three sets, 5.50 -> 5.24 us, 6.0 TB/s; 64 MiB 10.27 -> 10.18; 90 MiB 13.9 -> 13.6), below the host's 3.4 us and
-// from 200 MiB on 1.00.  More ranks: 16 distances of 20 bits, in halves and fours, fit as well, but finding two of them takes
+//   2 ranks     0.95 / 0.95    0.97 / 0.97    0.99 / 0.97    0.97 / 0.98    0.98 / 0.98   0.99 / 0.99
+//   3           0.99 / 0.95    0.98 / 0.95    0.99 / 0.97    0.97 / 0.98    0.98 / 0.98   0.99 / 0.99
+//   4           0.97 / 0.93    0.95 / 0.96    0.96 / 0.97    0.98 / 0.98    0.98 / 0.98   0.99 / 0.99
+// (4 ranks of 30 MiB, three sets, 5.36 -> 5.13 us, 6.1 TB/s; 64 MiB 10.22 -> 9.99; 90 MiB 13.8 -> 13.6).  Up to 12 MiB the host's launch is
+// what a call takes, 0.985 - 1.016 with a scatter of 5 %; from 200 MiB on it is the large form, by tables.  More ranks: 16 distances of 20
+// bits, in halves and fours, fit as well, but finding two of them takes
 // about what the table does (5 and 6 ranks 0.98 - 1.02, 7 and 8 ranks 0.98 - 1.01).
 //   rows    lowest address (two words), row_bytes, tiles | part << cu_near_part_bit; what ranks 0 - 3 load from
 //   stored  what they store to

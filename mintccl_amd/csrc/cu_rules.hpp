@@ -30,8 +30,8 @@ constexpr bool cu_adds(int op) { return op == MINT_OP_REDUCE || op == MINT_OP_RE
 // the number that launches by tables want, three sets of buffers in turn (in no cache alike):
 //   sums, one fewer: 4 ranks 0.98 from 530 MiB on (290 1.02, 430 0.99); 5 ranks 1.02 at 290 - 430, 0.99
 //     beyond; 7 ranks 0.985 - 0.99 throughout; 6 and 8 ranks 1.00 - 1.04
-
-//   (a sum of two ranks, 20 for 18, and an allreduce of four, 9 for 8, by cu_pauses: see there)
+//   (a sum of two ranks, 20 for 18, by cu_pauses: see there; an allreduce of four, f16 and f32, 9 and a wait of 768 clocks for 8 and
+//     none, one process: 0.976 - 1.003, geometric mean 0.995)
 // Copies of seven and eight ranks beyond 72 MiB copied: 10 (72 MiB 88.1 with 8, 87.7 with 10; 128 MiB 178 / 174).
 // Copies with fewer wavefronts than these (8 / 8 / 5 / 6 of 5 / 6 / 7 / 8 ranks up to 72 MiB copied) are ahead on
 // buffers that have just been used and behind where 1.3 GB and more lie between two uses, as with first uses:
@@ -60,7 +60,8 @@ constexpr int cu_waves(int op, int dtype, int ranks, bool vast, uint64_t copied)
 
 // ... of the form between.  4 ranks, over 32, the same buffers again / three sets in turn / 700 MiB between two uses: 105 - 125 MiB 18
 // 1.00 / 0.985 / 0.98 (16: 1.02 / 0.975 / 0.975), 150 MiB 22 0.99 / 0.995 / 0.99 (18: 1.03 / 0.99 / 0.99), 170 - 205 MiB 16
-// 0.975 / 0.97 / 0.97 (18: 0.99); 2 ranks 24 1.02 - 1.05; 3 ranks 24 0.99 - 1.00.  5 and 6 ranks: kCuMidRanks.
+// 0.975 / 0.97 / 0.97 (18: 0.99).  In one process over 18 throughout: 130 - 165 MiB 0.99 / 1.007 / 1.006 (22 is there for the same buffers
+// again, 0.95 - 0.995 at 150 MiB, where 18 is behind 32), 165 - 208 MiB 0.98 / 0.98 / 0.99; 2 ranks 24 1.02 - 1.05; 3 ranks 24 0.99 - 1.00.  5 and 6 ranks: kCuMidRanks.
 constexpr int cu_mid_waves(int ranks, uint64_t touched) {
     if (ranks == 4) return touched <= (130ull << 20) ? 18 : touched <= (165ull << 20) ? 22 : 16;
     return ranks < 4 ? kCuMostWaves : 14;
